@@ -19,12 +19,12 @@
 //     one 128-k scale group, so D[i][i] is a per-group sum of (code+136 or code+1032) * x and
 //     the lane holding it applies  scale * (D[i][i] - offset * sum_k x)  -- the post-scaled form
 //     (see caifx_gemv.hip for the numerics note).
-//   int8 (two to four activation rows, and one row when the shape does not fit the kernel below):
+//   int8 (two to four activation rows):
 //     a k-slot is 16 codes; float(code)*scale is rounded to the compute dtype exactly as the
 //     reference does.  With per-channel scales the index (n*K+k) % period depends on the
 //     row only through (n*K) % period, so a wave takes rows of one residue class
 //     n = v + V*i (V = period / gcd(K, period)) and keeps that class's scales in registers.
-//   int8, one activation row, K a multiple of 1024: the scales are folded into the activations and
+//   int8, one activation row: the scales are folded into the activations and
 //     the codes go into the integer matrix core as loaded (rowlin_int8_digits_kernel below).
 #include "caifx_internal.hpp"
 
@@ -69,7 +69,6 @@ struct RowArgs {
   int total_waves;
   int cpr;              // chunks (one load instruction of a wave) per weight row
   int xpitch;           // staged activations: elements per row (cpr * k-per-chunk)
-  int digits;           // int8, one activation row: take the integer-matrix-core kernel
   int round_x;          // that kernel only: activations pass through this dtype first (caifx_dtype), -1 = they are of it already
   int slices;           // its form for K > 4096: parts a weight row is cut into (2 or 4), 0 otherwise
 };
@@ -321,8 +320,12 @@ __global__ __launch_bounds__(256) void rowlin_int4_kernel(RowArgs a)
 }
 
 // ------------------------------------------------------------------ fixed-shape fast paths
-// Same arithmetic as the kernels above for rows made of whole chunks (K = CPR * 2048 for int4,
-// CPR * 1024 for int8).  Every inner trip count is a compile-time constant.  What the prologue needs
+// Same arithmetic as the kernels above for rows of CPR chunks (2048 codes each for int4, 1024 for int8; kTail: the
+// last chunk of a row is not whole, its missing lanes read the row's last piece again and multiply it with zeros).
+// Every inner trip count is a compile-time constant.  They take every result dtype and every reduction of whole groups:
+// with bf16 results, which used to run on the dynamic kernels above, K = 4096, N = 14336 takes 7.7 us instead of 12.0
+// (int4; 3.9 TB/s) and 12.4 instead of 18.0 (int8; 4.7 TB/s), and the K = 14336, N = 4096 way back 10.6 instead of
+// 12.0 (int4) and 16.1 instead of 14.7 + 4.3 for two launches of the row-block kernel (int8).  What the prologue needs
 // (activations, int8 scales) is requested BEFORE the first weight rows, because loads return in
 // order; a wave then walks `rows_per_wave` rows through a ring of D rows: it computes a row out of
 // the registers it arrived in and requests the row D further on into the same registers, so D-1
@@ -339,7 +342,7 @@ struct XPieces {
   typename Mfma16<CT>::vec_t v[kPerThread];
 };
 
-template <typename CT, int MT, int kPiecesPerRow, int kThreads = 256>
+template <typename CT, int MT, int kPiecesPerRow, bool kTail = false, int kThreads = 256>
 __device__ __forceinline__ void x_request(const RowArgs &a, XPieces<CT, MT, kPiecesPerRow, kThreads> &xp)
 {
   typedef typename Mfma16<CT>::vec_t vec_t;
@@ -350,8 +353,14 @@ __device__ __forceinline__ void x_request(const RowArgs &a, XPieces<CT, MT, kPie
     const int m = p / kPiecesPerRow;
     const int piece = p - m * kPiecesPerRow;
     const int msrc = m < a.M ? m : a.M - 1;
-    if (XPieces<CT, MT, kPiecesPerRow, kThreads>::kTotal % kThreads == 0 || p < MT * kPiecesPerRow)
-      xp.v[i] = *reinterpret_cast<const vec_t *>(xg + static_cast<int64_t>(msrc) * a.K + piece * 8);
+    const bool inside = !kTail || piece * 8 < a.K;
+    if (XPieces<CT, MT, kPiecesPerRow, kThreads>::kTotal % kThreads == 0 || p < MT * kPiecesPerRow) {
+      xp.v[i] = *reinterpret_cast<const vec_t *>(xg + static_cast<int64_t>(msrc) * a.K + (inside ? piece * 8 : 0));
+      if (kTail && !inside) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) xp.v[i][j] = from_f32<CT>(0.0f);
+      }
+    }
   }
 }
 
@@ -395,7 +404,7 @@ __device__ __forceinline__ void x_commit(const XPieces<CT, MT, kPiecesPerRow, kT
 
 constexpr int kInt4FastWaves = 4;   // waves per workgroup of the kernel below (8 and 16 measured no better)
 
-template <typename CT, int MT, int CPR>
+template <typename CT, int MT, int CPR, bool kTail>
 __global__ __launch_bounds__(kInt4FastWaves * 64) void rowlin_int4_fast_kernel(RowArgs a)
 {
   constexpr int kThreads = kInt4FastWaves * 64;
@@ -415,13 +424,13 @@ __global__ __launch_bounds__(kInt4FastWaves * 64) void rowlin_int4_fast_kernel(R
   const bool is_diag = (lane >> 4) == ((lane & 15) >> 2);
   const int di = lane & 15;
   const int pslot = di * 4 + (lane >> 4);
-  constexpr int64_t kRowBytes = static_cast<int64_t>(CPR) * 1024;
-  constexpr int groups_per_row = CPR * 16;       // group size 128
+  const int64_t kRowBytes = kTail ? a.K >> 1 : static_cast<int64_t>(CPR) * 1024;
+  const int groups_per_row = kTail ? static_cast<int>(a.K >> 7) : CPR * 16;       // group size 128
 
   XPieces<CT, MT, kPieces, kThreads> xp;
-  x_request<CT, MT, kPieces, kThreads>(a, xp);
+  x_request<CT, MT, kPieces, kTail, kThreads>(a, xp);
 
-  const uint8_t *wp = a.wq + row0 * kRowBytes + pslot * 16;
+  const uint8_t *wp = a.wq + row0 * kRowBytes + (kTail ? 0 : pslot * 16);
   const f16_t *sp = static_cast<const f16_t *>(a.scales) + row0 * groups_per_row;
   u32x4_t w[D][CPR];
   f16_t sc[D][CPR];
@@ -429,16 +438,27 @@ __global__ __launch_bounds__(kInt4FastWaves * 64) void rowlin_int4_fast_kernel(R
   // the activation row instead, which is cache resident and large enough): with no branch around a
   // load the compiler knows how many requests are in flight at every wait and lets the newer ones
   // stay outstanding, which is what keeps the ring of rows in flight.
-  const uint8_t *wdummy = static_cast<const uint8_t *>(a.x) + pslot * 16;
-  const f16_t *sdummy = static_cast<const f16_t *>(a.x) + di;
+  // With a partial last chunk the dummy is weight row 0 (the activation row may be shorter than CPR KiB); lanes past
+  // the row's end repeat its last piece and last group, and the group's scale is dropped (below).
+  const uint8_t *wdummy = kTail ? a.wq : static_cast<const uint8_t *>(a.x) + pslot * 16;
+  const f16_t *sdummy = kTail ? static_cast<const f16_t *>(a.scales) : static_cast<const f16_t *>(a.x) + di;
+  const int last_piece = kTail ? static_cast<int>(a.K >> 5) - 1 : 0;
+  const int tail_off = kTail ? min((CPR - 1) * 64 + pslot, last_piece) * 16 : 0;
+  const int tail_group = kTail ? min((CPR - 1) * 16 + di, groups_per_row - 1) : 0;
+  const bool tail_inside = !kTail || (CPR - 1) * 16 + di < groups_per_row;
   auto issue = [&](int d, int r) {
     const bool ok = r < nrows;
     const uint8_t *wsrc = ok ? wp + r * kRowBytes : wdummy;
-    const f16_t *ssrc = ok ? sp + r * groups_per_row + di : sdummy;
+    const f16_t *ssrc = ok ? sp + r * groups_per_row + (kTail ? 0 : di) : sdummy;
 #pragma unroll
     for (int c = 0; c < CPR; ++c) {
-      w[d][c] = *reinterpret_cast<const u32x4_t *>(wsrc + c * 1024);
-      sc[d][c] = ssrc[c * 16];
+      if constexpr (kTail) {
+        w[d][c] = *reinterpret_cast<const u32x4_t *>(wsrc + (c == CPR - 1 ? tail_off : c * 1024 + pslot * 16));
+        sc[d][c] = ssrc[c == CPR - 1 ? tail_group : c * 16 + di];
+      } else {
+        w[d][c] = *reinterpret_cast<const u32x4_t *>(wsrc + c * 1024);
+        sc[d][c] = ssrc[c * 16];
+      }
     }
   };
 #pragma unroll
@@ -496,7 +516,9 @@ __global__ __launch_bounds__(kInt4FastWaves * 64) void rowlin_int4_fast_kernel(R
             dsel = (tsel == 1) ? part[m][1] : dsel;
             dsel = (tsel == 2) ? part[m][2] : dsel;
             dsel = (tsel == 3) ? part[m][3] : dsel;
-            tot[m] = __builtin_fmaf(to_f32(sc[d][c]), dsel - corr[m][c], tot[m]);
+            float scale = to_f32(sc[d][c]);
+            if (kTail && c == CPR - 1) scale = tail_inside ? scale : 0.0f;
+            tot[m] = __builtin_fmaf(scale, dsel - corr[m][c], tot[m]);
           }
         }
 #pragma unroll
@@ -511,7 +533,7 @@ __global__ __launch_bounds__(kInt4FastWaves * 64) void rowlin_int4_fast_kernel(R
   if (lane < nrows) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
-      if (MT != 4 || m < a.M) static_cast<float *>(a.y)[static_cast<int64_t>(m) * a.N + row0 + lane] = res[m];
+      if (MT != 4 || m < a.M) store_y(a.y, a.y_dtype, static_cast<int64_t>(m) * a.N + row0 + lane, res[m]);
   }
 }
 
@@ -623,7 +645,7 @@ __global__ __launch_bounds__(256) void rowlin_int8_fast_kernel(RowArgs a)
   if (lane < nrows) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
-      if (MT != 4 || m < a.M) static_cast<float *>(a.y)[static_cast<int64_t>(m) * a.N + cls + V * (i0 + lane)] = res[m];
+      if (MT != 4 || m < a.M) store_y(a.y, a.y_dtype, static_cast<int64_t>(m) * a.N + cls + V * (i0 + lane), res[m]);
   }
 }
 
@@ -646,7 +668,7 @@ typedef int i32x4_t __attribute__((ext_vector_type(4)));
 // measured 12.2 us against 12.9 (8) and 13.1 (4) on the K=4096, N=14336 case.
 constexpr int kDigitWaves = 16;
 
-template <typename XT, bool kVec, int CPR>
+template <typename XT, bool kVec, int CPR, bool kTail>
 __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(RowArgs a)
 {
   constexpr int D = (CPR >= 4) ? 2 : 4;   // rows in the ring (2 for K = 4096 measured best against 1 and 4)
@@ -667,7 +689,7 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
       nrows = static_cast<int>(avail < a.rows_per_wave ? avail : a.rows_per_wave);
     }
   }
-  constexpr int64_t kRowBytes = static_cast<int64_t>(CPR) * 1024;
+  const int64_t kRowBytes = kTail ? a.K : static_cast<int64_t>(CPR) * 1024;
 
   // this lane's activations of chunk `wave` (chunks beyond CPR do not exist; their waves only join the
   // barriers) and their scales are requested BEFORE the first weight rows: loads return in order, so
@@ -676,9 +698,14 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
   floatx4_t scv[4];
   const bool has_chunk = wave < CPR;
   if (has_chunk) {
-    const XT *xg = static_cast<const XT *>(a.x) + (wave * 64 + lane) * 16;
+    const bool inside = !kTail || (wave * 64 + lane) * 16 < a.K;
+    const XT *xg = static_cast<const XT *>(a.x) + (inside ? (wave * 64 + lane) * 16 : 0);
 #pragma unroll
     for (int t = 0; t < 16; ++t) xv[t] = to_f32<XT>(xg[t]);
+    if (kTail && !inside) {
+#pragma unroll
+      for (int t = 0; t < 16; ++t) xv[t] = 0.0f;
+    }
     // the layer casts its input to the compute dtype before the GEMM (src/caif_device_frozen_linear.cpp:459)
     if (a.round_x == CAIFX_BF16) {
 #pragma unroll
@@ -690,7 +717,7 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
     if constexpr (kVec) {
       const float *sp = static_cast<const float *>(a.scales);
       // 32-bit arithmetic: cls < N / 256 and K <= 4096, so cls * K + k stays far below 2^31
-      const int idx = static_cast<int>((static_cast<uint32_t>(cls) * (CPR * 1024) + (wave * 64 + lane) * 16) % static_cast<uint32_t>(a.period));
+      const int idx = static_cast<int>((static_cast<uint32_t>(cls) * static_cast<uint32_t>(kRowBytes) + (wave * 64 + lane) * 16) % static_cast<uint32_t>(a.period));
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         int i = idx + 4 * q;
@@ -704,16 +731,18 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
     if (a.scales) s_scalar = static_cast<const float *>(a.scales)[0];
   }
 
-  const uint8_t *wp = a.wq + (cls + V * i0) * kRowBytes + lane * 16;
+  const uint8_t *wp = a.wq + (cls + V * i0) * kRowBytes + (kTail ? 0 : lane * 16);
   const int64_t rstep = V * kRowBytes;
   i32x4_t w[D][CPR];
   // unconditional loads (a row past the wave's range reads the start of the activation row): see the
-  // int4 kernel above
-  const uint8_t *wdummy = static_cast<const uint8_t *>(a.x) + lane * 16;
+  // int4 kernel above; with a partial last chunk the dummy is weight row 0, and lanes past the end repeat the last piece
+  const uint8_t *wdummy = kTail ? a.wq : static_cast<const uint8_t *>(a.x) + lane * 16;
+  const int tail_off = kTail ? min((CPR - 1) * 1024 + lane * 16, static_cast<int>(a.K) - 16) : 0;
   auto issue = [&](int d, int r) {
     const uint8_t *wsrc = r < nrows ? wp + r * rstep : wdummy;
 #pragma unroll
-    for (int c = 0; c < CPR; ++c) w[d][c] = *reinterpret_cast<const i32x4_t *>(wsrc + c * 1024);
+    for (int c = 0; c < CPR; ++c)
+      w[d][c] = *reinterpret_cast<const i32x4_t *>(wsrc + (!kTail ? c * 1024 : c == CPR - 1 ? tail_off : c * 1024 + lane * 16));
   };
 #pragma unroll
   for (int d = 0; d < D; ++d) issue(d, d);
@@ -814,7 +843,7 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
       issue(d, r + D);
     }
   }
-  if (lane < nrows) static_cast<float *>(a.y)[cls + V * (i0 + lane)] = poisoned ? __builtin_nanf("") : res;
+  if (lane < nrows) store_y(a.y, a.y_dtype, cls + V * (i0 + lane), poisoned ? __builtin_nanf("") : res);
 }
 
 
@@ -824,7 +853,7 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
 // registers for the whole kernel.  The power-of-two unit is taken per slice.  The nsl partial sums of a row meet in
 // LDS after the loop and are added in slice order.  a.cpr = chunks per row (K / 1024 <= 16), a.slices = nsl (2 or
 // 4), a.waves_per_class = row groups per residue class (a multiple of 16 / nsl).
-template <typename XT, bool kVec>
+template <typename XT, bool kVec, bool kTail>
 __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_long_kernel(RowArgs a)
 {
   constexpr int CPS = 4;                  // chunks per slice at most
@@ -861,9 +890,10 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_long_kern
   floatx4_t scv[4];
   const bool has_chunk = wave < a.cpr;
   if (has_chunk) {
-    const XT *xg = static_cast<const XT *>(a.x) + (wave * 64 + lane) * 16;
+    const bool inside = !kTail || (wave * 64 + lane) * 16 < a.K;
+    const XT *xg = static_cast<const XT *>(a.x) + (inside ? (wave * 64 + lane) * 16 : 0);
 #pragma unroll
-    for (int t = 0; t < 16; ++t) xv[t] = to_f32<XT>(xg[t]);
+    for (int t = 0; t < 16; ++t) xv[t] = inside ? to_f32<XT>(xg[t]) : 0.0f;
     if (a.round_x == CAIFX_BF16) {
 #pragma unroll
       for (int t = 0; t < 16; ++t) xv[t] = round_through<bf16_t>(xv[t]);
@@ -890,12 +920,18 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_long_kern
   const uint8_t *wp = a.wq + (cls + V * i0) * row_bytes + first_chunk * 1024 + lane * 16;
   const int64_t rstep = V * row_bytes;
   i32x4_t w[D][CPS];
-  // unconditional loads: a row past the wave's range, or a chunk past the slice, reads the activation row
+  // unconditional loads: a row past the wave's range, or a chunk past the slice, reads the activation row; lanes past
+  // the end of a partial last chunk repeat the row's last piece
   const uint8_t *wdummy = static_cast<const uint8_t *>(a.x) + lane * 16;
+  const int tail_back = kTail && lane * 16 >= static_cast<int>(a.K & 1023) ? lane * 16 + 16 - static_cast<int>(a.K & 1023) : 0;
   auto issue = [&](int d, int r) {
     const uint8_t *wsrc = r < nrows ? wp + r * rstep : wdummy;
 #pragma unroll
-    for (int c = 0; c < CPS; ++c) w[d][c] = *reinterpret_cast<const i32x4_t *>(c < my_chunks ? wsrc + c * 1024 : wdummy);
+    for (int c = 0; c < CPS; ++c) {
+      const uint8_t *src = c < my_chunks ? wsrc + c * 1024 : wdummy;
+      if (kTail && r < nrows && first_chunk + c == a.cpr - 1) src -= tail_back;
+      w[d][c] = *reinterpret_cast<const i32x4_t *>(src);
+    }
   };
 #pragma unroll
   for (int d = 0; d < D; ++d) issue(d, d);
@@ -1002,7 +1038,7 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_long_kern
   if (slice == 0 && lane < nrows) {
     float v = res;
     for (int sl = 1; sl < nsl; ++sl) v += red[wave + sl][lane];
-    static_cast<float *>(a.y)[cls + V * (i0 + lane)] = poisoned ? __builtin_nanf("") : v;
+    store_y(a.y, a.y_dtype, cls + V * (i0 + lane), poisoned ? __builtin_nanf("") : v);
   }
 }
 
@@ -1119,11 +1155,11 @@ __global__ __launch_bounds__(256) void rowlin_int8_kernel(RowArgs a)
   }
 }
 
-template <typename CT, int MT, int CPR>
+template <typename CT, int MT, int CPR, bool kTail>
 int launch_int4_fast(const RowArgs &ra, hipStream_t s)
 {
   const size_t lds = static_cast<size_t>((MT * CPR * 16 + 3) & ~3) * 4 + static_cast<size_t>(MT) * CPR * 2048 * 2;
-  hipLaunchKernelGGL((rowlin_int4_fast_kernel<CT, MT, CPR>),
+  hipLaunchKernelGGL((rowlin_int4_fast_kernel<CT, MT, CPR, kTail>),
                      dim3(static_cast<unsigned>((ra.total_waves + kInt4FastWaves - 1) / kInt4FastWaves)), dim3(kInt4FastWaves * 64),
                      lds, s, ra);
   return launch_status();
@@ -1138,17 +1174,37 @@ int launch_int8_fast(const RowArgs &ra, hipStream_t s)
   return launch_status();
 }
 
+// One or two activation rows: up to eight chunks per row (K <= 16384; two rows: 14336, what fits 64 KB of LDS).  More
+// rows come here only where the row-block kernel does not fit, and take the fixed-shape form at K <= 8192.
+template <typename CT, int MT, bool kTail>
+int pick_int4_fast(const RowArgs &ra, hipStream_t s)
+{
+  switch (ra.cpr) {
+    case 1: return launch_int4_fast<CT, MT, 1, kTail>(ra, s);
+    case 2: return launch_int4_fast<CT, MT, 2, kTail>(ra, s);
+    case 4: return launch_int4_fast<CT, MT, 4, kTail>(ra, s);
+    default: break;
+  }
+  if constexpr (MT <= 2) {
+    switch (ra.cpr) {
+      case 3: return launch_int4_fast<CT, MT, 3, kTail>(ra, s);
+      case 5: return launch_int4_fast<CT, MT, 5, kTail>(ra, s);
+      case 6: return launch_int4_fast<CT, MT, 6, kTail>(ra, s);
+      case 7: return launch_int4_fast<CT, MT, 7, kTail>(ra, s);
+      case 8: return launch_int4_fast<CT, MT, 8, kTail>(ra, s);
+      default: break;
+    }
+  }
+  return CAIFX_ERR_UNSUPPORTED;
+}
+
 template <typename CT, typename XT, int MT>
 int launch_int4(const RowArgs &ra, hipStream_t s)
 {
   if constexpr (dtype_code<XT>::value == dtype_code<CT>::value) {
-    const bool full = (ra.K % 2048 == 0) && ra.group_shift == 7 && ra.y_dtype == CAIFX_F32;
-    if (full && ra.cpr == 1) return launch_int4_fast<CT, MT, 1>(ra, s);
-    if (full && ra.cpr == 2) return launch_int4_fast<CT, MT, 2>(ra, s);
-    if (full && ra.cpr == 4) return launch_int4_fast<CT, MT, 4>(ra, s);
-    if constexpr (MT == 1) {      // long reductions with one activation row (a down projection at decode time)
-      if (full && ra.cpr == 7) return launch_int4_fast<CT, MT, 7>(ra, s);
-      if (full && ra.cpr == 8) return launch_int4_fast<CT, MT, 8>(ra, s);
+    if (ra.group_shift == 7) {
+      const int st = ra.K % 2048 == 0 ? pick_int4_fast<CT, MT, false>(ra, s) : pick_int4_fast<CT, MT, true>(ra, s);
+      if (st != CAIFX_ERR_UNSUPPORTED) return st;
     }
   }
   const size_t lds = static_cast<size_t>((MT * (ra.xpitch >> 7) + 3) & ~3) * 4 + static_cast<size_t>(MT) * ra.xpitch * 2;
@@ -1160,41 +1216,51 @@ int launch_int4(const RowArgs &ra, hipStream_t s)
 template <typename XT, bool kVec, int CPR>
 int launch_int8_digits(const RowArgs &ra, hipStream_t s)
 {
-  hipLaunchKernelGGL((rowlin_int8_digits_kernel<XT, kVec, CPR>), dim3(static_cast<unsigned>(ra.total_waves / kDigitWaves)), dim3(kDigitWaves * 64), 0, s, ra);
+  if (ra.K % 1024 != 0) {
+    hipLaunchKernelGGL((rowlin_int8_digits_kernel<XT, kVec, CPR, true>), dim3(static_cast<unsigned>(ra.total_waves / kDigitWaves)), dim3(kDigitWaves * 64), 0, s, ra);
+    return launch_status();
+  }
+  hipLaunchKernelGGL((rowlin_int8_digits_kernel<XT, kVec, CPR, false>), dim3(static_cast<unsigned>(ra.total_waves / kDigitWaves)), dim3(kDigitWaves * 64), 0, s, ra);
   return launch_status();
 }
 
 template <typename CT, typename XT, int MT, bool kVec>
 int launch_int8(const RowArgs &ra, hipStream_t s)
 {
-  if constexpr (MT == 1) {
-    if (ra.digits && ra.slices > 0) {
-      hipLaunchKernelGGL((rowlin_int8_digits_long_kernel<XT, kVec>),
-                         dim3(static_cast<unsigned>(ra.total_waves / (kDigitWaves / ra.slices))), dim3(kDigitWaves * 64), 0, s, ra);
+  if constexpr (MT == 1) {          // always the integer-matrix-core kernels
+    if (ra.slices > 0) {
+      const dim3 grid(static_cast<unsigned>(ra.total_waves / (kDigitWaves / ra.slices)));
+      if (ra.K % 1024 == 0)
+        hipLaunchKernelGGL((rowlin_int8_digits_long_kernel<XT, kVec, false>), grid, dim3(kDigitWaves * 64), 0, s, ra);
+      else
+        hipLaunchKernelGGL((rowlin_int8_digits_long_kernel<XT, kVec, true>), grid, dim3(kDigitWaves * 64), 0, s, ra);
       return launch_status();
     }
-    if (ra.digits) {
-      if (ra.cpr == 1) return launch_int8_digits<XT, kVec, 1>(ra, s);
-      if (ra.cpr == 2) return launch_int8_digits<XT, kVec, 2>(ra, s);
-      return launch_int8_digits<XT, kVec, 4>(ra, s);
+    switch (ra.cpr) {
+      case 1: return launch_int8_digits<XT, kVec, 1>(ra, s);
+      case 2: return launch_int8_digits<XT, kVec, 2>(ra, s);
+      case 3: return launch_int8_digits<XT, kVec, 3>(ra, s);
+      case 4: return launch_int8_digits<XT, kVec, 4>(ra, s);
+      default: return CAIFX_ERR_UNSUPPORTED;
     }
+  } else {
+    if constexpr (dtype_code<XT>::value == dtype_code<CT>::value) {
+      const bool full = ra.K % 1024 == 0;
+      if (full && ra.cpr == 1) return launch_int8_fast<CT, MT, kVec, 1>(ra, s);
+      if (full && ra.cpr == 2) return launch_int8_fast<CT, MT, kVec, 2>(ra, s);
+      if (full && ra.cpr == 4) return launch_int8_fast<CT, MT, kVec, 4>(ra, s);
+    }
+    const size_t lds = static_cast<size_t>(MT) * ra.xpitch * 2;
+    const unsigned grid = static_cast<unsigned>((ra.total_waves + 3) / 4);
+    switch (ra.cpr) {
+      case 1: hipLaunchKernelGGL((rowlin_int8_kernel<CT, XT, MT, kVec, 1>), dim3(grid), dim3(256), lds, s, ra); break;
+      case 2: hipLaunchKernelGGL((rowlin_int8_kernel<CT, XT, MT, kVec, 2>), dim3(grid), dim3(256), lds, s, ra); break;
+      case 3: hipLaunchKernelGGL((rowlin_int8_kernel<CT, XT, MT, kVec, 3>), dim3(grid), dim3(256), lds, s, ra); break;
+      case 4: hipLaunchKernelGGL((rowlin_int8_kernel<CT, XT, MT, kVec, 4>), dim3(grid), dim3(256), lds, s, ra); break;
+      default: return CAIFX_ERR_UNSUPPORTED;
+    }
+    return launch_status();
   }
-  if constexpr (dtype_code<XT>::value == dtype_code<CT>::value) {
-    const bool full = (ra.K % 1024 == 0) && ra.y_dtype == CAIFX_F32;
-    if (full && ra.cpr == 1) return launch_int8_fast<CT, MT, kVec, 1>(ra, s);
-    if (full && ra.cpr == 2) return launch_int8_fast<CT, MT, kVec, 2>(ra, s);
-    if (full && ra.cpr == 4) return launch_int8_fast<CT, MT, kVec, 4>(ra, s);
-  }
-  const size_t lds = static_cast<size_t>(MT) * ra.xpitch * 2;
-  const unsigned grid = static_cast<unsigned>((ra.total_waves + 3) / 4);
-  switch (ra.cpr) {
-    case 1: hipLaunchKernelGGL((rowlin_int8_kernel<CT, XT, MT, kVec, 1>), dim3(grid), dim3(256), lds, s, ra); break;
-    case 2: hipLaunchKernelGGL((rowlin_int8_kernel<CT, XT, MT, kVec, 2>), dim3(grid), dim3(256), lds, s, ra); break;
-    case 3: hipLaunchKernelGGL((rowlin_int8_kernel<CT, XT, MT, kVec, 3>), dim3(grid), dim3(256), lds, s, ra); break;
-    case 4: hipLaunchKernelGGL((rowlin_int8_kernel<CT, XT, MT, kVec, 4>), dim3(grid), dim3(256), lds, s, ra); break;
-    default: return CAIFX_ERR_UNSUPPORTED;
-  }
-  return launch_status();
 }
 
 template <typename CT, typename XT, int MT>
@@ -1289,7 +1355,7 @@ int rowlin_forward(const GemmArgs &g, hipStream_t s)
     if (static_cast<size_t>(mt) * ra.xpitch * 2 + 4096 > 64 * 1024) return CAIFX_ERR_UNSUPPORTED;
   } else {
     // one activation row and 4096 < K <= 16384: the integer-matrix-core kernel with the row split among waves
-    const bool long_digits = g.M == 1 && g.K > 4096 && g.K <= 16384 && g.K % 1024 == 0 && g.y_dtype == CAIFX_F32;
+    const bool long_digits = g.M == 1 && g.K > 4096 && g.K <= 16384;
     if (g.K % 16 != 0 || (g.K > 4096 && !long_digits)) return CAIFX_ERR_UNSUPPORTED;
     ra.cpr = static_cast<int>((g.K + 1023) / 1024);
     ra.xpitch = ra.cpr * 1024;
@@ -1306,12 +1372,11 @@ int rowlin_forward(const GemmArgs &g, hipStream_t s)
     }
     const int64_t rows_class = (g.N + ra.row_stride - 1) / ra.row_stride;
     const int rb = ra.cpr == 1 ? 8 : (ra.cpr == 2 ? 4 : 2);
-    const bool digits = long_digits || (g.M == 1 && g.K % 1024 == 0 && (ra.cpr == 1 || ra.cpr == 2 || ra.cpr == 4) && g.y_dtype == CAIFX_F32);
+    const bool digits = long_digits || g.M == 1;      // K <= 4096 from here on
     if (long_digits) {
       // wave w of a workgroup takes slice w % slices of the rows of row group w / slices; waves_per_class and
       // total_waves count row groups here
       ra.slices = ra.cpr > 8 ? 4 : 2;
-      ra.digits = 1;
       ra.round_x = g.x_dtype != g.compute_dtype ? g.compute_dtype : -1;
       const int groups_per_block = kDigitWaves / ra.slices;
       const int64_t cus = compute_unit_count();
@@ -1336,7 +1401,6 @@ int rowlin_forward(const GemmArgs &g, hipStream_t s)
     }
     ra.waves_per_class = static_cast<int>((rows_class + ra.rows_per_wave - 1) / ra.rows_per_wave);
     if (digits) {
-      ra.digits = 1;
       ra.round_x = g.x_dtype != g.compute_dtype ? g.compute_dtype : -1;
       ra.waves_per_class = (ra.waves_per_class + kDigitWaves - 1) / kDigitWaves * kDigitWaves;      // a workgroup stays inside one class
     }
