@@ -107,8 +107,10 @@ const char *caifx_status_string(int status)
 
 int caifx_version(void) { return 1000; }
 
-size_t caifx_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype, int compute_dtype, int w_kind,
-                                     int backward)
+// `dense_copy`: count the large-M path's dequantised copy of the weight too (it is optional: with less workspace the
+// kernels that dequantise inside the product run)
+static size_t workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype, int compute_dtype, int w_kind, bool backward,
+                              bool dense_copy)
 {
   GemmArgs a{};
   a.M = M;
@@ -117,14 +119,21 @@ size_t caifx_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtyp
   a.x_dtype = x_dtype;
   a.compute_dtype = compute_dtype;
   a.w.kind = w_kind;
-  const size_t f32_bytes = mfma_f32_workspace_bytes(a, backward != 0);
+  const size_t f32_bytes = mfma_f32_workspace_bytes(a, backward);
   // float storage runs on the fp32 matrix-core kernel unless it is stored in the 16-bit compute type itself
   if (float_kind(w_kind) && !same_16bit(w_kind, compute_dtype)) return f32_bytes;
-  size_t bytes = mfma_workspace_bytes(a, backward != 0);
-  if (float_kind(w_kind)) return f32_bytes > bytes ? f32_bytes : bytes;
-  const size_t decode_bytes = backward ? dxrows_workspace_bytes(a) : mblock_workspace_bytes(a);
-  if (decode_bytes > bytes) bytes = decode_bytes;
-  return f32_bytes > bytes ? f32_bytes : bytes;
+  size_t bytes = mfma_workspace_bytes(a, backward);
+  const auto at_least = [&bytes](size_t b) { bytes = b > bytes ? b : bytes; };
+  if (dense_copy) at_least(mfma_wide_workspace_bytes(a, backward));
+  at_least(f32_bytes);
+  if (!float_kind(w_kind)) at_least(backward ? dxrows_workspace_bytes(a) : mblock_workspace_bytes(a));
+  return bytes;
+}
+
+size_t caifx_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype, int compute_dtype, int w_kind,
+                                     int backward)
+{
+  return workspace_bytes(M, N, K, x_dtype, compute_dtype, w_kind, backward != 0, true);
 }
 
 // `addend` (optional): the matrix-core GEMM adds it in its store; every other path runs as usual and is
@@ -236,7 +245,7 @@ int caifx_qlinear_forward_static(int64_t M, int64_t N, int64_t K, const void *x,
                                  void *y, int y_dtype, caifx_stream_t stream)
 {
   const size_t need = (M > 0 && N > 0 && K > 0 && valid_dtype(x_dtype) && valid_dtype(compute_dtype))
-                          ? caifx_qlinear_workspace_bytes(M, N, K, x_dtype, compute_dtype, w_kind, 0)
+                          ? workspace_bytes(M, N, K, x_dtype, compute_dtype, w_kind, false, false)
                           : 0;
   if (need > CAIFX_STATIC_SCRATCH_BYTES) return CAIFX_ERR_SCRATCH_EXCEEDED;
   void *ws = nullptr;

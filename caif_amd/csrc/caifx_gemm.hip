@@ -225,8 +225,12 @@ int splitk_reduce(const float *partial, int parts, int64_t n, void *y, int y_dty
   return launch_status();
 }
 
-int mfma_tiled_forward(const GemmArgs &a, hipStream_t s) { return run(a, false, s); }
-int mfma_backward(const GemmArgs &a, hipStream_t s) { return run(a, true, s); }
+int mfma_tiled(const GemmArgs &a, bool backward, hipStream_t s) { return run(a, backward, s); }
+int mfma_backward(const GemmArgs &a, hipStream_t s)
+{
+  const int st = mfma_wide(a, true, s);
+  return st == CAIFX_ERR_UNSUPPORTED ? mfma_tiled(a, true, s) : st;
+}
 void mfma_grouped_stamp_target(unsigned long long **buf, long long *capacity)
 {
   *buf = g_stamps.load(std::memory_order_relaxed);

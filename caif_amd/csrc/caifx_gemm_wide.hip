@@ -1,0 +1,543 @@
+// Large-M dequant-GEMM, forward and input gradient, in two launches: the weight is dequantised once into the caller's
+// workspace as a dense matrix of the compute type, [columns of the result, reduction] row-major (the input gradient's
+// transposed on the way), and a dense kernel multiplies it with the activations.  A weight stored in the 16-bit compute
+// type needs no first launch in the forward direction.
+//
+// What bounds it: the power the chip may draw.  On all-zero operands the kernel runs at 2.0-2.1 PFLOP/s, on N(0,1)
+// activations x N(0,0.02) weights at 1.53-1.56 (M = 4096, C = 4096, R = 11008: 236 us), so what counts is work per
+// flop, not only what waits for what:
+//  - v_mfma_f32_16x16x32 instead of 32x32x16: the same loop without any memory traffic runs at 2.07 instead of 1.80
+//    PFLOP/s on those values (a 16 x 16 result is read and written once per 32 reduction elements, a 32 x 32 one once
+//    per 16), the whole kernel at 236 instead of 254 us.
+//  - four waves with 128 x 128 of the 256 x 256 tile each (one wave per SIMD, 256 accumulators in the accumulation
+//    registers): 128 KB of operand reads from LDS per 64-deep step; eight waves of 128 x 64 read 192 KB (262 us).
+//  - the weight is dequantised once per call instead of once per row tile.
+// Against the kernels that dequantise inside the product (forward 380 us, input gradient 385 us at M = 4096, N = 11008,
+// K = 4096, int4, bf16) the two launches take 290 and 257 us.
+#include "caifx_internal.hpp"
+
+#include <atomic>
+#include <type_traits>
+
+namespace caifx {
+namespace {
+
+constexpr int kBK = 64;                    // reduction extent of a step: one 128-byte line of every row
+constexpr int kBandRows = 1024;            // rows of a band of the tile order
+
+struct WideArgs {
+  const void *a;        // [M, R] activations / gradients of the compute type
+  const void *b;        // [C, R] dense weight of the compute type
+  void *d;              // [M, C]
+  const void *addend;
+  int64_t M, C, R;
+  int d_dtype;
+};
+
+// acc += a b, 16 x 16 x 32: lane l supplies row (column) l % 16, reduction elements 8 (l / 16) .. + 7; the result's
+// register r holds row 4 (l / 16) + r, column l % 16.  Written as asm so that the accumulators stay in accumulation
+// registers: with the builtin the compiler moves a part of the 256 between the two files in every step.
+template <typename CT> __device__ __forceinline__ void mfma16(floatx4_t &acc, const typename Mfma32<CT>::vec_t &a, const typename Mfma32<CT>::vec_t &b)
+{
+  if constexpr (std::is_same<CT, bf16_t>::value)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+
+// A result tile has 64 WI rows and 64 WJ columns.  Wave (wm, wn) owns rows h 32 WI + wm 16 WI + [0, 16 WI) and columns
+// g 32 WJ + wn 16 WJ + [0, 16 WJ) of it for h, g in {0, 1}: four quadrants of WI x WJ products.  LDS holds four half
+// tiles per operand: half h of step s in slot 2 (s & 1) + h.  A step runs through the quadrants (h, g) = (0,0) (0,1)
+// (1,1) (1,0); the operands of a quadrant are read during the one before it, so half 1 of step s has been read by
+// everybody in the middle of quadrant (1,1) and half 0 in the middle of the next step's (0,0).  There, and only there,
+// the waves meet; behind the barrier the freed slot is requested for step s + 2, three half tiles (96 KB per compute
+// unit for 256 x 256) are on their way at any time, and every request has one and a half steps to arrive.  Requests
+// complete in issue order, so the wait for the half tile that is read next is an exact count (a wave issues WI + WJ
+// per half).
+template <typename CT, int WI, int WJ>
+__global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(WideArgs g)
+{
+  typedef typename Mfma32<CT>::vec_t vec_t;
+  constexpr int BM = 64 * WI, BN = 64 * WJ;
+  constexpr int kASlot = BM / 2 * 128, kBSlot = BN / 2 * 128;      // LDS bytes of half an operand tile
+  constexpr int kBBase = 4 * kASlot;
+  constexpr int kBand = kBandRows / BM;
+  constexpr int kReq = WI + WJ;            // requests of a wave per half step
+  constexpr int Q = 2 * WI * WJ;           // products per quadrant
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int r16 = lane & 15, kq = lane >> 4;
+
+  // XCD x (workgroup id mod 8, each with its own L2) walks the x-th contiguous eighth of a list that runs through bands
+  // of 1024 rows column by column: the 256 x 256 tiles it works on at a time share 4 row and 8 column panels
+  const int64_t col_tiles = (g.C + BN - 1) / BN, row_tiles = (g.M + BM - 1) / BM;
+  int64_t row0, col0;
+  {
+    const unsigned bid = blockIdx.x;
+    const int64_t per_xcd = gridDim.x >> 3;
+    const int64_t pos = static_cast<int64_t>(bid & 7) * per_xcd + (bid >> 3);
+    if (pos >= row_tiles * col_tiles) return;
+    const int64_t band = pos / (kBand * col_tiles);
+    const int64_t within = pos - band * kBand * col_tiles;
+    const int64_t left = row_tiles - band * kBand;
+    const int64_t band_rows = left < kBand ? left : kBand;
+    col0 = (within / band_rows) * BN;
+    row0 = (band * kBand + within % band_rows) * BM;
+  }
+
+  // request i of a wave for half h of an operand: 8 rows x 128 bytes; LDS position p of row r holds 16-byte chunk
+  // p ^ (r ^ r >> 3) & 7 of the row (operand reads without bank conflicts), so that is the chunk a lane asks for.  Rows
+  // and columns past the end are loaded from the last one and never stored.
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+  uint32_t a_voff[2][WI], b_voff[2][WJ];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+      const int lrow = 8 * (wave + 4 * i) + (lane >> 3);
+      int64_t m = row0 + h * (BM / 2) + lrow;
+      if (m >= g.M) m = g.M - 1;
+      a_voff[h][i] = static_cast<uint32_t>((m - row0) * g.R * 2 + (((lane & 7) ^ ((lrow ^ (lrow >> 3)) & 7)) << 4));
+    }
+#pragma unroll
+    for (int i = 0; i < WJ; ++i) {
+      const int lrow = 8 * (wave + 4 * i) + (lane >> 3);
+      int64_t c = col0 + h * (BN / 2) + lrow;
+      if (c >= g.C) c = g.C - 1;
+      b_voff[h][i] = static_cast<uint32_t>((c - col0) * g.R * 2 + (((lane & 7) ^ ((lrow ^ (lrow >> 3)) & 7)) << 4));
+    }
+  }
+  const uint64_t a_base = reinterpret_cast<uint64_t>(g.a) + static_cast<uint64_t>(row0 * g.R * 2);
+  const uint64_t b_base = reinterpret_cast<uint64_t>(g.b) + static_cast<uint64_t>(col0 * g.R * 2);
+  const int steps = static_cast<int>(g.R / kBK);
+  const int last = steps - 1;
+  auto request = [&](int s, int h, int slot, int x) __attribute__((always_inline)) {
+    const uint32_t k0 = static_cast<uint32_t>(s < last ? s : last) * 128;          // past the end: the last step again
+    const bool is_a = x < WI;
+    const int i = is_a ? x : x - WI;
+    const uint64_t src = (is_a ? a_base : b_base) + k0;
+    const uint32_t dst = lds0 + (is_a ? slot * kASlot : kBBase + slot * kBSlot) + (wave + 4 * i) * 1024;
+    const uint32_t voff = is_a ? a_voff[h][is_a ? i : 0] : b_voff[h][is_a ? 0 : i];
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(src) : "memory");
+  };
+
+  // operand (row tile i of 16 rows, reduction half kk): tiles i and i + 2 lie 32 rows apart, which flips the
+  // swizzle's third bit, the one that kk selects
+  uint32_t a_addr[2][2], b_addr[2][2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int ra = wm * 16 * WI + i * 16 + r16;
+      a_addr[i][kk] = ra * 128 + (((4 * kk + kq) ^ ((ra ^ (ra >> 3)) & 7)) << 4);
+      const int rb = wn * 16 * WJ + i * 16 + r16;
+      b_addr[i][kk] = kBBase + rb * 128 + (((4 * kk + kq) ^ ((rb ^ (rb >> 3)) & 7)) << 4);
+    }
+  auto read_a = [&](int slot, int i, int kk) __attribute__((always_inline)) {
+    return *reinterpret_cast<const vec_t *>(smem + slot * kASlot + (i >> 1) * 4096 + a_addr[i & 1][kk ^ (i >> 1)]);
+  };
+  auto read_b = [&](int slot, int i, int kk) __attribute__((always_inline)) {
+    return *reinterpret_cast<const vec_t *>(smem + slot * kBSlot + (i >> 1) * 4096 + b_addr[i & 1][kk ^ (i >> 1)]);
+  };
+
+  floatx4_t acc[2][2][WI][WJ];     // [h][g][row tile][column tile]
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int i = 0; i < WI; ++i)
+#pragma unroll
+        for (int c = 0; c < WJ; ++c) acc[h][q][i][c] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int x = 0; x < kReq; ++x) request(u >> 1, u & 1, u, x);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * kReq) : "memory");
+  vec_t a0[WI][2], a1[WI][2], b0[WJ][2], b1[WJ][2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+    for (int i = 0; i < WJ; ++i) b0[i][kk] = read_b(0, i, kk);
+#pragma unroll
+    for (int i = 0; i < WI; ++i) a0[i][kk] = read_a(0, i, kk);
+  }
+
+  // one quadrant: its products run to and fro over the row tiles so that one operand stays from product to product;
+  // `first` runs in front of the second half, `each` behind every product
+  auto quadrant = [&](floatx4_t(&d)[WI][WJ], const vec_t(&a)[WI][2], const vec_t(&b)[WJ][2], auto first, auto each) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < Q; ++t) {
+      if (t == Q / 2) first();
+      const int u = t % (WI * WJ), kk = t / (WI * WJ);
+      const int c = u / WI, i = (c & 1) ? WI - 1 - u % WI : u % WI;
+      mfma16<CT>(d[i][c], a[i][kk], b[c][kk]);
+      each(t);
+      if (t & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // the n reads or requests of half a quadrant, spread over its Q / 2 products (t = 0 .. Q / 2 - 1)
+  auto spread = [&](int t, int n, auto op) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < n; ++x)
+      if (x * (Q / 2) / n == t) op(x);
+  };
+  auto meet = [&]() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kReq) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto nothing = []() __attribute__((always_inline)) {};
+  auto step = [&](auto par_, int s) __attribute__((always_inline)) {
+    constexpr int p = decltype(par_)::value;
+    constexpr int S0 = 2 * p, S1 = 2 * p + 1, S0n = 2 * (p ^ 1);
+    quadrant(acc[0][0], a0, b0, meet, [&](int t) __attribute__((always_inline)) {
+      spread(t - Q / 2, 2 * WJ, [&](int x) __attribute__((always_inline)) { b1[x % WJ][x / WJ] = read_b(S1, x % WJ, x / WJ); });
+      spread(t - Q / 2, kReq, [&](int x) __attribute__((always_inline)) { request(s + 2, 0, S0, x); });
+    });
+    quadrant(acc[0][1], a0, b1, nothing, [&](int t) __attribute__((always_inline)) {
+      spread(t, 2 * WI, [&](int x) __attribute__((always_inline)) { a1[x % WI][x / WI] = read_a(S1, x % WI, x / WI); });
+    });
+    quadrant(acc[1][1], a1, b1, meet, [&](int t) __attribute__((always_inline)) {
+      spread(t - Q / 2, 2 * WI, [&](int x) __attribute__((always_inline)) { a0[x % WI][x / WI] = read_a(S0n, x % WI, x / WI); });
+      spread(t - Q / 2, kReq, [&](int x) __attribute__((always_inline)) { request(s + 2, 1, S1, x); });
+    });
+    quadrant(acc[1][0], a1, b0, nothing, [&](int t) __attribute__((always_inline)) {
+      if (t % WI == WI - 1) b0[(t / WI) % WJ][t / (WI * WJ)] = read_b(S0n, (t / WI) % WJ, t / (WI * WJ));
+    });
+  };
+  int s = 0;
+  for (; s + 2 <= steps; s += 2) {
+    step(std::integral_constant<int, 0>{}, s);
+    step(std::integral_constant<int, 1>{}, s + 1);
+  }
+  if (s < steps) step(std::integral_constant<int, 0>{}, s);
+  // the last products have to leave the pipe before their registers are read (the compiler does not see the asm's
+  // latency), requests past the last step may still be writing LDS, and other waves may still be reading
+  asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // store through LDS: a pass of whole tile rows (16-bit results: all of them, fp32: one half), row pitch = row + 32
+  // bytes so that the four row groups of a wave's registers spread over the banks, then whole rows, 16 bytes per lane;
+  // the optional addend is read the same way
+  auto store = [&](auto type_) __attribute__((always_inline)) {
+    typedef decltype(type_) T;
+    constexpr int kPitch = BN * sizeof(T) + 32;
+    constexpr int kPer16 = 16 / sizeof(T);
+    constexpr int kLanesPerRow = BN / kPer16;            // 16, 32 or 64
+    constexpr int kPassHalves = sizeof(T) == 2 ? 2 : 1;
+    T *dp = static_cast<T *>(g.d);
+    const T *ap = static_cast<const T *>(g.addend);
+    const int chunk = lane % kLanesPerRow;
+    const int64_t gcol = col0 + chunk * kPer16;
+#pragma unroll
+    for (int pass = 0; pass < 2 / kPassHalves; ++pass) {
+      if (pass > 0) __syncthreads();
+#pragma unroll
+      for (int hh = 0; hh < kPassHalves; ++hh)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int i = 0; i < WI; ++i)
+#pragma unroll
+            for (int c = 0; c < WJ; ++c)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const int lrow = hh * (BM / 2) + wm * 16 * WI + i * 16 + 4 * kq + r;
+                *reinterpret_cast<T *>(smem + lrow * kPitch + (q * (BN / 2) + wn * 16 * WJ + c * 16 + r16) * sizeof(T)) =
+                    from_f32<T>(acc[pass * kPassHalves + hh][q][i][c][r]);
+              }
+      __syncthreads();
+      constexpr int kRows = kPassHalves * (BM / 2);
+      constexpr int kRowsPerInstr = 64 / kLanesPerRow;
+#pragma unroll 4
+      for (int it = 0; it < kRows / (4 * kRowsPerInstr); ++it) {
+        const int lrow = (it * 4 + wave) * kRowsPerInstr + lane / kLanesPerRow;
+        const int64_t grow = row0 + pass * (BM / 2) + lrow;
+        if (grow >= g.M || gcol >= g.C) continue;        // C is a multiple of 8
+        u32x4_t v = *reinterpret_cast<const u32x4_t *>(smem + lrow * kPitch + chunk * 16);
+        const int64_t o = grow * g.C + gcol;
+        if (ap) {
+          const u32x4_t av = *reinterpret_cast<const u32x4_t *>(ap + o);
+          const T *vp = reinterpret_cast<const T *>(&v);
+          const T *aq = reinterpret_cast<const T *>(&av);
+          u32x4_t w;
+          T *wp = reinterpret_cast<T *>(&w);
+#pragma unroll
+          for (int e = 0; e < kPer16; ++e) wp[e] = from_f32<T>(to_f32<T>(vp[e]) + to_f32<T>(aq[e]));
+          v = w;
+        }
+        *reinterpret_cast<u32x4_t *>(dp + o) = v;
+      }
+    }
+  };
+  if (g.d_dtype == CAIFX_BF16) store(bf16_t{});
+  else if (g.d_dtype == CAIFX_F16) store(f16_t{});
+  else store(float{});
+}
+
+// ------------------------------------------------------------------ the weight as a dense matrix of the compute type
+struct DenseArgs {
+  const void *q;
+  const void *scales;
+  void *out;
+  int64_t N, K;
+  int group_shift;         // int4
+  uint32_t period;         // int8; 0 = no scales
+};
+
+enum { DK_INT8 = 0, DK_INT4 = 1, DK_16 = 2 };
+
+// eight consecutive weights of flat index f (a multiple of 8) as fp32, the reference's code * scale
+template <typename CT, int kKind>
+__device__ __forceinline__ void load_weights8(const DenseArgs &g, int64_t f, float (&e)[8])
+{
+  if constexpr (kKind == DK_INT4) {
+    const uint32_t p = *reinterpret_cast<const uint32_t *>(static_cast<const uint8_t *>(g.q) + (f >> 1));
+    dequant_int4x8(p, to_f32(static_cast<const f16_t *>(g.scales)[f >> g.group_shift]), e);
+  } else if constexpr (kKind == DK_INT8) {
+    const u32x2_t p = *reinterpret_cast<const u32x2_t *>(static_cast<const uint8_t *>(g.q) + f);
+    float lo[4], hi[4];
+    int8x4_to_f32(p[0], lo);
+    int8x4_to_f32(p[1], hi);
+    const float *sp = static_cast<const float *>(g.scales);
+    if (g.period > 1) {          // a multiple of 4: neither quad wraps inside
+      const uint32_t i0 = static_cast<uint32_t>(f) % g.period;      // N * K < 2^32 (host)
+      const uint32_t i1 = i0 + 4 < g.period ? i0 + 4 : i0 + 4 - g.period;
+      const floatx4_t s0 = *reinterpret_cast<const floatx4_t *>(sp + i0), s1 = *reinterpret_cast<const floatx4_t *>(sp + i1);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        e[t] = lo[t] * s0[t];
+        e[4 + t] = hi[t] * s1[t];
+      }
+    } else {
+      const float s = g.period == 1 ? sp[0] : 1.0f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        e[t] = lo[t] * s;
+        e[4 + t] = hi[t] * s;
+      }
+    }
+  } else {
+    const u32x4_t p = *reinterpret_cast<const u32x4_t *>(static_cast<const CT *>(g.q) + f);
+    const CT *v = reinterpret_cast<const CT *>(&p);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) e[t] = to_f32<CT>(v[t]);
+  }
+}
+
+// [N, K] as stored: eight values per thread and round, four rounds requested ahead.  Bound by HBM.
+template <typename CT, int kKind>
+__global__ __launch_bounds__(256) void dense_rows_kernel(DenseArgs g)
+{
+  constexpr int kRounds = 4;
+  const int64_t pieces = g.N * g.K / 8;
+  const int64_t p0 = static_cast<int64_t>(blockIdx.x) * (256 * kRounds) + threadIdx.x;
+  float e[kRounds][8];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int64_t p = p0 + r * 256;
+    load_weights8<CT, kKind>(g, (p < pieces ? p : pieces - 1) * 8, e[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int64_t p = p0 + r * 256;
+    if (p >= pieces) continue;
+    u32x4_t v;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = pack2<CT>(e[r][2 * t], e[r][2 * t + 1]);
+    *reinterpret_cast<u32x4_t *>(static_cast<CT *>(g.out) + p * 8) = v;
+  }
+}
+
+// [K, N], transposed: a workgroup takes 64 rows n x 256 columns k.  A thread reads eight columns of eight rows (the
+// 32 lanes of a row together 128 bytes of int4 codes), packs them into eight pieces of eight n and lays them out in
+// LDS as rows of 64 n; the rows are then written in whole 128-byte lines.  The piece position is rotated by the
+// thread's k so that the eight lanes of a group use different banks.
+template <typename CT, int kKind>
+__global__ __launch_bounds__(256) void dense_transposed_kernel(DenseArgs g)
+{
+  __shared__ __attribute__((aligned(16))) unsigned char tile[256 * 128];
+  const int kl = threadIdx.x & 31, ng = threadIdx.x >> 5;
+  const int64_t n0 = static_cast<int64_t>(blockIdx.y) * 64, k0 = static_cast<int64_t>(blockIdx.x) * 256;
+  if (k0 + 8 * kl < g.K) {
+    float e[8][8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) load_weights8<CT, kKind>(g, (n0 + 8 * ng + r) * g.K + k0 + 8 * kl, e[r]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      u32x4_t v;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) v[t] = pack2<CT>(e[2 * t][j], e[2 * t + 1][j]);
+      *reinterpret_cast<u32x4_t *>(tile + (8 * kl + j) * 128 + (((ng + kl) & 7) << 4)) = v;
+    }
+  }
+  __syncthreads();
+  const int piece = threadIdx.x & 7;
+#pragma unroll
+  for (int it = 0; it < 8; ++it) {
+    const int k = it * 32 + (threadIdx.x >> 3);
+    if (k0 + k >= g.K) continue;
+    const u32x4_t v = *reinterpret_cast<const u32x4_t *>(tile + k * 128 + (((piece + (k >> 3)) & 7) << 4));
+    *reinterpret_cast<u32x4_t *>(static_cast<CT *>(g.out) + (k0 + k) * g.N + n0 + 8 * piece) = v;
+  }
+}
+
+template <typename CT>
+int launch_dense(const DenseArgs &g, int kind, bool transposed, hipStream_t s)
+{
+  if (transposed) {
+    const dim3 grid(static_cast<unsigned>((g.K + 255) / 256), static_cast<unsigned>(g.N / 64));
+    if (kind == DK_INT4) hipLaunchKernelGGL((dense_transposed_kernel<CT, DK_INT4>), grid, dim3(256), 0, s, g);
+    else if (kind == DK_INT8) hipLaunchKernelGGL((dense_transposed_kernel<CT, DK_INT8>), grid, dim3(256), 0, s, g);
+    else hipLaunchKernelGGL((dense_transposed_kernel<CT, DK_16>), grid, dim3(256), 0, s, g);
+  } else {
+    const dim3 grid(static_cast<unsigned>((g.N * g.K / 8 + 1023) / 1024));
+    if (kind == DK_INT4) hipLaunchKernelGGL((dense_rows_kernel<CT, DK_INT4>), grid, dim3(256), 0, s, g);
+    else hipLaunchKernelGGL((dense_rows_kernel<CT, DK_INT8>), grid, dim3(256), 0, s, g);
+  }
+  return launch_status();
+}
+
+template <typename CT, int WI, int WJ>
+int launch_wide(const WideArgs &g, hipStream_t s)
+{
+  constexpr int BM = 64 * WI, BN = 64 * WJ;
+  constexpr int kRing = (BM + BN) * 256, kStore16 = BM * (BN * 2 + 32), kStore32 = BM / 2 * (BN * 4 + 32);
+  constexpr int kStore = kStore16 > kStore32 ? kStore16 : kStore32;
+  constexpr int kLds = kRing > kStore ? kRing : kStore;
+  auto kern = wide_gemm_kernel<CT, WI, WJ>;
+  static std::atomic<bool> raised{false};
+  if (!raised.load(std::memory_order_relaxed)) {
+    // the attribute is per kernel and sticky; two threads racing here both set it, which is harmless
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+      return CAIFX_ERR_LAUNCH_FAILED;
+    raised.store(true, std::memory_order_relaxed);
+  }
+  const int64_t tiles = ((g.M + BM - 1) / BM) * ((g.C + BN - 1) / BN);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((tiles + 7) / 8 * 8)), dim3(256), kLds, s, g);
+  return launch_status();
+}
+
+// What a 64-deep step of the whole launch costs with one of the three tiles, in us: the number of rounds the tiles take
+// times the time of one, measured on N(0,1) x N(0,0.02) bf16 values at R = 4096.  256 x 256 (one workgroup per compute
+// unit) 1.39 per round of 256, 128 x 256 (one) 0.87, 128 x 128 (two) 0.91 per round of 512 and 0.49 for a last round of
+// at most 256.  M = 4096, C = 11008: 265 / 300 / 300 us; M = 2048, C = 11008: 166 / 149 / 162; M = 1024, C = 4096: 72 /
+// 44 / 32.
+enum { TILE_256 = 0, TILE_128x256 = 1, TILE_128 = 2 };
+double step_cost(int tile, int64_t M, int64_t C)
+{
+  const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((C + bn - 1) / bn); };
+  if (tile == TILE_256) return 1.39 * static_cast<double>((tiles(256, 256) + 255) / 256);
+  if (tile == TILE_128x256) return 0.87 * static_cast<double>((tiles(128, 256) + 255) / 256);
+  const int64_t t = tiles(128, 128), rest = t % 512;
+  return 0.91 * static_cast<double>(t / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.49 : 0.91);
+}
+int best_tile(int64_t M, int64_t C)
+{
+  int best = TILE_256;
+  for (int t = TILE_128x256; t <= TILE_128; ++t)
+    if (step_cost(t, M, C) < step_cost(best, M, C)) best = t;
+  return best;
+}
+
+template <typename CT>
+int pick_wide(const WideArgs &g, hipStream_t s)
+{
+  switch (best_tile(g.M, g.C)) {
+    case TILE_256: return launch_wide<CT, 4, 4>(g, s);
+    case TILE_128x256: return launch_wide<CT, 2, 4>(g, s);
+    default: return launch_wide<CT, 2, 2>(g, s);
+  }
+}
+
+bool dense16(const GemmArgs &a)
+{
+  return (a.w.kind == CAIFX_W_BF16 && a.compute_dtype == CAIFX_BF16) || (a.w.kind == CAIFX_W_F16 && a.compute_dtype == CAIFX_F16);
+}
+
+// The rule on sizes and types alone (the workspace query knows nothing else).
+bool wide_shape(const GemmArgs &a, bool backward)
+{
+  if (a.compute_dtype == CAIFX_F32 || a.x_dtype != a.compute_dtype || a.offsets || a.epilogue != 0) return false;
+  const bool codes = a.w.kind == CAIFX_W_INT8 || a.w.kind == CAIFX_W_INT4_GROUP;
+  if (!codes && !dense16(a)) return false;
+  const int64_t C = backward ? a.K : a.N, R = backward ? a.N : a.K;
+  if (R % kBK != 0 || C % 8 != 0 || a.K % 8 != 0 || a.M < 1 || R < 2 * kBK) return false;
+  if (a.N * a.K >= (int64_t{1} << 32) || a.M > (int64_t{1} << 30) || R > (int64_t{1} << 22)) return false;
+  const int64_t tiles = ((a.M + 127) / 128) * ((C + 127) / 128);
+  if (tiles > (int64_t{1} << 30)) return false;
+  // Is it worth it?  `tiles` counts 128 x 128 tiles.  A stored 16-bit weight needs no extra pass in the forward
+  // direction: from 100 tiles on (128: 25.8 against 27.4 us, 256: 31.5 against 39.4; 80: 26.1 against 24.2, where the
+  // tiled kernel shares each tile's reduction among workgroups).
+  if (!codes && !backward) return tiles >= 100;
+  // int4 forward with whole 256-code blocks has a kernel of its own (caifx_gemm_regw.hip): per round of 256 tiles of 128
+  // x 256 about 0.9 us a step and 6 us.  The dense pass costs 3.5 us and 0.33 us per million weights (18 us at 11008 x
+  // 4096), the rest 3 us.  M = 512, N = 11008, K = 4096: 55 against 65 us, M = 2048: 186 against 167.  Calls of up to
+  // one 128 x 128 tile per compute unit go on without a workspace, with the same bits from caifx_qlinear_forward_static
+  // as from here (M = 1024, N = K = 4096: 51 us where this would take 41).
+  const int64_t regw_tiles = ((a.M + 127) / 128) * ((C + 255) / 256);
+  if (!backward && a.w.kind == CAIFX_W_INT4_GROUP && a.K % 256 == 0 && regw_tiles >= 128) {
+    const double steps = static_cast<double>(R / kBK);
+    return tiles > 256 &&
+           3.0 + step_cost(best_tile(a.M, C), a.M, C) * steps + 3.5 + 0.33e-6 * static_cast<double>(a.N) * static_cast<double>(a.K) <
+               (0.9 * steps + 6.0) * static_cast<double>((regw_tiles + 255) / 256);
+  }
+  // Everything else runs on the tiled kernel otherwise (or int8 forward with a short scale vector on
+  // caifx_gemm_regw8.hip): int4 and 16-bit input gradients from 190 tiles on (198: 30.4 against 37.4 us at M = 1367, N =
+  // 2880, K = 2304; 128: 85 against 76), int8, whose unpacking costs those kernels more, from 90 (96 tiles of the
+  // input gradient at N = 5952, K = 2048: 43 against 66 us; 64: 61 against 50).
+  return tiles >= (a.w.kind == CAIFX_W_INT8 ? 90 : 190);
+}
+
+}  // namespace
+
+size_t mfma_wide_workspace_bytes(const GemmArgs &a, bool backward)
+{
+  if (!wide_shape(a, backward) || (dense16(a) && !backward)) return 0;
+  return static_cast<size_t>(a.N) * static_cast<size_t>(a.K) * 2;
+}
+
+int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s)
+{
+  if (!wide_shape(a, backward)) return CAIFX_ERR_UNSUPPORTED;
+  if (!aligned_to(a.x, 16) || !aligned_to(a.w.q, 16) || !aligned_to(a.y, 16) || (a.addend && !aligned_to(a.addend, 16))) return CAIFX_ERR_UNSUPPORTED;
+  WideArgs g{};
+  g.a = a.x;
+  g.d = a.y;
+  g.addend = a.addend;
+  g.M = a.M;
+  g.C = backward ? a.K : a.N;
+  g.R = backward ? a.N : a.K;
+  g.d_dtype = a.y_dtype;
+  g.b = a.w.q;
+  const size_t need = mfma_wide_workspace_bytes(a, backward);
+  if (need > 0) {
+    if (!a.workspace || a.workspace_bytes < need || !aligned_to(a.workspace, 16)) return CAIFX_ERR_UNSUPPORTED;
+    DenseArgs d{};
+    d.q = a.w.q;
+    d.scales = a.w.scales;
+    d.out = a.workspace;
+    d.N = a.N;
+    d.K = a.K;
+    int kind = DK_16;
+    if (a.w.kind == CAIFX_W_INT4_GROUP) {
+      const int gs = a.w.group_size;
+      if (gs < 8 || (gs & (gs - 1)) != 0) return CAIFX_ERR_UNSUPPORTED;
+      d.group_shift = __builtin_ctz(static_cast<unsigned>(gs));
+      kind = DK_INT4;
+    } else if (a.w.kind == CAIFX_W_INT8) {
+      d.period = a.w.scales ? static_cast<uint32_t>(a.w.scale_period) : 0;
+      if (d.period > 1 && (a.w.scale_period % 4 != 0 || a.w.scale_period < 8 || a.w.scale_period > a.N * a.K || !aligned_to(a.w.scales, 16)))
+        return CAIFX_ERR_UNSUPPORTED;
+      kind = DK_INT8;
+    }
+    const int st = a.compute_dtype == CAIFX_BF16 ? launch_dense<bf16_t>(d, kind, backward, s) : launch_dense<f16_t>(d, kind, backward, s);
+    if (st != CAIFX_OK) return st;
+    g.b = a.workspace;
+  }
+  return a.compute_dtype == CAIFX_BF16 ? pick_wide<bf16_t>(g, s) : pick_wide<f16_t>(g, s);
+}
+
+}  // namespace caifx

@@ -61,12 +61,18 @@ size_t mblock_workspace_bytes(const GemmArgs &a);
 int dxrows_backward(const GemmArgs &a, hipStream_t s);
 size_t dxrows_workspace_bytes(const GemmArgs &a);
 
-// Large-M MFMA path (compute bound), forward and input gradient, plain and grouped.  mfma_forward picks between
-// the forward kernels (mfma_regw_forward where it applies, else mfma_tiled_forward).
+// Large-M MFMA path (compute bound), forward and input gradient, plain and grouped.  mfma_forward and mfma_backward
+// pick between the kernels (mfma_wide, then the forward's register-weight forms, then mfma_tiled).
 int mfma_forward(const GemmArgs &a, hipStream_t s);
-int mfma_tiled_forward(const GemmArgs &a, hipStream_t s);
 int mfma_backward(const GemmArgs &a, hipStream_t s);
+int mfma_tiled(const GemmArgs &a, bool backward, hipStream_t s);
+// Workspace of the tiled kernel's shared reduction.
 size_t mfma_workspace_bytes(const GemmArgs &a, bool backward);
+// The weight dequantised once into the workspace (mfma_wide_workspace_bytes, 0 where it does not apply or where the
+// stored weight is used as it is), then a dense 256 x 256 tile kernel.  Without that workspace, or for shapes it does
+// not take, CAIFX_ERR_UNSUPPORTED.
+int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s);
+size_t mfma_wide_workspace_bytes(const GemmArgs &a, bool backward);
 // Measurement only: grouped launches of the matrix-core GEMM issued after this call record, per tile of their own
 // numbering (expert by expert, row tile by row tile, column tile last), four 64-bit words {expert, rows in the
 // tile, start, end} with the times in ticks of the 100 MHz wall clock, into buf (device memory for `tiles` tiles);

@@ -4,7 +4,7 @@ fixed-shape kernels, and every result dtype, against the CPU oracle (src/caif_de
 
 Bound: these kernels multiply codes with scales folded in afterwards (or into the activations), the oracle rounds
 code * scale to the compute dtype first: 4e-3 of the largest result at bf16, as in test_gpu_qlinear_skinny.py; a 16-bit
-result adds its own rounding, half a unit in the last place of 8 bits (2^-9)."""
+bf16 result adds its own rounding, half the spacing of 8-bit significands (2^-8)."""
 import numpy as np
 import pytest
 import torch
@@ -29,4 +29,4 @@ def test_reduction_tails(orc, kind, K):
             y = T.qlinear_forward(x, dw, cd, yd)
             want = orc.frozen_linear_forward(host(x), ow, cd)
             assert np.isfinite(host(y)).all()
-            assert max_rel_err(host(y), want) <= 4e-3 + (2.0 ** -9 if yd == 2 else 0), (M, cd, yd)
+            assert max_rel_err(host(y), want) <= 4e-3 + (2.0 ** -8 if yd == 2 else 0), (M, cd, yd)

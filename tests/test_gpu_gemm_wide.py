@@ -1,0 +1,68 @@
+"""The large-M path through a dense copy of the weight in the workspace (caifx_gemm_wide.hip): each of its three tile
+shapes with partial tiles in both directions, odd and even step counts, every weight kind, forward and input gradient,
+every result dtype and the fused addend, against the CPU oracle (src/caif_device_frozen_linear.cpp:382-524, :528-660).
+
+Bound: the operands are the oracle's (the weight rounded to the compute type once), the products are summed in fp32 in
+another order: 2e-5 of the largest result, as for the other matrix-core kernels; a 16-bit result adds half the spacing of
+its values, which for a significand of p bits is 2^-p of the value at most (bf16: p = 8, fp16: p = 11), the addend's
+rounding once more."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from caif_amd import capi, torch_ops as T                             # noqa: E402
+from gpu_helpers import dev_as, host, make_weight, max_rel_err        # noqa: E402
+
+ULP = {0: 0.0, 1: 2.0 ** -11, 2: 2.0 ** -8}
+
+# (M, N, K): 256 x 256, 128 x 256 and 128 x 128 tiles, ragged against them; 2, 3 and many 64-deep steps
+SHAPES = [(3900, 4040, 128), (2049, 4104, 192), (1160, 3080, 320), (2300, 1920, 448), (1500, 2112, 192), (2500, 1408, 320)]
+
+
+def _rows(m):
+    return np.unique(np.concatenate([np.arange(2), [m // 2, m - 1], np.arange(120, 132), np.arange(250, 260)]))
+
+
+@pytest.mark.parametrize("kind", ["int4", "int8pc", "int8pt", "int8none", "bf16"])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_against_the_oracle(orc, kind, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    cd = 2 if kind == "bf16" or (M + K) % 3 else 1
+    for backward in (False, True):
+        n, k = (K, N // 64 * 64) if backward else (N, K)        # the reduction is K forward, N backward
+        if kind == "int4":
+            k = max(128, k // 128 * 128)
+        if kind == "bf16":
+            w = torch.from_numpy(rng.normal(0, 0.02, (n, k)).astype(np.float32)).cuda().to(torch.bfloat16)
+            dw = T.FrozenWeight(w.reshape(-1), T.W_BF16, None, n, k)
+        else:
+            ow, dw = make_weight(orc, rng, n, k, kind)
+        R, C = (n, k) if backward else (k, n)
+        x = dev_as(rng.normal(0, 1, (M, R)), cd)
+        run = T.qlinear_backward_input if backward else T.qlinear_forward
+        sel = _rows(M)
+        if kind == "bf16":
+            want = host(x)[sel].astype(np.float64) @ (host(w).astype(np.float64) if backward else host(w).astype(np.float64).T)
+        else:
+            want = (orc.frozen_linear_backward if backward else orc.frozen_linear_forward)(host(x)[sel], ow, cd)
+        for yd in (0, cd):
+            assert max_rel_err(host(run(x, dw, cd, yd))[sel], want) <= 2e-5 + ULP[yd], (backward, yd)
+        add = dev_as(rng.normal(0, 1, (M, C)), cd)
+        got = host(run(x, dw, cd, cd, addend=add))[sel]
+        plain = host(run(x, dw, cd, cd))[sel]
+        assert max_rel_err(got, plain + host(add)[sel]) <= ULP[cd], backward      # one rounding of the sum
+
+
+@pytest.mark.parametrize("kind", ["int4", "int8pc"])
+def test_smaller_workspace_falls_back(orc, kind):
+    # the dense copy is optional: with less (or no) workspace the kernels that dequantise inside the product run
+    rng = np.random.default_rng(5)
+    M, N, K = 2048, 2048, 2048
+    ow, dw = make_weight(orc, rng, N, K, kind)
+    assert capi.lib().caifx_qlinear_workspace_bytes(M, N, K, T.BF16, T.BF16, dw.w_kind, 1) >= 2 * N * K
+    x = dev_as(rng.normal(0, 1, (M, N)), 2)
+    small = torch.empty(16, dtype=torch.uint8, device="cuda")
+    got, want = T.qlinear_backward_input(x, dw, T.BF16, workspace=small), T.qlinear_backward_input(x, dw, T.BF16)
+    assert max_rel_err(host(got), host(want)) <= 2e-5
