@@ -219,21 +219,38 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   // store through LDS: a pass of whole tile rows (16-bit results: all of them, fp32: one half), row pitch = row + 32
-  // bytes so that the four row groups of a wave's registers spread over the banks, then whole rows, 16 bytes per lane;
-  // the optional addend is read the same way
-  auto store = [&](auto type_) __attribute__((always_inline)) {
+  // bytes so that the four row groups of a wave's registers spread over the banks, then whole rows, 16 bytes per lane.
+  // The optional addend is read the same way, a batch of rows ahead (the operand registers are free by now): read row
+  // by row in front of each store it took 46 us of 322 at M = 4096, C = 11008, R = 4096.
+  auto store = [&](auto type_, auto add_) __attribute__((always_inline)) {
     typedef decltype(type_) T;
+    constexpr bool kAdd = decltype(add_)::value;
     constexpr int kPitch = BN * sizeof(T) + 32;
     constexpr int kPer16 = 16 / sizeof(T);
     constexpr int kLanesPerRow = BN / kPer16;            // 16, 32 or 64
     constexpr int kPassHalves = sizeof(T) == 2 ? 2 : 1;
+    constexpr int kRows = kPassHalves * (BM / 2);
+    constexpr int kRowsPerInstr = 64 / kLanesPerRow;
+    constexpr int kInstr = kRows / (4 * kRowsPerInstr);  // rows of a wave per pass, in instructions
+    constexpr int kBatch = kInstr < 8 ? kInstr : 8;
     T *dp = static_cast<T *>(g.d);
     const T *ap = static_cast<const T *>(g.addend);
     const int chunk = lane % kLanesPerRow;
     const int64_t gcol = col0 + chunk * kPer16;
+    const int64_t acol = gcol < g.C ? gcol : 0;          // C is a multiple of 8
+    u32x4_t add[2][kBatch];
+    auto fetch = [&](u32x4_t(&to)[kBatch], int pass, int batch) __attribute__((always_inline)) {
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        int64_t grow = row0 + pass * (BM / 2) + ((batch * kBatch + b) * 4 + wave) * kRowsPerInstr + lane / kLanesPerRow;
+        if (grow >= g.M) grow = g.M - 1;
+        to[b] = *reinterpret_cast<const u32x4_t *>(ap + grow * g.C + acol);
+      }
+    };
 #pragma unroll
     for (int pass = 0; pass < 2 / kPassHalves; ++pass) {
       if (pass > 0) __syncthreads();
+      if constexpr (kAdd) fetch(add[0], pass, 0);
 #pragma unroll
       for (int hh = 0; hh < kPassHalves; ++hh)
 #pragma unroll
@@ -249,32 +266,37 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
                     from_f32<T>(acc[pass * kPassHalves + hh][q][i][c][r]);
               }
       __syncthreads();
-      constexpr int kRows = kPassHalves * (BM / 2);
-      constexpr int kRowsPerInstr = 64 / kLanesPerRow;
-#pragma unroll 4
-      for (int it = 0; it < kRows / (4 * kRowsPerInstr); ++it) {
-        const int lrow = (it * 4 + wave) * kRowsPerInstr + lane / kLanesPerRow;
-        const int64_t grow = row0 + pass * (BM / 2) + lrow;
-        if (grow >= g.M || gcol >= g.C) continue;        // C is a multiple of 8
-        u32x4_t v = *reinterpret_cast<const u32x4_t *>(smem + lrow * kPitch + chunk * 16);
-        const int64_t o = grow * g.C + gcol;
-        if (ap) {
-          const u32x4_t av = *reinterpret_cast<const u32x4_t *>(ap + o);
-          const T *vp = reinterpret_cast<const T *>(&v);
-          const T *aq = reinterpret_cast<const T *>(&av);
-          u32x4_t w;
-          T *wp = reinterpret_cast<T *>(&w);
 #pragma unroll
-          for (int e = 0; e < kPer16; ++e) wp[e] = from_f32<T>(to_f32<T>(vp[e]) + to_f32<T>(aq[e]));
-          v = w;
+      for (int batch = 0; batch < kInstr / kBatch; ++batch) {
+        if constexpr (kAdd) {
+          if (batch + 1 < kInstr / kBatch) fetch(add[(batch + 1) & 1], pass, batch + 1);
         }
-        *reinterpret_cast<u32x4_t *>(dp + o) = v;
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+          const int lrow = ((batch * kBatch + b) * 4 + wave) * kRowsPerInstr + lane / kLanesPerRow;
+          const int64_t grow = row0 + pass * (BM / 2) + lrow;
+          u32x4_t v = *reinterpret_cast<const u32x4_t *>(smem + lrow * kPitch + chunk * 16);
+          if constexpr (kAdd) {
+            const T *vp = reinterpret_cast<const T *>(&v);
+            const T *aq = reinterpret_cast<const T *>(&add[batch & 1][b]);
+            u32x4_t w;
+            T *wp = reinterpret_cast<T *>(&w);
+#pragma unroll
+            for (int e = 0; e < kPer16; ++e) wp[e] = from_f32<T>(to_f32<T>(vp[e]) + to_f32<T>(aq[e]));
+            v = w;
+          }
+          if (grow < g.M && gcol < g.C) *reinterpret_cast<u32x4_t *>(dp + grow * g.C + gcol) = v;
+        }
       }
     }
   };
-  if (g.d_dtype == CAIFX_BF16) store(bf16_t{});
-  else if (g.d_dtype == CAIFX_F16) store(f16_t{});
-  else store(float{});
+  auto store_as = [&](auto type_) __attribute__((always_inline)) {
+    if (g.addend) store(type_, std::true_type{});
+    else store(type_, std::false_type{});
+  };
+  if (g.d_dtype == CAIFX_BF16) store_as(bf16_t{});
+  else if (g.d_dtype == CAIFX_F16) store_as(f16_t{});
+  else store_as(float{});
 }
 
 // ------------------------------------------------------------------ the weight as a dense matrix of the compute type
