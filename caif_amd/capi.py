@@ -14,6 +14,7 @@ W_INT8, W_INT4_GROUP, W_F32, W_F16, W_BF16 = 0, 1, 2, 3, 4
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libcaifx.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "caifx_torch_calls.so")
 CSRC = os.path.join(_HERE, "csrc")
 
 EXPORTS = [
@@ -111,6 +112,33 @@ def lib():
         L.caifx_moe_dispatch_backward.argtypes = [_p, _p, _p, _p, _p, _i64, _i64, _int, _int, _int, _p]
         _lib = L
     return _lib
+
+
+def addresses():
+    """Entry point name -> address in the loaded library."""
+    L = lib()
+    return {name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value for name in EXPORTS}
+
+
+_calls = None
+
+
+def calls():
+    """The native side of torch_ops (csrc/torch_calls.cpp), bound to the loaded library.  Raises if it has not been
+    built: there is no Python form of that work."""
+    global _calls
+    if _calls is None:
+        if not os.path.exists(CALLS_PATH):
+            raise RuntimeError(
+                f"{CALLS_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`.")
+        import importlib.util
+        import torch  # noqa: F401  (its libraries are what the module links against)
+        spec = importlib.util.spec_from_file_location("caifx_torch_calls", CALLS_PATH)
+        m = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(m)
+        m.bind(addresses())
+        _calls = m
+    return _calls
 
 
 def status_string(status):

@@ -1,7 +1,8 @@
 """Thin callers of the C ABI for torch-owned device buffers (tests and bench.py plumbing).
 
 torch supplies device memory and the current HIP stream; every computation is a
-call into libcaifx.so.  Function names follow the reference's CAIF_Ops entry
+call into libcaifx.so.  The calls of a training or serving step go through native code
+(csrc/torch_calls.cpp: checks, result and workspace allocation, stream), the rest through ctypes.  Function names follow the reference's CAIF_Ops entry
 points (src/caif_ops.cpp:504-680); argument meaning is the same.
 """
 import torch
@@ -120,30 +121,28 @@ class FrozenWeight:
         self.N, self.K, self.scale_period, self.group_size = N, K, scale_period, group_size
 
 
-def _workspace(nbytes, device):
-    return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+_native = None
+
+
+def _calls():
+    global _native
+    if _native is None:
+        _native = capi.calls()
+    return _native
+
+
+def _done(r, name):
+    """The native call's result; a status other than CAIFX_OK comes back as an int."""
+    if r.__class__ is int:
+        capi.check(r, name)
+    return r
 
 
 def qlinear_forward(x, fw, compute_dtype, y_dtype=F32, out=None, workspace=None, addend=None):
     """caifx_qlinear_forward on x [..., K]; returns y [M, N].  With `addend` [M, N] of y_dtype:
     caifx_qlinear_forward_add, y = T(float(T(x W^T)) + float(addend))."""
-    _need_cuda(x)
-    M = x.numel() // fw.K
-    y = out if out is not None else torch.empty((M, fw.N), dtype=TORCH_DTYPE[y_dtype], device=x.device)
-    xd = CODE_OF[x.dtype]
-    if workspace is None:
-        workspace = _workspace(capi.lib().caifx_qlinear_workspace_bytes(M, fw.N, fw.K, xd, compute_dtype,
-                                                                       fw.w_kind, 0), x.device)
-    if addend is not None:
-        assert addend.dtype == y.dtype and addend.numel() == y.numel()
-        capi.call("caifx_qlinear_forward_add", M, fw.N, fw.K, _ptr(x), xd, compute_dtype, _ptr(fw.wq), fw.w_kind,
-                  _ptr(fw.scales), fw.scale_period, fw.group_size, _ptr(y), y_dtype, _ptr(addend), _ptr(workspace),
-                  workspace.numel(), _stream())
-        return y
-    capi.call("caifx_qlinear_forward", M, fw.N, fw.K, _ptr(x), xd, compute_dtype, _ptr(fw.wq), fw.w_kind,
-              _ptr(fw.scales), fw.scale_period, fw.group_size, _ptr(y), y_dtype, _ptr(workspace),
-              workspace.numel(), _stream())
-    return y
+    return _done((_native or _calls()).qlinear(0, x, fw, compute_dtype, y_dtype, out, workspace, addend),
+                 "caifx_qlinear_forward")
 
 
 def probe_mfma_bf16(a_values, b_values, iters):
@@ -162,23 +161,8 @@ def probe_mfma_bf16(a_values, b_values, iters):
 
 def qlinear_backward_input(dy, fw, compute_dtype, dx_dtype=F32, out=None, workspace=None, addend=None):
     """caifx_qlinear_backward_input on dy [..., N]; returns dx [M, K] (plus `addend` [M, K], see qlinear_forward)."""
-    _need_cuda(dy)
-    M = dy.numel() // fw.N
-    dx = out if out is not None else torch.empty((M, fw.K), dtype=TORCH_DTYPE[dx_dtype], device=dy.device)
-    yd = CODE_OF[dy.dtype]
-    if workspace is None:
-        workspace = _workspace(capi.lib().caifx_qlinear_workspace_bytes(M, fw.N, fw.K, yd, compute_dtype,
-                                                                       fw.w_kind, 1), dy.device)
-    if addend is not None:
-        assert addend.dtype == dx.dtype and addend.numel() == dx.numel()
-        capi.call("caifx_qlinear_backward_input_add", M, fw.N, fw.K, _ptr(dy), yd, compute_dtype, _ptr(fw.wq),
-                  fw.w_kind, _ptr(fw.scales), fw.scale_period, fw.group_size, _ptr(dx), dx_dtype, _ptr(addend),
-                  _ptr(workspace), workspace.numel(), _stream())
-        return dx
-    capi.call("caifx_qlinear_backward_input", M, fw.N, fw.K, _ptr(dy), yd, compute_dtype, _ptr(fw.wq),
-              fw.w_kind, _ptr(fw.scales), fw.scale_period, fw.group_size, _ptr(dx), dx_dtype,
-              _ptr(workspace), workspace.numel(), _stream())
-    return dx
+    return _done((_native or _calls()).qlinear(1, dy, fw, compute_dtype, dx_dtype, out, workspace, addend),
+                 "caifx_qlinear_backward_input")
 
 
 class GroupedFrozenWeights:
@@ -208,38 +192,15 @@ def _check_grouped(x, in_dim, rows, offsets, E, results, out_dim, out_dtype):
             raise ValueError(f"result / gating tensors must be {out_dtype} with {rows} x {out_dim} elements")
 
 
-def _grouped(name, backward, x, offsets, gw, compute_dtype, out_dtype, out, workspace, addend=None):
-    _need_cuda(x, offsets)
-    in_dim = gw.N if backward else gw.K
-    out_dim = gw.K if backward else gw.N
-    rows = x.numel() // in_dim
-    y = out if out is not None else torch.zeros((rows, out_dim), dtype=TORCH_DTYPE[out_dtype], device=x.device)
-    xd = CODE_OF[x.dtype]
-    E = len(gw.weights)
-    _check_grouped(x, in_dim, rows, offsets, E, (y,), out_dim, TORCH_DTYPE[out_dtype])
-    if workspace is None:
-        workspace = _workspace(capi.lib().caifx_qlinear_grouped_workspace_bytes(
-            E, rows, gw.N, gw.K, xd, compute_dtype, gw.w_kind, int(backward)), x.device)
-    if addend is not None:
-        assert addend.dtype == y.dtype and addend.numel() == y.numel()
-        capi.call(name + "_add", E, _ptr(offsets), rows, gw.N, gw.K, _ptr(x), xd, compute_dtype, _ptr(gw.wq_ptrs),
-                  gw.w_kind, _ptr(gw.scales_ptrs), gw.scale_period, gw.group_size, _ptr(y), out_dtype, _ptr(addend),
-                  _ptr(workspace), workspace.numel(), _stream())
-        return y
-    capi.call(name, E, _ptr(offsets), rows, gw.N, gw.K, _ptr(x), xd, compute_dtype, _ptr(gw.wq_ptrs), gw.w_kind,
-              _ptr(gw.scales_ptrs), gw.scale_period, gw.group_size, _ptr(y), out_dtype, _ptr(workspace),
-              workspace.numel(), _stream())
-    return y
-
-
 def qlinear_grouped_forward(x, offsets, gw, compute_dtype, y_dtype=F32, out=None, workspace=None):
-    return _grouped("caifx_qlinear_grouped_forward", False, x, offsets, gw, compute_dtype, y_dtype, out, workspace)
+    return _done((_native or _calls()).grouped(0, x, offsets, gw, compute_dtype, y_dtype, out, workspace, None),
+                 "caifx_qlinear_grouped_forward")
 
 
 def qlinear_grouped_backward_input(dy, offsets, gw, compute_dtype, dx_dtype=F32, out=None, workspace=None,
                                    addend=None):
-    return _grouped("caifx_qlinear_grouped_backward_input", True, dy, offsets, gw, compute_dtype, dx_dtype, out,
-                    workspace, addend)
+    return _done((_native or _calls()).grouped(1, dy, offsets, gw, compute_dtype, dx_dtype, out, workspace, addend),
+                 "caifx_qlinear_grouped_backward_input")
 
 
 def qlinear_grouped_forward_swiglu(x, offsets, gw_up, gate, compute_dtype, out=None):
@@ -268,119 +229,67 @@ def qlinear_grouped_backward_input_swiglu(dy, offsets, gw_down, gate, up, comput
 
 
 # ------------------------------------------------------------------ element-wise
-def _ew(name, n_in, a, b=None, out=None):
-    _need_cuda(a, b, out)
-    if out is None:
-        out = torch.empty_like(a)
-    elif out.dtype != a.dtype or out.numel() != a.numel() or not out.is_contiguous():
-        raise ValueError("out must be a contiguous tensor of the input's dtype and size")
-    dt = CODE_OF[a.dtype]
-    if n_in == 1:
-        capi.call(name, _ptr(a), _ptr(out), a.numel(), dt, _stream())
-    else:
-        capi.call(name, _ptr(a), _ptr(b), _ptr(out), a.numel(), dt, _stream())
-    return out
+def _ew(op, name, a, b=None, out=None):
+    return _done((_native or _calls()).elementwise(op, a, b, out), name)
 
 
 def silu(x):
-    return _ew("caifx_silu", 1, x)
+    return _ew(0, "caifx_silu", x)
 
 
 def silu_backward(x, grad_out):
-    return _ew("caifx_silu_backward", 2, x, grad_out)
+    return _ew(1, "caifx_silu_backward", x, grad_out)
 
 
 def multiply(a, b):
-    return _ew("caifx_multiply", 2, a, b)
+    return _ew(2, "caifx_multiply", a, b)
 
 
 def add(a, b):
-    return _ew("caifx_add", 2, a, b)
+    return _ew(3, "caifx_add", a, b)
 
 
 def silu_multiply(gate, up, out=None):
-    return _ew("caifx_silu_multiply", 2, gate, up, out)
+    return _ew(4, "caifx_silu_multiply", gate, up, out)
 
 
 def swiglu_backward(gate, up, grad_hidden, out_gate=None, out_up=None):
     """(grad_gate, grad_up) of hidden = silu(gate) * up in one pass, bit-identical to
     multiply(grad_hidden, silu(gate)) and silu_backward(gate, multiply(grad_hidden, up))."""
-    _need_cuda(gate, up, grad_hidden)
-    assert gate.shape == up.shape == grad_hidden.shape and gate.dtype == up.dtype == grad_hidden.dtype
-    grad_gate = torch.empty_like(gate) if out_gate is None else out_gate
-    grad_up = torch.empty_like(gate) if out_up is None else out_up
-    capi.call("caifx_swiglu_backward", _ptr(gate), _ptr(up), _ptr(grad_hidden), _ptr(grad_gate), _ptr(grad_up),
-              gate.numel(), CODE_OF[gate.dtype], _stream())
-    return grad_gate, grad_up
+    return _done((_native or _calls()).swiglu_backward(gate, up, grad_hidden, out_gate, out_up), "caifx_swiglu_backward")
 
 
 # ------------------------------------------------------------------ MoE token routing
 def moe_build_dispatch_map(expert_indices, num_experts, capacity_per_expert=0):
     """(dispatch_map [T, top_k] int32, expert_offsets [E+1] int32), built on the device without a host
     round trip; expert_offsets[-1] is the number of assigned rows."""
-    _need_cuda(expert_indices)
-    assert expert_indices.dtype == torch.int32 and expert_indices.dim() == 2
-    T_, top_k = expert_indices.shape
-    dmap = torch.empty_like(expert_indices)
-    offsets = torch.empty(num_experts + 1, dtype=torch.int32, device=expert_indices.device)
-    nb = capi.lib().caifx_moe_dispatch_map_workspace_bytes(T_, top_k, num_experts)
-    ws = torch.empty(max(nb, 4 * num_experts), dtype=torch.uint8, device=expert_indices.device)
-    capi.call("caifx_moe_build_dispatch_map", _ptr(expert_indices), T_, top_k, num_experts, capacity_per_expert,
-              _ptr(dmap), _ptr(offsets), _ptr(ws), ws.numel(), _stream())
-    return dmap, offsets
+    return _done((_native or _calls()).moe_build_dispatch_map(expert_indices, num_experts, capacity_per_expert),
+                 "caifx_moe_build_dispatch_map")
 
 
 def moe_dispatch(x, expert_indices, dispatch_map, expert_offsets, total_rows, out=None):
-    _need_cuda(x, expert_indices, dispatch_map, expert_offsets)
-    T_, dim = x.shape
-    top_k = expert_indices.shape[1]
-    buf = out if out is not None else torch.zeros((total_rows, dim), dtype=x.dtype, device=x.device)
-    capi.call("caifx_moe_dispatch", _ptr(x), _ptr(expert_indices), _ptr(dispatch_map), _ptr(expert_offsets), _ptr(buf),
-              T_, dim, top_k, expert_offsets.numel() - 1, CODE_OF[x.dtype], _stream())
-    return buf
+    return _done((_native or _calls()).moe_dispatch(x, expert_indices, dispatch_map, expert_offsets, total_rows, out),
+                 "caifx_moe_dispatch")
 
 
 def moe_combine(expert_buffer, expert_indices, expert_weights, dispatch_map, expert_offsets, out=None):
-    _need_cuda(expert_buffer, expert_indices, expert_weights, dispatch_map, expert_offsets)
-    T_, top_k = expert_indices.shape
-    dim = expert_buffer.shape[1]
-    y = out if out is not None else torch.empty((T_, dim), dtype=expert_buffer.dtype, device=expert_buffer.device)
-    capi.call("caifx_moe_combine", _ptr(expert_buffer), _ptr(expert_indices), _ptr(expert_weights), _ptr(dispatch_map),
-              _ptr(expert_offsets), _ptr(y), T_, dim, top_k, expert_offsets.numel() - 1, CODE_OF[expert_buffer.dtype],
-              _stream())
-    return y
+    return _done((_native or _calls()).moe_combine(expert_buffer, expert_indices, expert_weights, dispatch_map,
+                                                   expert_offsets, out), "caifx_moe_combine")
 
 
 def moe_combine_backward_grad_expert(grad_output, expert_indices, expert_weights, dispatch_map, expert_offsets,
                                      total_rows, out=None):
-    _need_cuda(grad_output, expert_indices, expert_weights, dispatch_map, expert_offsets)
-    T_, dim = grad_output.shape
-    top_k = expert_indices.shape[1]
-    gb = out if out is not None else torch.zeros((total_rows, dim), dtype=grad_output.dtype, device=grad_output.device)
-    capi.call("caifx_moe_combine_backward_grad_expert", _ptr(grad_output), _ptr(expert_indices), _ptr(expert_weights),
-              _ptr(dispatch_map), _ptr(expert_offsets), _ptr(gb), T_, dim, top_k, expert_offsets.numel() - 1,
-              CODE_OF[grad_output.dtype], _stream())
-    return gb
+    return _done((_native or _calls()).moe_combine_backward_grad_expert(
+        grad_output, expert_indices, expert_weights, dispatch_map, expert_offsets, total_rows, out),
+        "caifx_moe_combine_backward_grad_expert")
 
 
 def moe_dispatch_backward(grad_expert_buffer, expert_indices, dispatch_map, expert_offsets, out=None):
-    _need_cuda(grad_expert_buffer, expert_indices, dispatch_map, expert_offsets)
-    T_, top_k = expert_indices.shape
-    dim = grad_expert_buffer.shape[1]
-    gi = out if out is not None else torch.empty((T_, dim), dtype=grad_expert_buffer.dtype,
-                                                 device=grad_expert_buffer.device)
-    capi.call("caifx_moe_dispatch_backward", _ptr(grad_expert_buffer), _ptr(expert_indices), _ptr(dispatch_map),
-              _ptr(expert_offsets), _ptr(gi), T_, dim, top_k, expert_offsets.numel() - 1,
-              CODE_OF[grad_expert_buffer.dtype], _stream())
-    return gi
+    return _done((_native or _calls()).moe_dispatch_backward(grad_expert_buffer, expert_indices, dispatch_map,
+                                                             expert_offsets, out), "caifx_moe_dispatch_backward")
 
 
 def moe_combine_backward_grad_weights(grad_output, expert_buffer, expert_indices, dispatch_map, expert_offsets):
-    _need_cuda(grad_output, expert_buffer, expert_indices, dispatch_map, expert_offsets)
-    T_, top_k = expert_indices.shape
-    dim = grad_output.shape[1]
-    gw = torch.empty((T_, top_k), dtype=grad_output.dtype, device=grad_output.device)
-    capi.call("caifx_moe_combine_backward_grad_weights", _ptr(grad_output), _ptr(expert_buffer), _ptr(expert_indices),
-              _ptr(dispatch_map), _ptr(expert_offsets), _ptr(gw), T_, dim, top_k, expert_offsets.numel() - 1,
-              CODE_OF[grad_output.dtype], _stream())
-    return gw
+    return _done((_native or _calls()).moe_combine_backward_grad_weights(
+        grad_output, expert_buffer, expert_indices, dispatch_map, expert_offsets),
+        "caifx_moe_combine_backward_grad_weights")
