@@ -28,7 +28,8 @@ namespace {
   X(caifx_qlinear_grouped_workspace_bytes) X(caifx_silu) X(caifx_silu_backward) X(caifx_multiply) X(caifx_add)           \
   X(caifx_silu_multiply) X(caifx_swiglu_backward) X(caifx_moe_dispatch_map_workspace_bytes)                              \
   X(caifx_moe_build_dispatch_map) X(caifx_moe_dispatch) X(caifx_moe_combine) X(caifx_moe_combine_backward_grad_expert)   \
-  X(caifx_moe_combine_backward_grad_weights) X(caifx_moe_dispatch_backward)
+  X(caifx_moe_combine_backward_grad_weights) X(caifx_moe_dispatch_backward) X(caifx_quantize_int8_per_channel)           \
+  X(caifx_quantize_int8_per_tensor) X(caifx_quantize_to_int4)
 
 struct Api {
 #define X(name) decltype(&::name) name = nullptr;
@@ -297,6 +298,53 @@ PyObject *grouped(PyObject *, PyObject *const *a, Py_ssize_t n)
   });
 }
 
+PyObject *pair(int status, const at::Tensor &x, const at::Tensor &y)
+{
+  if (status != CAIFX_OK) return PyLong_FromLong(status);
+  Owned p(THPVariable_Wrap(x)), q(THPVariable_Wrap(y));
+  return PyTuple_Pack(2, p.p, q.p);
+}
+
+// ------------------------------------------------------------------ quantise
+// quantize_int8(x, per_channel) -> (codes, scales) or status
+PyObject *quantize_int8(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+  return guarded(n, 2, [&]() -> PyObject * {
+    const at::Tensor &x = device_tensor(a[0]);
+    if (x.scalar_type() != at::kFloat) throw Error{PyExc_RuntimeError, "QuantizeInt8: input must be fp32"};
+    const int per_channel = PyObject_IsTrue(a[1]);
+    if (per_channel < 0) throw Error{nullptr, nullptr};
+    if (per_channel && x.dim() != 2) throw Error{PyExc_RuntimeError, "QuantizeInt8 PerChannel: input must be 2D"};
+    const at::Tensor q = at::empty(x.sizes(), x.options().dtype(at::kChar));
+    const at::Tensor s = at::empty({per_channel ? x.size(1) : 1}, x.options());
+    const auto in = static_cast<const float *>(x.data_ptr());
+    if (!per_channel) return pair(launch([&] { return api.caifx_quantize_int8_per_tensor(in, q.data_ptr(), s.data_ptr(), x.numel(), stream()); }), q, s);
+    const int64_t rows = x.size(0), cols = x.size(1);
+    if (rows > INT32_MAX || cols > INT32_MAX) throw Error{PyExc_OverflowError, "QuantizeInt8 PerChannel: too many rows or columns"};
+    return pair(launch([&] {
+      return api.caifx_quantize_int8_per_channel(in, q.data_ptr(), s.data_ptr(), static_cast<int>(rows), static_cast<int>(cols), stream());
+    }), q, s);
+  });
+}
+
+// quantize_int4(x, group_size) -> (packed, fp16 scales) or status
+PyObject *quantize_int4(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+  return guarded(n, 2, [&]() -> PyObject * {
+    const at::Tensor &x = device_tensor(a[0]);
+    if (x.scalar_type() != at::kFloat) throw Error{PyExc_RuntimeError, "QuantizeInt4PerGroup: input must be fp32"};
+    const int64_t group = integer(a[1]), count = x.numel();
+    if (group == 0) throw Error{PyExc_RuntimeError, "QuantizeInt4PerGroup: group_size must be > 0"};
+    if (group > INT32_MAX || group < INT32_MIN) throw Error{PyExc_OverflowError, "QuantizeInt4PerGroup: group_size out of range"};
+    const int64_t groups = group > 0 ? (count + group - 1) / group : 0;      // a negative size is the library's error
+    const at::Tensor packed = at::empty({(count + 1) / 2}, x.options().dtype(at::kByte));
+    const at::Tensor s = at::empty({groups}, x.options().dtype(at::kHalf));
+    return pair(launch([&] {
+      return api.caifx_quantize_to_int4(static_cast<const float *>(x.data_ptr()), packed.data_ptr(), s.data_ptr(), count, static_cast<int>(group), stream());
+    }), packed, s);
+  });
+}
+
 // ------------------------------------------------------------------ element-wise
 // elementwise(op, a, b or None, out or None): 0 silu, 1 silu_backward, 2 multiply, 3 add, 4 silu_multiply
 PyObject *elementwise(PyObject *, PyObject *const *a, Py_ssize_t n)
@@ -340,13 +388,6 @@ PyObject *swiglu_backward(PyObject *, PyObject *const *a, Py_ssize_t n)
 }
 
 // ------------------------------------------------------------------ MoE token routing
-PyObject *pair(int status, const at::Tensor &x, const at::Tensor &y)
-{
-  if (status != CAIFX_OK) return PyLong_FromLong(status);
-  Owned p(THPVariable_Wrap(x)), q(THPVariable_Wrap(y));
-  return PyTuple_Pack(2, p.p, q.p);
-}
-
 // moe_build_dispatch_map(expert_indices, num_experts, capacity) -> (map, offsets) or status
 PyObject *moe_build_dispatch_map(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
@@ -440,7 +481,7 @@ PyObject *moe_combine_backward_grad_weights(PyObject *, PyObject *const *a, Py_s
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, nullptr},
 #define M(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr},
-    M(qlinear) M(grouped) M(elementwise) M(swiglu_backward) M(moe_build_dispatch_map) M(moe_dispatch) M(moe_combine)
+    M(qlinear) M(grouped) M(quantize_int8) M(quantize_int4) M(elementwise) M(swiglu_backward) M(moe_build_dispatch_map) M(moe_dispatch) M(moe_combine)
     M(moe_combine_backward_grad_expert) M(moe_dispatch_backward) M(moe_combine_backward_grad_weights)
 #undef M
     {nullptr, nullptr, 0, nullptr}};

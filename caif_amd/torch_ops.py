@@ -31,23 +31,28 @@ def _need_cuda(*ts):
             raise RuntimeError("tensor must be contiguous")
 
 
+_native = None
+
+
+def _calls():
+    global _native
+    if _native is None:
+        _native = capi.calls()
+    return _native
+
+
+def _done(r, name):
+    """The native call's result; a status other than CAIFX_OK comes back as an int."""
+    if r.__class__ is int:
+        capi.check(r, name)
+    return r
+
+
 # ------------------------------------------------------------------ CAIF_Ops::Quantize* / Dequantize*
 def quantize_int8(x, per_channel):
     """CAIF_Ops::QuantizeInt8 (src/caif_ops_device.cpp:1517-1573).  Returns (codes, scales)."""
-    _need_cuda(x)
-    if x.dtype != torch.float32:
-        raise RuntimeError("QuantizeInt8: input must be fp32")
-    q = torch.empty(x.shape, dtype=torch.int8, device=x.device)
-    if not per_channel:
-        s = torch.empty(1, dtype=torch.float32, device=x.device)
-        capi.call("caifx_quantize_int8_per_tensor", _ptr(x), _ptr(q), _ptr(s), x.numel(), _stream())
-        return q, s
-    if x.dim() != 2:
-        raise RuntimeError("QuantizeInt8 PerChannel: input must be 2D")
-    rows, cols = x.shape
-    s = torch.empty(cols, dtype=torch.float32, device=x.device)
-    capi.call("caifx_quantize_int8_per_channel", _ptr(x), _ptr(q), _ptr(s), rows, cols, _stream())
-    return q, s
+    return _done((_native or _calls()).quantize_int8(x, per_channel),
+                 "caifx_quantize_int8_per_channel" if per_channel else "caifx_quantize_int8_per_tensor")
 
 
 def dequantize_int8(q, scales, per_channel):
@@ -70,16 +75,7 @@ def dequantize_int8(q, scales, per_channel):
 
 def quantize_int4_per_group(x, group_size):
     """CAIF_Ops::QuantizeInt4PerGroup (src/caif_ops_device.cpp:1651-1687).  Returns (packed, fp16 scales)."""
-    _need_cuda(x)
-    if x.dtype != torch.float32:
-        raise RuntimeError("QuantizeInt4PerGroup: input must be fp32")
-    if group_size == 0:
-        raise RuntimeError("QuantizeInt4PerGroup: group_size must be > 0")
-    n = x.numel()
-    packed = torch.empty((n + 1) // 2, dtype=torch.uint8, device=x.device)
-    scales = torch.empty((n + group_size - 1) // group_size, dtype=torch.float16, device=x.device)
-    capi.call("caifx_quantize_to_int4", _ptr(x), _ptr(packed), _ptr(scales), n, group_size, _stream())
-    return packed, scales
+    return _done((_native or _calls()).quantize_int4(x, group_size), "caifx_quantize_to_int4")
 
 
 def dequantize_int4_per_group(packed, scales, n, group_size):
@@ -119,23 +115,6 @@ class FrozenWeight:
     def __init__(self, wq, w_kind, scales, N, K, scale_period=1, group_size=128):
         self.wq, self.w_kind, self.scales = wq, w_kind, scales
         self.N, self.K, self.scale_period, self.group_size = N, K, scale_period, group_size
-
-
-_native = None
-
-
-def _calls():
-    global _native
-    if _native is None:
-        _native = capi.calls()
-    return _native
-
-
-def _done(r, name):
-    """The native call's result; a status other than CAIFX_OK comes back as an int."""
-    if r.__class__ is int:
-        capi.check(r, name)
-    return r
 
 
 def qlinear_forward(x, fw, compute_dtype, y_dtype=F32, out=None, workspace=None, addend=None):

@@ -1,0 +1,29 @@
+"""Per-column int8 quantisation around the edges of its workgroups (256 columns, chunks of 32 to 256 rows whose partial
+maxima wait in the codes' memory, 64-row blocks), bit-exact against the oracle (src/caif_cuda_kernels_quant.cu:515-560)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from caif_amd import torch_ops as T                                  # noqa: E402
+from gpu_helpers import dev                                           # noqa: E402
+
+
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 31, 32, 33, 63, 65, 257, 1031])
+@pytest.mark.parametrize("cols", [3, 4, 8, 252, 256, 260, 1028])
+def test_bit_exact(orc, rows, cols):
+    rng = np.random.default_rng(rows * 2000 + cols)
+    w = rng.normal(0, 0.02, (rows, cols)).astype(np.float32)
+    w[:, 0] = 0.0                                      # a column without a maximum: scale 1
+    w[rows - 1, cols - 1] = -3.0                        # the maxima of the last row and the last column count
+    w[rows // 2, cols // 2] = 2.0
+    q, s = T.quantize_int8(dev(w), True)
+    qo, so = orc.quantize_int8_per_channel(w)
+    assert np.array_equal(s.cpu().numpy(), so) and np.array_equal(q.cpu().numpy(), qo)
+    # a source that is not 16-byte aligned takes the element-wise kernels: same bits
+    buf = torch.empty(rows * cols + 1, dtype=torch.float32, device="cuda")
+    x = buf[1:].reshape(rows, cols)
+    x.copy_(dev(w))
+    q2, s2 = T.quantize_int8(x, True)
+    assert torch.equal(q2, q) and torch.equal(s2, s)
