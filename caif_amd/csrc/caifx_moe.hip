@@ -280,9 +280,17 @@ __global__ __launch_bounds__(kRouteThreads) void combine_bwd_kernel(const T *gou
   }
 }
 
-// one wave per token: out[t] = T(sum_k w[t,k] * buf[row(t,k)])  (kWeighted) or T(sum_k buf[row(t,k)]);
-// per element the additions run over k in order.  The rows and weights of a token are fetched once per
-// batch of 8 assignments by lanes 0..7 and broadcast.
+// out[t] = T(sum_k w[t,k] * buf[row(t,k)])  (kWeighted) or T(sum_k buf[row(t,k)]); per element the additions run over k in
+// order.  A wave takes one 64-lane piece of a token's row (and every gather_waves-th after it), so that a decode step's few
+// tokens still spread over the chip, and asks for the pieces of up to eight rows before it adds the first: with one wave per
+// token and one row at a time 16 tokens of 2048 took 14.4 us, a chain of 24 memory round trips.
+// The rows and weights of a token are fetched once per batch of 8 assignments by lanes 0..7 and broadcast.
+constexpr int kGatherWavesMax = 8;
+__host__ __device__ inline int gather_waves(int64_t dim, int n)
+{
+  const int64_t pieces = (dim + 64 * n - 1) / (64 * n);
+  return pieces < kGatherWavesMax ? static_cast<int>(pieces) : kGatherWavesMax;
+}
 template <typename T, bool kWeighted, bool kVec>
 __global__ __launch_bounds__(kRouteThreads) void gather_sum_kernel(const T *buf, const int32_t *idx, const T *w,
                                                                     const int32_t *map, const int32_t *offsets, T *out,
@@ -292,9 +300,11 @@ __global__ __launch_bounds__(kRouteThreads) void gather_sum_kernel(const T *buf,
   constexpr int n = kVec ? Vec16<T>::kN : 1;
   typedef typename Vec16<T>::type v_t;
   const int lane = threadIdx.x & 63;
-  const int64_t t = (static_cast<int64_t>(blockIdx.x) * kRouteThreads + threadIdx.x) >> 6;
+  const int per_token = gather_waves(dim, n);
+  const int64_t wave = (static_cast<int64_t>(blockIdx.x) * kRouteThreads + threadIdx.x) >> 6;
+  const int64_t t = wave / per_token;
   if (t >= num_tokens) return;
-  for (int64_t d0 = 0; d0 < dim; d0 += 64 * n) {          // the whole wave walks the row together
+  for (int64_t d0 = (wave - t * per_token) * 64 * n; d0 < dim; d0 += static_cast<int64_t>(per_token) * 64 * n) {
     const int64_t d = d0 + static_cast<int64_t>(lane) * n;
     float sum[n];
 #pragma unroll
@@ -307,22 +317,24 @@ __global__ __launch_bounds__(kRouteThreads) void gather_sum_kernel(const T *buf,
         my_row = routed_row(idx, map, offsets, a, num_experts);
         if constexpr (kWeighted) my_w = to_f32<T>(w[a]);
       }
-      const int kn = top_k - k0 < 8 ? top_k - k0 : 8;
-      for (int k = 0; k < kn; ++k) {
-        const int64_t row = __shfl(my_row, k, 64);
-        const float wt = __shfl(my_w, k, 64);
-        if (row < 0 || d >= dim) continue;
-        if constexpr (kVec) {
-          const v_t v = *reinterpret_cast<const v_t *>(buf + row * dim + d);
+      int64_t row[8];
+      v_t v[8];          // (element 0 alone when not kVec)
 #pragma unroll
-          for (int i = 0; i < n; ++i) {
-            if constexpr (kWeighted) sum[i] = __builtin_fmaf(wt, to_f32<T>(v[i]), sum[i]);
-            else sum[i] += to_f32<T>(v[i]);
-          }
-        } else {
-          const float v = to_f32<T>(buf[row * dim + d]);
-          if constexpr (kWeighted) sum[0] = __builtin_fmaf(wt, v, sum[0]);
-          else sum[0] += v;
+      for (int k = 0; k < 8; ++k) {
+        row[k] = __shfl(my_row, k, 64);          // -1 past top_k
+        if (row[k] >= 0 && d < dim) {
+          if constexpr (kVec) v[k] = *reinterpret_cast<const v_t *>(buf + row[k] * dim + d);
+          else v[k][0] = buf[row[k] * dim + d];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const float wt = __shfl(my_w, k, 64);
+        if (row[k] < 0 || d >= dim) continue;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+          if constexpr (kWeighted) sum[i] = __builtin_fmaf(wt, to_f32<T>(v[k][i]), sum[i]);
+          else sum[i] += to_f32<T>(v[k][i]);
         }
       }
     }
@@ -356,7 +368,29 @@ __global__ __launch_bounds__(kRouteThreads) void combine_bwd_weights_kernel(cons
   if (row >= 0) {
     const T *g = gout + (a / top_k) * dim;
     const T *b = buf + row * dim;
-    for (int64_t d = lane; d < dim; d += 64) sum = __builtin_fmaf(to_f32<T>(g[d]), to_f32<T>(b[d]), sum);
+    int64_t d = lane;
+    // sixteen pairs asked for before the first is added: the order of the additions is a chain, the loads need not be
+    for (; d - lane + 16 * 64 <= dim; d += 16 * 64) {
+      T x[16], y[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        x[i] = g[d + 64 * i];
+        y[i] = b[d + 64 * i];
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum = __builtin_fmaf(to_f32<T>(x[i]), to_f32<T>(y[i]), sum);
+    }
+    for (; d - lane + 4 * 64 <= dim; d += 4 * 64) {
+      T x[4], y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = g[d + 64 * i];
+        y[i] = b[d + 64 * i];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum = __builtin_fmaf(to_f32<T>(x[i]), to_f32<T>(y[i]), sum);
+    }
+    for (; d < dim; d += 64) sum = __builtin_fmaf(to_f32<T>(g[d]), to_f32<T>(b[d]), sum);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
   }
@@ -468,9 +502,9 @@ int caifx_moe_combine(const void *expert_buffer, const int32_t *expert_indices, 
                              num_experts, dtype);
   if (st >= 0) return st;
   if (!expert_weights) return CAIFX_ERR_INVALID_ARGUMENT;
-  const dim3 grid(wave_blocks(num_tokens)), block(kRouteThreads);
   hipStream_t s = as_stream(stream);
   const bool vec = (dim * dtype_size(dtype)) % 16 == 0 && aligned_to(expert_buffer, 16) && aligned_to(output, 16);
+  const dim3 grid(wave_blocks(num_tokens * gather_waves(dim, vec ? 16 / static_cast<int>(dtype_size(dtype)) : 1))), block(kRouteThreads);
 #define CAIFX_GO(T)                                                                                                    \
   if (vec)                                                                                                             \
     hipLaunchKernelGGL((gather_sum_kernel<T, true, true>), grid, block, 0, s, static_cast<const T *>(expert_buffer),   \
@@ -558,9 +592,9 @@ int caifx_moe_dispatch_backward(const void *grad_expert_buffer, const int32_t *e
   const int st = check_route(grad_expert_buffer, grad_input, expert_indices, dispatch_map, expert_offsets, num_tokens, dim,
                              top_k, num_experts, dtype);
   if (st >= 0) return st;
-  const dim3 grid(wave_blocks(num_tokens)), block(kRouteThreads);
   hipStream_t s = as_stream(stream);
   const bool vec = (dim * dtype_size(dtype)) % 16 == 0 && aligned_to(grad_expert_buffer, 16) && aligned_to(grad_input, 16);
+  const dim3 grid(wave_blocks(num_tokens * gather_waves(dim, vec ? 16 / static_cast<int>(dtype_size(dtype)) : 1))), block(kRouteThreads);
 #define CAIFX_GO(T)                                                                                                    \
   if (vec)                                                                                                             \
     hipLaunchKernelGGL((gather_sum_kernel<T, false, true>), grid, block, 0, s,                                         \
