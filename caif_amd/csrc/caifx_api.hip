@@ -339,7 +339,8 @@ size_t caifx_qlinear_grouped_workspace_bytes(int num_experts, int64_t total_rows
   a.w.kind = w_kind;
   a.num_experts = num_experts;
   a.offsets = reinterpret_cast<const int32_t *>(uintptr_t{1});   // marks the grouped form for the size query
-  return mfma_workspace_bytes(a, backward != 0);
+  const size_t bytes = mfma_workspace_bytes(a, backward != 0), dense = mfma_wide_workspace_bytes(a, backward != 0);
+  return bytes > dense ? bytes : dense;
 }
 
 static int grouped(bool backward, int num_experts, const int32_t *offsets, int64_t total_rows, int64_t N, int64_t K,

@@ -123,6 +123,14 @@ __device__ __forceinline__ void segment_rows(const int32_t *offsets, int e, int6
   hi = hi < lo ? lo : (hi > m ? m : hi);
 }
 
+// a 64-bit value every lane holds alike, moved to scalar registers (the direct-to-LDS requests take their base there)
+__device__ __forceinline__ uint64_t uniform64(uint64_t v)
+{
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+  return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
 // Which tile of a grouped launch a workgroup owns.  Row tiles of BM rows are counted over all experts, expert by
 // expert, and crossed with col_tiles column tiles, column tile last; XCD x (workgroup id mod 8, each XCD has its own
 // L2) takes the x-th contiguous eighth of that list, so one expert's weight and one row tile's activations are

@@ -66,14 +66,6 @@ struct Regw8Args {
   long long stamps_capacity;
 };
 
-// a 64-bit value every lane holds alike, moved to scalar registers (the direct-to-LDS requests take their base there)
-__device__ __forceinline__ uint64_t uniform64(uint64_t v)
-{
-  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
-  return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-
 template <typename CT, bool kGrouped>
 __global__ __launch_bounds__(512, 2) void qgemm_regw8_kernel(Regw8Args g)
 {

@@ -14,7 +14,7 @@
 //  - the weight is dequantised once per call instead of once per row tile.
 // Against the kernels that dequantise inside the product (forward 380 us, input gradient 385 us at M = 4096, N = 11008,
 // K = 4096, int4, bf16) the two launches take 290 and 257 us.
-#include "caifx_internal.hpp"
+#include "caifx_gemm_regw.hpp"
 
 #include <atomic>
 #include <type_traits>
@@ -32,6 +32,12 @@ struct WideArgs {
   const void *addend;
   int64_t M, C, R;
   int d_dtype;
+  // grouped form: rows [offsets[e], offsets[e + 1]) times the e-th [C, R] matrix behind b
+  const int32_t *offsets;
+  const void *const *wq_ptrs;
+  int num_experts;
+  unsigned long long *stamps;      // measurement only, see mfma_grouped_tile_stamps
+  long long stamps_capacity;
 };
 
 // acc += a b, 16 x 16 x 32: lane l supplies row (column) l % 16, reduction elements 8 (l / 16) .. + 7; the result's
@@ -54,7 +60,7 @@ template <typename CT> __device__ __forceinline__ void mfma16(floatx4_t &acc, co
 // unit for 256 x 256) are on their way at any time, and every request has one and a half steps to arrive.  Requests
 // complete in issue order, so the wait for the half tile that is read next is an exact count (a wave issues WI + WJ
 // per half).
-template <typename CT, int WI, int WJ>
+template <typename CT, int WI, int WJ, bool kGrouped>
 __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(WideArgs g)
 {
   typedef typename Mfma32<CT>::vec_t vec_t;
@@ -73,8 +79,25 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
   // XCD x (workgroup id mod 8, each with its own L2) walks the x-th contiguous eighth of a list that runs through bands
   // of 1024 rows column by column: the 256 x 256 tiles it works on at a time share 4 row and 8 column panels
   const int64_t col_tiles = (g.C + BN - 1) / BN, row_tiles = (g.M + BM - 1) / BM;
-  int64_t row0, col0;
-  {
+  int64_t row0, col0, row_end = g.M;
+  uint64_t b_ptr = reinterpret_cast<uint64_t>(g.b);
+  int64_t stamp_pos = -1;
+  if constexpr (kGrouped) {
+    GroupedTile gt;
+    if (!grouped_tile<BM>(g.offsets, g.num_experts, g.M, col_tiles, g.wq_ptrs, nullptr, lane, gt)) return;
+    // the search's results are the same in every lane: into scalar registers with them
+    row0 = uniform64(static_cast<uint64_t>(gt.row0));
+    row_end = uniform64(static_cast<uint64_t>(gt.row_end));
+    col0 = uniform64(static_cast<uint64_t>(gt.col_tile * BN));
+    b_ptr = uniform64(b_ptr + static_cast<uint64_t>(gt.e) * static_cast<uint64_t>(g.C * g.R * 2));
+    if (g.stamps && threadIdx.x == 0 && gt.pos < g.stamps_capacity) {
+      stamp_pos = gt.pos;
+      const int64_t rows = row_end - row0 < BM ? row_end - row0 : BM;
+      g.stamps[4 * stamp_pos] = static_cast<unsigned long long>(gt.e);
+      g.stamps[4 * stamp_pos + 1] = static_cast<unsigned long long>(rows) | (WI + WJ <= 4 ? 0ull : 1ull << 32);      // one or two workgroups per compute unit
+      g.stamps[4 * stamp_pos + 2] = wall_clock64();
+    }
+  } else {
     const unsigned bid = blockIdx.x;
     const int64_t per_xcd = gridDim.x >> 3;
     const int64_t pos = static_cast<int64_t>(bid & 7) * per_xcd + (bid >> 3);
@@ -98,7 +121,7 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
     for (int i = 0; i < WI; ++i) {
       const int lrow = 8 * (wave + 4 * i) + (lane >> 3);
       int64_t m = row0 + h * (BM / 2) + lrow;
-      if (m >= g.M) m = g.M - 1;
+      if (m >= row_end) m = row_end - 1;
       a_voff[h][i] = static_cast<uint32_t>((m - row0) * g.R * 2 + (((lane & 7) ^ ((lrow ^ (lrow >> 3)) & 7)) << 4));
     }
 #pragma unroll
@@ -109,8 +132,8 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
       b_voff[h][i] = static_cast<uint32_t>((c - col0) * g.R * 2 + (((lane & 7) ^ ((lrow ^ (lrow >> 3)) & 7)) << 4));
     }
   }
-  const uint64_t a_base = reinterpret_cast<uint64_t>(g.a) + static_cast<uint64_t>(row0 * g.R * 2);
-  const uint64_t b_base = reinterpret_cast<uint64_t>(g.b) + static_cast<uint64_t>(col0 * g.R * 2);
+  const uint64_t a_base = uniform64(reinterpret_cast<uint64_t>(g.a) + static_cast<uint64_t>(row0 * g.R * 2));
+  const uint64_t b_base = uniform64(b_ptr + static_cast<uint64_t>(col0 * g.R * 2));
   const int steps = static_cast<int>(g.R / kBK);
   const int last = steps - 1;
   auto request = [&](int s, int h, int slot, int x) __attribute__((always_inline)) {
@@ -243,7 +266,7 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
 #pragma unroll
       for (int b = 0; b < kBatch; ++b) {
         int64_t grow = row0 + pass * (BM / 2) + ((batch * kBatch + b) * 4 + wave) * kRowsPerInstr + lane / kLanesPerRow;
-        if (grow >= g.M) grow = g.M - 1;
+        if (grow >= row_end) grow = row_end - 1;
         to[b] = *reinterpret_cast<const u32x4_t *>(ap + grow * g.C + acol);
       }
     };
@@ -285,7 +308,7 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
             for (int e = 0; e < kPer16; ++e) wp[e] = from_f32<T>(to_f32<T>(vp[e]) + to_f32<T>(aq[e]));
             v = w;
           }
-          if (grow < g.M && gcol < g.C) *reinterpret_cast<u32x4_t *>(dp + grow * g.C + gcol) = v;
+          if (grow < row_end && gcol < g.C) *reinterpret_cast<u32x4_t *>(dp + grow * g.C + gcol) = v;
         }
       }
     }
@@ -297,6 +320,9 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
   if (g.d_dtype == CAIFX_BF16) store_as(bf16_t{});
   else if (g.d_dtype == CAIFX_F16) store_as(f16_t{});
   else store_as(float{});
+  if constexpr (kGrouped) {
+    if (stamp_pos >= 0) g.stamps[4 * stamp_pos + 3] = wall_clock64();
+  }
 }
 
 // ------------------------------------------------------------------ the weight as a dense matrix of the compute type
@@ -307,7 +333,26 @@ struct DenseArgs {
   int64_t N, K;
   int group_shift;         // int4
   uint32_t period;         // int8; 0 = no scales
+  // grouped form: expert blockIdx.z, skipped when it has no rows; its copy is the z-th [N, K] behind out
+  const int32_t *offsets;
+  const void *const *wq_ptrs;
+  const void *const *scales_ptrs;
+  int64_t M;
 };
+
+// the grouped form's weight of this workgroup; false: nothing to do
+__device__ __forceinline__ bool dense_expert(DenseArgs &g)
+{
+  if (!g.offsets) return true;
+  const int e = static_cast<int>(blockIdx.z);
+  int lo, hi;
+  segment_rows(g.offsets, e, g.M, lo, hi);
+  if (lo >= hi) return false;
+  g.q = g.wq_ptrs[e];
+  g.scales = g.scales_ptrs ? g.scales_ptrs[e] : nullptr;
+  g.out = static_cast<char *>(g.out) + static_cast<int64_t>(e) * g.N * g.K * 2;
+  return true;
+}
 
 enum { DK_INT8 = 0, DK_INT4 = 1, DK_16 = 2 };
 
@@ -354,6 +399,7 @@ template <typename CT, int kKind>
 __global__ __launch_bounds__(256) void dense_rows_kernel(DenseArgs g)
 {
   constexpr int kRounds = 4;
+  if (!dense_expert(g)) return;
   const int64_t pieces = g.N * g.K / 8;
   const int64_t p0 = static_cast<int64_t>(blockIdx.x) * (256 * kRounds) + threadIdx.x;
   float e[kRounds][8];
@@ -381,6 +427,7 @@ template <typename CT, int kKind>
 __global__ __launch_bounds__(256) void dense_transposed_kernel(DenseArgs g)
 {
   __shared__ __attribute__((aligned(16))) unsigned char tile[256 * 128];
+  if (!dense_expert(g)) return;
   const int kl = threadIdx.x & 31, ng = threadIdx.x >> 5;
   const int64_t n0 = static_cast<int64_t>(blockIdx.y) * 64, k0 = static_cast<int64_t>(blockIdx.x) * 256;
   if (k0 + 8 * kl < g.K) {
@@ -407,29 +454,29 @@ __global__ __launch_bounds__(256) void dense_transposed_kernel(DenseArgs g)
 }
 
 template <typename CT>
-int launch_dense(const DenseArgs &g, int kind, bool transposed, hipStream_t s)
+int launch_dense(const DenseArgs &g, int kind, bool transposed, int experts, hipStream_t s)
 {
   if (transposed) {
-    const dim3 grid(static_cast<unsigned>((g.K + 255) / 256), static_cast<unsigned>(g.N / 64));
+    const dim3 grid(static_cast<unsigned>((g.K + 255) / 256), static_cast<unsigned>(g.N / 64), static_cast<unsigned>(experts));
     if (kind == DK_INT4) hipLaunchKernelGGL((dense_transposed_kernel<CT, DK_INT4>), grid, dim3(256), 0, s, g);
     else if (kind == DK_INT8) hipLaunchKernelGGL((dense_transposed_kernel<CT, DK_INT8>), grid, dim3(256), 0, s, g);
     else hipLaunchKernelGGL((dense_transposed_kernel<CT, DK_16>), grid, dim3(256), 0, s, g);
   } else {
-    const dim3 grid(static_cast<unsigned>((g.N * g.K / 8 + 1023) / 1024));
+    const dim3 grid(static_cast<unsigned>((g.N * g.K / 8 + 1023) / 1024), 1, static_cast<unsigned>(experts));
     if (kind == DK_INT4) hipLaunchKernelGGL((dense_rows_kernel<CT, DK_INT4>), grid, dim3(256), 0, s, g);
     else hipLaunchKernelGGL((dense_rows_kernel<CT, DK_INT8>), grid, dim3(256), 0, s, g);
   }
   return launch_status();
 }
 
-template <typename CT, int WI, int WJ>
+template <typename CT, int WI, int WJ, bool kGrouped>
 int launch_wide(const WideArgs &g, hipStream_t s)
 {
   constexpr int BM = 64 * WI, BN = 64 * WJ;
   constexpr int kRing = (BM + BN) * 256, kStore16 = BM * (BN * 2 + 32), kStore32 = BM / 2 * (BN * 4 + 32);
   constexpr int kStore = kStore16 > kStore32 ? kStore16 : kStore32;
   constexpr int kLds = kRing > kStore ? kRing : kStore;
-  auto kern = wide_gemm_kernel<CT, WI, WJ>;
+  auto kern = wide_gemm_kernel<CT, WI, WJ, kGrouped>;
   static std::atomic<bool> raised{false};
   if (!raised.load(std::memory_order_relaxed)) {
     // the attribute is per kernel and sticky; two threads racing here both set it, which is harmless
@@ -437,7 +484,8 @@ int launch_wide(const WideArgs &g, hipStream_t s)
       return CAIFX_ERR_LAUNCH_FAILED;
     raised.store(true, std::memory_order_relaxed);
   }
-  const int64_t tiles = ((g.M + BM - 1) / BM) * ((g.C + BN - 1) / BN);
+  // grouped: segment lengths live on the device; an upper bound, every expert can add one partial tile
+  const int64_t tiles = ((g.M + BM - 1) / BM + (kGrouped ? g.num_experts : 0)) * ((g.C + BN - 1) / BN);
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((tiles + 7) / 8 * 8)), dim3(256), kLds, s, g);
   return launch_status();
 }
@@ -448,30 +496,42 @@ int launch_wide(const WideArgs &g, hipStream_t s)
 // at most 256.  M = 4096, C = 11008: 265 / 300 / 300 us; M = 2048, C = 11008: 166 / 149 / 162; M = 1024, C = 4096: 72 /
 // 44 / 32.
 enum { TILE_256 = 0, TILE_128x256 = 1, TILE_128 = 2 };
-double step_cost(int tile, int64_t M, int64_t C)
+// row tiles of bm rows; over expert segments of unknown lengths the last tile of each is taken as half full
+int64_t row_tiles_of(int64_t M, int experts, int64_t bm)
 {
-  const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((C + bn - 1) / bn); };
+  if (experts == 0) return (M + bm - 1) / bm;
+  const int64_t t = (M + bm - 1) / bm + experts / 2, least = M < experts ? M : experts;
+  return t > least ? t : least;
+}
+double step_cost(int tile, int64_t M, int64_t C, int experts)
+{
+  const auto tiles = [&](int64_t bm, int64_t bn) { return row_tiles_of(M, experts, bm) * ((C + bn - 1) / bn); };
   if (tile == TILE_256) return 1.39 * static_cast<double>((tiles(256, 256) + 255) / 256);
   if (tile == TILE_128x256) return 0.87 * static_cast<double>((tiles(128, 256) + 255) / 256);
   const int64_t t = tiles(128, 128), rest = t % 512;
   return 0.91 * static_cast<double>(t / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.49 : 0.91);
 }
-int best_tile(int64_t M, int64_t C)
+int best_tile(int64_t M, int64_t C, int experts)
 {
   int best = TILE_256;
   for (int t = TILE_128x256; t <= TILE_128; ++t)
-    if (step_cost(t, M, C) < step_cost(best, M, C)) best = t;
+    if (step_cost(t, M, C, experts) < step_cost(best, M, C, experts)) best = t;
   return best;
 }
 
-template <typename CT>
+template <typename CT, bool kGrouped>
 int pick_wide(const WideArgs &g, hipStream_t s)
 {
-  switch (best_tile(g.M, g.C)) {
-    case TILE_256: return launch_wide<CT, 4, 4>(g, s);
-    case TILE_128x256: return launch_wide<CT, 2, 4>(g, s);
-    default: return launch_wide<CT, 2, 2>(g, s);
+  switch (best_tile(g.M, g.C, g.num_experts)) {
+    case TILE_256: return launch_wide<CT, 4, 4, kGrouped>(g, s);
+    case TILE_128x256: return launch_wide<CT, 2, 4, kGrouped>(g, s);
+    default: return launch_wide<CT, 2, 2, kGrouped>(g, s);
   }
+}
+template <typename CT>
+int pick_form(const WideArgs &g, hipStream_t s)
+{
+  return g.offsets ? pick_wide<CT, true>(g, s) : pick_wide<CT, false>(g, s);
 }
 
 bool dense16(const GemmArgs &a)
@@ -482,7 +542,7 @@ bool dense16(const GemmArgs &a)
 // The rule on sizes and types alone (the workspace query knows nothing else).
 bool wide_shape(const GemmArgs &a, bool backward)
 {
-  if (a.compute_dtype == CAIFX_F32 || a.x_dtype != a.compute_dtype || a.offsets || a.epilogue != 0) return false;
+  if (a.compute_dtype == CAIFX_F32 || a.x_dtype != a.compute_dtype || a.epilogue != 0) return false;
   const bool codes = a.w.kind == CAIFX_W_INT8 || a.w.kind == CAIFX_W_INT4_GROUP;
   if (!codes && !dense16(a)) return false;
   const int64_t C = backward ? a.K : a.N, R = backward ? a.N : a.K;
@@ -490,6 +550,20 @@ bool wide_shape(const GemmArgs &a, bool backward)
   if (a.N * a.K >= (int64_t{1} << 32) || a.M > (int64_t{1} << 30) || R > (int64_t{1} << 22)) return false;
   const int64_t tiles = ((a.M + 127) / 128) * ((C + 127) / 128);
   if (tiles > (int64_t{1} << 30)) return false;
+  if (a.offsets) {
+    // Experts with long segments, and copies of all their weights within half of the memory-side cache (128 MB): the
+    // dense pass then costs 10 to 20 us and the product gains a quarter.  Forward / input gradient in us, dequantised
+    // inside the product against here, int8, N = 1408, K = 2048: 8 experts, 24576 rows 198 / 216 against 156 / 158, 6000 rows
+    // 80 / 71 against 62 / 55, 4096 rows 42 / 58 against 45 / 52; 16 experts, 12288 rows 126 / 130 against 102 / 104, 8192
+    // rows 81 / 94 against 77 / 94; 33 experts (190 MB), 24576 rows 218 / 243 against 244 / 235; 64 experts (369 MB),
+    // 24576 rows 260 / 283 against 294 / 297, and no better in chunks of experts (8: 432 / 502, 32: 325 / 310, the launches'
+    // ends add up).  Small products: 8 experts, 512 x 512, 8192 rows 14.6 / 18.0 against 16.9 / 18.1, 24576 rows 29.3 / 34.7
+    // against 28.1 / 29.2.  Stored 16-bit weights stay on the tiled kernel (input gradient, 16 experts: 188 against 215 us
+    // with 24576 rows, 157 against 147 with 16384).
+    if (!codes || a.num_experts < 1 || a.num_experts > 65535) return false;
+    return a.M >= 750 * static_cast<int64_t>(a.num_experts) && a.num_experts * a.N * a.K * 2 <= (int64_t{1} << 27) &&
+           static_cast<double>(a.M) * static_cast<double>(a.N) * static_cast<double>(a.K) >= 5e9;
+  }
   // Is it worth it?  `tiles` counts 128 x 128 tiles.  A stored 16-bit weight needs no extra pass in the forward
   // direction: from 100 tiles on (128: 25.8 against 27.4 us, 256: 31.5 against 39.4; 80: 26.1 against 24.2, where the
   // tiled kernel shares each tile's reduction among workgroups).
@@ -503,7 +577,7 @@ bool wide_shape(const GemmArgs &a, bool backward)
   if (!backward && a.w.kind == CAIFX_W_INT4_GROUP && a.K % 256 == 0 && regw_tiles >= 128) {
     const double steps = static_cast<double>(R / kBK);
     return tiles > 256 &&
-           3.0 + step_cost(best_tile(a.M, C), a.M, C) * steps + 3.5 + 0.33e-6 * static_cast<double>(a.N) * static_cast<double>(a.K) <
+           3.0 + step_cost(best_tile(a.M, C, 0), a.M, C, 0) * steps + 3.5 + 0.33e-6 * static_cast<double>(a.N) * static_cast<double>(a.K) <
                (0.9 * steps + 6.0) * static_cast<double>((regw_tiles + 255) / 256);
   }
   // Everything else runs on the tiled kernel otherwise (or int8 forward with a short scale vector on
@@ -518,13 +592,14 @@ bool wide_shape(const GemmArgs &a, bool backward)
 size_t mfma_wide_workspace_bytes(const GemmArgs &a, bool backward)
 {
   if (!wide_shape(a, backward) || (dense16(a) && !backward)) return 0;
-  return static_cast<size_t>(a.N) * static_cast<size_t>(a.K) * 2;
+  return static_cast<size_t>(a.offsets ? a.num_experts : 1) * static_cast<size_t>(a.N) * static_cast<size_t>(a.K) * 2;
 }
 
 int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s)
 {
   if (!wide_shape(a, backward)) return CAIFX_ERR_UNSUPPORTED;
-  if (!aligned_to(a.x, 16) || !aligned_to(a.w.q, 16) || !aligned_to(a.y, 16) || (a.addend && !aligned_to(a.addend, 16))) return CAIFX_ERR_UNSUPPORTED;
+  const bool grouped = a.offsets != nullptr;      // (the tuned kernels take expert weights to be aligned to 16 bytes)
+  if (!aligned_to(a.x, 16) || (!grouped && !aligned_to(a.w.q, 16)) || !aligned_to(a.y, 16) || (a.addend && !aligned_to(a.addend, 16))) return CAIFX_ERR_UNSUPPORTED;
   WideArgs g{};
   g.a = a.x;
   g.d = a.y;
@@ -533,33 +608,44 @@ int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s)
   g.C = backward ? a.K : a.N;
   g.R = backward ? a.N : a.K;
   g.d_dtype = a.y_dtype;
-  g.b = a.w.q;
-  const size_t need = mfma_wide_workspace_bytes(a, backward);
-  if (need > 0) {
-    if (!a.workspace || a.workspace_bytes < need || !aligned_to(a.workspace, 16)) return CAIFX_ERR_UNSUPPORTED;
-    DenseArgs d{};
-    d.q = a.w.q;
-    d.scales = a.w.scales;
-    d.out = a.workspace;
-    d.N = a.N;
-    d.K = a.K;
-    int kind = DK_16;
-    if (a.w.kind == CAIFX_W_INT4_GROUP) {
-      const int gs = a.w.group_size;
-      if (gs < 8 || (gs & (gs - 1)) != 0) return CAIFX_ERR_UNSUPPORTED;
-      d.group_shift = __builtin_ctz(static_cast<unsigned>(gs));
-      kind = DK_INT4;
-    } else if (a.w.kind == CAIFX_W_INT8) {
-      d.period = a.w.scales ? static_cast<uint32_t>(a.w.scale_period) : 0;
-      if (d.period > 1 && (a.w.scale_period % 4 != 0 || a.w.scale_period < 8 || a.w.scale_period > a.N * a.K || !aligned_to(a.w.scales, 16)))
-        return CAIFX_ERR_UNSUPPORTED;
-      kind = DK_INT8;
-    }
-    const int st = a.compute_dtype == CAIFX_BF16 ? launch_dense<bf16_t>(d, kind, backward, s) : launch_dense<f16_t>(d, kind, backward, s);
-    if (st != CAIFX_OK) return st;
-    g.b = a.workspace;
+  g.b = grouped ? nullptr : a.w.q;
+  if (grouped) {
+    if (!a.wq_ptrs) return CAIFX_ERR_UNSUPPORTED;
+    g.offsets = a.offsets;
+    g.wq_ptrs = a.wq_ptrs;
+    g.num_experts = a.num_experts;
+    mfma_grouped_stamp_target(&g.stamps, &g.stamps_capacity);
   }
-  return a.compute_dtype == CAIFX_BF16 ? pick_wide<bf16_t>(g, s) : pick_wide<f16_t>(g, s);
+  const auto product = [&]() { return a.compute_dtype == CAIFX_BF16 ? pick_form<bf16_t>(g, s) : pick_form<f16_t>(g, s); };
+  if (dense16(a) && !backward) return product();
+  if (!a.workspace || a.workspace_bytes < mfma_wide_workspace_bytes(a, backward) || !aligned_to(a.workspace, 16)) return CAIFX_ERR_UNSUPPORTED;
+  DenseArgs d{};
+  d.q = a.w.q;
+  d.scales = a.w.scales;
+  d.out = a.workspace;
+  d.N = a.N;
+  d.K = a.K;
+  d.M = a.M;
+  d.offsets = a.offsets;
+  d.wq_ptrs = a.wq_ptrs;
+  d.scales_ptrs = a.scales_ptrs;
+  int kind = DK_16;
+  if (a.w.kind == CAIFX_W_INT4_GROUP) {
+    const int gs = a.w.group_size;
+    if (gs < 8 || (gs & (gs - 1)) != 0) return CAIFX_ERR_UNSUPPORTED;
+    d.group_shift = __builtin_ctz(static_cast<unsigned>(gs));
+    kind = DK_INT4;
+  } else if (a.w.kind == CAIFX_W_INT8) {
+    d.period = (grouped ? a.scales_ptrs != nullptr : a.w.scales != nullptr) ? static_cast<uint32_t>(a.w.scale_period) : 0;
+    if (d.period > 1 && (a.w.scale_period % 4 != 0 || a.w.scale_period < 8 || a.w.scale_period > a.N * a.K || (!grouped && !aligned_to(a.w.scales, 16))))
+      return CAIFX_ERR_UNSUPPORTED;
+    kind = DK_INT8;
+  }
+  const int experts = grouped ? a.num_experts : 1;
+  const int st = a.compute_dtype == CAIFX_BF16 ? launch_dense<bf16_t>(d, kind, backward, experts, s) : launch_dense<f16_t>(d, kind, backward, experts, s);
+  if (st != CAIFX_OK) return st;
+  g.b = a.workspace;
+  return product();
 }
 
 }  // namespace caifx
