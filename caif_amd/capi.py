@@ -29,7 +29,7 @@ EXPORTS = [
     "caifx_qlinear_forward_add", "caifx_qlinear_backward_input_add", "caifx_qlinear_grouped_backward_input_add",
     "caifx_qlinear_grouped_forward", "caifx_qlinear_grouped_backward_input",
     "caifx_qlinear_grouped_workspace_bytes", "caifx_qlinear_grouped_forward_swiglu",
-    "caifx_qlinear_grouped_backward_input_swiglu",
+    "caifx_qlinear_grouped_backward_input_swiglu", "caifx_qlinear_grouped_zero_rest",
     "caifx_silu", "caifx_silu_backward", "caifx_multiply", "caifx_add", "caifx_silu_multiply",
     "caifx_swiglu_backward",
     "caifx_moe_dispatch_map_workspace_bytes", "caifx_moe_build_dispatch_map", "caifx_moe_dispatch",
@@ -102,6 +102,7 @@ def lib():
         L.caifx_add.argtypes = [_p, _p, _p, _i64, _int, _p]
         L.caifx_silu_multiply.argtypes = [_p, _p, _p, _i64, _int, _p]
         L.caifx_swiglu_backward.argtypes = [_p, _p, _p, _p, _p, _i64, _int, _p]
+        L.caifx_qlinear_grouped_zero_rest.argtypes = [_int, _p, _i64, _i64, _p, _p]
         L.caifx_moe_dispatch_map_workspace_bytes.restype = _sz
         L.caifx_moe_dispatch_map_workspace_bytes.argtypes = [_i64, _int, _int]
         L.caifx_moe_build_dispatch_map.argtypes = [_p, _i64, _int, _int, _int, _p, _p, _p, _sz, _p]

@@ -416,7 +416,49 @@ unsigned wave_blocks(int64_t waves) { return static_cast<unsigned>((waves * 64 +
 
 using namespace caifx;
 
+namespace caifx {
+namespace {
+
+// Zeroes rows [0, offsets[0]) and [offsets[E], rows) of a grouped result: the segments' rows are all written by the
+// launch behind it (the steps upwards from offsets[0] to offsets[E] cover every row between the two, whatever the order
+// of the entries).  Usually there is nothing to do and the launch takes 2 us, where clearing the whole result took 11
+// (24576 x 1408 bf16) to 15 us (24576 x 2048).
+__global__ __launch_bounds__(256) void zero_rest_kernel(const int32_t *offsets, int num_experts, int64_t rows, int64_t row_bytes,
+                                                        unsigned char *y)
+{
+  const int64_t first = offsets[0], end = offsets[num_experts];
+  const int64_t lo = first < 0 ? 0 : first > rows ? rows : first, hi = end < 0 ? 0 : end > rows ? rows : end;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, threads = static_cast<int64_t>(gridDim.x) * 256;
+  const int64_t shift = reinterpret_cast<uintptr_t>(y) & 15;
+  const auto zero = [&](int64_t a, int64_t b) {        // bytes [a, b): whole aligned 16-byte pieces, single bytes at the ends
+    if (a >= b) return;
+    const int64_t up = ((a + shift + 15) & ~int64_t{15}) - shift, down = ((b + shift) & ~int64_t{15}) - shift;
+    const int64_t a16 = up < b ? up : b, b16 = down > a16 ? down : a16;
+    for (int64_t i = a16 + 16 * t; i < b16; i += 16 * threads) *reinterpret_cast<u32x4_t *>(y + i) = u32x4_t{0, 0, 0, 0};
+    if (a + t < a16) y[a + t] = 0;
+    if (b16 + t < b) y[b16 + t] = 0;
+  };
+  zero(0, lo * row_bytes);
+  zero((hi > lo ? hi : lo) * row_bytes, rows * row_bytes);
+}
+
+}  // namespace
+}  // namespace caifx
+
 extern "C" {
+
+int caifx_qlinear_grouped_zero_rest(int num_experts, const int32_t *offsets, int64_t total_rows, int64_t row_bytes, void *y,
+                                    caifx_stream_t stream)
+{
+  if (num_experts < 0 || total_rows < 0 || row_bytes < 0) return CAIFX_ERR_INVALID_ARGUMENT;
+  if (total_rows == 0 || row_bytes == 0) return CAIFX_OK;
+  if (!offsets || !y || total_rows > INT64_MAX / row_bytes) return CAIFX_ERR_INVALID_ARGUMENT;
+  // 8 pieces a thread where everything is to be cleared; never more than 1024 workgroups, which mostly find nothing to do
+  const int64_t blocks = total_rows * row_bytes / (256 * 16 * 8) + 1;
+  hipLaunchKernelGGL(caifx::zero_rest_kernel, dim3(static_cast<unsigned>(blocks < 1024 ? blocks : 1024)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), offsets, num_experts, total_rows, row_bytes, static_cast<unsigned char *>(y));
+  return caifx::launch_status();
+}
 
 size_t caifx_moe_dispatch_map_workspace_bytes(int64_t num_tokens, int top_k, int num_experts)
 {

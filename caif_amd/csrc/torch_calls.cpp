@@ -25,7 +25,7 @@ namespace {
   X(caifx_qlinear_forward) X(caifx_qlinear_forward_add) X(caifx_qlinear_backward_input)                                  \
   X(caifx_qlinear_backward_input_add) X(caifx_qlinear_workspace_bytes) X(caifx_qlinear_grouped_forward)                  \
   X(caifx_qlinear_grouped_backward_input) X(caifx_qlinear_grouped_backward_input_add)                                    \
-  X(caifx_qlinear_grouped_workspace_bytes) X(caifx_silu) X(caifx_silu_backward) X(caifx_multiply) X(caifx_add)           \
+  X(caifx_qlinear_grouped_workspace_bytes) X(caifx_qlinear_grouped_zero_rest) X(caifx_silu) X(caifx_silu_backward) X(caifx_multiply) X(caifx_add)           \
   X(caifx_silu_multiply) X(caifx_swiglu_backward) X(caifx_moe_dispatch_map_workspace_bytes)                              \
   X(caifx_moe_build_dispatch_map) X(caifx_moe_dispatch) X(caifx_moe_combine) X(caifx_moe_combine_backward_grad_expert)   \
   X(caifx_moe_combine_backward_grad_weights) X(caifx_moe_dispatch_backward) X(caifx_quantize_int8_per_channel)           \
@@ -275,7 +275,7 @@ PyObject *grouped(PyObject *, PyObject *const *a, Py_ssize_t n)
       if (o.scalar_type() != type_of(od) || o.numel() != rows * out_dim)
         throw Error{PyExc_ValueError, "the result tensor must have the result's dtype and rows x columns elements"};
     }
-    const at::Tensor y = a[6] != Py_None ? tensor(a[6]) : at::zeros({rows, out_dim}, x.options().dtype(type_of(od)));
+    const at::Tensor y = a[6] != Py_None ? tensor(a[6]) : at::empty({rows, out_dim}, x.options().dtype(type_of(od)));
     const int64_t period = int_attr(w, at_.period);
     const int group = static_cast<int>(int_attr(w, at_.group));
     const auto wq = static_cast<const void *const *>(ptr_attr(w, at_.wq_ptrs));
@@ -284,6 +284,12 @@ PyObject *grouped(PyObject *, PyObject *const *a, Py_ssize_t n)
       return api.caifx_qlinear_grouped_workspace_bytes(static_cast<int>(E), rows, N, K, xd, compute, kind, backward ? 1 : 0);
     });
     const auto off = static_cast<const int32_t *>(offsets.data_ptr());
+    if (a[6] == Py_None && y.numel() > 0) {      // a fresh result's rows outside the segments are zero
+      const int status = launch([&] {
+        return api.caifx_qlinear_grouped_zero_rest(static_cast<int>(E), off, rows, out_dim * static_cast<int64_t>(y.element_size()), y.data_ptr(), stream());
+      });
+      if (status != CAIFX_OK) return PyLong_FromLong(status);
+    }
     if (a[8] != Py_None) {
       if (!backward) throw Error{PyExc_AssertionError, "the forward takes no addend"};
       const at::Tensor &add = tensor(a[8]);

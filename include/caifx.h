@@ -383,6 +383,11 @@ CAIFX_API int caifx_moe_dispatch(const void *input, const int32_t *expert_indice
                        const int32_t *expert_offsets, void *expert_buffer, int64_t num_tokens, int64_t dim,
                        int top_k, int num_experts, int dtype, caifx_stream_t stream);
 
+/* Zeroes the rows of a grouped result that no segment covers, [0, offsets[0]) and [offsets[num_experts], total_rows), each
+ * row_bytes long: what a result tensor that was not cleared as a whole needs in front of the launch that fills it. */
+CAIFX_API int caifx_qlinear_grouped_zero_rest(int num_experts, const int32_t *offsets, int64_t total_rows, int64_t row_bytes,
+                                    void *y, caifx_stream_t stream);
+
 /* launch_moe_combine (caif_cuda_kernels_moe.cuh:317-326, caif_cuda_kernels_moe.cu:705-745):
  * output[t,d] = T( sum over k in order of float(w[t,k]) * float(buffer[row(t,k), d]) ), fp32
  * accumulation with one fused multiply-add per k, one rounding to T. */
