@@ -414,6 +414,13 @@ PyObject *moe_build_dispatch_map(PyObject *, PyObject *const *a, Py_ssize_t n)
   });
 }
 
+// rows x columns: the routing entry points take no other rank
+const at::Tensor &matrix(const at::Tensor &t)
+{
+  if (t.dim() != 2) throw Error{PyExc_ValueError, "expected a two-dimensional tensor"};
+  return t;
+}
+
 const int32_t *ints(PyObject *o) { return static_cast<const int32_t *>(device_tensor(o).data_ptr()); }
 
 // moe_dispatch(x, ids, map, offsets, total_rows, out)
@@ -421,7 +428,7 @@ PyObject *moe_dispatch(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
   return guarded(n, 6, [&]() -> PyObject * {
     const at::Tensor &x = device_tensor(a[0]), &ids = device_tensor(a[1]), &offsets = device_tensor(a[3]);
-    const int64_t tokens = x.size(0), dim = x.size(1);
+    const int64_t tokens = matrix(x).size(0), dim = x.size(1);
     const at::Tensor buf = a[5] != Py_None ? tensor(a[5]) : at::zeros({integer(a[4]), dim}, x.options());
     const int32_t *i1 = ints(a[1]); const int32_t *i2 = ints(a[2]); const int32_t *i3 = ints(a[3]); const int dt = code_of(x.scalar_type());
     return result(launch([&] { return api.caifx_moe_dispatch(x.data_ptr(), i1, i2, i3, buf.data_ptr(), tokens, dim,
@@ -434,7 +441,7 @@ PyObject *moe_combine(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
   return guarded(n, 6, [&]() -> PyObject * {
     const at::Tensor &buf = device_tensor(a[0]), &ids = device_tensor(a[1]), &w = device_tensor(a[2]), &offsets = device_tensor(a[4]);
-    const int64_t tokens = ids.size(0), dim = buf.size(1);
+    const int64_t tokens = matrix(ids).size(0), dim = buf.size(1);
     const at::Tensor y = a[5] != Py_None ? tensor(a[5]) : at::empty({tokens, dim}, buf.options());
     const int32_t *i1 = ints(a[1]); const int32_t *i3 = ints(a[3]); const int32_t *i4 = ints(a[4]); const int dt = code_of(buf.scalar_type());
     return result(launch([&] { return api.caifx_moe_combine(buf.data_ptr(), i1, w.data_ptr(), i3, i4, y.data_ptr(), tokens, dim,
@@ -447,7 +454,7 @@ PyObject *moe_combine_backward_grad_expert(PyObject *, PyObject *const *a, Py_ss
 {
   return guarded(n, 7, [&]() -> PyObject * {
     const at::Tensor &g = device_tensor(a[0]), &ids = device_tensor(a[1]), &w = device_tensor(a[2]), &offsets = device_tensor(a[4]);
-    const int64_t tokens = g.size(0), dim = g.size(1);
+    const int64_t tokens = matrix(g).size(0), dim = g.size(1);
     const at::Tensor buf = a[6] != Py_None ? tensor(a[6]) : at::zeros({integer(a[5]), dim}, g.options());
     const int32_t *i1 = ints(a[1]); const int32_t *i3 = ints(a[3]); const int32_t *i4 = ints(a[4]); const int dt = code_of(g.scalar_type());
     return result(launch([&] { return api.caifx_moe_combine_backward_grad_expert(g.data_ptr(), i1, w.data_ptr(), i3, i4, buf.data_ptr(), tokens, dim,
@@ -461,7 +468,7 @@ PyObject *moe_dispatch_backward(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
   return guarded(n, 5, [&]() -> PyObject * {
     const at::Tensor &g = device_tensor(a[0]), &ids = device_tensor(a[1]), &offsets = device_tensor(a[3]);
-    const int64_t tokens = ids.size(0), dim = g.size(1);
+    const int64_t tokens = matrix(ids).size(0), dim = g.size(1);
     const at::Tensor y = a[4] != Py_None ? tensor(a[4]) : at::empty({tokens, dim}, g.options());
     const int32_t *i1 = ints(a[1]); const int32_t *i2 = ints(a[2]); const int32_t *i3 = ints(a[3]); const int dt = code_of(g.scalar_type());
     return result(launch([&] { return api.caifx_moe_dispatch_backward(g.data_ptr(), i1, i2, i3, y.data_ptr(), tokens, dim,
@@ -475,7 +482,7 @@ PyObject *moe_combine_backward_grad_weights(PyObject *, PyObject *const *a, Py_s
 {
   return guarded(n, 5, [&]() -> PyObject * {
     const at::Tensor &g = device_tensor(a[0]), &buf = device_tensor(a[1]), &ids = device_tensor(a[2]), &offsets = device_tensor(a[4]);
-    const int64_t tokens = ids.size(0), top_k = ids.size(1), dim = g.size(1);
+    const int64_t tokens = matrix(ids).size(0), top_k = ids.size(1), dim = g.size(1);
     const at::Tensor y = at::empty({tokens, top_k}, g.options());
     const int32_t *i2 = ints(a[2]); const int32_t *i3 = ints(a[3]); const int32_t *i4 = ints(a[4]); const int dt = code_of(g.scalar_type());
     return result(launch([&] { return api.caifx_moe_combine_backward_grad_weights(g.data_ptr(), buf.data_ptr(), i2, i3, i4, y.data_ptr(), tokens, dim,
