@@ -652,14 +652,15 @@ __global__ __launch_bounds__(256) void rowlin_int8_fast_kernel(RowArgs a)
 // ------------------------------------------------------------------ int8, one activation row, integer matrix core
 // Y[n] = sum_k q[n,k] * scale[(n*K+k) mod P] * x[k].  All rows of one residue class see the same
 // scales along k, so the scales are folded into the activations once per workgroup:
-// x'[k] = scale[(cls*K+k) mod P] * x[k] (fp32), and x' is split into three signed 7-bit "digits"
-// relative to a power-of-two scale per diagonal element (the 256 k values of lanes i, i+16, i+32,
-// i+48): x' ~ 2^(e-6) * (d0 + d1/128 + d2/16384), |error| <= 2^(e-21).  The int8 codes then go into
+// x'[k] = scale[(cls*K+k) mod P] * x[k] (fp32), and x' is split into three signed 8-bit "digits"
+// relative to a power-of-two scale per diagonal element (the 64 k values per chunk of lanes i, i+16,
+// i+32, i+48, 256 at most): x' ~ 2^(e-6) * (d0 + d1/256 + d2/65536), |error| <= 2^(e-23) where the
+// largest |x'| is below 2^e (the row-block kernel's digits, caifx_gemv_mblock.hip: 2^(e-22)).  The int8 codes then go into
 // v_mfma_i32_16x16x64_i8 exactly as they were loaded (one 16-byte load = one A operand, no
 // unpacking arithmetic at all) against the digit planes as B operands; the three int32 sums are exact
 // and are combined in fp32 once per weight row.  As in the kernels above only the diagonal of the
-// 16x16 result is used.  The result is sum_k q*scale*x with every product exact to ~2^-21 of the
-// largest |x'| of its 256-k set; it differs from the reference's dequantise-round-GEMM by the rounding
+// 16x16 result is used.  The result is sum_k q*scale*x with every factor exact to 2^-22 of the
+// largest |x'| of its set of at most 256; it differs from the reference's dequantise-round-GEMM by the rounding
 // of q*scale to the compute dtype that the reference applies and this kernel does not.
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 
@@ -667,6 +668,23 @@ typedef int i32x4_t __attribute__((ext_vector_type(4)));
 // paid once per workgroup and reads 24 KB for K = 4096, so a workgroup should own many rows: 16 waves
 // measured 12.2 us against 12.9 (8) and 13.1 (4) on the K=4096, N=14336 case.
 constexpr int kDigitWaves = 16;
+
+// Byte q of the digit words: four values x' as three digits.  n = round(x' / unit * 2^16), |n| <= 2^22, is the difference of
+// the bit patterns of x' * (2^16 / unit) + 1.5 * 2^23 and of 1.5 * 2^23, whose low 16 bits are zero; n = 2^16 d0 + 2^8 d1 +
+// d2 with d1, d2 in [-128, 127] and |d0| <= 64, the carries supplied by adding half a digit below each field.
+__device__ __forceinline__ void cut_digits(const float *x, float inv16, int q, i32x4_t &d0, i32x4_t &d1, i32x4_t &d2)
+{
+  int b0[4], b1[4], b2[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    b2[t] = __builtin_bit_cast(int, __builtin_fmaf(x[t], inv16, 12582912.0f));
+    b1[t] = (b2[t] + 0x80) >> 8;
+    b0[t] = (b2[t] + (0x8080 - 0x4B400000)) >> 16;
+  }
+  d0[q] = static_cast<int>(pack_low_bytes(b0[0], b0[1], b0[2], b0[3]));
+  d1[q] = static_cast<int>(pack_low_bytes(b1[0], b1[1], b1[2], b1[3]));
+  d2[q] = static_cast<int>(pack_low_bytes(b2[0], b2[1], b2[2], b2[3]));
+}
 
 template <typename XT, bool kVec, int CPR, bool kTail>
 __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(RowArgs a)
@@ -783,25 +801,10 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
     unit = (m > 0.0f && !poisoned) ? ldexpf(1.0f, e - 6) : 1.0f;
   }
   if (has_chunk) {
-    // n = round(x' / unit * 2^14) as the low mantissa bits of x' * (2^14 / unit) + 1.5 * 2^23 (|n| <= 2^20);
-    // n = 2^14 d0 + 2^7 d1 + d2 with d1, d2 in [-64, 63]: three signed bit-field extracts, the carries
-    // supplied by adding half a digit below each field
-    const float inv14 = 16384.0f / unit;      // exact: a power of two
+    const float inv16 = 65536.0f / unit;      // exact: a power of two
     i32x4_t d0, d1, d2;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      int e0[4], e1[4], e2[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int b = __builtin_bit_cast(int, __builtin_fmaf(xv[4 * q + t], inv14, 12582912.0f));
-        e2[t] = __builtin_amdgcn_sbfe(b, 0, 7);
-        e1[t] = __builtin_amdgcn_sbfe(b + 64, 7, 7);
-        e0[t] = __builtin_amdgcn_sbfe(b + 64 + 8192, 14, 8);
-      }
-      d0[q] = static_cast<int>(pack_low_bytes(e0[0], e0[1], e0[2], e0[3]));
-      d1[q] = static_cast<int>(pack_low_bytes(e1[0], e1[1], e1[2], e1[3]));
-      d2[q] = static_cast<int>(pack_low_bytes(e2[0], e2[1], e2[2], e2[3]));
-    }
+    for (int q = 0; q < 4; ++q) cut_digits(&xv[4 * q], inv16, q, d0, d1, d2);
     dig[wave][0][lane] = d0;
     dig[wave][1][lane] = d1;
     dig[wave][2][lane] = d2;
@@ -812,7 +815,7 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
   for (int c = 0; c < CPR; ++c)
 #pragma unroll
     for (int d = 0; d < 3; ++d) xb[c][d] = dig[c][d][lane];
-  const float u0 = unit * s_scalar, u1 = u0 * (1.0f / 128.0f), u2 = u0 * (1.0f / 16384.0f);
+  const float u0 = unit * s_scalar, u1 = u0 * (1.0f / 256.0f), u2 = u0 * (1.0f / 65536.0f);
   const int tsel = lane & 3;
   const bool is_diag = (lane >> 4) == ((lane & 15) >> 2);
 
@@ -976,22 +979,10 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_long_kern
   }
   if (has_chunk) {
     const float unit_c = poisoned ? 1.0f : unit_of(slice_max(wave / cps));
-    const float inv14 = 16384.0f / unit_c;
+    const float inv16 = 65536.0f / unit_c;
     i32x4_t d0, d1, d2;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      int e0[4], e1[4], e2[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int b = __builtin_bit_cast(int, __builtin_fmaf(xv[4 * q + t], inv14, 12582912.0f));
-        e2[t] = __builtin_amdgcn_sbfe(b, 0, 7);
-        e1[t] = __builtin_amdgcn_sbfe(b + 64, 7, 7);
-        e0[t] = __builtin_amdgcn_sbfe(b + 64 + 8192, 14, 8);
-      }
-      d0[q] = static_cast<int>(pack_low_bytes(e0[0], e0[1], e0[2], e0[3]));
-      d1[q] = static_cast<int>(pack_low_bytes(e1[0], e1[1], e1[2], e1[3]));
-      d2[q] = static_cast<int>(pack_low_bytes(e2[0], e2[1], e2[2], e2[3]));
-    }
+    for (int q = 0; q < 4; ++q) cut_digits(&xv[4 * q], inv16, q, d0, d1, d2);
     dig[wave][0][lane] = d0;
     dig[wave][1][lane] = d1;
     dig[wave][2][lane] = d2;
@@ -1003,7 +994,7 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_long_kern
   for (int c = 0; c < CPS; ++c)
 #pragma unroll
     for (int d = 0; d < 3; ++d) xb[c][d] = c < my_chunks ? dig[first_chunk + c][d][lane] : i32x4_t{0, 0, 0, 0};
-  const float u0 = unit * s_scalar, u1 = u0 * (1.0f / 128.0f), u2 = u0 * (1.0f / 16384.0f);
+  const float u0 = unit * s_scalar, u1 = u0 * (1.0f / 256.0f), u2 = u0 * (1.0f / 65536.0f);
   const int tsel = lane & 3;
   const bool is_diag = (lane >> 4) == ((lane & 15) >> 2);
 
