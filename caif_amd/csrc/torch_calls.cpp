@@ -141,13 +141,16 @@ const WeightAttrs &attrs()
   return a;
 }
 
-// the launch itself without the interpreter lock: it can wait for room in the queue
-template <typename F> int launch(F f)
+// the launch itself without the interpreter lock: it can wait for room in the queue.  It takes the entry point and its
+// arguments, so whatever can throw (sizes, data pointers, the stream) is evaluated while the lock is held.
+struct Unlocked {
+  PyThreadState *state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <typename... P, typename... A> int launch(int (*entry)(P...), A... args)
 {
-  PyThreadState *st = PyEval_SaveThread();
-  const int status = f();
-  PyEval_RestoreThread(st);
-  return status;
+  const Unlocked without_lock;
+  return entry(args...);
 }
 
 void *stream() { return static_cast<void *>(c10::hip::getCurrentHIPStream().stream()); }
@@ -241,10 +244,10 @@ PyObject *qlinear(PyObject *, PyObject *const *a, Py_ssize_t n)
       if (add.scalar_type() != y.scalar_type() || add.numel() != y.numel())
         throw Error{PyExc_AssertionError, "the addend must have the result's dtype and size"};
       const auto fn = backward ? api.caifx_qlinear_backward_input_add : api.caifx_qlinear_forward_add;
-      return result(launch([&] { return fn(M, N, K, x.data_ptr(), xd, compute, wq, kind, scales, period, group, y.data_ptr(), od, add.data_ptr(), ws.p, ws.bytes, stream()); }), y);
+      return result(launch(fn, M, N, K, x.data_ptr(), xd, compute, wq, kind, scales, period, group, y.data_ptr(), od, add.data_ptr(), ws.p, ws.bytes, stream()), y);
     }
     const auto fn = backward ? api.caifx_qlinear_backward_input : api.caifx_qlinear_forward;
-    return result(launch([&] { return fn(M, N, K, x.data_ptr(), xd, compute, wq, kind, scales, period, group, y.data_ptr(), od, ws.p, ws.bytes, stream()); }), y);
+    return result(launch(fn, M, N, K, x.data_ptr(), xd, compute, wq, kind, scales, period, group, y.data_ptr(), od, ws.p, ws.bytes, stream()), y);
   });
 }
 
@@ -285,9 +288,7 @@ PyObject *grouped(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
     const auto off = static_cast<const int32_t *>(offsets.data_ptr());
     if (a[6] == Py_None && y.numel() > 0) {      // a fresh result's rows outside the segments are zero
-      const int status = launch([&] {
-        return api.caifx_qlinear_grouped_zero_rest(static_cast<int>(E), off, rows, out_dim * static_cast<int64_t>(y.element_size()), y.data_ptr(), stream());
-      });
+      const int status = launch(api.caifx_qlinear_grouped_zero_rest, static_cast<int>(E), off, rows, out_dim * static_cast<int64_t>(y.element_size()), y.data_ptr(), stream());
       if (status != CAIFX_OK) return PyLong_FromLong(status);
     }
     if (a[8] != Py_None) {
@@ -295,12 +296,12 @@ PyObject *grouped(PyObject *, PyObject *const *a, Py_ssize_t n)
       const at::Tensor &add = tensor(a[8]);
       if (add.scalar_type() != y.scalar_type() || add.numel() != y.numel())
         throw Error{PyExc_AssertionError, "the addend must have the result's dtype and size"};
-      return result(launch([&] { return api.caifx_qlinear_grouped_backward_input_add(static_cast<int>(E), off, rows, N, K, x.data_ptr(), xd, compute, wq, kind, scales,
-                                                                 period, group, y.data_ptr(), od, add.data_ptr(), ws.p, ws.bytes, stream()); }), y);
+      return result(launch(api.caifx_qlinear_grouped_backward_input_add, static_cast<int>(E), off, rows, N, K, x.data_ptr(), xd, compute, wq, kind, scales,
+                                                                 period, group, y.data_ptr(), od, add.data_ptr(), ws.p, ws.bytes, stream()), y);
     }
     const auto fn = backward ? api.caifx_qlinear_grouped_backward_input : api.caifx_qlinear_grouped_forward;
-    return result(launch([&] { return fn(static_cast<int>(E), off, rows, N, K, x.data_ptr(), xd, compute, wq, kind, scales, period, group, y.data_ptr(), od, ws.p,
-                     ws.bytes, stream()); }), y);
+    return result(launch(fn, static_cast<int>(E), off, rows, N, K, x.data_ptr(), xd, compute, wq, kind, scales, period, group, y.data_ptr(), od, ws.p,
+                     ws.bytes, stream()), y);
   });
 }
 
@@ -324,12 +325,10 @@ PyObject *quantize_int8(PyObject *, PyObject *const *a, Py_ssize_t n)
     const at::Tensor q = at::empty(x.sizes(), x.options().dtype(at::kChar));
     const at::Tensor s = at::empty({per_channel ? x.size(1) : 1}, x.options());
     const auto in = static_cast<const float *>(x.data_ptr());
-    if (!per_channel) return pair(launch([&] { return api.caifx_quantize_int8_per_tensor(in, q.data_ptr(), s.data_ptr(), x.numel(), stream()); }), q, s);
+    if (!per_channel) return pair(launch(api.caifx_quantize_int8_per_tensor, in, q.data_ptr(), s.data_ptr(), x.numel(), stream()), q, s);
     const int64_t rows = x.size(0), cols = x.size(1);
     if (rows > INT32_MAX || cols > INT32_MAX) throw Error{PyExc_OverflowError, "QuantizeInt8 PerChannel: too many rows or columns"};
-    return pair(launch([&] {
-      return api.caifx_quantize_int8_per_channel(in, q.data_ptr(), s.data_ptr(), static_cast<int>(rows), static_cast<int>(cols), stream());
-    }), q, s);
+    return pair(launch(api.caifx_quantize_int8_per_channel, in, q.data_ptr(), s.data_ptr(), static_cast<int>(rows), static_cast<int>(cols), stream()), q, s);
   });
 }
 
@@ -345,9 +344,7 @@ PyObject *quantize_int4(PyObject *, PyObject *const *a, Py_ssize_t n)
     const int64_t groups = group > 0 ? (count + group - 1) / group : 0;      // a negative size is the library's error
     const at::Tensor packed = at::empty({(count + 1) / 2}, x.options().dtype(at::kByte));
     const at::Tensor s = at::empty({groups}, x.options().dtype(at::kHalf));
-    return pair(launch([&] {
-      return api.caifx_quantize_to_int4(static_cast<const float *>(x.data_ptr()), packed.data_ptr(), s.data_ptr(), count, static_cast<int>(group), stream());
-    }), packed, s);
+    return pair(launch(api.caifx_quantize_to_int4, static_cast<const float *>(x.data_ptr()), packed.data_ptr(), s.data_ptr(), count, static_cast<int>(group), stream()), packed, s);
   });
 }
 
@@ -368,9 +365,9 @@ PyObject *elementwise(PyObject *, PyObject *const *a, Py_ssize_t n)
     const at::Tensor y = a[3] != Py_None ? tensor(a[3]) : at::empty_like(x);
     const int dt = code_of(x.scalar_type());
     const int64_t op = integer(a[0]);
-    if (op == 0) return result(launch([&] { return api.caifx_silu(x.data_ptr(), y.data_ptr(), x.numel(), dt, stream()); }), y);
+    if (op == 0) return result(launch(api.caifx_silu, x.data_ptr(), y.data_ptr(), x.numel(), dt, stream()), y);
     const auto fn = op == 1 ? api.caifx_silu_backward : op == 2 ? api.caifx_multiply : op == 3 ? api.caifx_add : api.caifx_silu_multiply;
-    return result(launch([&] { return fn(x.data_ptr(), b, y.data_ptr(), x.numel(), dt, stream()); }), y);
+    return result(launch(fn, x.data_ptr(), b, y.data_ptr(), x.numel(), dt, stream()), y);
   });
 }
 
@@ -384,9 +381,7 @@ PyObject *swiglu_backward(PyObject *, PyObject *const *a, Py_ssize_t n)
     const at::Tensor gg = a[3] != Py_None ? tensor(a[3]) : at::empty_like(gate);
     const at::Tensor gu = a[4] != Py_None ? tensor(a[4]) : at::empty_like(gate);
     const int dt = code_of(gate.scalar_type());
-    const int st = launch([&] {
-      return api.caifx_swiglu_backward(gate.data_ptr(), up.data_ptr(), gh.data_ptr(), gg.data_ptr(), gu.data_ptr(), gate.numel(), dt, stream());
-    });
+    const int st = launch(api.caifx_swiglu_backward, gate.data_ptr(), up.data_ptr(), gh.data_ptr(), gg.data_ptr(), gu.data_ptr(), gate.numel(), dt, stream());
     if (st != CAIFX_OK) return PyLong_FromLong(st);
     Owned p(THPVariable_Wrap(gg)), q(THPVariable_Wrap(gu));
     return PyTuple_Pack(2, p.p, q.p);
@@ -408,17 +403,24 @@ PyObject *moe_build_dispatch_map(PyObject *, PyObject *const *a, Py_ssize_t n)
     if (nb < 4 * static_cast<size_t>(E)) nb = 4 * static_cast<size_t>(E);
     const at::Tensor ws = bytes_like(ids, nb);
     const int capacity = static_cast<int>(integer(a[2]));
-    return pair(launch([&] { return api.caifx_moe_build_dispatch_map(static_cast<const int32_t *>(ids.data_ptr()), tokens, top_k, E, capacity,
+    return pair(launch(api.caifx_moe_build_dispatch_map, static_cast<const int32_t *>(ids.data_ptr()), tokens, top_k, E, capacity,
                                                  static_cast<int32_t *>(map.data_ptr()), static_cast<int32_t *>(offsets.data_ptr()), ws.data_ptr(),
-                                                 nb, stream()); }), map, offsets);
+                                                 nb, stream()), map, offsets);
   });
 }
 
-// rows x columns: the routing entry points take no other rank
+// rows x columns: the tensor that gives the number of tokens has no other rank
 const at::Tensor &matrix(const at::Tensor &t)
 {
   if (t.dim() != 2) throw Error{PyExc_ValueError, "expected a two-dimensional tensor"};
   return t;
+}
+
+// the second extent of a tensor of two dimensions or more
+int64_t columns(const at::Tensor &t)
+{
+  if (t.dim() < 2) throw Error{PyExc_IndexError, "expected a tensor of at least two dimensions"};
+  return t.size(1);
 }
 
 const int32_t *ints(PyObject *o) { return static_cast<const int32_t *>(device_tensor(o).data_ptr()); }
@@ -428,11 +430,11 @@ PyObject *moe_dispatch(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
   return guarded(n, 6, [&]() -> PyObject * {
     const at::Tensor &x = device_tensor(a[0]), &ids = device_tensor(a[1]), &offsets = device_tensor(a[3]);
-    const int64_t tokens = matrix(x).size(0), dim = x.size(1);
+    const int64_t tokens = matrix(x).size(0), dim = x.size(1), top_k = columns(ids);
     const at::Tensor buf = a[5] != Py_None ? tensor(a[5]) : at::zeros({integer(a[4]), dim}, x.options());
     const int32_t *i1 = ints(a[1]); const int32_t *i2 = ints(a[2]); const int32_t *i3 = ints(a[3]); const int dt = code_of(x.scalar_type());
-    return result(launch([&] { return api.caifx_moe_dispatch(x.data_ptr(), i1, i2, i3, buf.data_ptr(), tokens, dim,
-                                         static_cast<int>(ids.size(1)), static_cast<int>(offsets.numel() - 1), dt, stream()); }), buf);
+    return result(launch(api.caifx_moe_dispatch, x.data_ptr(), i1, i2, i3, buf.data_ptr(), tokens, dim,
+                                         static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1), dt, stream()), buf);
   });
 }
 
@@ -441,11 +443,11 @@ PyObject *moe_combine(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
   return guarded(n, 6, [&]() -> PyObject * {
     const at::Tensor &buf = device_tensor(a[0]), &ids = device_tensor(a[1]), &w = device_tensor(a[2]), &offsets = device_tensor(a[4]);
-    const int64_t tokens = matrix(ids).size(0), dim = buf.size(1);
+    const int64_t tokens = matrix(ids).size(0), dim = columns(buf), top_k = ids.size(1);
     const at::Tensor y = a[5] != Py_None ? tensor(a[5]) : at::empty({tokens, dim}, buf.options());
     const int32_t *i1 = ints(a[1]); const int32_t *i3 = ints(a[3]); const int32_t *i4 = ints(a[4]); const int dt = code_of(buf.scalar_type());
-    return result(launch([&] { return api.caifx_moe_combine(buf.data_ptr(), i1, w.data_ptr(), i3, i4, y.data_ptr(), tokens, dim,
-                                        static_cast<int>(ids.size(1)), static_cast<int>(offsets.numel() - 1), dt, stream()); }), y);
+    return result(launch(api.caifx_moe_combine, buf.data_ptr(), i1, w.data_ptr(), i3, i4, y.data_ptr(), tokens, dim,
+                                        static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1), dt, stream()), y);
   });
 }
 
@@ -454,12 +456,12 @@ PyObject *moe_combine_backward_grad_expert(PyObject *, PyObject *const *a, Py_ss
 {
   return guarded(n, 7, [&]() -> PyObject * {
     const at::Tensor &g = device_tensor(a[0]), &ids = device_tensor(a[1]), &w = device_tensor(a[2]), &offsets = device_tensor(a[4]);
-    const int64_t tokens = matrix(g).size(0), dim = g.size(1);
+    const int64_t tokens = matrix(g).size(0), dim = g.size(1), top_k = columns(ids);
     const at::Tensor buf = a[6] != Py_None ? tensor(a[6]) : at::zeros({integer(a[5]), dim}, g.options());
     const int32_t *i1 = ints(a[1]); const int32_t *i3 = ints(a[3]); const int32_t *i4 = ints(a[4]); const int dt = code_of(g.scalar_type());
-    return result(launch([&] { return api.caifx_moe_combine_backward_grad_expert(g.data_ptr(), i1, w.data_ptr(), i3, i4, buf.data_ptr(), tokens, dim,
-                                                             static_cast<int>(ids.size(1)), static_cast<int>(offsets.numel() - 1),
-                                                             dt, stream()); }), buf);
+    return result(launch(api.caifx_moe_combine_backward_grad_expert, g.data_ptr(), i1, w.data_ptr(), i3, i4, buf.data_ptr(), tokens, dim,
+                                                             static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1),
+                                                             dt, stream()), buf);
   });
 }
 
@@ -468,12 +470,12 @@ PyObject *moe_dispatch_backward(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
   return guarded(n, 5, [&]() -> PyObject * {
     const at::Tensor &g = device_tensor(a[0]), &ids = device_tensor(a[1]), &offsets = device_tensor(a[3]);
-    const int64_t tokens = matrix(ids).size(0), dim = g.size(1);
+    const int64_t tokens = matrix(ids).size(0), dim = columns(g), top_k = ids.size(1);
     const at::Tensor y = a[4] != Py_None ? tensor(a[4]) : at::empty({tokens, dim}, g.options());
     const int32_t *i1 = ints(a[1]); const int32_t *i2 = ints(a[2]); const int32_t *i3 = ints(a[3]); const int dt = code_of(g.scalar_type());
-    return result(launch([&] { return api.caifx_moe_dispatch_backward(g.data_ptr(), i1, i2, i3, y.data_ptr(), tokens, dim,
-                                                  static_cast<int>(ids.size(1)), static_cast<int>(offsets.numel() - 1), dt,
-                                                  stream()); }), y);
+    return result(launch(api.caifx_moe_dispatch_backward, g.data_ptr(), i1, i2, i3, y.data_ptr(), tokens, dim,
+                                                  static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1), dt,
+                                                  stream()), y);
   });
 }
 
@@ -482,12 +484,12 @@ PyObject *moe_combine_backward_grad_weights(PyObject *, PyObject *const *a, Py_s
 {
   return guarded(n, 5, [&]() -> PyObject * {
     const at::Tensor &g = device_tensor(a[0]), &buf = device_tensor(a[1]), &ids = device_tensor(a[2]), &offsets = device_tensor(a[4]);
-    const int64_t tokens = matrix(ids).size(0), top_k = ids.size(1), dim = g.size(1);
+    const int64_t tokens = matrix(ids).size(0), top_k = ids.size(1), dim = columns(g);
     const at::Tensor y = at::empty({tokens, top_k}, g.options());
     const int32_t *i2 = ints(a[2]); const int32_t *i3 = ints(a[3]); const int32_t *i4 = ints(a[4]); const int dt = code_of(g.scalar_type());
-    return result(launch([&] { return api.caifx_moe_combine_backward_grad_weights(g.data_ptr(), buf.data_ptr(), i2, i3, i4, y.data_ptr(), tokens, dim,
+    return result(launch(api.caifx_moe_combine_backward_grad_weights, g.data_ptr(), buf.data_ptr(), i2, i3, i4, y.data_ptr(), tokens, dim,
                                                               static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1),
-                                                              dt, stream()); }), y);
+                                                              dt, stream()), y);
   });
 }
 
