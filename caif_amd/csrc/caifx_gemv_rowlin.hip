@@ -301,8 +301,8 @@ __global__ __launch_bounds__(256) void rowlin_int4_kernel(RowArgs a)
         }
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-          const float corr = Mfma16<CT>::kOffset * xsum[m * groups_pad + cchunk * 16 + di];
-          tot[m] = __builtin_fmaf(s, diag_of(part[m], lane) - corr, tot[m]);
+          const float sum = xsum[m * groups_pad + cchunk * 16 + di];
+          tot[m] = __builtin_fmaf(s, __builtin_fmaf(-Mfma16<CT>::kOffset, sum, diag_of(part[m], lane)), tot[m]);
         }
         if (++cchunk == cpr) {
           cchunk = 0;
@@ -467,11 +467,13 @@ __global__ __launch_bounds__(kInt4FastWaves * 64) void rowlin_int4_fast_kernel(R
   x_commit<CT, MT, kPieces, true, kThreads>(xp, xs, xsum);
   __syncthreads();
 
-  float corr[MT][CPR];
+  // The offset times a group's sum of activations is up to 1000 times the group's result: it is taken off in one fused
+  // step, like in the dynamic kernel above (rounding the product first cost 15 % of the error against 64 bits).
+  float gsum[MT][CPR];
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int c = 0; c < CPR; ++c) corr[m][c] = Mfma16<CT>::kOffset * xsum[m * kGroupsPad + c * 16 + di];
+    for (int c = 0; c < CPR; ++c) gsum[m][c] = xsum[m * kGroupsPad + c * 16 + di];
   const int tsel = di & 3;
   // lane r keeps the result of the wave's row r: one coalesced store per wave after the loop, and no
   // store (which would count against the same in-flight counter as the loads) inside it
@@ -518,7 +520,7 @@ __global__ __launch_bounds__(kInt4FastWaves * 64) void rowlin_int4_fast_kernel(R
             dsel = (tsel == 3) ? part[m][3] : dsel;
             float scale = to_f32(sc[d][c]);
             if (kTail && c == CPR - 1) scale = tail_inside ? scale : 0.0f;
-            tot[m] = __builtin_fmaf(scale, dsel - corr[m][c], tot[m]);
+            tot[m] = __builtin_fmaf(scale, __builtin_fmaf(-Mfma16<CT>::kOffset, gsum[m][c], dsel), tot[m]);
           }
         }
 #pragma unroll
@@ -1193,8 +1195,8 @@ template <typename CT, typename XT, int MT>
 int launch_int4(const RowArgs &ra, hipStream_t s)
 {
   if constexpr (dtype_code<XT>::value == dtype_code<CT>::value) {
-    // fp32 results with a partial last chunk stay on the dynamic kernel: error against 64 bits 3.9e-5 against 4.5e-5 (fp16,
-    // K = 7168, N = 2048; a 16-bit result's own rounding is 2.1e-4)
+    // fp32 results with a partial last chunk stay on the dynamic kernel: the same bits, and only whole chunks and 16-bit
+    // results have been timed on both
     if (ra.group_shift == 7 && (ra.K % 2048 == 0 || ra.y_dtype != CAIFX_F32)) {
       const int st = ra.K % 2048 == 0 ? pick_int4_fast<CT, MT, false>(ra, s) : pick_int4_fast<CT, MT, true>(ra, s);
       if (st != CAIFX_ERR_UNSUPPORTED) return st;
@@ -1348,8 +1350,8 @@ int rowlin_forward(const GemmArgs &g, hipStream_t s)
     if (static_cast<size_t>(mt) * ra.xpitch * 2 + 4096 > 64 * 1024) return CAIFX_ERR_UNSUPPORTED;
   } else {
     // one activation row and 4096 < K <= 16384: the integer-matrix-core kernel with the row split among waves.  fp32 results
-    // with a partial last chunk stay on the row-block kernel, whose digits share a unit over 128 or 256 elements instead
-    // of a slice: error against 64 bits 6.0e-7 there, 1.35e-6 here (K = 6400, N = 4096), which 16-bit results do not see
+    // with a partial last chunk stay on the row-block kernel, the one they have been timed on (error against 64 bits 5.8e-7
+    // there; here 3.0e-7 to 3.5e-7, measured with whole chunks)
     const bool long_digits = g.M == 1 && g.K > 4096 && g.K <= 16384 && (g.K % 1024 == 0 || g.y_dtype != CAIFX_F32);
     if (g.K % 16 != 0 || (g.K > 4096 && !long_digits)) return CAIFX_ERR_UNSUPPORTED;
     ra.cpr = static_cast<int>((g.K + 1023) / 1024);

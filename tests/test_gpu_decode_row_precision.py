@@ -29,3 +29,20 @@ def test_int8_digits_reach_2_to_the_minus_21_of_the_largest_activation(K, period
     for yd in ((T.F32, T.BF16) if K % 1024 == 0 else (T.BF16,)):
         got = host(T.qlinear_forward(xd, w, T.BF16, yd))[0]
         assert max_rel_err(got, want) <= 2.0 ** -20 + (2.0 ** -8 if yd == T.BF16 else 0), yd
+
+
+@pytest.mark.parametrize("cd", [T.BF16, T.F16])
+@pytest.mark.parametrize("K", [256, 2048, 2304, 3840, 4096, 6144, 6400, 8192, 10240, 12288, 14336, 16384])
+def test_int4_groups_of_128_and_of_256_give_the_same_bits(orc, K, cd):
+    # The same codes and scales as groups of 256 (the kernel for any group size) and of 128 (the fixed-shape kernels, also
+    # with a partial last chunk where the result has 16 bits): the same sums in the same order, so the same bits.
+    rng = np.random.default_rng(K)
+    N = 1037
+    p, s = orc.quantize_to_int4(rng.normal(0, 0.02, (N, K)).astype(np.float32), 256)
+    s = s.view(np.float16)
+    wide = T.FrozenWeight(dev(p), T.W_INT4_GROUP, dev(s), N, K, 1, 256)
+    narrow = T.FrozenWeight(dev(p), T.W_INT4_GROUP, dev(np.repeat(s, 2)), N, K, 1, 128)
+    for M in (1, 2) if K <= 14336 else (1,):
+        x = dev_as(rng.normal(0, 1, (M, K)), cd)
+        for yd in (T.F32, cd):
+            assert torch.equal(T.qlinear_forward(x, wide, cd, yd), T.qlinear_forward(x, narrow, cd, yd)), (M, yd)
