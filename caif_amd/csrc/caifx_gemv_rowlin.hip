@@ -671,6 +671,15 @@ typedef int i32x4_t __attribute__((ext_vector_type(4)));
 // measured 12.2 us against 12.9 (8) and 13.1 (4) on the K=4096, N=14336 case.
 constexpr int kDigitWaves = 16;
 
+// power-of-two unit of a set of values whose largest magnitude is m (0 < m finite): maps m into [32, 64).  Not below 2^-111,
+// so that 2^16 / unit stays finite; sets that small next to larger ones lose bits below 2^-127.
+__device__ __forceinline__ float digit_unit(float m)
+{
+  int e = 0;
+  (void)frexpf(m, &e);      // m = f * 2^e, f in [0.5, 1)
+  return ldexpf(1.0f, (e > -105 ? e : -105) - 6);
+}
+
 // Byte q of the digit words: four values x' as three digits.  n = round(x' / unit * 2^16), |n| <= 2^22, is the difference of
 // the bit patterns of x' * (2^16 / unit) + 1.5 * 2^23 and of 1.5 * 2^23, whose low 16 bits are zero; n = 2^16 d0 + 2^8 d1 +
 // d2 with d1, d2 in [-128, 127] and |d0| <= 64, the carries supplied by adding half a digit below each field.
@@ -686,6 +695,29 @@ __device__ __forceinline__ void cut_digits(const float *x, float inv16, int q, i
   d0[q] = static_cast<int>(pack_low_bytes(b0[0], b0[1], b0[2], b0[3]));
   d1[q] = static_cast<int>(pack_low_bytes(b1[0], b1[1], b1[2], b1[3]));
   d2[q] = static_cast<int>(pack_low_bytes(b2[0], b2[1], b2[2], b2[3]));
+}
+
+// Lane r: result of row cls + V * (i0 + r) as the reference forms it, sum of x[k] * CT(code * scale) in fp32.  For the few
+// inputs whose products have no digits; the whole wave takes part (nrows is wave uniform).
+template <typename XT>
+__device__ __forceinline__ float rowlin_int8_plain_rows(const RowArgs &a, int cls, int64_t i0, int nrows)
+{
+  const int lane = threadIdx.x & 63;
+  const int ct = a.round_x >= 0 ? a.round_x : dtype_code<XT>::value;      // the compute dtype
+  const XT *x = static_cast<const XT *>(a.x);
+  const float *scales = static_cast<const float *>(a.scales);
+  const auto rounded = [&](float v) { return ct == CAIFX_BF16 ? round_through<bf16_t>(v) : round_through<f16_t>(v); };
+  float res = 0.0f;
+  for (int r = 0; r < nrows; ++r) {
+    const int64_t first = (cls + a.row_stride * (i0 + r)) * a.K;
+    float sum = 0.0f;
+    for (int64_t k = lane; k < a.K; k += 64) {
+      const float scale = !scales ? 1.0f : a.period > 1 ? scales[(first + k) % a.period] : scales[0];
+      sum = __builtin_fmaf(rounded(to_f32<XT>(x[k])), rounded(static_cast<float>(static_cast<int8_t>(a.wq[first + k])) * scale), sum);
+    }
+    res = lane_insert(res, wave_sum_hi(sum), r);
+  }
+  return res;
 }
 
 template <typename XT, bool kVec, int CPR, bool kTail>
@@ -788,19 +820,17 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
   }
   __syncthreads();
 
-  // power-of-two unit of diagonal element i: the largest |x'| of its CPR*64 values maps into [32, 64]
+  // unit of diagonal element i: from the largest |x'| of its CPR*64 values
   float unit;
-  bool poisoned;       // wave uniform, and the same in every wave of the workgroup
+  bool no_digits;      // wave uniform, and the same in every wave of the workgroup
   {
     float m = 0.0f;
 #pragma unroll
     for (int c = 0; c < CPR; ++c) m = fmaxf(m, mx[c][lane & 15]);
-    // A NaN or an infinity among the scaled activations has no digits.  The reference's GEMM returns NaN or an
-    // infinity in every output then (each output multiplies every activation); here every output becomes NaN.
-    poisoned = __any(!(m <= 3.4028235e38f));
-    int e = 0;
-    (void)frexpf(poisoned ? 1.0f : m, &e);    // m = f * 2^e, f in [0.5, 1)
-    unit = (m > 0.0f && !poisoned) ? ldexpf(1.0f, e - 6) : 1.0f;
+    // A NaN or an infinity among the scaled activations has no digits, and where even the largest is below 2^-90 the
+    // digits would run out of the exponent range: the results are summed value by value at the end then.
+    no_digits = __any(!(m <= 3.4028235e38f)) || (__any(m > 0.0f) && !__any(m >= 0x1p-90f));
+    unit = (m > 0.0f && !no_digits) ? digit_unit(m) : 1.0f;
   }
   if (has_chunk) {
     const float inv16 = 65536.0f / unit;      // exact: a power of two
@@ -848,7 +878,8 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_kernel(Ro
       issue(d, r + D);
     }
   }
-  if (lane < nrows) store_y(a.y, a.y_dtype, cls + V * (i0 + lane), poisoned ? __builtin_nanf("") : res);
+  if (no_digits) res = rowlin_int8_plain_rows<XT>(a, cls, i0, nrows);
+  if (lane < nrows) store_y(a.y, a.y_dtype, cls + V * (i0 + lane), res);
 }
 
 
@@ -968,11 +999,7 @@ __global__ __launch_bounds__(kDigitWaves * 64) void rowlin_int8_digits_long_kern
     for (int c = sl * cps; c < (sl + 1) * cps && c < a.cpr; ++c) m = fmaxf(m, mx[c][lane & 15]);
     return m;
   };
-  auto unit_of = [&](float m) {
-    int e = 0;
-    (void)frexpf(m, &e);
-    return (m > 0.0f && m <= 3.4028235e38f) ? ldexpf(1.0f, e - 6) : 1.0f;
-  };
+  auto unit_of = [&](float m) { return (m > 0.0f && m <= 3.4028235e38f) ? digit_unit(m) : 1.0f; };
   bool poisoned;       // the same in every wave of the workgroup
   {
     float m = 0.0f;

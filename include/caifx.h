@@ -134,7 +134,9 @@ CAIFX_API int caifx_dequantize_int4(const void *packed_data, const void *scales,
  * to the compute type for int8 and for int4 with groups of 128 or more (the products with x are formed
  * exactly instead): results then differ from the formula above by that rounding, about 2e-3 of max|y|.
  * In the int8 kernels of that class a NaN or an infinity among the activations of a row turns every result of
- * that row into NaN (the formula above gives NaN or an infinity in each of them). */
+ * that row into NaN (the formula above gives NaN or an infinity in each of them), except with one row and K <= 4096
+ * where the kernel for whole weight rows runs (groups of 256 rows or more with equal scales along k): there the
+ * results are the formula's. */
 CAIFX_API int caifx_qlinear_forward(int64_t M, int64_t N, int64_t K,
                           const void *x, int x_dtype, int compute_dtype,
                           const void *wq, int w_kind, const void *scales, int64_t scale_period,

@@ -46,3 +46,39 @@ def test_int4_groups_of_128_and_of_256_give_the_same_bits(orc, K, cd):
         x = dev_as(rng.normal(0, 1, (M, K)), cd)
         for yd in (T.F32, cd):
             assert torch.equal(T.qlinear_forward(x, wide, cd, yd), T.qlinear_forward(x, narrow, cd, yd)), (M, yd)
+
+
+def _int8(rng, N, K, period):
+    codes = rng.integers(-127, 128, (N, K)).astype(np.int8)
+    scales = rng.uniform(1e-4, 2e-4, period).astype(np.float32)
+    w = T.FrozenWeight(dev(codes).reshape(-1), T.W_INT8, dev(scales), N, K, period)
+    return codes * scales[np.arange(N * K) % period].reshape(N, K).astype(np.float64), w
+
+
+@pytest.mark.parametrize("yd", [T.F32, T.BF16])
+@pytest.mark.parametrize("N,K,period", [(777, 1024, 1), (1408, 2176, 1), (1000, 3072, 3072), (2048, 3968, 496), (768, 4096, 4096)])
+def test_int8_infinities_come_out_as_the_products_give_them(N, K, period, yd):
+    rng = np.random.default_rng(N + K)
+    w64, w = _int8(rng, N, K, period)
+    for values in ({5: np.inf}, {K - 1: -np.inf}, {0: np.inf, K // 2: np.inf}, {7: np.nan}):
+        x = rng.normal(0, 1, (1, K)).astype(np.float32)
+        for k, v in values.items():
+            x[0, k] = v
+        for xd in (T.BF16, T.F32):
+            got = host(T.qlinear_forward(dev_as(x, xd), w, T.BF16, yd))[0]
+            with np.errstate(invalid="ignore"):
+                want = (x[0].astype(np.float64) * w64).sum(axis=1)
+            assert not np.isfinite(want).any() and np.array_equal(got, want, equal_nan=True), (values, xd)
+
+
+@pytest.mark.parametrize("N,K,period", [(777, 1024, 1), (1408, 2176, 1), (2048, 3968, 496)])
+def test_int8_activations_near_the_end_of_the_exponent_range(N, K, period):
+    # 2^-100 times ordinary values: the same results times 2^-100, to the rounding of code * scale to bf16 (2^-9 each, 4e-3 of the
+    # largest result as for the other decode kernels) and the result's own
+    rng = np.random.default_rng(K)
+    w64, w = _int8(rng, N, K, period)
+    x = dev_as(rng.normal(0, 1, (1, K)), 2)
+    want = w64 @ host(x)[0].astype(np.float64)
+    for shift in (-80, -100, -108):
+        got = host(T.qlinear_forward(x * 2.0 ** shift, w, T.BF16, T.BF16))[0].astype(np.float64) * 2.0 ** -shift
+        assert max_rel_err(got, want) <= 4e-3 + 2.0 ** -8, shift
