@@ -417,7 +417,8 @@ template <typename CT, bool kGrouped> int launch(const Regw8Args &t, int64_t row
 
 }  // namespace
 
-int mfma_regw8_forward(const GemmArgs &a, hipStream_t s)
+// CAIFX_OK and the kernel's arguments where it takes the call
+static int prepare(const GemmArgs &a, Regw8Args &t)
 {
   const bool grouped = a.offsets != nullptr;
   if (a.w.kind != CAIFX_W_INT8) return CAIFX_ERR_UNSUPPORTED;
@@ -440,7 +441,7 @@ int mfma_regw8_forward(const GemmArgs &a, hipStream_t s)
   const int64_t col_tiles = (a.N + kBN - 1) / kBN;
   if (((a.M + BM - 1) / BM) * col_tiles < 128) return CAIFX_ERR_UNSUPPORTED;
 
-  Regw8Args t{};
+  t = Regw8Args{};
   t.M = a.M;
   t.N = a.N;
   t.K = a.K;
@@ -483,7 +484,21 @@ int mfma_regw8_forward(const GemmArgs &a, hipStream_t s)
     t.row_len = static_cast<int>(len);
     t.row_pitch = static_cast<int>(pitch);
   }
-  if (grouped) {
+  return CAIFX_OK;
+}
+
+bool mfma_regw8_takes(const GemmArgs &a)
+{
+  Regw8Args t;
+  return prepare(a, t) == CAIFX_OK;
+}
+
+int mfma_regw8_forward(const GemmArgs &a, hipStream_t s)
+{
+  Regw8Args t;
+  const int st = prepare(a, t);
+  if (st != CAIFX_OK) return st;
+  if (a.offsets) {
     mfma_grouped_stamp_target(&t.stamps, &t.stamps_capacity);
     // segment lengths live on the device: the grid is an upper bound, every expert can add one partial tile
     const int64_t row_tiles = (a.M + BM - 1) / BM + a.num_experts;

@@ -519,6 +519,71 @@ int best_tile(int64_t M, int64_t C, int experts)
   return best;
 }
 
+// What a call costs on this path and on the kernels that dequantise inside the product, in us, for the choice between them
+// (plain form; measured on N(0,1) x N(0,0.02) bf16 values for eleven weights from 2048 x 2048 to 14336 x 4096, 33 to 2048
+// rows, both directions).  A partly filled round costs less than a full one: `base` + `per` for each of its tiles.
+double rounds_cost(int64_t tiles, int64_t slots, double full, double base, double per)
+{
+  const int64_t rest = tiles % slots;
+  return full * static_cast<double>(tiles / slots) + (rest == 0 ? 0.0 : base + per * static_cast<double>(rest));
+}
+double wide_us(const GemmArgs &a, bool backward)
+{
+  const int64_t C = backward ? a.K : a.N, R = backward ? a.N : a.K;
+  const auto tiles = [&](int64_t bm, int64_t bn) { return (a.M + bm - 1) / bm * ((C + bn - 1) / bn); };
+  double step;
+  switch (best_tile(a.M, C, 0)) {
+    case TILE_256: step = rounds_cost(tiles(256, 256), 256, 1.42, 0.75, 0.0026); break;
+    case TILE_128x256: step = rounds_cost(tiles(128, 256), 256, 0.81, 0.25, 0.0022); break;
+    default: {
+      const int64_t t = tiles(128, 128);
+      step = t % 512 <= 256 ? rounds_cost(t, 512, 0.82, 0.24, 0.0008) : rounds_cost(t, 512, 0.82, 0.30, 0.0010);
+    }
+  }
+  // the dense copy, per million weights; of a 16-bit weight beyond 48 million it no longer stays in the memory-side cache
+  const double millions = 1e-6 * static_cast<double>(a.N) * static_cast<double>(a.K);
+  const double copy = a.w.kind == CAIFX_W_INT8          ? 10.0 + 0.42 * millions
+                      : a.w.kind == CAIFX_W_INT4_GROUP ? 10.0 + 0.34 * millions
+                                                       : 6.0 + (millions > 48.0 ? 0.78 : 0.40) * millions;
+  return step * static_cast<double>(R / kBK) + copy;
+}
+// caifx_gemm.hip: 256 x 128 tiles for long reductions with enough of them, else 128 x 128, whose reduction is shared out
+// where at most 128 of them leave compute units idle
+double tiled_us(const GemmArgs &a, bool backward)
+{
+  const int64_t C = backward ? a.K : a.N, R = backward ? a.N : a.K;
+  const bool int8 = a.w.kind == CAIFX_W_INT8, int4 = a.w.kind == CAIFX_W_INT4_GROUP;
+  const int64_t cols = (C + 127) / 128, tall = (a.M + 255) / 256 * cols, tiles = (a.M + 127) / 128 * cols;
+  const double steps = static_cast<double>(R / kBK);
+  // int8 codes with one scale or none are unpacked more slowly than those with a scale vector; without a call's scales (the
+  // workspace query) they are taken to be such
+  const double slower = int8 && a.w.scale_period <= 1 ? 2.3 : 1.0;
+  if (tall >= 200 && R > 2048) return static_cast<double>((tall + 255) / 256) * ((int8 ? 1.10 * slower : int4 ? 1.07 : 1.04) * steps + 2.0);
+  const auto one_each = [&](int64_t t) {       // us per step with up to 256 workgroups
+    return int8 ? 1.07 * slower : int4 ? 0.35 + 0.0015 * static_cast<double>(t) : 0.40 + 0.0009 * static_cast<double>(t);
+  };
+  if (tiles <= 128) {
+    int64_t parts = 256 / tiles;
+    if (parts > 8) parts = 8;
+    if (parts > R / kBK / 8) parts = R / kBK / 8;
+    if (parts >= 2) {
+      const int64_t per = (R / kBK + parts - 1) / parts;
+      return one_each(tiles * parts) * static_cast<double>(per) + 10.0 + 1.6e-6 * static_cast<double>(parts * a.M) * static_cast<double>(C);
+    }
+  }
+  const double two_each = int8 ? 2.14 * slower : int4 ? 1.18 : 1.20;
+  const int64_t rest = tiles % 512;
+  return 5.0 + steps * (two_each * static_cast<double>(tiles / 512) + (rest == 0 ? 0.0 : rest <= 256 ? one_each(rest) : two_each));
+}
+// caifx_gemm_regw.hip and caifx_gemm_regw8.hip: 128 x 256 tiles, one workgroup per compute unit
+double regw_us(const GemmArgs &a)
+{
+  const int64_t tiles = (a.M + 127) / 128 * ((a.N + 255) / 256);
+  const double steps = static_cast<double>(a.K / kBK);
+  if (a.w.kind == CAIFX_W_INT8) return 4.0 + steps * rounds_cost(tiles, 256, 1.10, 0.75, 0.0013);
+  return 4.0 * static_cast<double>((tiles + 255) / 256) + steps * rounds_cost(tiles, 256, 0.90, 0.55, 0.0014);
+}
+
 template <typename CT, bool kGrouped>
 int pick_wide(const WideArgs &g, hipStream_t s)
 {
@@ -539,7 +604,7 @@ bool dense16(const GemmArgs &a)
   return (a.w.kind == CAIFX_W_BF16 && a.compute_dtype == CAIFX_BF16) || (a.w.kind == CAIFX_W_F16 && a.compute_dtype == CAIFX_F16);
 }
 
-// The rule on sizes and types alone (the workspace query knows nothing else).
+// The rule on sizes and types (the workspace query knows nothing else: scale_period is 0 there).
 bool wide_shape(const GemmArgs &a, bool backward)
 {
   if (a.compute_dtype == CAIFX_F32 || a.x_dtype != a.compute_dtype || a.epilogue != 0) return false;
@@ -553,38 +618,39 @@ bool wide_shape(const GemmArgs &a, bool backward)
   if (a.offsets) {
     // Experts with long segments, and copies of all their weights within half of the memory-side cache (128 MB): the
     // dense pass then costs 10 to 20 us and the product gains a quarter.  Forward / input gradient in us, dequantised
-    // inside the product against here, int8, N = 1408, K = 2048: 8 experts, 24576 rows 198 / 216 against 156 / 158, 6000 rows
-    // 80 / 71 against 62 / 55, 4096 rows 42 / 58 against 45 / 52; 16 experts, 12288 rows 126 / 130 against 102 / 104, 8192
-    // rows 81 / 94 against 77 / 94; 33 experts (190 MB), 24576 rows 218 / 243 against 244 / 235; 64 experts (369 MB),
-    // 24576 rows 260 / 283 against 294 / 297, and no better in chunks of experts (8: 432 / 502, 32: 325 / 310, the launches'
-    // ends add up).  Small products: 8 experts, 512 x 512, 8192 rows 14.6 / 18.0 against 16.9 / 18.1, 24576 rows 29.3 / 34.7
-    // against 28.1 / 29.2.  Stored 16-bit weights stay on the tiled kernel (input gradient, 16 experts: 188 against 215 us
-    // with 24576 rows, 157 against 147 with 16384).
+    // inside the product against here, with uniformly drawn ids: N = 1408, K = 2048, 8 experts, 24576 rows, int8 198 / 216
+    // against 156 / 158, int4 190 / 203 against 156 / 137; 33 experts (190 MB), 24576 rows, int8 218 / 243 against 244 / 235.
+    // Over 840 calls (2 to 64 experts, 512 x 512 to 4096 x 4096, 760 to 4096 rows per expert, even and uneven segments, both
+    // storages and directions) the rule below takes 17 % off the mean call it admits; it is slower by more than 2.5 % in six
+    // of them, by up to 16 %, where one more row tile than estimated starts another round (int8, 2 experts, 4096 x 4096, 4000
+    // rows: 148 against 171).  What it leaves out: fewer rows (33 experts, 1024 x 1536, 29700 rows, int8 forward 122 against
+    // 149), reductions of 512 (16 experts, 512 x 2048, 14400 rows, int4 gradient 58 against 64), small products (8 experts,
+    // 512 x 1024, 16000 rows 27 against 36).  Stored 16-bit weights stay on the tiled kernel (input gradient, 16 experts: 188
+    // against 215 us with 24576 rows, 157 against 147 with 16384).
     if (!codes || a.num_experts < 1 || a.num_experts > 65535) return false;
-    return a.M >= 750 * static_cast<int64_t>(a.num_experts) && a.num_experts * a.N * a.K * 2 <= (int64_t{1} << 27) &&
-           static_cast<double>(a.M) * static_cast<double>(a.N) * static_cast<double>(a.K) >= 5e9;
+    const int64_t E = a.num_experts;
+    const double product = static_cast<double>(a.M) * static_cast<double>(a.N) * static_cast<double>(a.K);
+    return a.M >= (a.w.kind == CAIFX_W_INT8 && !backward ? 1250 : 1000) * E && E * a.N * a.K * 2 <= (int64_t{1} << 27) && R >= 768 &&
+           product >= (a.M >= 3000 * E ? 5e9 : 1e10);
   }
   // Is it worth it?  `tiles` counts 128 x 128 tiles.  A stored 16-bit weight needs no extra pass in the forward
   // direction: from 100 tiles on (128: 25.8 against 27.4 us, 256: 31.5 against 39.4; 80: 26.1 against 24.2, where the
-  // tiled kernel shares each tile's reduction among workgroups).
-  if (!codes && !backward) return tiles >= 100;
-  // int4 forward with whole 256-code blocks has a kernel of its own (caifx_gemm_regw.hip): per round of 256 tiles of 128
-  // x 256 about 0.9 us a step and 6 us.  The dense pass costs 3.5 us and 0.33 us per million weights (18 us at 11008 x
-  // 4096), the rest 3 us.  M = 512, N = 11008, K = 4096: 55 against 65 us, M = 2048: 186 against 167.  Calls of up to
-  // one 128 x 128 tile per compute unit go on without a workspace, with the same bits from caifx_qlinear_forward_static
-  // as from here (M = 1024, N = K = 4096: 51 us where this would take 41).
-  const int64_t regw_tiles = ((a.M + 127) / 128) * ((C + 255) / 256);
-  if (!backward && a.w.kind == CAIFX_W_INT4_GROUP && a.K % 256 == 0 && regw_tiles >= 128) {
-    const double steps = static_cast<double>(R / kBK);
-    return tiles > 256 &&
-           3.0 + step_cost(best_tile(a.M, C, 0), a.M, C, 0) * steps + 3.5 + 0.33e-6 * static_cast<double>(a.N) * static_cast<double>(a.K) <
-               (0.9 * steps + 6.0) * static_cast<double>((regw_tiles + 255) / 256);
-  }
-  // Everything else runs on the tiled kernel otherwise (or int8 forward with a short scale vector on
-  // caifx_gemm_regw8.hip): int4 and 16-bit input gradients from 190 tiles on (198: 30.4 against 37.4 us at M = 1367, N =
-  // 2880, K = 2304; 128: 85 against 76), int8, whose unpacking costs those kernels more, from 90 (96 tiles of the
-  // input gradient at N = 5952, K = 2048: 43 against 66 us; 64: 61 against 50).
-  return tiles >= (a.w.kind == CAIFX_W_INT8 ? 90 : 190);
+  // tiled kernel shares each tile's reduction among workgroups; with up to 128 tiles and long reductions that sharing wins:
+  // M = 512, N = 4096, K = 14336 67 against 79 us, K = 11008 57 against 63, K = 4096 27.6 against 24.8).
+  if (!codes && !backward) return tiles >= 100 && (tiles > 128 || R <= 6400);
+  // int4 forward with whole 256-code blocks has a kernel of its own (caifx_gemm_regw.hip).  M = 512, N = 11008, K = 4096: 55
+  // there against 65 us here, M = 2048: 180 against 173, M = 1024: 112 against 94.  K < 2048 stays there (M = 1536, N = 8192,
+  // K = 1024: 37 against 39), and so do calls of up to one 128 x 128 tile per compute unit, which go on without a workspace
+  // and with the same bits from caifx_qlinear_forward_static as from here (M = 1024, N = K = 4096: 51 us where this takes 41).
+  if (!backward && a.w.kind == CAIFX_W_INT4_GROUP && a.K % 256 == 0 && (a.M + 127) / 128 * ((C + 255) / 256) >= 128)
+    return tiles > 256 && a.K >= 2048 && wide_us(a, backward) < regw_us(a);
+  // Everything else runs on the tiled kernel otherwise: int4 and 16-bit input gradients from 190 tiles on (198: 30.4 against
+  // 37.4 us at M = 1367, N = 2880, K = 2304; 128: 85 against 76), int8, whose unpacking costs those kernels more, from 90
+  // (96 tiles of the input gradient at N = 5952, K = 2048: 43 against 66 us; 64: 61 against 50), where the copy is used often
+  // enough to pay: with one or two row tiles of a large weight it is not (N = 14336, K = 4096: int8, M = 64, 47 us there
+  // against 52 here, M = 512 75 against 83; int4, M = 256, 44 against 53; K = 2048 25 against 37; the 16-bit gradient to 14336
+  // columns, M = 256, 43 against 65).
+  return tiles >= (a.w.kind == CAIFX_W_INT8 ? 90 : 190) && wide_us(a, backward) < tiled_us(a, backward);
 }
 
 }  // namespace
@@ -600,6 +666,9 @@ int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s)
   if (!wide_shape(a, backward)) return CAIFX_ERR_UNSUPPORTED;
   const bool grouped = a.offsets != nullptr;      // (the tuned kernels take expert weights to be aligned to 16 bytes)
   if (!aligned_to(a.x, 16) || (!grouped && !aligned_to(a.w.q, 16)) || !aligned_to(a.y, 16) || (a.addend && !aligned_to(a.addend, 16))) return CAIFX_ERR_UNSUPPORTED;
+  // what the workspace query cannot know: int8 forward with one scale, or with a scale vector that fits its LDS table, has a
+  // kernel of its own (one scale, N = 14336, K = 4096, M = 320 59 us there against 75 here, K = 2048, M = 512 41 against 46)
+  if (!grouped && !backward && a.w.kind == CAIFX_W_INT8 && mfma_regw8_takes(a) && regw_us(a) < wide_us(a, false)) return CAIFX_ERR_UNSUPPORTED;
   WideArgs g{};
   g.a = a.x;
   g.d = a.y;
