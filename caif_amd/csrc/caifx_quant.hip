@@ -133,6 +133,9 @@ __global__ void absmax_columns_kernel(const float *__restrict__ in, uint32_t *__
   if (m > 0.0f) atomicMax(acc + c, __float_as_uint(m));
 }
 
+// four floats at any float's alignment: the partial maxima lie in the codes' memory, which needs no more than that
+typedef floatx4_t floatx4_any_t __attribute__((aligned(4)));
+
 // The same with four adjacent columns per thread (cols % 4 == 0, 16-byte aligned input).  A workgroup takes 256 columns of
 // `chunk` rows, its four waves every fourth row with eight 16-byte loads in flight per lane, and writes one partial
 // maximum per column: partial[chunk index][column].  No accumulator to clear and no atomics: the form before this one
@@ -170,7 +173,7 @@ __global__ __launch_bounds__(256) void absmax_columns_x4_kernel(const float *__r
   if (wave == 0 && c < cols) {
 #pragma unroll
     for (int w = 1; w < 4; ++w) take(part[w][lane]);
-    *reinterpret_cast<floatx4_t *>(partial + static_cast<int64_t>(blockIdx.y) * cols + c) = m;
+    *reinterpret_cast<floatx4_any_t *>(partial + static_cast<int64_t>(blockIdx.y) * cols + c) = m;
   }
 }
 

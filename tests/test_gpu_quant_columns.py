@@ -6,7 +6,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-from caif_amd import torch_ops as T                                  # noqa: E402
+from caif_amd import capi, torch_ops as T                                  # noqa: E402
 from gpu_helpers import dev                                           # noqa: E402
 
 
@@ -27,3 +27,18 @@ def test_bit_exact(orc, rows, cols):
     x.copy_(dev(w))
     q2, s2 = T.quantize_int8(x, True)
     assert torch.equal(q2, q) and torch.equal(s2, s)
+
+
+@pytest.mark.parametrize("offset", [4, 8, 12, 1])
+@pytest.mark.parametrize("rows,cols", [(8, 4), (65, 260), (1031, 1028)])
+def test_codes_at_any_address(orc, rows, cols, offset):
+    # a slice of a packed checkpoint: the partial maxima wait in the codes' memory whatever its alignment
+    w = np.random.default_rng(rows + cols).normal(0, 0.02, (rows, cols)).astype(np.float32)
+    src, scales = dev(w), torch.empty(cols, device="cuda")
+    held = torch.full((rows * cols + 32,), 99, dtype=torch.int8, device="cuda")
+    codes = held[offset:offset + rows * cols]
+    capi.call("caifx_quantize_int8_per_channel", src.data_ptr(), codes.data_ptr(), scales.data_ptr(), rows, cols,
+              torch.cuda.current_stream().cuda_stream)
+    qo, so = orc.quantize_int8_per_channel(w)
+    assert np.array_equal(codes.cpu().numpy().reshape(rows, cols), qo) and np.array_equal(scales.cpu().numpy(), so)
+    assert bool((held[:offset] == 99).all()) and bool((held[offset + rows * cols:] == 99).all())
