@@ -286,10 +286,12 @@ __global__ __launch_bounds__(kRouteThreads) void combine_bwd_kernel(const T *gou
 // token and one row at a time 16 tokens of 2048 took 14.4 us, a chain of 24 memory round trips.
 // The rows and weights of a token are fetched once per batch of 8 assignments by lanes 0..7 and broadcast.
 constexpr int kGatherWavesMax = 8;
-__host__ __device__ inline int gather_waves(int64_t dim, int n)
+__host__ __device__ inline int gather_waves(int64_t dim, int n, int64_t num_tokens)
 {
   const int64_t pieces = (dim + 64 * n - 1) / (64 * n);
-  return pieces < kGatherWavesMax ? static_cast<int>(pieces) : kGatherWavesMax;
+  int waves = pieces < kGatherWavesMax ? static_cast<int>(pieces) : kGatherWavesMax;
+  while (waves > 1 && num_tokens * waves > (int64_t{1} << 26) - 4) waves /= 2;      // a grid has fewer than 2^32 threads
+  return waves;
 }
 template <typename T, bool kWeighted, bool kVec>
 __global__ __launch_bounds__(kRouteThreads) void gather_sum_kernel(const T *buf, const int32_t *idx, const T *w,
@@ -300,7 +302,7 @@ __global__ __launch_bounds__(kRouteThreads) void gather_sum_kernel(const T *buf,
   constexpr int n = kVec ? Vec16<T>::kN : 1;
   typedef typename Vec16<T>::type v_t;
   const int lane = threadIdx.x & 63;
-  const int per_token = gather_waves(dim, n);
+  const int per_token = gather_waves(dim, n, num_tokens);
   const int64_t wave = (static_cast<int64_t>(blockIdx.x) * kRouteThreads + threadIdx.x) >> 6;
   const int64_t t = wave / per_token;
   if (t >= num_tokens) return;
@@ -546,7 +548,7 @@ int caifx_moe_combine(const void *expert_buffer, const int32_t *expert_indices, 
   if (!expert_weights) return CAIFX_ERR_INVALID_ARGUMENT;
   hipStream_t s = as_stream(stream);
   const bool vec = (dim * dtype_size(dtype)) % 16 == 0 && aligned_to(expert_buffer, 16) && aligned_to(output, 16);
-  const dim3 grid(wave_blocks(num_tokens * gather_waves(dim, vec ? 16 / static_cast<int>(dtype_size(dtype)) : 1))), block(kRouteThreads);
+  const dim3 grid(wave_blocks(num_tokens * gather_waves(dim, vec ? 16 / static_cast<int>(dtype_size(dtype)) : 1, num_tokens))), block(kRouteThreads);
 #define CAIFX_GO(T)                                                                                                    \
   if (vec)                                                                                                             \
     hipLaunchKernelGGL((gather_sum_kernel<T, true, true>), grid, block, 0, s, static_cast<const T *>(expert_buffer),   \
@@ -636,7 +638,7 @@ int caifx_moe_dispatch_backward(const void *grad_expert_buffer, const int32_t *e
   if (st >= 0) return st;
   hipStream_t s = as_stream(stream);
   const bool vec = (dim * dtype_size(dtype)) % 16 == 0 && aligned_to(grad_expert_buffer, 16) && aligned_to(grad_input, 16);
-  const dim3 grid(wave_blocks(num_tokens * gather_waves(dim, vec ? 16 / static_cast<int>(dtype_size(dtype)) : 1))), block(kRouteThreads);
+  const dim3 grid(wave_blocks(num_tokens * gather_waves(dim, vec ? 16 / static_cast<int>(dtype_size(dtype)) : 1, num_tokens))), block(kRouteThreads);
 #define CAIFX_GO(T)                                                                                                    \
   if (vec)                                                                                                             \
     hipLaunchKernelGGL((gather_sum_kernel<T, false, true>), grid, block, 0, s,                                         \
