@@ -45,8 +45,8 @@ class CaifxError(RuntimeError):
 
 
 def build(jobs=8):
-    """Compile every HIP source for gfx950 into caif_amd/lib/libcaifx.so (always recompiles)."""
-    subprocess.check_call(["make", "-C", CSRC, "-B", f"-j{jobs}", "all"],
+    """Compile every HIP source for gfx950 into caif_amd/lib/libcaifx.so, and the native side of torch_ops (always recompiles)."""
+    subprocess.check_call(["make", "-C", CSRC, "-B", f"-j{jobs}", "all", "torch_calls"],
                           stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
     return LIB_PATH
 
