@@ -172,8 +172,14 @@ struct Workspace {
       p = t.data_ptr();
       bytes = static_cast<size_t>(t.numel());
     } else if ((bytes = query()) > 0) {
-      held = bytes_like(x, bytes);
-      p = held.data_ptr();
+      // the workspace is optional: on a card that is full up to the result the calls run without it, as those kernels do that
+      // never asked for one
+      try {
+        held = bytes_like(x, bytes);
+        p = held.data_ptr();
+      } catch (const c10::OutOfMemoryError &) {
+        bytes = 0;
+      }
     }
   }
 };

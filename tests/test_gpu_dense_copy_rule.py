@@ -24,3 +24,24 @@ def test_the_scales_decide(M, N, K, backward, per_channel, copies):
     workspace = torch.zeros(2 * N * K, dtype=torch.uint8, device="cuda")
     run(x, w, T.BF16, workspace=workspace)
     assert bool(workspace[-4096:].any()) == copies
+
+
+def test_a_full_card_does_without_the_copy():
+    # the copy is 128 MB more than the call needs: where they cannot be had the call runs on the kernels without it
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    M, N, K = 2048, 8192, 8192
+    codes, scales = T.quantize_int8(torch.empty(K, N, device="cuda").normal_(generator=gen), True)
+    w = T.FrozenWeight(codes.reshape(-1), T.W_INT8, scales, N, K, N)
+    x = torch.empty(M, N, device="cuda").normal_(generator=gen).to(torch.bfloat16)
+    out = torch.empty(M, K, device="cuda", dtype=torch.bfloat16)
+    want = T.qlinear_backward_input(x, w, T.BF16, T.BF16, workspace=torch.empty(0, dtype=torch.uint8, device="cuda"))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (32 << 20)) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(2 * N * K, dtype=torch.uint8, device="cuda")
+        assert torch.equal(T.qlinear_backward_input(x, w, T.BF16, T.BF16, out=out), want)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
