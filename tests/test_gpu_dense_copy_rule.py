@@ -28,11 +28,14 @@ def test_the_scales_decide(M, N, K, backward, per_channel, copies):
 
 def test_a_full_card_does_without_the_copy():
     # the copy is 128 MB more than the call needs: where they cannot be had the call runs on the kernels without it
+    # tensors made in place, without larger temporaries: blocks they left behind would have room for the copy
     gen = torch.Generator(device="cuda").manual_seed(3)
     M, N, K = 2048, 8192, 8192
-    codes, scales = T.quantize_int8(torch.empty(K, N, device="cuda").normal_(generator=gen), True)
-    w = T.FrozenWeight(codes.reshape(-1), T.W_INT8, scales, N, K, N)
-    x = torch.empty(M, N, device="cuda").normal_(generator=gen).to(torch.bfloat16)
+    torch.cuda.empty_cache()
+    codes = torch.randint(-127, 128, (N * K,), device="cuda", dtype=torch.int8, generator=gen)
+    scales = torch.full((N,), 1e-3, device="cuda")
+    w = T.FrozenWeight(codes, T.W_INT8, scales, N, K, N)
+    x = torch.empty(M, N, device="cuda", dtype=torch.bfloat16).normal_(generator=gen)
     out = torch.empty(M, K, device="cuda", dtype=torch.bfloat16)
     want = T.qlinear_backward_input(x, w, T.BF16, T.BF16, workspace=torch.empty(0, dtype=torch.uint8, device="cuda"))
     torch.cuda.synchronize()
