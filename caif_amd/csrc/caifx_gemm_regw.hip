@@ -347,24 +347,19 @@ template <typename CT, int WR> int launch(const RegwArgs &t, hipStream_t s)
 
 }  // namespace
 
-bool mfma_regw_takes(const GemmArgs &a)
-{
-  if (a.w.kind != CAIFX_W_INT4_GROUP || a.offsets != nullptr || a.epilogue != 0) return false;
-  if (a.compute_dtype == CAIFX_F32 || a.x_dtype != a.compute_dtype) return false;
-  if (a.w.group_size != kGroup) return false;
-  if (a.K % 256 != 0 || a.K < 512 || a.K > (int64_t{1} << 22)) return false;
-  if (a.N * a.K >= (int64_t{1} << 32) || a.M > (int64_t{1} << 30)) return false;
-  if (!aligned_to(a.x, 16) || !aligned_to(a.w.q, 16) || !aligned_to(a.w.scales, 4) || !aligned_to(a.y, 16) ||
-      (a.addend && !aligned_to(a.addend, 16)))
-    return false;
-  // enough 128 x 256 tiles to give most compute units one; below that the tiled kernel's shared reduction wins
-  const int64_t tiles128 = ((a.M + 127) / 128) * ((a.N + kBN - 1) / kBN);
-  return tiles128 >= 128;
-}
-
 int mfma_regw_forward(const GemmArgs &a, hipStream_t s)
 {
-  if (!mfma_regw_takes(a)) return CAIFX_ERR_UNSUPPORTED;
+  if (a.w.kind != CAIFX_W_INT4_GROUP || a.offsets != nullptr || a.epilogue != 0) return CAIFX_ERR_UNSUPPORTED;
+  if (a.compute_dtype == CAIFX_F32 || a.x_dtype != a.compute_dtype) return CAIFX_ERR_UNSUPPORTED;
+  if (a.w.group_size != kGroup) return CAIFX_ERR_UNSUPPORTED;
+  if (a.K % 256 != 0 || a.K < 512 || a.K > (int64_t{1} << 22)) return CAIFX_ERR_UNSUPPORTED;
+  if (a.N * a.K >= (int64_t{1} << 32) || a.M > (int64_t{1} << 30)) return CAIFX_ERR_UNSUPPORTED;
+  if (!aligned_to(a.x, 16) || !aligned_to(a.w.q, 16) || !aligned_to(a.w.scales, 4) || !aligned_to(a.y, 16) ||
+      (a.addend && !aligned_to(a.addend, 16)))
+    return CAIFX_ERR_UNSUPPORTED;
+  // enough 128 x 256 tiles to give most compute units one; below that the tiled kernel's shared reduction wins
+  const int64_t tiles128 = ((a.M + 127) / 128) * ((a.N + kBN - 1) / kBN);
+  if (tiles128 < 128) return CAIFX_ERR_UNSUPPORTED;
   RegwArgs t{};
   t.M = a.M;
   t.N = a.N;

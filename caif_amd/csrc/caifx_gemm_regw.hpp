@@ -114,8 +114,7 @@ __device__ __forceinline__ void store_tile(unsigned char *smem, const floatx16_t
 // int8 counterpart of mfma_regw_forward, plain and grouped: scale vectors (or one scale, or none) whose table fits
 // 16 KiB of LDS, K a multiple of 128.  CAIFX_ERR_UNSUPPORTED for everything else.
 int mfma_regw8_forward(const GemmArgs &a, hipStream_t s);
-// Whether mfma_regw_forward (caifx_gemm_regw.hip) and mfma_regw8_forward take the call.
-bool mfma_regw_takes(const GemmArgs &a);
+// Whether mfma_regw8_forward takes the call.
 bool mfma_regw8_takes(const GemmArgs &a);
 // where grouped launches record their tiles (see mfma_grouped_tile_stamps); null when switched off
 void mfma_grouped_stamp_target(unsigned long long **buf, long long *capacity);

@@ -666,15 +666,9 @@ int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s)
   if (!wide_shape(a, backward)) return CAIFX_ERR_UNSUPPORTED;
   const bool grouped = a.offsets != nullptr;      // (the tuned kernels take expert weights to be aligned to 16 bytes)
   if (!aligned_to(a.x, 16) || (!grouped && !aligned_to(a.w.q, 16)) || !aligned_to(a.y, 16) || (a.addend && !aligned_to(a.addend, 16))) return CAIFX_ERR_UNSUPPORTED;
-  // What the workspace query cannot know.  int8 forward with one scale, or with a scale vector that fits its LDS table, has a
-  // kernel of its own (one scale, N = 14336, K = 4096, M = 320 59 us there against 75 here, K = 2048, M = 512 41 against 46).
-  // The 128 x 256 tile stores fp32 results in two passes with nothing else on the compute unit, 8 us a round: against the
-  // int4 forward kernel that decides (M = 2048, N = 11008, K = 4096: 186 us there, 202 here; bf16 results 180 and 171).
-  if (!grouped && !backward && (a.w.kind == CAIFX_W_INT8 ? mfma_regw8_takes(a) : a.w.kind == CAIFX_W_INT4_GROUP && mfma_regw_takes(a))) {
-    const int64_t tiles = (a.M + 127) / 128 * ((a.N + 255) / 256);
-    const bool slow_store = a.y_dtype == CAIFX_F32 && best_tile(a.M, a.N, 0) == TILE_128x256;
-    if (regw_us(a) < wide_us(a, false) + (slow_store ? 8.0 * static_cast<double>((tiles + 255) / 256) : 0.0)) return CAIFX_ERR_UNSUPPORTED;
-  }
+  // what the workspace query cannot know: int8 forward with one scale, or with a scale vector that fits its LDS table, has a
+  // kernel of its own (one scale, N = 14336, K = 4096, M = 320 59 us there against 75 here, K = 2048, M = 512 41 against 46)
+  if (!grouped && !backward && a.w.kind == CAIFX_W_INT8 && mfma_regw8_takes(a) && regw_us(a) < wide_us(a, false)) return CAIFX_ERR_UNSUPPORTED;
   WideArgs g{};
   g.a = a.x;
   g.d = a.y;
