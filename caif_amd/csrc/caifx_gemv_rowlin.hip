@@ -1222,9 +1222,7 @@ template <typename CT, typename XT, int MT>
 int launch_int4(const RowArgs &ra, hipStream_t s)
 {
   if constexpr (dtype_code<XT>::value == dtype_code<CT>::value) {
-    // fp32 results with a partial last chunk stay on the dynamic kernel: the same bits, and only whole chunks and 16-bit
-    // results have been timed on both
-    if (ra.group_shift == 7 && (ra.K % 2048 == 0 || ra.y_dtype != CAIFX_F32)) {
+    if (ra.group_shift == 7) {
       const int st = ra.K % 2048 == 0 ? pick_int4_fast<CT, MT, false>(ra, s) : pick_int4_fast<CT, MT, true>(ra, s);
       if (st != CAIFX_ERR_UNSUPPORTED) return st;
     }
@@ -1376,10 +1374,9 @@ int rowlin_forward(const GemmArgs &g, hipStream_t s)
     ra.waves_per_class = ra.total_waves;
     if (static_cast<size_t>(mt) * ra.xpitch * 2 + 4096 > 64 * 1024) return CAIFX_ERR_UNSUPPORTED;
   } else {
-    // one activation row and 4096 < K <= 16384: the integer-matrix-core kernel with the row split among waves.  fp32 results
-    // with a partial last chunk stay on the row-block kernel, the one they have been timed on (error against 64 bits 5.8e-7
-    // there; here 3.0e-7 to 3.5e-7, measured with whole chunks)
-    const bool long_digits = g.M == 1 && g.K > 4096 && g.K <= 16384 && (g.K % 1024 == 0 || g.y_dtype != CAIFX_F32);
+    // one activation row and 4096 < K <= 16384: the integer-matrix-core kernel with the row split among waves.  The
+    // result's type does not decide: a 16-bit result is the fp32 result rounded
+    const bool long_digits = g.M == 1 && g.K > 4096 && g.K <= 16384;
     if (g.K % 16 != 0 || (g.K > 4096 && !long_digits)) return CAIFX_ERR_UNSUPPORTED;
     ra.cpr = static_cast<int>((g.K + 1023) / 1024);
     ra.xpitch = ra.cpr * 1024;
