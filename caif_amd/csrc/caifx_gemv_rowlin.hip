@@ -1374,9 +1374,13 @@ int rowlin_forward(const GemmArgs &g, hipStream_t s)
     ra.waves_per_class = ra.total_waves;
     if (static_cast<size_t>(mt) * ra.xpitch * 2 + 4096 > 64 * 1024) return CAIFX_ERR_UNSUPPORTED;
   } else {
-    // one activation row and 4096 < K <= 16384: the integer-matrix-core kernel with the row split among waves.  The
-    // result's type does not decide: a 16-bit result is the fp32 result rounded
-    const bool long_digits = g.M == 1 && g.K > 4096 && g.K <= 16384;
+    // One activation row and 4096 < K <= 16384: the integer-matrix-core kernel with the row split among waves (whole chunks: 1.0
+    // to 2.1 times as fast as the row-block kernel).  With a partial last chunk it loads less evenly and wins where the rows
+    // are many or short (K = 6400, N = 14336 22.7 against 26.3 us, K = 4224, N = 3072 10.2 against 11.6, K = 11008, N = 11008 30.7
+    // against 48.3) and loses in between (K = 11008, N = 4096 17.6 against 16.2, K = 13824, N = 5120 23.4 against 20.1).
+    // The result's type does not decide: a 16-bit result is the fp32 result rounded.
+    const bool whole = g.K % 1024 == 0, many_or_short = g.N >= 11008 || (g.K <= 8192 && (g.N >= 6144 || g.K <= 6144));
+    const bool long_digits = g.M == 1 && g.K > 4096 && g.K <= 16384 && (whole || many_or_short);
     if (g.K % 16 != 0 || (g.K > 4096 && !long_digits)) return CAIFX_ERR_UNSUPPORTED;
     ra.cpr = static_cast<int>((g.K + 1023) / 1024);
     ra.xpitch = ra.cpr * 1024;

@@ -9,13 +9,13 @@ from caif_amd import torch_ops as T                                  # noqa: E40
 from gpu_helpers import dev, dev_as, host, max_rel_err               # noqa: E402
 
 
-@pytest.mark.parametrize("K", [1024, 2048, 3072, 4096, 5120, 11264, 14336, 16384, 3968, 11008])
+@pytest.mark.parametrize("K", [1024, 2048, 3072, 4096, 5120, 11264, 14336, 16384, 3968, 5504])
 @pytest.mark.parametrize("period", [1, 0])
 def test_int8_digits_reach_2_to_the_minus_21_of_the_largest_activation(K, period):
     # One activation of 1 meets a code of 0 in every row and each lane's unit is set by others like it; the rest are odd
     # multiples of 2^-21, which digits of 2^-21 or finer hold exactly: what is left is the fp32 sum of at most 16384
-    # terms in a tree (2^-20 of the largest result), and for whole chunks the fp32 result shows it.  A partial last chunk takes
-    # these kernels with 16-bit results only (half the spacing of 8-bit significands, 2^-8).
+    # terms in a tree (2^-20 of the largest result), and a 16-bit result's rounding (half the spacing of 8-bit significands, 2^-8).
+    # Partial last chunks beyond K = 6144 need more rows than these for the kernel to be chosen.
     rng = np.random.default_rng(K)
     N = 1500                            # one residue class of 256 rows or more: the row-linear kernels are taken
     codes = rng.integers(-127, 128, (N, K)).astype(np.int8)
@@ -26,7 +26,7 @@ def test_int8_digits_reach_2_to_the_minus_21_of_the_largest_activation(K, period
     w = T.FrozenWeight(dev(codes).reshape(-1), T.W_INT8, scales, N, K, 1 if period == 1 else K)
     want = codes.astype(np.float64) @ x
     xd = dev_as(x[None], 2)
-    for yd in ((T.F32, T.BF16) if K % 1024 == 0 else (T.BF16,)):
+    for yd in (T.F32, T.BF16):
         got = host(T.qlinear_forward(xd, w, T.BF16, yd))[0]
         assert max_rel_err(got, want) <= 2.0 ** -20 + (2.0 ** -8 if yd == T.BF16 else 0), yd
 
