@@ -24,7 +24,7 @@ EXPORTS = [
     "caifx_quantize_int8_per_tensor", "caifx_dequantize_int8_per_tensor",
     "caifx_quantize_int8_per_channel", "caifx_dequantize_int8_per_channel",
     "caifx_quantize_to_int4", "caifx_dequantize_int4",
-    "caifx_qlinear_forward", "caifx_qlinear_backward_input", "caifx_qlinear_workspace_bytes",
+    "caifx_qlinear_forward", "caifx_qlinear_backward_input", "caifx_qlinear_workspace_bytes", "caifx_qlinear_partials_workspace_bytes",
     "caifx_qlinear_forward_static", "caifx_static_scratch_prepare", "caifx_probe_mfma_bf16", "caifx_qlinear_grouped_tile_stamps",
     "caifx_qlinear_forward_add", "caifx_qlinear_backward_input_add", "caifx_qlinear_grouped_backward_input_add",
     "caifx_qlinear_grouped_forward", "caifx_qlinear_grouped_backward_input",
@@ -88,6 +88,8 @@ def lib():
         L.caifx_qlinear_backward_input_add.argtypes = gemm_add
         L.caifx_qlinear_workspace_bytes.restype = _sz
         L.caifx_qlinear_workspace_bytes.argtypes = [_i64, _i64, _i64, _int, _int, _int, _int]
+        L.caifx_qlinear_partials_workspace_bytes.restype = _sz
+        L.caifx_qlinear_partials_workspace_bytes.argtypes = [_i64, _i64, _i64, _int, _int, _int, _int]
         grouped = [_int, _p, _i64, _i64, _i64, _p, _int, _int, _p, _int, _p, _i64, _int, _p, _int, _p, _sz, _p]
         L.caifx_qlinear_grouped_forward.argtypes = grouped
         L.caifx_qlinear_grouped_backward_input.argtypes = grouped

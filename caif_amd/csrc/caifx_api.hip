@@ -136,6 +136,12 @@ size_t caifx_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtyp
   return workspace_bytes(M, N, K, x_dtype, compute_dtype, w_kind, backward != 0, true);
 }
 
+size_t caifx_qlinear_partials_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype, int compute_dtype, int w_kind,
+                                     int backward)
+{
+  return workspace_bytes(M, N, K, x_dtype, compute_dtype, w_kind, backward != 0, false);
+}
+
 // `addend` (optional): the matrix-core GEMM adds it in its store; every other path runs as usual and is
 // followed by the element-wise Add in place, which rounds in the same two places
 static int finish_add(int st, const void *addend, void *y, int y_dtype, int64_t n, caifx_stream_t stream)

@@ -129,7 +129,8 @@ CAIFX_API int caifx_dequantize_int4(const void *packed_data, const void *scales,
  * output type (:442), F16/BF16 fold the caller's following `.To(StorageT)` cast
  * (src/caif_device_moe_frozen_expert.cpp:119-126) into the store and give the
  * same bits as writing fp32 and casting.
- * compute_dtype is the layer's ComputeT.  No dense copy of W is ever written.
+ * compute_dtype is the layer's ComputeT.  A dense copy of W is written by large calls only, into the caller's workspace
+ * (see caifx_qlinear_workspace_bytes).
  * With up to 32 rows and a 16-bit compute type the memory-bound kernels skip the rounding of code * scale
  * to the compute type for int8 and for int4 with groups of 128 or more (the products with x are formed
  * exactly instead): results then differ from the formula above by that rounding, about 2e-3 of max|y|.
@@ -184,8 +185,15 @@ CAIFX_API int caifx_qlinear_backward_input_add(int64_t M, int64_t N, int64_t K,
                                      void *workspace, size_t workspace_bytes, caifx_stream_t stream);
 
 /* Bytes of workspace the calls above can use for this problem (may be 0).
- * backward != 0 asks for caifx_qlinear_backward_input.  Nonzero for 16-bit compute types when the result has
- * fewer 128 x 128 tiles than the chip has compute units: up to 8 workgroups then share a tile's reduction through
+ * backward != 0 asks for caifx_qlinear_backward_input.  Two things use it: partial tiles of shared reductions, and in
+ * large calls a dense copy of the weight.
+ * The dense copy: int8 and int4 codes, and the input gradient of a weight stored in the 16-bit compute type, with activations
+ * of that type, when the result has enough tiles (90 of 128 x 128 or more for int8, 190 otherwise) that the copy, 2 N K bytes,
+ * is made up for by the faster product behind it (N K < 2^32: 8 GiB at most, 90 MB for 11008 x 4096).  The size does not
+ * know the scales: a call whose scales make another kernel the faster one leaves that part unused.  With less workspace the
+ * large calls run on the kernels that dequantise inside the product, up to three times as slow, their sums in another order.
+ * The partial tiles (caifx_qlinear_partials_workspace_bytes asks for them alone): nonzero for 16-bit compute types when the
+ * result has fewer 128 x 128 tiles than the chip has compute units: up to 8 workgroups then share a tile's reduction through
  * fp32 partial tiles in the workspace (16-byte aligned) and a second launch adds them in a fixed order (results do
  * not depend on scheduling).  The fp32 compute type does the same for up to 128 rows.  The forward with up to
  * 32 rows cuts a reduction longer than one workgroup covers into slices whose sums meet there (K > 4096 with up
@@ -201,14 +209,20 @@ CAIFX_API int caifx_qlinear_backward_input_add(int64_t M, int64_t N, int64_t K,
  * int4 with a 16-bit compute type multiplies the rounded weight either way). */
 CAIFX_API size_t caifx_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype, int compute_dtype,
                                      int w_kind, int backward);
+/* The same without the dense copy of large calls: what is left is a few partial tiles, at most 16 MiB for the 16-bit compute
+ * types' tiled kernel.  For callers that pay for every allocation (a pool that returns its memory at each synchronisation). */
+CAIFX_API size_t caifx_qlinear_partials_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype, int compute_dtype,
+                                     int w_kind, int backward);
 
 /* caifx_qlinear_forward for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc) and so have no workspace to pass: the fp32 partial tiles of a
  * shared reduction go to a buffer of CAIFX_STATIC_SCRATCH_BYTES that is part of the library's device image (one
  * copy per GPU, held until the process ends) instead of the caller's workspace.  It has no counterpart in the
  * reference, whose layers allocate freely.  Same arguments, kernels and results (bit for bit) as
- * caifx_qlinear_forward called with a workspace of caifx_qlinear_workspace_bytes(..., backward = 0) bytes.
- * A problem for which that size exceeds CAIFX_STATIC_SCRATCH_BYTES returns CAIFX_ERR_SCRATCH_EXCEEDED and
+ * caifx_qlinear_forward called with a workspace of caifx_qlinear_partials_workspace_bytes(..., backward = 0) bytes:
+ * everything but the dense copy that large calls make in the larger workspace of caifx_qlinear_workspace_bytes, with
+ * which their last bits differ (fp32 sums in another order).
+ * A problem whose partial tiles exceed CAIFX_STATIC_SCRATCH_BYTES returns CAIFX_ERR_SCRATCH_EXCEEDED and
  * launches nothing (use caifx_qlinear_forward then; with a null workspace it runs without sharing).
  * The call itself allocates and frees nothing.  Every call on one GPU uses that GPU's one buffer: calls on
  * different streams of the same GPU that may overlap race on it; calls on one stream are ordered and need no
@@ -227,11 +241,11 @@ CAIFX_API int caifx_qlinear_forward_static(int64_t M, int64_t N, int64_t K,
 
 /* Measurement only, no counterpart in the reference (whose per-expert loop, src/caif_device_moe_layer.cpp:534-557,
  * can simply be timed expert by expert on the host): grouped launches of the matrix-core GEMM issued after this
- * call record four 64-bit words per tile (128 rows x 128 columns, or x 256 for the int8 forward kernel that keeps
- * the weight out of LDS) - {expert, rows of the segment inside the tile (low 32 bits; from bit 32 up, when not 0,
- * how many workgroups of that kernel share a compute unit instead of two), start, end}, times in ticks of the
+ * call record four 64-bit words per tile (128 rows x 128 columns, x 256 for the int8 forward kernel that keeps
+ * the weight out of LDS, and 128 x 128, 128 x 256 or 256 x 256 where the experts' weights are copied first) - {expert, rows of the segment inside the tile (low 32 bits; from bit 32 up, when not 0,
+ * how many workgroups share a compute unit instead of two), start, end}, times in ticks of the
  * GPU's 100 MHz wall clock - into `stamps` (device memory for `tiles` tiles, 32 bytes each; sizing for 128 x 128
- * tiles covers both; tiles are numbered expert by expert, row tile by row tile, column tile last; clear it before
+ * tiles covers all of them; tiles are numbered expert by expert, row tile by row tile, column tile last; clear it before
  * a launch, words of tiles that do not exist stay as they are).  stamps = NULL switches the recording off.
  * Process-wide state; not meant for timed runs (one more store per workgroup). */
 CAIFX_API int caifx_qlinear_grouped_tile_stamps(void *stamps, int64_t tiles);
@@ -295,8 +309,8 @@ CAIFX_API int caifx_qlinear_grouped_backward_input_add(int num_experts, const in
 /* The up projection of CAIF_DeviceMoEFrozenExpert::ForwardImpl with the expert's gating folded into its store
  * (src/caif_device_moe_frozen_expert.cpp:119-153: up_out.To(StorageT); SiLU(gate); Multiply): for the rows of
  * the segments up[r,:] = T(x[r,:] * W_e^T) and hidden[r,:] = T(T(silu(gate[r,:])) * up[r,:]), with the cast
- * points of the three separate launches (the result equals caifx_qlinear_grouped_forward followed by
- * caifx_silu_mul bit for bit).  gate, up, hidden: [total_rows,N] of out_dtype (CAIFX_F16 or CAIFX_BF16),
+ * points of the three separate launches (the result equals caifx_qlinear_grouped_forward without a workspace followed
+ * by caifx_silu_multiply bit for bit).  gate, up, hidden: [total_rows,N] of out_dtype (CAIFX_F16 or CAIFX_BF16),
  * pairwise distinct.  CAIFX_ERR_UNSUPPORTED for shapes the matrix-core kernel does not take or results that
  * are not 16-byte aligned with N % 8 == 0 (the caller then uses the separate calls).  This form and the one
  * below save a launch and, in the backward, the grad-of-hidden buffer; at 64 experts x 24576 rows (2048 <-> 1408)
@@ -312,7 +326,7 @@ CAIFX_API int caifx_qlinear_grouped_forward_swiglu(int num_experts, const int32_
 /* The input gradient of the down projection in CAIF_DeviceMoEFrozenExpert::BackwardImpl with the gating's
  * backward folded into its store (src/caif_device_moe_frozen_expert.cpp:252-290): with h = T(dy[r,:] * W_e)
  * (never written), grad_up[r,:] = T(h * T(silu(gate[r,:]))) and grad_gate[r,:] = T(silu'(gate[r,:]) * T(h * up[r,:]))
- * (equal to caifx_qlinear_grouped_backward_input followed by caifx_swiglu_backward bit for bit).  gate, up,
+ * (equal to caifx_qlinear_grouped_backward_input without a workspace followed by caifx_swiglu_backward bit for bit).  gate, up,
  * grad_gate, grad_up: [total_rows,K] of out_dtype (16-bit), pairwise distinct.  CAIFX_ERR_UNSUPPORTED as above. */
 CAIFX_API int caifx_qlinear_grouped_backward_input_swiglu(int num_experts, const int32_t *offsets, int64_t total_rows,
                                                 int64_t N, int64_t K,
@@ -322,6 +336,9 @@ CAIFX_API int caifx_qlinear_grouped_backward_input_swiglu(int num_experts, const
                                                 int group_size,
                                                 const void *gate, const void *up, void *grad_gate, void *grad_up,
                                                 int out_dtype, caifx_stream_t stream);
+/* Bytes of workspace the grouped forward and input gradient can use (may be 0): dense copies of all the experts' weights,
+ * 2 E N K bytes, for int8 and int4 codes with long segments (1000 rows per expert and more) whose copies stay below 128 MB.
+ * Without it they run on the kernels that dequantise inside the product. */
 CAIFX_API size_t caifx_qlinear_grouped_workspace_bytes(int num_experts, int64_t total_rows, int64_t N, int64_t K,
                                              int x_dtype, int compute_dtype, int w_kind, int backward);
 
