@@ -170,6 +170,27 @@ static void GpuTests()
     base->SetOffloadPolicy(CAIF_OffloadPolicy::CAIF_OffloadPolicy_e::GpuResident_e);
     Report("back to GpuResident works",Download(layer->Forward(in,infer))==before);
   }
+  {
+    // per call the layer allocates its result and partial tiles, no dense copy of the weight (32 MiB here)
+    const uint32_t k=2048,n=8192,m=1024;
+    std::unique_ptr<CAIF_DeviceLayer> layer=CAIF_DeviceFrozenLinearFactory::Create(k,n,Dtype_e::Int8,stream,128,true,Dtype_e::BFloat16,Scheme::PerTensor_e);
+    CAIF_DeviceFrozenLinearBase *base=dynamic_cast<CAIF_DeviceFrozenLinearBase*>(layer.get());
+    base->LoadFromTensor(CAIF_DeviceTensor::Zeros({k,n},stream,Dtype_e::Int8));
+    const float scale=1.0f;
+    base->LoadScalesFromHost(&scale,sizeof(scale));
+    CAIF_DeviceTensor in=CAIF_DeviceTensor::Zeros({m,k},stream,Dtype_e::BFloat16);
+    layer->Forward(in,infer);
+    stream.Synchronize();
+    hipMemPool_t pool;
+    uint64_t zero=0,used=0,high=0;
+    bool ok=hipDeviceGetDefaultMemPool(&pool,0)==hipSuccess&&
+            hipMemPoolGetAttribute(pool,hipMemPoolAttrUsedMemCurrent,&used)==hipSuccess&&
+            hipMemPoolSetAttribute(pool,hipMemPoolAttrUsedMemHigh,&zero)==hipSuccess;
+    layer->Forward(in,infer);
+    stream.Synchronize();
+    ok=ok&&hipMemPoolGetAttribute(pool,hipMemPoolAttrUsedMemHigh,&high)==hipSuccess;
+    Report("a large forward allocates no copy of the weight",ok&&high>used&&high-used<=static_cast<uint64_t>(m)*n*4+(16u<<20));
+  }
   stream.Synchronize();
 }
 
