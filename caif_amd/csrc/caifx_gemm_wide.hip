@@ -3,17 +3,18 @@
 // transposed on the way), and a dense kernel multiplies it with the activations.  A weight stored in the 16-bit compute
 // type needs no first launch in the forward direction.
 //
-// What bounds it: the power the chip may draw.  On all-zero operands the kernel runs at 2.0-2.1 PFLOP/s, on N(0,1)
-// activations x N(0,0.02) weights at 1.53-1.56 (M = 4096, C = 4096, R = 11008: 236 us), so what counts is work per
-// flop, not only what waits for what:
+// What bounds it: the power the chip may draw.  On all-zero operands the kernel runs at 2.03 PFLOP/s and a clock of 2.47
+// GHz, on N(0,1) activations x N(0,0.02) weights at 1.50 to 1.56 and 1.99 GHz, in the same number of cycles (M = 4096, C =
+// 4096, R = 11008: 236 to 247 us), so what counts is work per flop, not only what waits
+// for what:
 //  - v_mfma_f32_16x16x32 instead of 32x32x16: the same loop without any memory traffic runs at 2.07 instead of 1.80
 //    PFLOP/s on those values (a 16 x 16 result is read and written once per 32 reduction elements, a 32 x 32 one once
 //    per 16), the whole kernel at 236 instead of 254 us.
 //  - four waves with 128 x 128 of the 256 x 256 tile each (one wave per SIMD, 256 accumulators in the accumulation
 //    registers): 128 KB of operand reads from LDS per 64-deep step; eight waves of 128 x 64 read 192 KB (262 us).
 //  - the weight is dequantised once per call instead of once per row tile.
-// Against the kernels that dequantise inside the product (forward 380 us, input gradient 385 us at M = 4096, N = 11008,
-// K = 4096, int4, bf16) the two launches take 290 and 257 us.
+// Against the kernels that dequantise inside the product (forward 361 us, input gradient 390 us at M = 4096, N = 11008,
+// K = 4096, int4, bf16) the two launches take 293 and 251 us in the same run.
 #include "caifx_gemm_regw.hpp"
 
 #include <atomic>
@@ -621,8 +622,8 @@ bool wide_shape(const GemmArgs &a, bool backward)
     // inside the product against here, with uniformly drawn ids: N = 1408, K = 2048, 8 experts, 24576 rows, int8 198 / 216
     // against 156 / 158, int4 190 / 203 against 156 / 137; 33 experts (190 MB), 24576 rows, int8 218 / 243 against 244 / 235.
     // Over 840 calls (2 to 64 experts, 512 x 512 to 4096 x 4096, 760 to 4096 rows per expert, even and uneven segments, both
-    // storages and directions) the rule below takes 17 % off the mean call it admits; it is slower by more than 2.5 % in six
-    // of them, by up to 16 %, where one more row tile than estimated starts another round (int8, 2 experts, 4096 x 4096, 4000
+    // storages and directions) the 546 that the rule below admits are 1.26 times as fast in the mean; six are slower by more
+    // than 2.5 %, by up to 16 %, where one more row tile than estimated starts another round (int8, 2 experts, 4096 x 4096, 4000
     // rows: 148 against 171).  What it leaves out: fewer rows (33 experts, 1024 x 1536, 29700 rows, int8 forward 122 against
     // 149), reductions of 512 (16 experts, 512 x 2048, 14400 rows, int4 gradient 58 against 64), small products (8 experts,
     // 512 x 1024, 16000 rows 27 against 36).  Stored 16-bit weights stay on the tiled kernel (input gradient, 16 experts: 188

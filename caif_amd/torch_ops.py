@@ -1,9 +1,10 @@
-"""Thin callers of the C ABI for torch-owned device buffers (tests and bench.py plumbing).
+"""Callers of the C ABI for torch-owned device buffers: the library's Python entry points.
 
 torch supplies device memory and the current HIP stream; every computation is a
 call into libcaifx.so.  The calls of a training or serving step go through native code
-(csrc/torch_calls.cpp: checks, result and workspace allocation, stream), the rest through ctypes.  Function names follow the reference's CAIF_Ops entry
-points (src/caif_ops.cpp:504-680); argument meaning is the same.
+(csrc/torch_calls.cpp: checks, result and workspace allocation, stream), the rest through
+ctypes.  Function names follow the reference's CAIF_Ops entry points
+(src/caif_ops.cpp:504-680); argument meaning is the same.
 """
 import torch
 
