@@ -613,7 +613,8 @@ bool wide_shape(const GemmArgs &a, bool backward)
   if (!codes && !dense16(a)) return false;
   const int64_t C = backward ? a.K : a.N, R = backward ? a.N : a.K;
   if (R % kBK != 0 || C % 8 != 0 || a.K % 8 != 0 || a.M < 1 || R < 2 * kBK) return false;
-  if (a.N * a.K >= (int64_t{1} << 32) || a.M > (int64_t{1} << 30) || R > (int64_t{1} << 22)) return false;
+  // (the transposing pass has R / 64 rows of workgroups, kept below the 65536 of a grid)
+  if (a.N * a.K >= (int64_t{1} << 32) || a.M > (int64_t{1} << 30) || R >= (int64_t{1} << 22)) return false;
   const int64_t tiles = ((a.M + 127) / 128) * ((C + 127) / 128);
   if (tiles > (int64_t{1} << 30)) return false;
   if (a.offsets) {

@@ -30,6 +30,10 @@ def test_a_copy_that_pays_is_made(kind, backward, M, N, K):
     assert _copies(M, N, K, kind, backward)
 
 
+def test_reductions_longer_than_a_grid_of_the_transposing_pass():
+    assert _copies(8192, (1 << 22) - 64, 512, INT8, 1) and not _copies(8192, 1 << 22, 512, INT8, 1)
+
+
 def _grouped_copies(E, rows, N, K, kind, backward):
     return capi.lib().caifx_qlinear_grouped_workspace_bytes(E, rows, N, K, BF16, BF16, kind, backward) == 2 * E * N * K
 
