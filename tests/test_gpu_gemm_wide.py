@@ -106,3 +106,28 @@ def test_the_copy_is_made_and_used(orc, kind, backward, M, N, K):
     add = dev_as(rng.normal(0, 1, (M, C)), cd)
     plain = host(run(x, dw, cd, cd))[sel]
     assert max_rel_err(host(run(x, dw, cd, cd, addend=add))[sel], plain + host(add)[sel]) <= ULP[cd]
+
+
+@pytest.mark.parametrize("kind", ["int4", "int8pc"])
+def test_replays_of_a_captured_step(orc, kind):
+    # the copy and the product of both directions in one graph: every replay, with new inputs in the captured buffers and eager
+    # work in between, gives the eager call's bits
+    rng = np.random.default_rng(77)
+    M, N, K = 2049, 4096, 4096
+    _, dw = make_weight(orc, rng, N, K, kind)
+    x, dy = (torch.empty(M, n, device="cuda", dtype=torch.bfloat16) for n in (K, N))
+    a, b = (torch.empty(M, n, device="cuda", dtype=torch.bfloat16) for n in (N, K))
+    step = lambda: (T.qlinear_forward(x, dw, T.BF16, T.BF16, addend=a), T.qlinear_backward_input(dy, dw, T.BF16, T.BF16, addend=b))      # noqa: E731
+    fill = lambda: [t.normal_() for t in (x, dy, a, b)]      # noqa: E731
+    fill()
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step()
+    for _ in range(4):
+        fill()
+        graph.replay()
+        want = step()
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, w) for g, w in zip(got, want))

@@ -22,8 +22,7 @@ def test_16_bit_results_are_the_fp32_results_rounded(kind, M, N, K):
     if kind == "bf16":
         w = T.FrozenWeight(normal(N, K).to(torch.bfloat16).reshape(-1), T.W_BF16, None, N, K)
     elif kind == "int4":
-        if K % 128:
-            pytest.skip("groups of 128")
+        K = max(K // 128 * 128, 128)
         p, s = T.quantize_int4_per_group(normal(N, K), 128)
         w = T.FrozenWeight(p, T.W_INT4_GROUP, s, N, K, 1, 128)
     else:
