@@ -67,7 +67,7 @@ struct MbArgs {
   int period;            // int8: length of the scale vector, 0 = one scale (or none)
   int V;                 // residue classes the rows are split into (1 unless period > 0)
   int blocks_per_class;  // gridDim.x = blocks_per_class * V
-  int scale_step;        // int8 scale vector: 1024 mod period (staging stride of the workgroup)
+  int scale_step;        // int8 scale vector: 64 mod period (staging stride of a wave)
   // K beyond one workgroup's reach: blockIdx.y takes the k range [y * slice_groups * 128, ...) and writes its
   // share of the sums as fp32 to partial + y * M * N; a second launch adds the shares in a fixed order
   int slice_groups;      // 128-k groups per slice (= groups when there is one slice)
@@ -159,8 +159,8 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   float *partial = reinterpret_cast<float *>(smem);      // [RBB][MT][16 waves][4][64]
   float *ybuf = partial + RBB * MT * kPartialFloats;     // [16 * MT activation rows][kSegRows]
-  float *svec = ybuf + 16 * MT * kSegRows;               // int8: the scale vector of this slice [slice k]; int4 with
-                                                         // MT > 1: the group-sum corrections [MT][GPW][16 waves][16]
+  float *svec = ybuf + 16 * MT * kSegRows;               // int8: the scales of every wave's k range [16 waves][GPW * 128];
+                                                         // int4 with MT > 1: the group-sum corrections [MT][GPW][16 waves][16]
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -210,7 +210,14 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
     xg[mt] = static_cast<const XT *>(xrows) + static_cast<int64_t>(16 * mt + j < M ? 16 * mt + j : M - 1) * a.K + kbase;
-  if constexpr (!kF32) {
+  // fp32 compute type: the values themselves where they fit the registers (fp32 activations, one tile, one group per wave)
+  constexpr bool kHoldF32 = kF32 && sizeof(XT) == 4 && MT == 1 && GPW == 1;
+  floatx4_t xf[kHoldF32 ? 8 : 1];
+  if constexpr (kHoldF32) {
+    const int gg = g0 < groups ? g0 : groups - 1;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) xf[c] = *reinterpret_cast<const floatx4_t *>(xg[0] + gg * 128 + (c >> 2) * 64 + q * 16 + 4 * (c & 3));
+  } else if constexpr (!kF32) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -223,14 +230,21 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
         }
       }
   }
-  // int8 scale vector of this residue class: svec[k] = scales[(cls*K + k) mod period], K <= 4096
+  // int8 scales of this residue class, scales[(cls*K + k) mod period], for this wave's own k range: a wave reads back
+  // only what it staged, so nobody waits for the slowest wave's scales (with the vector staged by the whole workgroup
+  // and a barrier behind it, 16 rows: N = 4096, K = 2048 8.1 -> 7.0 us, N = 13568, K = 1280 10.1 -> 8.8, N = 14336, K = 4096
+  // 18.9 -> 18.0).  Waves past the last group stage in-range entries that meet zero activations.
   float s_one = 1.0f;
-  float sv[4] = {1.0f, 1.0f, 1.0f, 1.0f};     // without a scale vector the staged scales are 1
+  constexpr int kScaleLoads = 2 * GPW;
+  float sv[kScaleLoads];
+#pragma unroll
+  for (int t = 0; t < kScaleLoads; ++t) sv[t] = 1.0f;     // without a scale vector the staged scales are 1
+  float *swave = svec + wave * (GPW * 128);
   if constexpr (!kInt4) {
     if (a.period > 0) {
-      int idx = static_cast<int>((static_cast<int64_t>(cls) * a.K + kbase + threadIdx.x) % a.period);
+      int idx = static_cast<int>((static_cast<int64_t>(cls) * a.K + kbase + g0 * 128 + lane) % a.period);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < kScaleLoads; ++t) {
         sv[t] = s32[idx];
         idx += a.scale_step;
         if (idx >= a.period) idx -= a.period;
@@ -257,10 +271,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
   }
   if constexpr (!kInt4) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int k = threadIdx.x + t * kMbThreads;
-      if (k < groups * 128) svec[k] = sv[t];
-    }
+    for (int t = 0; t < kScaleLoads; ++t) swave[64 * t + lane] = sv[t];
   }
 
   // int4: the nibbles unpack in the order 0,4,1,5,2,6,3,7, so X is stored that way; and
@@ -315,13 +326,17 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
       poison[mt][r] = false;
     }
   if constexpr (!kInt4) {
-    __syncthreads();       // svec is complete
+    __builtin_amdgcn_wave_barrier();       // the wave's scales are staged
     // four consecutive x' values: quad c (0..3) of step t of tile mt
     auto xprime4 = [&](int mt, int t, int c, float (&v)[4]) {
       const int g = t >> 1;
-      const int gg = g0 + g < groups ? g0 + g : groups - 1;
       if constexpr (kF32) {
+        const int gg = g0 + g < groups ? g0 + g : groups - 1;
         const bool live = g0 + g < groups && 16 * mt + j < M;
+        if constexpr (kHoldF32) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = live ? xf[4 * (t & 1) + c][i] : 0.0f;
+        } else {
         const XT *px = xg[mt] + gg * 128 + (t & 1) * 64 + q * 16 + 4 * c;
         if constexpr (sizeof(XT) == 4) {
           const floatx4_t xv = *reinterpret_cast<const floatx4_t *>(px);
@@ -333,12 +348,13 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
 #pragma unroll
           for (int i = 0; i < 4; ++i) v[i] = live ? to_f32<XT>(h[i]) : 0.0f;
         }
+        }
       } else {
         const vec_t xv = xa[mt][g][2 * (t & 1) + (c >> 1)];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = to_f32<CT>(xv[4 * (c & 1) + i]);
       }
-      const floatx4_t sc4 = *reinterpret_cast<const floatx4_t *>(svec + gg * 128 + (t & 1) * 64 + q * 16 + 4 * c);
+      const floatx4_t sc4 = *reinterpret_cast<const floatx4_t *>(swave + g * 128 + (t & 1) * 64 + q * 16 + 4 * c);
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] *= sc4[i];
     };
@@ -353,7 +369,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
       // first pass: x' = x * scale, kept in registers for the second pass; the largest |x'| and whether all are finite
       float xp[kSteps][16];
       float mx = 0.0f;
-      bool finite = true;
+      float nan_if_bad = 0.0f;
 #pragma unroll
       for (int t = 0; t < kSteps; ++t)
 #pragma unroll
@@ -364,14 +380,14 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
           for (int i = 0; i < 4; ++i) {
             xp[t][4 * c + i] = v[i];
             mx = fmaxf(mx, fabsf(v[i]));                       // ignores a NaN
-            finite = finite && fabsf(v[i]) <= 3.4028235e38f;    // false for NaN and infinities
+            nan_if_bad = __builtin_fmaf(v[i], 0.0f, nan_if_bad);      // NaN from a NaN or an infinity on
           }
         }
       mx = fmaxf(mx, __shfl_xor(mx, 16));
       mx = fmaxf(mx, __shfl_xor(mx, 32));      // over the four k quarters: row j's largest |x'| in this wave's k range
       // A NaN or an infinity among row j's scaled activations has no digits.  The reference's GEMM returns NaN or an
       // infinity in every output of that activation row; here this wave's share of them, and so their sum, is NaN.
-      const int bad = (__ballot(!finite) >> j & 0x0001000100010001ull) != 0 ? 1 : 0;
+      const int bad = (__ballot(!(nan_if_bad == 0.0f)) >> j & 0x0001000100010001ull) != 0 ? 1 : 0;
       mx = bad ? 1.0f : mx;
 #pragma unroll
       for (int r = 0; r < 4; ++r) poison[mt][r] = __shfl(bad, 4 * q + r) != 0;
@@ -669,7 +685,7 @@ static int64_t mb_slice_k(const GemmArgs &g)
 static size_t mb_lds_bytes(bool int4, int mt, int slice_groups)
 {
   size_t floats = static_cast<size_t>(mb_reduce_blocks(int4, mt)) * mt * kPartialFloats + static_cast<size_t>(16) * mt * kSegRows;
-  if (!int4) floats += static_cast<size_t>(slice_groups) * 128;      // staged scales (ones without a scale vector)
+  if (!int4) floats += static_cast<size_t>((slice_groups + kMbWaves - 1) / kMbWaves) * kMbWaves * 128;      // staged scales (ones without a scale vector)
   else if (mt > 1) floats += static_cast<size_t>(mt) * mb_max_gpw(true, mt) * kMbWaves * 16;      // group-sum corrections
   return floats * sizeof(float);
 }
@@ -736,7 +752,7 @@ int mblock_forward(const GemmArgs &g, hipStream_t s)
     const int64_t V = P / gcd64(g.K % P == 0 ? P : g.K % P, P);
     if (V * 64 > g.N) return CAIFX_ERR_UNSUPPORTED;      // too few rows per residue class
     m.period = static_cast<int>(P);
-    m.scale_step = static_cast<int>(kMbThreads % P);
+    m.scale_step = static_cast<int>(64 % P);
     m.V = static_cast<int>(V);
   }
   const size_t lds = mb_lds_bytes(int4, mt, m.slice_groups);
@@ -789,7 +805,7 @@ int mblock_grouped_forward(const GemmArgs &g, hipStream_t s)
     const int64_t V = P / gcd64(g.K % P == 0 ? P : g.K % P, P);
     if (V * 64 > g.N) return CAIFX_ERR_UNSUPPORTED;
     m.period = static_cast<int>(P);
-    m.scale_step = static_cast<int>(kMbThreads % P);
+    m.scale_step = static_cast<int>(64 % P);
     m.V = static_cast<int>(V);
   }
   const size_t lds = mb_lds_bytes(int4, 1, m.groups);
