@@ -52,7 +52,7 @@ template <> struct Mfma16<f16_t> {
 
 constexpr int kMbWaves = 16;
 constexpr int kMbThreads = kMbWaves * 64;
-constexpr int kPartialFloats = kMbWaves * 4 * 64;     // one buffer of per-wave partial tiles
+constexpr int kPartialFloats(int waves) { return waves * 4 * 64; }     // one buffer of per-wave partial tiles
 
 struct MbArgs {
   const uint8_t *wq;
@@ -145,11 +145,11 @@ constexpr int kSegRows = kSegBlocks * 16;
 // MT: tiles of 16 activation rows that share one pass over the weight (M <= 16 * MT); every weight fragment is
 // unpacked once and multiplied with each tile's operands.
 // wq / scales: the weight; xrows / yrows: the first of the M activation and result rows; slice: which part of
-// the reduction (see MbArgs).  Every thread of the workgroup makes the same calls (the body has barriers).
+// the reduction (see MbArgs); rows n = cls + V * i of the weight for i in [i_lo, i_hi).  Every thread of the workgroup makes the same calls (the body has barriers).
 // D: row blocks a wave keeps requested (1 or 2; the launch code picks by measurement)
-template <typename CT, typename XT, bool kInt4, int GPW, bool kF32, int MT = 1, int D = 2>
+template <typename CT, typename XT, bool kInt4, int GPW, bool kF32, int MT = 1, int D = 2, int W = kMbWaves>
 __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, const void *scales, const void *xrows,
-                                            void *yrows, int M, int slice)
+                                            void *yrows, int M, int slice, int cls, int64_t i_lo, int64_t i_hi)
 {
   static_assert(!(kF32 && kInt4), "the fp32 compute type is for int8 storage");
   typedef typename Mfma16<CT>::vec_t vec_t;
@@ -157,23 +157,15 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
   constexpr int LPR = GPW * LPG;               // ... per block of 16 weight rows
   constexpr int RBB = mb_reduce_blocks(kInt4, MT);      // row blocks between two reductions (a multiple of D, divides kSegBlocks)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  float *partial = reinterpret_cast<float *>(smem);      // [RBB][MT][16 waves][4][64]
-  float *ybuf = partial + RBB * MT * kPartialFloats;     // [16 * MT activation rows][kSegRows]
-  float *svec = ybuf + 16 * MT * kSegRows;               // int8: the scales of every wave's k range [16 waves][GPW * 128];
-                                                         // int4 with MT > 1: the group-sum corrections [MT][GPW][16 waves][16]
+  float *partial = reinterpret_cast<float *>(smem);      // [RBB][MT][W waves][4][64]
+  float *ybuf = partial + RBB * MT * kPartialFloats(W);     // [16 * MT activation rows][kSegRows]
+  float *svec = ybuf + 16 * MT * kSegRows;               // int8: the scales of every wave's k range [W waves][GPW * 128];
+                                                         // int4 with MT > 1: the group-sum corrections [MT][GPW][W waves][16]
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15;        // weight row within the block (B column) / activation row (A row)
   const int q = lane >> 4;        // quarter of the 32-wide k step
-  const int cls = blockIdx.x / a.blocks_per_class;
-  const int bc = blockIdx.x - cls * a.blocks_per_class;
-  const int64_t rows_class = (a.N - cls + a.V - 1) / a.V;          // rows n = cls + V*i, i < rows_class
-  // every workgroup of a class takes the same number of consecutive rows (the last block of 16 may
-  // be partly masked): equal bytes per compute unit matter more than full MFMA tiles
-  const int64_t per_block = (rows_class + a.blocks_per_class - 1) / a.blocks_per_class;
-  const int64_t i_lo = bc * per_block;
-  const int64_t i_hi = i_lo + per_block < rows_class ? i_lo + per_block : rows_class;
   const int nrb = i_hi > i_lo ? static_cast<int>((i_hi - i_lo + 15) / 16) : 0;
   if (nrb == 0) return;           // the whole workgroup; nothing has been started yet
   const int g0 = wave * GPW;
@@ -306,7 +298,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
           for (int r = 0; r < 4; ++r) cor[g][r] = Mfma16<CT>::kOffset * xsum[r];
         } else if (j == 0) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) corbuf[(mt * GPW + g) * (kMbWaves * 16) + 4 * q + r] = Mfma16<CT>::kOffset * xsum[r];
+          for (int r = 0; r < 4; ++r) corbuf[(mt * GPW + g) * (W * 16) + 4 * q + r] = Mfma16<CT>::kOffset * xsum[r];
         }
       }
     if constexpr (MT > 1) __syncthreads();
@@ -461,7 +453,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
 #pragma unroll
                   for (int r = 0; r < 4; ++r) tot[u][mt][r] = __builtin_fmaf(sr, acc[mt][r] - cor[g][r], tot[u][mt][r]);
                 } else {
-                  const floatx4_t cr = *reinterpret_cast<const floatx4_t *>(corbuf + (mt * GPW + g) * (kMbWaves * 16) + 4 * q);
+                  const floatx4_t cr = *reinterpret_cast<const floatx4_t *>(corbuf + (mt * GPW + g) * (W * 16) + 4 * q);
 #pragma unroll
                   for (int r = 0; r < 4; ++r) tot[u][mt][r] = __builtin_fmaf(sr, acc[mt][r] - cr[r], tot[u][mt][r]);
                 }
@@ -501,15 +493,15 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) partial[(((u * MT + mt) * kMbWaves + wave) * 4 + r) * 64 + lane] = tot[u][mt][r];
+          for (int r = 0; r < 4; ++r) partial[(((u * MT + mt) * W + wave) * 4 + r) * 64 + lane] = tot[u][mt][r];
       __syncthreads();
-      for (int idx = threadIdx.x; idx < RBB * MT * 256; idx += kMbThreads) {
+      for (int idx = threadIdx.x; idx < RBB * MT * 256; idx += (64 * W)) {
         const int um = idx >> 8;             // u * MT + mt
         const int r = (idx >> 6) & 3;
         const int l = idx & 63;
         float v = 0.0f;
 #pragma unroll
-        for (int wv = 0; wv < kMbWaves; ++wv) v += partial[((um * kMbWaves + wv) * 4 + r) * 64 + l];
+        for (int wv = 0; wv < W; ++wv) v += partial[((um * W + wv) * 4 + r) * 64 + l];
         const int m = 16 * (um % MT) + 4 * (l >> 4) + r;
         ybuf[m * kSegRows + (base - seg0 + um / MT) * 16 + (l & 15)] = v;
       }
@@ -519,7 +511,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
     const int64_t i_seg = i_lo + static_cast<int64_t>(seg0) * 16;
     const int seg_rows = static_cast<int>(i_hi - i_seg < kSegRows ? i_hi - i_seg : kSegRows);
     float *part = a.partial ? a.partial + static_cast<int64_t>(slice) * M * a.N : nullptr;
-    for (int idx = threadIdx.x; idx < M * seg_rows; idx += kMbThreads) {
+    for (int idx = threadIdx.x; idx < M * seg_rows; idx += (64 * W)) {
       const int m = idx / seg_rows;
       const int r = idx - m * seg_rows;
       const int64_t o = static_cast<int64_t>(m) * a.N + cls + a.V * (i_seg + r);
@@ -532,36 +524,90 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
 template <typename CT, typename XT, bool kInt4, int GPW, bool kF32 = false, int MT = 1, int D = 2>
 __global__ __launch_bounds__(kMbThreads) void mblock_kernel(MbArgs a)
 {
-  mblock_body<CT, XT, kInt4, GPW, kF32, MT, D>(a, a.wq, a.scales, a.x, a.y, a.M, blockIdx.y);
+  const int cls = blockIdx.x / a.blocks_per_class;
+  const int bc = blockIdx.x - cls * a.blocks_per_class;
+  const int64_t rows_class = (a.N - cls + a.V - 1) / a.V;          // rows n = cls + V*i, i < rows_class
+  // every workgroup of a class takes the same number of consecutive rows (the last block of 16 may
+  // be partly masked): equal bytes per compute unit matter more than full MFMA tiles
+  const int64_t per_block = (rows_class + a.blocks_per_class - 1) / a.blocks_per_class;
+  const int64_t i_lo = bc * per_block;
+  const int64_t i_hi = i_lo + per_block < rows_class ? i_lo + per_block : rows_class;
+  mblock_body<CT, XT, kInt4, GPW, kF32, MT, D>(a, a.wq, a.scales, a.x, a.y, a.M, blockIdx.y, cls, i_lo, i_hi);
 }
 
-// Token-sorted expert segments with few rows each (MoE decode): blockIdx.y is the expert, whose weight is streamed
-// once per 16 rows of its segment; an expert without rows costs nothing.  The host only knows the total row
-// count, so routing may hand one expert most of the rows: the 16-row passes of a segment are dealt out over
-// blockIdx.z, and a long segment is worked on by gridDim.z times as many workgroups instead of gridDim.z times
-// as long (its weight then comes from L2 after the first pass).
+// Token-sorted expert segments with few rows each (MoE decode).  An expert's weight is streamed once per 16 rows of its
+// segment (a pass); an expert without rows costs nothing.  Every pass is V units, one per residue class of the weight's
+// rows, of `unit` blocks of 16 weight rows, listed expert by expert, class by class, pass by pass (a class's passes side by
+// side: the second finds the weight in L2).  The list of blocks is cut into equal runs, one per workgroup and one workgroup
+// per compute unit: with a workgroup per expert and class the 550 that 16 tokens x 6 of 64 experts (2048 -> 1408) wake
+// made 2.15 rounds of the chip and were paid as three.  A workgroup prepares its activations once per unit it touches.
 struct MbGroup {
   const int32_t *offsets;
   const void *const *wq_ptrs;
   const void *const *scales_ptrs;
   int64_t total_rows;
+  int num_experts;
+  unsigned unit_blocks, pass_blocks;      // blocks of 16 rows in a unit, and in a pass (V units)
 };
 template <typename CT, typename XT, bool kInt4, int GPW>
 __global__ __launch_bounds__(kMbThreads) void mblock_grouped_kernel(MbArgs a, MbGroup g)
 {
-  const int e = blockIdx.y;
-  int lo, hi;
-  segment_rows(g.offsets, e, g.total_rows, lo, hi);
-  if (hi <= lo) return;
-  const uint8_t *wq = static_cast<const uint8_t *>(g.wq_ptrs[e]);
-  const void *scales = g.scales_ptrs ? g.scales_ptrs[e] : nullptr;
+  const int lane = threadIdx.x & 63;
+  // passes of experts base + lane, and their running count within the 64
+  int lo = 0, hi = 0, passes = 0, incl = 0;
+  auto look = [&](int base) __attribute__((always_inline)) {
+    lo = hi = 0;
+    if (base + lane < g.num_experts) segment_rows(g.offsets, base + lane, g.total_rows, lo, hi);
+    passes = (hi - lo + 15) / 16;
+    incl = passes;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += up;
+    }
+    return __builtin_amdgcn_readlane(incl, 63);       // (scalar: everything derived from it stays out of the lanes' registers)
+  };
+  int total = 0;
+  for (int base = 0; base < g.num_experts; base += 64) total += look(base);
+  const unsigned blocks = static_cast<unsigned>(total) * g.pass_blocks;          // < 2^31 (host)
+  const unsigned per = (blocks + gridDim.x - 1) / gridDim.x;
+  const unsigned start = blockIdx.x * per;
+  int todo = start < blocks ? static_cast<int>(blocks - start < per ? blocks - start : per) : 0;
+  int u = static_cast<int>(start / g.unit_blocks);                               // unit, and the run's first block in it
+  int first = static_cast<int>(start - u * g.unit_blocks);
   const size_t ybytes = a.y_dtype == CAIFX_F32 ? 4 : 2;
-  const int first = lo + 16 * static_cast<int>(blockIdx.z);
-  for (int r = first; r < hi; r += 16 * static_cast<int>(gridDim.z)) {
-    if (r > first) __syncthreads();      // the pass before has read its staging buffers
-    mblock_body<CT, XT, kInt4, GPW, false>(a, wq, scales, static_cast<const XT *>(a.x) + static_cast<int64_t>(r) * a.K,
+  int base = g.num_experts <= 64 ? 0 : -1;          // which 64 experts the lanes hold
+  int before = 0;                                   // units of the experts in front of them
+  while (todo > 0) {
+    const int count = static_cast<int>(g.unit_blocks) - first < todo ? static_cast<int>(g.unit_blocks) - first : todo;
+    if (base < 0 || u >= before + __builtin_amdgcn_readlane(incl, 63) * a.V) {      // more than 64 experts: find the group of 64
+      before = 0;
+      for (base = 0;; base += 64) {
+        const int n = look(base) * a.V;
+        if (u < before + n) break;          // u < total * V
+        before += n;
+      }
+    }
+    const int in_group = u - before;
+    const unsigned long long owners = __ballot(incl * a.V > in_group);
+    const int src = __builtin_ctzll(owners);
+    const int e = base + src;
+    const int np = __builtin_amdgcn_readlane(passes, src);
+    const int within = in_group - (__builtin_amdgcn_readlane(incl, src) - np) * a.V;
+    const int cls = __builtin_amdgcn_readfirstlane(within / np);
+    const int r = __builtin_amdgcn_readlane(lo, src) + 16 * (within - cls * np);
+    const int end = __builtin_amdgcn_readlane(hi, src);
+    const int rows_class = (static_cast<int>(a.N) - cls + a.V - 1) / a.V;          // N <= 2^30 (host)
+    const int i_lo = first * 16;
+    const int i_hi = i_lo + count * 16 < rows_class ? i_lo + count * 16 : rows_class;
+    // (no barrier between units: a unit's partial tiles and result staging are written behind barriers of its own)
+    mblock_body<CT, XT, kInt4, GPW, false>(a, static_cast<const uint8_t *>(g.wq_ptrs[e]), g.scales_ptrs ? g.scales_ptrs[e] : nullptr,
+                                           static_cast<const XT *>(a.x) + static_cast<int64_t>(r) * a.K,
                                            static_cast<char *>(a.y) + static_cast<int64_t>(r) * a.N * ybytes,
-                                           hi - r < 16 ? hi - r : 16, 0);
+                                           end - r < 16 ? end - r : 16, 0, cls, i_lo, i_hi);
+    todo -= count;
+    first = 0;
+    u += 1;
   }
 }
 
@@ -610,13 +656,23 @@ int launch_gpw(const MbArgs &m, size_t lds, hipStream_t s)
   return launch_status();
 }
 
-template <typename CT, typename XT, bool kInt4>
-int launch_grouped_gpw(const MbArgs &m, const MbGroup &g, int experts, size_t lds, hipStream_t s)
+int compute_units()
 {
-  // up to eight passes of a segment side by side: with every row in one expert a segment has g.total_rows / 16 passes
-  const int64_t passes = (g.total_rows + 15) / 16;
-  const dim3 grid(static_cast<unsigned>(m.blocks_per_class * m.V), static_cast<unsigned>(experts),
-                  static_cast<unsigned>(passes < 8 ? (passes < 1 ? 1 : passes) : 8));
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+      cus = n;
+    else
+      cus = 256;
+  }
+  return cus;
+}
+
+template <typename CT, typename XT, bool kInt4>
+int launch_grouped_gpw(const MbArgs &m, const MbGroup &g, size_t lds, hipStream_t s)
+{
+  const dim3 grid(static_cast<unsigned>(compute_units()));
   const int gpw = (m.groups + kMbWaves - 1) / kMbWaves;
   if (gpw <= 1) hipLaunchKernelGGL((mblock_grouped_kernel<CT, XT, kInt4, 1>), grid, dim3(kMbThreads), lds, s, m, g);
   else if (gpw <= 2) hipLaunchKernelGGL((mblock_grouped_kernel<CT, XT, kInt4, 2>), grid, dim3(kMbThreads), lds, s, m, g);
@@ -625,13 +681,13 @@ int launch_grouped_gpw(const MbArgs &m, const MbGroup &g, int experts, size_t ld
 }
 
 template <typename CT>
-int launch_grouped_xt(const MbArgs &m, const MbGroup &g, int experts, int x_dtype, bool int4, size_t lds, hipStream_t s)
+int launch_grouped_xt(const MbArgs &m, const MbGroup &g, int x_dtype, bool int4, size_t lds, hipStream_t s)
 {
   if (x_dtype == CAIFX_F32)
-    return int4 ? launch_grouped_gpw<CT, float, true>(m, g, experts, lds, s) : launch_grouped_gpw<CT, float, false>(m, g, experts, lds, s);
+    return int4 ? launch_grouped_gpw<CT, float, true>(m, g, lds, s) : launch_grouped_gpw<CT, float, false>(m, g, lds, s);
   if (x_dtype == CAIFX_F16)
-    return int4 ? launch_grouped_gpw<CT, f16_t, true>(m, g, experts, lds, s) : launch_grouped_gpw<CT, f16_t, false>(m, g, experts, lds, s);
-  return int4 ? launch_grouped_gpw<CT, bf16_t, true>(m, g, experts, lds, s) : launch_grouped_gpw<CT, bf16_t, false>(m, g, experts, lds, s);
+    return int4 ? launch_grouped_gpw<CT, f16_t, true>(m, g, lds, s) : launch_grouped_gpw<CT, f16_t, false>(m, g, lds, s);
+  return int4 ? launch_grouped_gpw<CT, bf16_t, true>(m, g, lds, s) : launch_grouped_gpw<CT, bf16_t, false>(m, g, lds, s);
 }
 
 template <typename XT>
@@ -646,19 +702,6 @@ int launch_xt(const MbArgs &m, int x_dtype, bool int4, size_t lds, hipStream_t s
   if (x_dtype == CAIFX_F32) return int4 ? launch_gpw<CT, float, true>(m, lds, s) : launch_gpw<CT, float, false>(m, lds, s);
   if (x_dtype == CAIFX_F16) return int4 ? launch_gpw<CT, f16_t, true>(m, lds, s) : launch_gpw<CT, f16_t, false>(m, lds, s);
   return int4 ? launch_gpw<CT, bf16_t, true>(m, lds, s) : launch_gpw<CT, bf16_t, false>(m, lds, s);
-}
-
-int compute_units()
-{
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-      cus = n;
-    else
-      cus = 256;
-  }
-  return cus;
 }
 
 }  // namespace
@@ -682,10 +725,10 @@ static int64_t mb_slice_k(const GemmArgs &g)
   return g.N <= n_max ? reach / 2 : reach;
 }
 
-static size_t mb_lds_bytes(bool int4, int mt, int slice_groups)
+static size_t mb_lds_bytes(bool int4, int mt, int slice_groups, int waves = kMbWaves)
 {
-  size_t floats = static_cast<size_t>(mb_reduce_blocks(int4, mt)) * mt * kPartialFloats + static_cast<size_t>(16) * mt * kSegRows;
-  if (!int4) floats += static_cast<size_t>((slice_groups + kMbWaves - 1) / kMbWaves) * kMbWaves * 128;      // staged scales (ones without a scale vector)
+  size_t floats = static_cast<size_t>(mb_reduce_blocks(int4, mt)) * mt * kPartialFloats(waves) + static_cast<size_t>(16) * mt * kSegRows;
+  if (!int4) floats += static_cast<size_t>((slice_groups + waves - 1) / waves) * waves * 128;      // staged scales (ones without a scale vector)
   else if (mt > 1) floats += static_cast<size_t>(mt) * mb_max_gpw(true, mt) * kMbWaves * 16;      // group-sum corrections
   return floats * sizeof(float);
 }
@@ -809,14 +852,11 @@ int mblock_grouped_forward(const GemmArgs &g, hipStream_t s)
     m.V = static_cast<int>(V);
   }
   const size_t lds = mb_lds_bytes(int4, 1, m.groups);
-  const int64_t nrb_class = ((g.N + m.V - 1) / m.V + 15) / 16;
-  int64_t bpc = 2 * static_cast<int64_t>(compute_units()) / (static_cast<int64_t>(g.num_experts) * m.V);
-  if (bpc < 1) bpc = 1;
-  if (bpc > nrb_class) bpc = nrb_class;
-  m.blocks_per_class = static_cast<int>(bpc);
-  MbGroup grp{g.offsets, g.wq_ptrs, g.scales_ptrs, g.M};
-  return g.compute_dtype == CAIFX_BF16 ? launch_grouped_xt<bf16_t>(m, grp, g.num_experts, g.x_dtype, int4, lds, s)
-                                       : launch_grouped_xt<f16_t>(m, grp, g.num_experts, g.x_dtype, int4, lds, s);
+  const int64_t unit = ((g.N + m.V - 1) / m.V + 15) / 16;
+  if (((g.M + 15) / 16 + g.num_experts) * unit * m.V >= (int64_t{1} << 31)) return CAIFX_ERR_UNSUPPORTED;
+  MbGroup grp{g.offsets, g.wq_ptrs, g.scales_ptrs, g.M, g.num_experts, static_cast<unsigned>(unit), static_cast<unsigned>(unit * m.V)};
+  return g.compute_dtype == CAIFX_BF16 ? launch_grouped_xt<bf16_t>(m, grp, g.x_dtype, int4, lds, s)
+                                       : launch_grouped_xt<f16_t>(m, grp, g.x_dtype, int4, lds, s);
 }
 
 }  // namespace caifx
