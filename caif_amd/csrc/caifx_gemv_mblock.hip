@@ -52,7 +52,7 @@ template <> struct Mfma16<f16_t> {
 
 constexpr int kMbWaves = 16;
 constexpr int kMbThreads = kMbWaves * 64;
-constexpr int kPartialFloats(int waves) { return waves * 4 * 64; }     // one buffer of per-wave partial tiles
+constexpr int kPartialFloats = kMbWaves * 4 * 64;     // one buffer of per-wave partial tiles
 
 struct MbArgs {
   const uint8_t *wq;
@@ -71,6 +71,9 @@ struct MbArgs {
   // K beyond one workgroup's reach: blockIdx.y takes the k range [y * slice_groups * 128, ...) and writes its
   // share of the sums as fp32 to partial + y * M * N; a second launch adds the shares in a fixed order
   int slice_groups;      // 128-k groups per slice (= groups when there is one slice)
+  // Waves of a workgroup: as many as a slice has shares of GPW groups.  Up to 16; a launch of sixteen whatever K is left up to
+  // half of them computing on zeros beside the others (us, 16 rows, eight launches: N = 2048, K = 1024 54.5 -> 42.7)
+  int waves;
   float *partial;        // null with one slice
 };
 
@@ -147,7 +150,7 @@ constexpr int kSegRows = kSegBlocks * 16;
 // wq / scales: the weight; xrows / yrows: the first of the M activation and result rows; slice: which part of
 // the reduction (see MbArgs); rows n = cls + V * i of the weight for i in [i_lo, i_hi).  Every thread of the workgroup makes the same calls (the body has barriers).
 // D: row blocks a wave keeps requested (1 or 2; the launch code picks by measurement)
-template <typename CT, typename XT, bool kInt4, int GPW, bool kF32, int MT = 1, int D = 2, int W = kMbWaves>
+template <typename CT, typename XT, bool kInt4, int GPW, bool kF32, int MT = 1, int D = 2>
 __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, const void *scales, const void *xrows,
                                             void *yrows, int M, int slice, int cls, int64_t i_lo, int64_t i_hi)
 {
@@ -157,13 +160,14 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
   constexpr int LPR = GPW * LPG;               // ... per block of 16 weight rows
   constexpr int RBB = mb_reduce_blocks(kInt4, MT);      // row blocks between two reductions (a multiple of D, divides kSegBlocks)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  float *partial = reinterpret_cast<float *>(smem);      // [RBB][MT][W waves][4][64]
-  float *ybuf = partial + RBB * MT * kPartialFloats(W);     // [16 * MT activation rows][kSegRows]
-  float *svec = ybuf + 16 * MT * kSegRows;               // int8: the scales of every wave's k range [W waves][GPW * 128];
-                                                         // int4 with MT > 1: the group-sum corrections [MT][GPW][W waves][16]
+  float *partial = reinterpret_cast<float *>(smem);      // [RBB][MT][16 waves][4][64]
+  float *ybuf = partial + RBB * MT * kPartialFloats;     // [16 * MT activation rows][kSegRows]
+  float *svec = ybuf + 16 * MT * kSegRows;               // int8: the scales of every wave's k range [16 waves][GPW * 128];
+                                                         // int4 with MT > 1: the group-sum corrections [MT][GPW][16 waves][16]
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int threads = 64 * a.waves;
   const int j = lane & 15;        // weight row within the block (B column) / activation row (A row)
   const int q = lane >> 4;        // quarter of the 32-wide k step
   const int nrb = i_hi > i_lo ? static_cast<int>((i_hi - i_lo + 15) / 16) : 0;
@@ -298,7 +302,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
           for (int r = 0; r < 4; ++r) cor[g][r] = Mfma16<CT>::kOffset * xsum[r];
         } else if (j == 0) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) corbuf[(mt * GPW + g) * (W * 16) + 4 * q + r] = Mfma16<CT>::kOffset * xsum[r];
+          for (int r = 0; r < 4; ++r) corbuf[(mt * GPW + g) * (kMbWaves * 16) + 4 * q + r] = Mfma16<CT>::kOffset * xsum[r];
         }
       }
     if constexpr (MT > 1) __syncthreads();
@@ -453,7 +457,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
 #pragma unroll
                   for (int r = 0; r < 4; ++r) tot[u][mt][r] = __builtin_fmaf(sr, acc[mt][r] - cor[g][r], tot[u][mt][r]);
                 } else {
-                  const floatx4_t cr = *reinterpret_cast<const floatx4_t *>(corbuf + (mt * GPW + g) * (W * 16) + 4 * q);
+                  const floatx4_t cr = *reinterpret_cast<const floatx4_t *>(corbuf + (mt * GPW + g) * (kMbWaves * 16) + 4 * q);
 #pragma unroll
                   for (int r = 0; r < 4; ++r) tot[u][mt][r] = __builtin_fmaf(sr, acc[mt][r] - cr[r], tot[u][mt][r]);
                 }
@@ -493,15 +497,18 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) partial[(((u * MT + mt) * W + wave) * 4 + r) * 64 + lane] = tot[u][mt][r];
+          for (int r = 0; r < 4; ++r) partial[(((u * MT + mt) * kMbWaves + wave) * 4 + r) * 64 + lane] = tot[u][mt][r];
       __syncthreads();
-      for (int idx = threadIdx.x; idx < RBB * MT * 256; idx += (64 * W)) {
+      for (int idx = threadIdx.x; idx < RBB * MT * 256; idx += threads) {
         const int um = idx >> 8;             // u * MT + mt
         const int r = (idx >> 6) & 3;
         const int l = idx & 63;
         float v = 0.0f;
 #pragma unroll
-        for (int wv = 0; wv < W; ++wv) v += partial[((um * W + wv) * 4 + r) * 64 + l];
+        for (int wv = 0; wv < kMbWaves; ++wv) {
+          const float p = partial[((um * kMbWaves + wv) * 4 + r) * 64 + l];      // (waves that were not launched: read, not added)
+          v += wv < a.waves ? p : 0.0f;
+        }
         const int m = 16 * (um % MT) + 4 * (l >> 4) + r;
         ybuf[m * kSegRows + (base - seg0 + um / MT) * 16 + (l & 15)] = v;
       }
@@ -511,7 +518,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
     const int64_t i_seg = i_lo + static_cast<int64_t>(seg0) * 16;
     const int seg_rows = static_cast<int>(i_hi - i_seg < kSegRows ? i_hi - i_seg : kSegRows);
     float *part = a.partial ? a.partial + static_cast<int64_t>(slice) * M * a.N : nullptr;
-    for (int idx = threadIdx.x; idx < M * seg_rows; idx += (64 * W)) {
+    for (int idx = threadIdx.x; idx < M * seg_rows; idx += threads) {
       const int m = idx / seg_rows;
       const int r = idx - m * seg_rows;
       const int64_t o = static_cast<int64_t>(m) * a.N + cls + a.V * (i_seg + r);
@@ -642,14 +649,14 @@ int launch_gpw(const MbArgs &m, size_t lds, hipStream_t s)
     const bool one_block = kInt4 ? (m.M <= 8 || rows_wg <= 32 || rows_wg > 64) : rows_wg <= 32;
     if (gpw > 2) return CAIFX_ERR_UNSUPPORTED;
     if (one_block) {
-      if (gpw <= 1) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 1, kF32, 1, 1>), grid, dim3(kMbThreads), lds, s, m);
-      else hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 2, kF32, 1, 1>), grid, dim3(kMbThreads), lds, s, m);
-    } else if (gpw <= 1) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 1, kF32>), grid, dim3(kMbThreads), lds, s, m);
-    else hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 2, kF32>), grid, dim3(kMbThreads), lds, s, m);
+      if (gpw <= 1) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 1, kF32, 1, 1>), grid, dim3(64 * m.waves), lds, s, m);
+      else hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 2, kF32, 1, 1>), grid, dim3(64 * m.waves), lds, s, m);
+    } else if (gpw <= 1) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 1, kF32>), grid, dim3(64 * m.waves), lds, s, m);
+    else hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 2, kF32>), grid, dim3(64 * m.waves), lds, s, m);
   } else {
-    if (gpw <= 1) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 1, kF32, 2>), grid, dim3(kMbThreads), lds, s, m);
+    if (gpw <= 1) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 1, kF32, 2>), grid, dim3(64 * m.waves), lds, s, m);
     else if constexpr (mb_max_gpw(kInt4, 2) >= 2) {
-      if (gpw <= 2) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 2, kF32, 2>), grid, dim3(kMbThreads), lds, s, m);
+      if (gpw <= 2) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 2, kF32, 2>), grid, dim3(64 * m.waves), lds, s, m);
       else return CAIFX_ERR_UNSUPPORTED;
     } else return CAIFX_ERR_UNSUPPORTED;
   }
@@ -674,8 +681,8 @@ int launch_grouped_gpw(const MbArgs &m, const MbGroup &g, size_t lds, hipStream_
 {
   const dim3 grid(static_cast<unsigned>(compute_units()));
   const int gpw = (m.groups + kMbWaves - 1) / kMbWaves;
-  if (gpw <= 1) hipLaunchKernelGGL((mblock_grouped_kernel<CT, XT, kInt4, 1>), grid, dim3(kMbThreads), lds, s, m, g);
-  else if (gpw <= 2) hipLaunchKernelGGL((mblock_grouped_kernel<CT, XT, kInt4, 2>), grid, dim3(kMbThreads), lds, s, m, g);
+  if (gpw <= 1) hipLaunchKernelGGL((mblock_grouped_kernel<CT, XT, kInt4, 1>), grid, dim3(64 * m.waves), lds, s, m, g);
+  else if (gpw <= 2) hipLaunchKernelGGL((mblock_grouped_kernel<CT, XT, kInt4, 2>), grid, dim3(64 * m.waves), lds, s, m, g);
   else return CAIFX_ERR_UNSUPPORTED;
   return launch_status();
 }
@@ -712,64 +719,110 @@ constexpr int64_t kMbMaxSlices = 64;
 // longest reduction one workgroup covers: 16 waves times the groups a wave can hold operands for
 static int64_t mb_reach(int64_t M) { return kMbWaves * 128 * mb_max_gpw(false, M > 16 ? 2 : 1); }
 
-// Reduction length per workgroup the launch is planned with.  The int8 prologue (scaled activations cut into digit
-// planes) costs a workgroup time in proportion to its k range, while its share of the weight shrinks with N: at
-// K = 4096, 16 rows, half the reach plus the pass that adds the two slices measured 17.6 -> 12.5 us (fp32 compute,
-// N = 4096), 26.1 -> 21.9 us (fp32, N = 14336), 13.5 -> 11.7 us (bf16, N = 4096), 18.7 -> 18.9 us (bf16, N = 14336).
-// int4 has no such prologue and loses (9.3 -> 9.0 us at N = 4096 but 14.4 -> 15.2 us at N = 14336).
-static int64_t mb_slice_k(const GemmArgs &g)
+// How a call's reduction is cut: slices of equal length (the last may be shorter), the residue classes' rows dealt to
+// `per_class` workgroups each so that all slices together are one workgroup per compute unit or fewer (seven slices of 37
+// workgroups, three more than the chip has units, measured 24 us where 36 measure 16: int4, N = 4096, K = 14336).
+struct MbPlan {
+  int slices, slice_groups, waves, per_class;
+};
+
+// slices of `length` or less, and the 128-k groups of one; K > 0
+static int64_t mb_slices(int64_t K, int64_t length, int64_t &slice_groups)
 {
-  const int64_t reach = mb_reach(g.M);
-  if (g.M > 16 || g.w.kind == CAIFX_W_INT4_GROUP) return reach;
-  const int64_t n_max = g.compute_dtype == CAIFX_F32 ? 32768 : 8192;
-  return g.N <= n_max ? reach / 2 : reach;
+  const int64_t groups = K / 128, wanted = (K + length - 1) / length;
+  slice_groups = (groups + wanted - 1) / wanted;
+  return (groups + slice_groups - 1) / slice_groups;
 }
 
-static size_t mb_lds_bytes(bool int4, int mt, int slice_groups, int waves = kMbWaves)
+static MbPlan mb_plan(const GemmArgs &g, int64_t V, int64_t length)
 {
-  size_t floats = static_cast<size_t>(mb_reduce_blocks(int4, mt)) * mt * kPartialFloats(waves) + static_cast<size_t>(16) * mt * kSegRows;
-  if (!int4) floats += static_cast<size_t>((slice_groups + waves - 1) / waves) * waves * 128;      // staged scales (ones without a scale vector)
+  MbPlan p;
+  int64_t slice_groups;
+  p.slices = static_cast<int>(mb_slices(g.K, length, slice_groups));
+  p.slice_groups = static_cast<int>(slice_groups);
+  const int gpw = (p.slice_groups + kMbWaves - 1) / kMbWaves;
+  p.waves = (p.slice_groups + gpw - 1) / gpw;
+  const int64_t blocks = ((g.N + V - 1) / V + 15) / 16;          // at least 16 rows per workgroup
+  int64_t bpc = compute_units() / (p.slices * V);
+  if (bpc < 1) bpc = 1;
+  p.per_class = static_cast<int>(bpc < blocks ? bpc : blocks);
+  return p;
+}
+
+static size_t mb_partial_bytes(const GemmArgs &g, int64_t slices)
+{
+  return slices < 2 ? 0 : static_cast<size_t>(slices) * static_cast<size_t>(g.M) * static_cast<size_t>(g.N) * sizeof(float);
+}
+
+// What a plan costs in us beyond what all plans of a call share, fitted to 20 weights from 1408 x 2048 to 14336 x 4096 and
+// 4096 x 14336, 3 to 32 rows: the launch that adds the slices, their sums, the activations a workgroup takes in, the rounds
+// of its weight blocks, and the preparation of its activations (for int8 the digits).  The cheapest plan by this measure is
+// within 1 % of the fastest in the mean, at most 10 % off it; one length for all (2048 for int8 with few columns, 4096) 3 to 5 %
+// and up to 23 %.  M = 16, us with slices of 1024 / 2048 / 4096: fp32 compute, N = K = 4096 10.9 / 12.4 / 15.8; int8, N = 14336,
+// K = 4096 22.8 / 20.2 / 20.3, N = K = 2304 8.2 / 8.6 / 8.0; int4, N = 4096, K = 8192 14.1 / 12.3 / 13.7, N = K = 4096 8.9 / 9.2 / 9.1.
+static double mb_cost(const GemmArgs &g, int64_t V, const MbPlan &p)
+{
+  const bool f32 = g.compute_dtype == CAIFX_F32, int4 = g.w.kind == CAIFX_W_INT4_GROUP;
+  const int mt = g.M > 16 ? 2 : 1, gpw = (p.slice_groups + kMbWaves - 1) / kMbWaves;
+  const int64_t rows = (g.N + V - 1) / V;
+  const double blocks = static_cast<double>(((rows + p.per_class - 1) / p.per_class + 15) / 16);
+  const double taken = static_cast<double>(g.M * p.slice_groups * 128 * (f32 ? 4 : 2)) / 32768.0;
+  const double sums = p.slices > 1 ? 1e-6 * static_cast<double>(p.slices * g.M) * static_cast<double>(g.N) : 0.0;
+  const double add = p.slices > 1 ? 1.7 : 0.0, streamed = blocks * static_cast<double>(p.slice_groups) / 16.0;
+  if (int4) return add + 4.5 * sums + 0.58 * taken + 0.735 * streamed + 0.15 * (gpw * mt);
+  if (f32) return add + 3.6 * sums + 0.70 * taken + 1.44 * streamed + (0.10 * blocks + 2.27) * (gpw * mt);
+  return add + 3.6 * sums + 0.53 * taken + 1.43 * streamed + (0.064 * blocks + 0.86) * (gpw * mt);
+}
+
+// Slice lengths worth a look beside the longest one a workgroup covers (mb_reach), where the sums of the slices stay within
+// the library's own buffer for callers without a workspace (half the reach for int8 with up to 8192 columns, fp32 compute 32768,
+// always counted: the size query has reported it since there were slices)
+template <typename F> static void mb_for_lengths(const GemmArgs &g, F f)
+{
+  const int64_t reach = mb_reach(g.M);
+  const bool f32 = g.compute_dtype == CAIFX_F32, int4 = g.w.kind == CAIFX_W_INT4_GROUP;
+  for (int64_t length = 1024; length < reach; length *= 2) {
+    if (g.M <= 16 && int4 && (length < 2048 || g.K <= reach)) continue;
+    if (g.M <= 16 && !int4 && !f32 && length < 2048 && g.K <= reach) continue;
+    if (g.K <= length || g.K > length * kMbMaxSlices) continue;
+    int64_t slice_groups;
+    const bool always = g.M <= 16 && !int4 && length == reach / 2 && g.N <= (f32 ? 32768 : 8192);
+    if (always || mb_partial_bytes(g, mb_slices(g.K, length, slice_groups)) <= CAIFX_STATIC_SCRATCH_BYTES) f(length);
+  }
+}
+
+static size_t mb_lds_bytes(bool int4, int mt, int slice_groups)
+{
+  size_t floats = static_cast<size_t>(mb_reduce_blocks(int4, mt)) * mt * kPartialFloats + static_cast<size_t>(16) * mt * kSegRows;
+  if (!int4) floats += static_cast<size_t>((slice_groups + kMbWaves - 1) / kMbWaves) * kMbWaves * 128;      // staged scales (ones without a scale vector)
   else if (mt > 1) floats += static_cast<size_t>(mt) * mb_max_gpw(true, mt) * kMbWaves * 16;      // group-sum corrections
   return floats * sizeof(float);
 }
 
 size_t mblock_workspace_bytes(const GemmArgs &g)
 {
-  if (g.offsets || g.M < 1 || g.M > kMbMaxRows || g.K % 128 != 0) return 0;
+  if (g.offsets || g.M < 1 || g.M > kMbMaxRows || g.N < 1 || g.K < 1 || g.K % 128 != 0) return 0;
   const bool int4 = g.w.kind == CAIFX_W_INT4_GROUP;
   if (g.compute_dtype == CAIFX_F32 && int4) return 0;
-  int64_t reach = mb_slice_k(g);
-  int64_t slices = (g.K + reach - 1) / reach;
-  if (slices > kMbMaxSlices) {
-    reach = mb_reach(g.M);
-    slices = (g.K + reach - 1) / reach;
-  }
-  if (slices < 2 || slices > kMbMaxSlices) return 0;
-  return static_cast<size_t>(slices) * static_cast<size_t>(g.M) * static_cast<size_t>(g.N) * sizeof(float);
+  int64_t slice_groups;
+  const int64_t slices = mb_slices(g.K, mb_reach(g.M), slice_groups);
+  if (slices > kMbMaxSlices) return 0;
+  size_t bytes = mb_partial_bytes(g, slices);
+  mb_for_lengths(g, [&](int64_t length) {          // (the scales, which also count for the choice, are not known here)
+    const size_t b = mb_partial_bytes(g, mb_slices(g.K, length, slice_groups));
+    bytes = b > bytes ? b : bytes;
+  });
+  return bytes;
 }
 
 int mblock_forward(const GemmArgs &g, hipStream_t s)
 {
   if (g.offsets || g.M < 1 || g.M > kMbMaxRows) return CAIFX_ERR_UNSUPPORTED;
-  if (g.N < 16 || g.N > (int64_t{1} << 30) || g.K % 128 != 0) return CAIFX_ERR_UNSUPPORTED;
+  if (g.N < 16 || g.N > (int64_t{1} << 30) || g.K % 128 != 0 || g.K / 128 > INT32_MAX) return CAIFX_ERR_UNSUPPORTED;
   if (!aligned_to(g.w.q, 16) || !aligned_to(g.x, 16)) return CAIFX_ERR_UNSUPPORTED;
   const bool int4 = g.w.kind == CAIFX_W_INT4_GROUP;
   if (g.compute_dtype == CAIFX_F32 && int4) return CAIFX_ERR_UNSUPPORTED;
-  // a reduction longer than one workgroup's reach is cut into slices whose sums meet in the caller's workspace
-  // (a shorter slice than the workgroup's reach is a choice: without room for its sums the full reach is used)
   const int mt = g.M > 16 ? 2 : 1;
-  int64_t reach = mb_slice_k(g);
-  int64_t slices = (g.K + reach - 1) / reach;
-  const bool room = g.workspace && aligned_to(g.workspace, 4) &&
-                    g.workspace_bytes / sizeof(float) / static_cast<size_t>(g.M) / static_cast<size_t>(g.N) >= static_cast<size_t>(slices);
-  if (slices > kMbMaxSlices || (slices > 1 && !room)) {
-    reach = mb_reach(g.M);
-    slices = (g.K + reach - 1) / reach;
-    if (slices > kMbMaxSlices) return CAIFX_ERR_UNSUPPORTED;
-    if (slices > 1 && (!g.workspace || !aligned_to(g.workspace, 4) ||
-                       g.workspace_bytes < static_cast<size_t>(slices) * static_cast<size_t>(g.M) * static_cast<size_t>(g.N) * sizeof(float)))
-      return CAIFX_ERR_UNSUPPORTED;
-  }
 
   MbArgs m{};
   m.wq = static_cast<const uint8_t *>(g.w.q);
@@ -781,9 +834,6 @@ int mblock_forward(const GemmArgs &g, hipStream_t s)
   m.N = g.N;
   m.K = g.K;
   m.groups = static_cast<int>(g.K / 128);
-  m.slice_groups = static_cast<int>((m.groups + slices - 1) / slices);      // slices of equal length, the last may be shorter
-  slices = (m.groups + m.slice_groups - 1) / m.slice_groups;
-  m.partial = slices > 1 ? static_cast<float *>(g.workspace) : nullptr;
   m.V = 1;
   if (int4) {
     const int gs = g.w.group_size;
@@ -798,15 +848,20 @@ int mblock_forward(const GemmArgs &g, hipStream_t s)
     m.scale_step = static_cast<int>(64 % P);
     m.V = static_cast<int>(V);
   }
+  // a reduction longer than one workgroup's reach is cut into slices whose sums meet in the caller's workspace; shorter slices
+  // than that are a choice, where there is room for their sums
+  const size_t room = g.workspace && aligned_to(g.workspace, 4) ? g.workspace_bytes : 0;
+  MbPlan plan = mb_plan(g, m.V, mb_reach(g.M));
+  if (plan.slices > kMbMaxSlices || mb_partial_bytes(g, plan.slices) > room) return CAIFX_ERR_UNSUPPORTED;
+  mb_for_lengths(g, [&](int64_t length) {
+    const MbPlan p = mb_plan(g, m.V, length);
+    if (mb_partial_bytes(g, p.slices) <= room && mb_cost(g, m.V, p) < mb_cost(g, m.V, plan)) plan = p;
+  });
+  m.slice_groups = plan.slice_groups;
+  m.waves = plan.waves;
+  m.blocks_per_class = plan.per_class;
+  m.partial = plan.slices > 1 ? static_cast<float *>(g.workspace) : nullptr;
   const size_t lds = mb_lds_bytes(int4, mt, m.slice_groups);
-  // one workgroup per compute unit over all slices: the prologue (the slice of X as operands, for int8 its digit
-  // planes) is paid per workgroup, so each should own as many rows as the chip allows
-  int target = static_cast<int>((compute_units() + slices - 1) / slices);
-  const int64_t nrb_class = ((g.N + m.V - 1) / m.V + 15) / 16;
-  int64_t bpc = target / m.V;
-  if (bpc < 1) bpc = 1;
-  if (bpc > nrb_class) bpc = nrb_class;        // at least 16 rows per workgroup
-  m.blocks_per_class = static_cast<int>(bpc);
   int st;
   if (g.compute_dtype == CAIFX_F32)
     st = g.x_dtype == CAIFX_F32 ? launch_f32<float>(m, lds, s)
@@ -814,8 +869,8 @@ int mblock_forward(const GemmArgs &g, hipStream_t s)
   else
     st = g.compute_dtype == CAIFX_BF16 ? launch_xt<bf16_t>(m, g.x_dtype, int4, lds, s)
                                        : launch_xt<f16_t>(m, g.x_dtype, int4, lds, s);
-  if (st != CAIFX_OK || slices == 1) return st;
-  return splitk_reduce(m.partial, static_cast<int>(slices), g.M * g.N, g.y, g.y_dtype, nullptr, s);
+  if (st != CAIFX_OK || plan.slices == 1) return st;
+  return splitk_reduce(m.partial, plan.slices, g.M * g.N, g.y, g.y_dtype, nullptr, s);
 }
 
 int mblock_grouped_forward(const GemmArgs &g, hipStream_t s)
@@ -851,6 +906,7 @@ int mblock_grouped_forward(const GemmArgs &g, hipStream_t s)
     m.scale_step = static_cast<int>(64 % P);
     m.V = static_cast<int>(V);
   }
+  m.waves = mb_plan(g, 1, g.K).waves;
   const size_t lds = mb_lds_bytes(int4, 1, m.groups);
   const int64_t unit = ((g.N + m.V - 1) / m.V + 15) / 16;
   if (((g.M + 15) / 16 + g.num_experts) * unit * m.V >= (int64_t{1} << 31)) return CAIFX_ERR_UNSUPPORTED;

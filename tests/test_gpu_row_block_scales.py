@@ -29,7 +29,8 @@ def _weight(N, K, period, seed):
 @pytest.mark.parametrize("compute", [T.F32, T.BF16])
 @pytest.mark.parametrize("M", [3, 16, 17, 32])
 @pytest.mark.parametrize("N,K,period", [(192, 128, 192), (320, 128, 10), (1408, 2048, 1408), (2048, 1408, 2048), (960, 384, 960),
-                                        (256, 4096, 256), (208, 3968, 1), (80, 2176, 0)])
+                                        (256, 4096, 256), (208, 3968, 1), (80, 2176, 0),
+                                        (1280, 5632, 1280), (640, 14336, 640)])
 def test_against_64_bits(N, K, period, M, compute):
     w, dense = _weight(N, K, period, N + K + M)
     g = torch.Generator(device="cuda").manual_seed(7)
