@@ -508,10 +508,19 @@ size_t mfma_f32_workspace_bytes(const GemmArgs &a, bool backward)
 {
   const bool float_w = a.w.kind == CAIFX_W_F32 || a.w.kind == CAIFX_W_F16 || a.w.kind == CAIFX_W_BF16;
   if (a.compute_dtype != CAIFX_F32 && !float_w) return 0;
-  return plan_f32(a.M, backward ? a.K : a.N, backward ? a.N : a.K, a.offsets != nullptr).bytes;
+  const size_t here = plan_f32(a.M, backward ? a.K : a.N, backward ? a.N : a.K, a.offsets != nullptr).bytes, pieces = pieces_workspace_bytes(a, backward);
+  return pieces > here ? pieces : here;
 }
 
-int mfma_f32_forward(const GemmArgs &a, hipStream_t s) { return run_f32(a, false, s); }
-int mfma_f32_backward(const GemmArgs &a, hipStream_t s) { return run_f32(a, true, s); }
+int mfma_f32_forward(const GemmArgs &a, hipStream_t s)
+{
+  const int st = pieces_gemm(a, false, s);
+  return st == CAIFX_ERR_UNSUPPORTED ? run_f32(a, false, s) : st;
+}
+int mfma_f32_backward(const GemmArgs &a, hipStream_t s)
+{
+  const int st = pieces_gemm(a, true, s);
+  return st == CAIFX_ERR_UNSUPPORTED ? run_f32(a, true, s) : st;
+}
 
 }  // namespace caifx
