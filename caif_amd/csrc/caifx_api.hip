@@ -352,11 +352,13 @@ size_t caifx_qlinear_grouped_workspace_bytes(int num_experts, int64_t total_rows
 static int grouped(bool backward, int num_experts, const int32_t *offsets, int64_t total_rows, int64_t N, int64_t K,
                    const void *x, int x_dtype, int compute_dtype, const void *const *wq_ptrs, int w_kind,
                    const void *const *scales_ptrs, int64_t scale_period, int group_size, void *y, int y_dtype,
-                   const void *addend, void *workspace, size_t workspace_bytes, caifx_stream_t stream)
+                   const void *addend, void *workspace, size_t workspace_bytes, bool zero_rest, caifx_stream_t stream)
 {
   int st = validate_common(total_rows, N, K, x, x_dtype, compute_dtype, y, y_dtype);
   if (st != CAIFX_OK) return st;
   if (num_experts < 0) return CAIFX_ERR_INVALID_ARGUMENT;
+  const int64_t row_bytes = (backward ? K : N) * static_cast<int64_t>(dtype_size(y_dtype));
+  if (num_experts == 0 && zero_rest) return caifx_qlinear_grouped_zero_rest(0, offsets, total_rows, row_bytes, y, stream);
   if (num_experts == 0 || total_rows == 0) return CAIFX_OK;
   if (!offsets || !wq_ptrs) return CAIFX_ERR_INVALID_ARGUMENT;
   if (w_kind == CAIFX_W_INT4_GROUP) {
@@ -377,6 +379,16 @@ static int grouped(bool backward, int num_experts, const int32_t *offsets, int64
   a.num_experts = num_experts;
   if (addend && (addend == y || !aligned_to(addend, dtype_size(y_dtype)))) return CAIFX_ERR_INVALID_ARGUMENT;
   hipStream_t s = as_stream(stream);
+  if (!backward && !addend && !float_kind(w_kind) && compute_dtype != CAIFX_F32) {
+    // few rows per expert (MoE decode): memory bound on the touched experts' weights; it clears the other rows itself
+    a.zero_rest = zero_rest;
+    st = mblock_grouped_forward(a, s);
+    if (st != CAIFX_ERR_UNSUPPORTED) return st;
+  }
+  if (zero_rest) {
+    st = caifx_qlinear_grouped_zero_rest(num_experts, offsets, total_rows, row_bytes, y, stream);
+    if (st != CAIFX_OK) return st;
+  }
   if (same_16bit(w_kind, compute_dtype)) {
     a.addend = addend;
     st = backward ? mfma_backward(a, s) : mfma_forward(a, s);
@@ -390,11 +402,6 @@ static int grouped(bool backward, int num_experts, const int32_t *offsets, int64
   if (float_kind(w_kind)) {
     if (addend) return CAIFX_ERR_UNSUPPORTED;
     return backward ? generic_backward(a, s) : generic_forward(a, s);
-  }
-  if (!backward && !addend) {
-    // few rows per expert (MoE decode): memory bound on the touched experts' weights
-    st = mblock_grouped_forward(a, s);
-    if (st != CAIFX_ERR_UNSUPPORTED) return st;
   }
   a.addend = addend;
   st = backward ? mfma_backward(a, s) : mfma_forward(a, s);
@@ -419,7 +426,7 @@ int caifx_qlinear_grouped_forward(int num_experts, const int32_t *offsets, int64
                                   caifx_stream_t stream)
 {
   return grouped(false, num_experts, offsets, total_rows, N, K, x, x_dtype, compute_dtype, wq_ptrs, w_kind,
-                 scales_ptrs, scale_period, group_size, y, y_dtype, nullptr, workspace, workspace_bytes, stream);
+                 scales_ptrs, scale_period, group_size, y, y_dtype, nullptr, workspace, workspace_bytes, false, stream);
 }
 
 int caifx_qlinear_grouped_backward_input(int num_experts, const int32_t *offsets, int64_t total_rows, int64_t N,
@@ -429,7 +436,7 @@ int caifx_qlinear_grouped_backward_input(int num_experts, const int32_t *offsets
                                          void *workspace, size_t workspace_bytes, caifx_stream_t stream)
 {
   return grouped(true, num_experts, offsets, total_rows, N, K, dy, dy_dtype, compute_dtype, wq_ptrs, w_kind,
-                 scales_ptrs, scale_period, group_size, dx, dx_dtype, nullptr, workspace, workspace_bytes, stream);
+                 scales_ptrs, scale_period, group_size, dx, dx_dtype, nullptr, workspace, workspace_bytes, false, stream);
 }
 
 int caifx_qlinear_grouped_backward_input_add(int num_experts, const int32_t *offsets, int64_t total_rows, int64_t N,
@@ -441,7 +448,17 @@ int caifx_qlinear_grouped_backward_input_add(int num_experts, const int32_t *off
 {
   if (total_rows > 0 && num_experts > 0 && !addend) return CAIFX_ERR_INVALID_ARGUMENT;
   return grouped(true, num_experts, offsets, total_rows, N, K, dy, dy_dtype, compute_dtype, wq_ptrs, w_kind,
-                 scales_ptrs, scale_period, group_size, dx, dx_dtype, addend, workspace, workspace_bytes, stream);
+                 scales_ptrs, scale_period, group_size, dx, dx_dtype, addend, workspace, workspace_bytes, false, stream);
+}
+
+int caifx_qlinear_grouped_fresh(int backward, int num_experts, const int32_t *offsets, int64_t total_rows, int64_t N, int64_t K,
+                                const void *x, int x_dtype, int compute_dtype, const void *const *wq_ptrs, int w_kind,
+                                const void *const *scales_ptrs, int64_t scale_period, int group_size, void *y, int y_dtype,
+                                const void *addend, void *workspace, size_t workspace_bytes, caifx_stream_t stream)
+{
+  if (!backward && addend) return CAIFX_ERR_INVALID_ARGUMENT;
+  return grouped(backward != 0, num_experts, offsets, total_rows, N, K, x, x_dtype, compute_dtype, wq_ptrs, w_kind, scales_ptrs,
+                 scale_period, group_size, y, y_dtype, addend, workspace, workspace_bytes, true, stream);
 }
 
 // Shared checks of the two gated-expert launches: 16-bit results, every tensor of the result's shape present,

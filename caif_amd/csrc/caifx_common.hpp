@@ -123,6 +123,18 @@ __device__ __forceinline__ void segment_rows(const int32_t *offsets, int e, int6
   hi = hi < lo ? lo : (hi > m ? m : hi);
 }
 
+// Zeroes bytes [a, b) of y by `threads` threads of which this is the t-th: whole aligned 16-byte pieces, single bytes at the ends.
+__device__ __forceinline__ void zero_bytes(unsigned char *y, int64_t a, int64_t b, int64_t t, int64_t threads)
+{
+  if (a >= b) return;
+  const int64_t shift = reinterpret_cast<uintptr_t>(y) & 15;
+  const int64_t up = ((a + shift + 15) & ~int64_t{15}) - shift, down = ((b + shift) & ~int64_t{15}) - shift;
+  const int64_t a16 = up < b ? up : b, b16 = down > a16 ? down : a16;
+  for (int64_t i = a16 + 16 * t; i < b16; i += 16 * threads) *reinterpret_cast<u32x4_t *>(y + i) = u32x4_t{0, 0, 0, 0};
+  if (a + t < a16) y[a + t] = 0;
+  if (b16 + t < b) y[b16 + t] = 0;
+}
+
 // a 64-bit value every lane holds alike, moved to scalar registers (the direct-to-LDS requests take their base there)
 __device__ __forceinline__ uint64_t uniform64(uint64_t v)
 {

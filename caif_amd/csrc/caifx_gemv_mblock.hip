@@ -555,7 +555,37 @@ struct MbGroup {
   int64_t total_rows;
   int num_experts;
   unsigned unit_blocks, pass_blocks;      // blocks of 16 rows in a unit, and in a pass (V units)
+  bool zero_rest;                         // zero the result's rows that no segment covers
 };
+
+// Zeroes the rows of a grouped result that no segment covers, the launch's workgroups sharing them: [0, offsets[0]) and
+// [offsets[E], rows), none of which a unit writes.  Offsets that step down somewhere (a caller's mistake) may also leave rows in
+// between, or cover some of those: then each row is looked up.  A launch of its own in front of the product took 4.7 us of a decode step.
+__device__ __forceinline__ void zero_uncovered(const MbGroup &g, unsigned char *y, int64_t row_bytes)
+{
+  const int lane = threadIdx.x & 63;
+  const int rows = static_cast<int>(g.total_rows);
+  const int first = g.offsets[0], end = g.offsets[g.num_experts];
+  bool down = false;
+  for (int e = lane; e < g.num_experts; e += 64) down = down || g.offsets[e + 1] < g.offsets[e];
+  if (__ballot(down) == 0) {
+    const int lo = first < 0 ? 0 : first > rows ? rows : first, hi = end < 0 ? 0 : end > rows ? rows : end;
+    if (lo == 0 && hi == rows) return;
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x, threads = static_cast<int64_t>(gridDim.x) * blockDim.x;
+    zero_bytes(y, 0, lo * row_bytes, t, threads);
+    zero_bytes(y, hi * row_bytes, rows * row_bytes, t, threads);
+    return;
+  }
+  for (int r = static_cast<int>(blockIdx.x); r < rows; r += static_cast<int>(gridDim.x)) {
+    bool covered = false;
+    for (int e = lane; e < g.num_experts; e += 64) {
+      int lo, hi;
+      segment_rows(g.offsets, e, g.total_rows, lo, hi);
+      covered = covered || (lo <= r && r < hi);
+    }
+    if (__ballot(covered) == 0) zero_bytes(y, r * row_bytes, (r + 1) * row_bytes, threadIdx.x, blockDim.x);
+  }
+}
 template <typename CT, typename XT, bool kInt4, int GPW>
 __global__ __launch_bounds__(kMbThreads) void mblock_grouped_kernel(MbArgs a, MbGroup g)
 {
@@ -583,6 +613,7 @@ __global__ __launch_bounds__(kMbThreads) void mblock_grouped_kernel(MbArgs a, Mb
   int u = static_cast<int>(start / g.unit_blocks);                               // unit, and the run's first block in it
   int first = static_cast<int>(start - u * g.unit_blocks);
   const size_t ybytes = a.y_dtype == CAIFX_F32 ? 4 : 2;
+  if (g.zero_rest) zero_uncovered(g, static_cast<unsigned char *>(a.y), a.N * static_cast<int64_t>(ybytes));
   int base = g.num_experts <= 64 ? 0 : -1;          // which 64 experts the lanes hold
   int before = 0;                                   // units of the experts in front of them
   while (todo > 0) {
@@ -910,7 +941,7 @@ int mblock_grouped_forward(const GemmArgs &g, hipStream_t s)
   const size_t lds = mb_lds_bytes(int4, 1, m.groups);
   const int64_t unit = ((g.N + m.V - 1) / m.V + 15) / 16;
   if (((g.M + 15) / 16 + g.num_experts) * unit * m.V >= (int64_t{1} << 31)) return CAIFX_ERR_UNSUPPORTED;
-  MbGroup grp{g.offsets, g.wq_ptrs, g.scales_ptrs, g.M, g.num_experts, static_cast<unsigned>(unit), static_cast<unsigned>(unit * m.V)};
+  MbGroup grp{g.offsets, g.wq_ptrs, g.scales_ptrs, g.M, g.num_experts, static_cast<unsigned>(unit), static_cast<unsigned>(unit * m.V), g.zero_rest};
   return g.compute_dtype == CAIFX_BF16 ? launch_grouped_xt<bf16_t>(m, grp, g.x_dtype, int4, lds, s)
                                        : launch_grouped_xt<f16_t>(m, grp, g.x_dtype, int4, lds, s);
 }

@@ -27,6 +27,7 @@ struct GemmArgs {
   const void *const *wq_ptrs;
   const void *const *scales_ptrs;
   int num_experts;
+  bool zero_rest;         // grouped: y holds nothing yet, rows that no segment covers are to be zero (mblock_grouped_forward alone looks)
   void *workspace;
   size_t workspace_bytes;
   // optional: y = T(float(T(acc)) + float(addend)), addend [M, columns of y] of y_dtype (may alias y)

@@ -431,17 +431,8 @@ __global__ __launch_bounds__(256) void zero_rest_kernel(const int32_t *offsets, 
   const int64_t first = offsets[0], end = offsets[num_experts];
   const int64_t lo = first < 0 ? 0 : first > rows ? rows : first, hi = end < 0 ? 0 : end > rows ? rows : end;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, threads = static_cast<int64_t>(gridDim.x) * 256;
-  const int64_t shift = reinterpret_cast<uintptr_t>(y) & 15;
-  const auto zero = [&](int64_t a, int64_t b) {        // bytes [a, b): whole aligned 16-byte pieces, single bytes at the ends
-    if (a >= b) return;
-    const int64_t up = ((a + shift + 15) & ~int64_t{15}) - shift, down = ((b + shift) & ~int64_t{15}) - shift;
-    const int64_t a16 = up < b ? up : b, b16 = down > a16 ? down : a16;
-    for (int64_t i = a16 + 16 * t; i < b16; i += 16 * threads) *reinterpret_cast<u32x4_t *>(y + i) = u32x4_t{0, 0, 0, 0};
-    if (a + t < a16) y[a + t] = 0;
-    if (b16 + t < b) y[b16 + t] = 0;
-  };
-  zero(0, lo * row_bytes);
-  zero((hi > lo ? hi : lo) * row_bytes, rows * row_bytes);
+  zero_bytes(y, 0, lo * row_bytes, t, threads);
+  zero_bytes(y, (hi > lo ? hi : lo) * row_bytes, rows * row_bytes, t, threads);
 }
 
 }  // namespace

@@ -25,7 +25,7 @@ namespace {
   X(caifx_qlinear_forward) X(caifx_qlinear_forward_add) X(caifx_qlinear_backward_input)                                  \
   X(caifx_qlinear_backward_input_add) X(caifx_qlinear_workspace_bytes) X(caifx_qlinear_grouped_forward)                  \
   X(caifx_qlinear_grouped_backward_input) X(caifx_qlinear_grouped_backward_input_add)                                    \
-  X(caifx_qlinear_grouped_workspace_bytes) X(caifx_qlinear_grouped_zero_rest) X(caifx_silu) X(caifx_silu_backward) X(caifx_multiply) X(caifx_add)           \
+  X(caifx_qlinear_grouped_workspace_bytes) X(caifx_qlinear_grouped_fresh) X(caifx_silu) X(caifx_silu_backward) X(caifx_multiply) X(caifx_add)           \
   X(caifx_silu_multiply) X(caifx_swiglu_backward) X(caifx_moe_dispatch_map_workspace_bytes)                              \
   X(caifx_moe_build_dispatch_map) X(caifx_moe_dispatch) X(caifx_moe_combine) X(caifx_moe_combine_backward_grad_expert)   \
   X(caifx_moe_combine_backward_grad_weights) X(caifx_moe_dispatch_backward) X(caifx_quantize_int8_per_channel)           \
@@ -293,17 +293,21 @@ PyObject *grouped(PyObject *, PyObject *const *a, Py_ssize_t n)
       return api.caifx_qlinear_grouped_workspace_bytes(static_cast<int>(E), rows, N, K, xd, compute, kind, backward ? 1 : 0);
     });
     const auto off = static_cast<const int32_t *>(offsets.data_ptr());
-    if (a[6] == Py_None && y.numel() > 0) {      // a fresh result's rows outside the segments are zero
-      const int status = launch(api.caifx_qlinear_grouped_zero_rest, static_cast<int>(E), off, rows, out_dim * static_cast<int64_t>(y.element_size()), y.data_ptr(), stream());
-      if (status != CAIFX_OK) return PyLong_FromLong(status);
-    }
+    const void *addend = nullptr;
     if (a[8] != Py_None) {
       if (!backward) throw Error{PyExc_AssertionError, "the forward takes no addend"};
       const at::Tensor &add = tensor(a[8]);
       if (add.scalar_type() != y.scalar_type() || add.numel() != y.numel())
         throw Error{PyExc_AssertionError, "the addend must have the result's dtype and size"};
+      addend = add.data_ptr();
+    }
+    // a fresh result's rows outside the segments are zero
+    if (a[6] == Py_None)
+      return result(launch(api.caifx_qlinear_grouped_fresh, backward ? 1 : 0, static_cast<int>(E), off, rows, N, K, x.data_ptr(), xd, compute, wq, kind, scales,
+                           period, group, y.data_ptr(), od, addend, ws.p, ws.bytes, stream()), y);
+    if (addend) {
       return result(launch(api.caifx_qlinear_grouped_backward_input_add, static_cast<int>(E), off, rows, N, K, x.data_ptr(), xd, compute, wq, kind, scales,
-                                                                 period, group, y.data_ptr(), od, add.data_ptr(), ws.p, ws.bytes, stream()), y);
+                                                                 period, group, y.data_ptr(), od, addend, ws.p, ws.bytes, stream()), y);
     }
     const auto fn = backward ? api.caifx_qlinear_grouped_backward_input : api.caifx_qlinear_grouped_forward;
     return result(launch(fn, static_cast<int>(E), off, rows, N, K, x.data_ptr(), xd, compute, wq, kind, scales, period, group, y.data_ptr(), od, ws.p,

@@ -407,6 +407,15 @@ CAIFX_API int caifx_moe_dispatch(const void *input, const int32_t *expert_indice
 CAIFX_API int caifx_qlinear_grouped_zero_rest(int num_experts, const int32_t *offsets, int64_t total_rows, int64_t row_bytes,
                                     void *y, caifx_stream_t stream);
 
+/* caifx_qlinear_grouped_forward (backward = 0), caifx_qlinear_grouped_backward_input or, with an addend, _backward_input_add (backward
+ * != 0) into a result that holds nothing yet: rows that no segment covers are zeroed too (caifx_qlinear_grouped_zero_rest), by the
+ * decode kernel in its own launch and in front of it otherwise. */
+CAIFX_API int caifx_qlinear_grouped_fresh(int backward, int num_experts, const int32_t *offsets, int64_t total_rows, int64_t N,
+                                int64_t K, const void *x, int x_dtype, int compute_dtype, const void *const *wq_ptrs,
+                                int w_kind, const void *const *scales_ptrs, int64_t scale_period, int group_size,
+                                void *y, int y_dtype, const void *addend, void *workspace, size_t workspace_bytes,
+                                caifx_stream_t stream);
+
 /* launch_moe_combine (caif_cuda_kernels_moe.cuh:317-326, caif_cuda_kernels_moe.cu:705-745):
  * output[t,d] = T( sum over k in order of float(w[t,k]) * float(buffer[row(t,k), d]) ), fp32
  * accumulation with one fused multiply-add per k, one rounding to T. */

@@ -50,3 +50,24 @@ def test_runs(kind, N, K, counts):
             bound = BOUND[kind] if rows + 2 <= 16 * E else 3e-3          # the tiled kernel rounds code * scale to bf16
             assert ((y[lo:lo + n].double() - want).norm() / want.norm()).item() <= bound, (e, n)
         lo += n
+
+
+@pytest.mark.parametrize("kind", ["int8", "int4"])
+@pytest.mark.parametrize("offsets,rows", [([0, 3, 7], 7), ([2, 3, 9], 14), ([0, 0, 0], 5), ([5, 5, 5], 9), ([5, 8, 2, 4], 11), ([-4, 6, 99], 8),
+                                          ([4, 2, 6], 9), ([3] + [4] * 70, 6)])
+def test_rows_outside_the_segments(kind, offsets, rows):
+    # cleared by the product's own launch; offsets out of range or order lose rows and leave the others zero
+    E, N, K = len(offsets) - 1, 192, 128
+    gw, dense = _bank(kind, E, N, K, 3)
+    x = torch.empty(rows, K, device="cuda").normal_(0, 1, generator=torch.Generator(device="cuda").manual_seed(1)).to(torch.bfloat16)
+    off = torch.tensor(offsets, device="cuda", dtype=torch.int32)
+    want = torch.zeros(rows, N, device="cuda", dtype=torch.bfloat16)
+    T.qlinear_grouped_forward(x, off, gw, T.BF16, T.BF16, out=want)       # into a result that is cleared already
+    dirty = torch.full((rows, N), float("nan"), device="cuda", dtype=torch.bfloat16)      # what a fresh result's memory may hold
+    del dirty
+    assert torch.equal(T.qlinear_grouped_forward(x, off, gw, T.BF16, T.BF16), want)
+    covered = torch.zeros(rows, dtype=torch.bool)
+    for e in range(E):
+        lo = min(max(offsets[e], 0), rows)
+        covered[lo:max(lo, min(max(offsets[e + 1], 0), rows))] = True
+    assert not want[~covered.cuda()].any()
