@@ -120,7 +120,7 @@ static size_t workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype, int 
   a.compute_dtype = compute_dtype;
   a.w.kind = w_kind;
   const size_t f32_bytes = mfma_f32_workspace_bytes(a, backward);
-  // float storage runs on the fp32 matrix-core kernel unless it is stored in the 16-bit compute type itself
+  // float storage runs on the fp32 matrix-core instruction unless it is stored in the 16-bit compute type itself
   if (float_kind(w_kind) && !same_16bit(w_kind, compute_dtype)) return f32_bytes;
   size_t bytes = mfma_workspace_bytes(a, backward);
   const auto at_least = [&bytes](size_t b) { bytes = b > bytes ? b : bytes; };
@@ -182,8 +182,9 @@ static int forward_impl(int64_t M, int64_t N, int64_t K, const void *x, int x_dt
   // matrix-core tiling (cost independent of M) is faster; both fall through when a shape does not fit
   st = CAIFX_ERR_UNSUPPORTED;
   // fp32 compute.  int8 storage with up to 32 rows: the row-block decode kernel on the integer matrix core (digit
-  // planes of the fp32 activations); otherwise from two rows on the fp32 matrix-core kernel (40-43 us at
-  // K = N = 4096 whatever M <= 32); the VALU decode kernel below takes 40-46 us for one row
+  // planes of the fp32 activations); otherwise from two rows on products of bf16 pieces, or the fp32 instruction where those
+  // do not fit (mfma_f32_forward chooses).  One row of int4 takes the VALU decode kernel below: the pieces would be up to
+  // 1.5 times as fast on large weights, but with an error of 1.1e-7 against its 8.5e-8
   if (compute_dtype == CAIFX_F32) {
     if (M <= 32 && w_kind == CAIFX_W_INT8) {
       st = mblock_forward(a, s);
@@ -202,7 +203,7 @@ static int forward_impl(int64_t M, int64_t N, int64_t K, const void *x, int x_dt
     if (st == CAIFX_ERR_UNSUPPORTED) st = skinny_forward(a, s);
   }
   if (M > 16 && M <= 32) {
-    // 17..32 rows: the decode kernel with two tiles of 16 rows reads the weight once; without the workspace its
+    // 17..32 rows: the decode kernel with two tiles of 16 rows reads the weight once; without the workspace the
     // reduction slices need, two launches of the 16-row form (2 x 14-17 us at K = 4096, N = 4096..14336) still
     // beat the tiled GEMM, whose shortest launch is one tile's reduction (43 us int4, 68 us int8 at K = 4096)
     st = mblock_forward(a, s);

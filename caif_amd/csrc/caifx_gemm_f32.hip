@@ -1,4 +1,6 @@
-// Dequant-GEMM for the fp32 compute type on the matrix cores: Y[M,N] = X[M,K] * W[N,K]^T and
+// Dequant-GEMM on the fp32 matrix-core instruction: what the products of pieces (caifx_gemm_pieces.hip) do not take, that is
+// float storage, expert segments, reductions that are no multiple of 64, up to 80 rows of a short reduction (640 at most), and
+// scale vectors or groups outside that kernel's forms.  Y[M,N] = X[M,K] * W[N,K]^T and
 // dX[M,K] = dY[M,N] * W[N,K] with W stored int8 or packed int4 and dequantised to fp32 exactly as the
 // reference's dequantise kernels do (fp32 code * scale, no further rounding; ConvertToComputeDtype with
 // ComputeT = float, src/caif_device_frozen_linear.cpp:289-378), activations widened to fp32, fp32
@@ -8,7 +10,8 @@
 // before anything else and is kept simple: 256 threads, one BM x 128 tile of the result per workgroup, 32
 // deep reduction steps, one LDS buffer per operand (the global loads of the next two steps are in flight in two
 // register sets while the matrix cores work on the current one; two barriers per step cost little against the
-// 1000-4000 MFMA cycles between them).  Plain and grouped (per-expert row segments) problems.  Both operands sit in LDS reduction-major ([r][row] with the row index contiguous),
+// 1000-4000 MFMA cycles between them).  Plain and grouped (per-expert row segments) problems.  Both operands sit in
+// LDS reduction-major ([r][row] with the row index contiguous),
 // which is what the MFMA operands read: lane (i, h) of a 32x32x2 step takes element [2p + h][i].
 // Up to 32 activation rows a workgroup takes a 32 x 32 tile with 128-deep steps and its four waves split each
 // step's reduction (partial tiles are added through LDS in a fixed order at the end): four times as many

@@ -7,7 +7,7 @@
 // the fp32 instruction.  Error against 64 bits (2-norm, relative; N(0,1) x N(0,0.02)), fp32 instruction -> here: M = 185, N = 3456,
 // K = 3712 int4 1.0e-6 -> 1.6e-7, int8 1.1e-6 -> 2.1e-7; M = 256, 8192 x 4096 1.1e-6 -> 3.3e-7 and 3.9e-7; M = 40, 1024 x 512 1.9e-7 ->
 // 7.4e-8 and 2.1e-7 -> 9.2e-8.  us, forward / gradient: M = 200, N = 3456, K = 3712, int4 120 / 123 -> 60 / 62; M = 66, 6720 x 3584
-// 85 / 235 -> 43 / 42; M = 2048, 4096 x 4096 549 / 570 -> 420 / 403.
+// 85 / 235 -> 43 / 42; M = 2048, 4096 x 4096 549 / 570 -> 420 / 403 (int8 590 / 594 -> 496 / 456).
 //
 // What bounds it with up to a few hundred rows is not the products but cutting the operands (6 to 8 VALU instructions a value,
 // a tile of 64 x 64 x 64 as long as its 48 products per wave) and the latency of a step, so two to four workgroups share a

@@ -1,9 +1,9 @@
-// Decode path for a handful of activation rows (2 <= M <= 16): Y[M,N] = X[M,K] * W[N,K]^T with W
+// Decode path for a handful of activation rows (M <= 32, in tiles of 16): Y[M,N] = X[M,K] * W[N,K]^T with W
 // stored int8 or packed int4, memory bound on the weight stream.
 //
 // The matrix cores do the dot products with the activation rows as the 16 rows of the A operand
 // of v_mfma_f32_16x16x32 (rows past M are zero) and 16 weight rows as the columns of B, so the
-// cost per weight byte does not depend on M.  A workgroup is 16 waves; wave w owns the k range
+// cost per weight byte does not depend on M.  A workgroup is up to 16 waves; wave w owns the k range
 // [w*GPW*128, (w+1)*GPW*128) for every weight row the workgroup visits and keeps the matching
 // slice of X in registers, already laid out as A operands, for the whole kernel.  Per block of 16
 // weight rows a lane (j = lane%16, q = lane/16) loads 16 bytes of row j:
@@ -17,7 +17,7 @@
 //         (no unpacking arithmetic).  The scales are folded into the activations instead: a scale
 //         vector of period P is addressed by the flat index n*K + k modulo P; rows n with equal
 //         n mod V, V = P / gcd(K mod P, P), see the same scales along k, so a workgroup only visits
-//         rows of one residue class, stages that class's K scales in LDS once and forms
+//         rows of one residue class; each of its waves stages that class's scales of its own k range in LDS and forms
 //         x'[m][k] = x[m][k] * scale[k] in fp32.  x' is split into three signed 8-bit digit planes
 //         relative to a power-of-two unit per activation row and wave (x' ~ unit * (d0 + d1/256 +
 //         d2/65536), |d0| <= 32, error <= unit * 2^-17); the three exact int32 sums are combined in fp32 per block.
@@ -143,8 +143,8 @@ constexpr int kSegRows = kSegBlocks * 16;
 // and written once per kSegRows rows).  A wait for one block of the ring then leaves the younger
 // block in flight instead of draining the queue.
 // kF32 (int8 only): fp32 compute type.  The activations are not rounded to a 16-bit type: the digit planes are cut
-// from x * scale in fp32, read from memory in both passes over them instead of being kept in registers (CT then
-// only names a vector type nothing is stored in).
+// from x * scale in fp32.  The activations are held in registers between the two passes over them where they fit
+// (kHoldF32) and read from memory twice otherwise (CT then only names a vector type nothing is stored in).
 // MT: tiles of 16 activation rows that share one pass over the weight (M <= 16 * MT); every weight fragment is
 // unpacked once and multiplied with each tile's operands.
 // wq / scales: the weight; xrows / yrows: the first of the M activation and result rows; slice: which part of
@@ -560,7 +560,8 @@ struct MbGroup {
 
 // Zeroes the rows of a grouped result that no segment covers, the launch's workgroups sharing them: [0, offsets[0]) and
 // [offsets[E], rows), none of which a unit writes.  Offsets that step down somewhere (a caller's mistake) may also leave rows in
-// between, or cover some of those: then each row is looked up.  A launch of its own in front of the product took 4.7 us of a decode step.
+// between, or cover some of those: then each row is looked up.  As a launch of its own in front of each
+// of the three products it was a quarter of the smallest MoE decode passes (ten of them, geometric mean: 1.25x without).
 __device__ __forceinline__ void zero_uncovered(const MbGroup &g, unsigned char *y, int64_t row_bytes)
 {
   const int lane = threadIdx.x & 63;
@@ -670,7 +671,8 @@ int launch_gpw(const MbArgs &m, size_t lds, hipStream_t s)
                   static_cast<unsigned>((m.groups + m.slice_groups - 1) / m.slice_groups));
   const int gpw = (m.slice_groups + kMbWaves - 1) / kMbWaves;
   if (m.M <= 16) {
-    // One row block requested at a time instead of two, by measurement (K = 4096, N = 2048 ... 28672, times in us):
+    // One row block requested at a time instead of two, by measurement with sixteen waves and one slice (K = 4096,
+    // N = 2048 ... 28672, times in us):
     // int4 with 4 rows 7.2 -> 6.6, 7.9 -> 7.1, 9.6 -> 9.1, 11.0 -> 10.6, 12.7 -> 12.4, 20.4 -> 19.7; with 16 rows
     // 9.0 -> 8.4, 9.4 -> 8.9, 11.3 -> 11.2, 12.8 -> 13.1, 14.7 -> 14.9, 23.0 -> 22.4, so two stay only for more than 8
     // rows with 33..64 weight rows per workgroup; int8 gains up to 32 weight rows per workgroup (10.8 -> 10.6,

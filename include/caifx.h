@@ -151,7 +151,7 @@ CAIFX_API int caifx_qlinear_forward(int64_t M, int64_t N, int64_t K,
  *   dX[M,K] = cast<compute>(dY)[M,N] * cast<compute>(dequant(W))[N,K], fp32 accumulate.
  * With up to 16 rows and int8 codes (any scale vector that leaves at most 64 residue classes of rows with
  * equal scales along k, each of 256 rows or more; one scale; none) or int4 codes in groups of 128 or more, the
- * weight is streamed once through the matrix cores (the 16-bit ones for a 16-bit compute type, the fp32 one
+ * weight is streamed once through the matrix cores (the 16-bit ones for a 16-bit compute type, the fp32 ones
  * for fp32).  For int8 codes the scale is applied outside the products: like the forward's memory-bound kernels
  * this skips the rounding of code * scale to a 16-bit compute type (about 2e-3 of max|dX| for bf16; for the
  * fp32 compute type the difference is fp32 rounding, 1e-7).  int4 codes with a 16-bit compute type meet their
@@ -195,10 +195,10 @@ CAIFX_API int caifx_qlinear_backward_input_add(int64_t M, int64_t N, int64_t K,
  * The partial tiles (caifx_qlinear_partials_workspace_bytes asks for them alone): nonzero for 16-bit compute types when the
  * result has fewer 128 x 128 tiles than the chip has compute units: up to 8 workgroups then share a tile's reduction through
  * fp32 partial tiles in the workspace (16-byte aligned) and a second launch adds them in a fixed order (results do
- * not depend on scheduling).  The fp32 compute type does the same for up to 128 rows.  The forward with up to
- * 32 rows cuts a reduction longer than one workgroup covers into slices whose sums meet there (K > 4096 with up
- * to 16 rows, K > 2048 with 17..32 rows or with int8 codes and N small enough that the activations' preparation
- * outweighs a workgroup's share of the weight), and the input gradient with up to 16 rows splits
+ * not depend on scheduling).  The fp32 compute type does the same (int8 and int4 codes: while there are too few tiles of 64
+ * columns; float storage: up to 128 rows).  The forward with up to 32 rows cuts the reduction into slices of 1024, 2048 or 4096
+ * whose sums meet there (always where K exceeds what one workgroup covers, 4096 with up to 16 rows and 2048 with more; in
+ * shorter ones where the estimated time falls), and the input gradient with up to 16 rows splits
  * the weight's rows among workgroups the same way.  With a smaller or null
  * workspace the calls run without that sharing, slower, and the sums are formed in a different order, so
  * the last bits of a result differ between a call with and a call without the workspace.  In two places the
