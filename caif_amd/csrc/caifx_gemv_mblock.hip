@@ -942,7 +942,8 @@ int mblock_grouped_forward(const GemmArgs &g, hipStream_t s)
   m.waves = mb_plan(g, 1, g.K).waves;
   const size_t lds = mb_lds_bytes(int4, 1, m.groups);
   const int64_t unit = ((g.N + m.V - 1) / m.V + 15) / 16;
-  if (((g.M + 15) / 16 + g.num_experts) * unit * m.V >= (int64_t{1} << 31)) return CAIFX_ERR_UNSUPPORTED;
+  // the kernel counts blocks in 32 bits, also where offsets that step down let every segment cover all rows
+  if ((g.M + 15) / 16 * g.num_experts * unit * m.V >= (int64_t{1} << 31)) return CAIFX_ERR_UNSUPPORTED;
   MbGroup grp{g.offsets, g.wq_ptrs, g.scales_ptrs, g.M, g.num_experts, static_cast<unsigned>(unit), static_cast<unsigned>(unit * m.V), g.zero_rest};
   return g.compute_dtype == CAIFX_BF16 ? launch_grouped_xt<bf16_t>(m, grp, g.x_dtype, int4, lds, s)
                                        : launch_grouped_xt<f16_t>(m, grp, g.x_dtype, int4, lds, s);
