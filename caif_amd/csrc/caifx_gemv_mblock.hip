@@ -129,6 +129,16 @@ __device__ __forceinline__ uint32_t pack_low_bytes(int a, int b, int c, int d)
   return __builtin_amdgcn_perm(cd, ab, 0x05040100u);
 }
 
+// Between LDS stores of a wave and its lanes' loads of what other lanes stored.  A wave's LDS operations are carried out in order,
+// so nothing is waited for: the fences keep the compiler from moving either past the other (the wave barrier alone does not, it
+// touches no memory).
+__device__ __forceinline__ void exchange_in_wave()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // row blocks between two additions of the waves' partial tiles
 constexpr int mb_reduce_blocks(bool int4, int mt) { return int4 && mt == 1 ? 4 : 2; }
 
@@ -322,7 +332,7 @@ __device__ __forceinline__ void mblock_body(const MbArgs &a, const uint8_t *wq, 
       poison[mt][r] = false;
     }
   if constexpr (!kInt4) {
-    __builtin_amdgcn_wave_barrier();       // the wave's scales are staged
+    exchange_in_wave();       // the wave's scales are staged
     // four consecutive x' values: quad c (0..3) of step t of tile mt
     auto xprime4 = [&](int mt, int t, int c, float (&v)[4]) {
       const int g = t >> 1;
