@@ -1,0 +1,15 @@
+// Prints the plan of the products of bf16 pieces for calls read from stdin, one a line: M C R int4 room.
+#include "caifx_gemm_pieces_plan.hpp"
+
+#include <cstdio>
+
+int main()
+{
+  long long M, C, R, int4;
+  unsigned long long room;
+  while (std::scanf("%lld %lld %lld %lld %llu", &M, &C, &R, &int4, &room) == 5) {
+    const caifx::PiecesPlan p = caifx::plan_pieces(M, C, R, int4 != 0, static_cast<size_t>(room));
+    std::printf("%d %d %d %zu\n", p.bm, p.parts, p.part_steps, p.bytes);
+  }
+  return 0;
+}
