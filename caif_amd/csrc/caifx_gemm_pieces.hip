@@ -49,52 +49,47 @@ __device__ __forceinline__ void store_result(void *p, int dt, int64_t i, float v
 __device__ __forceinline__ float low_bf16(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
 __device__ __forceinline__ float high_bf16(uint32_t p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
 
-// Two values as P pieces each, packed (the first value in the low half).
-// A value whose first piece is no number (an infinity, a NaN, or a finite value that bf16 would round to an infinity) turns its
-// remainder into NaN, which `odd` collects.
-template <int P> __device__ __forceinline__ void cut2(float x0, float x1, uint32_t (&p)[P], float &odd)
+// Pieces are the value where it is zero or its magnitude lies in these ranges.  Below, a piece or a product of first and last pieces
+// would be a subnormal number (2^-64 * 2^-38 = 2^-102, its last bits 2^-125); above, sums of fewer than 2^22 products could pass the
+// largest number in acc and its negative in rest.  Weights are held to theirs by their scales (int8 codes: 2^-38 to 2^43; every finite
+// fp16 scale does).  A step of a tile that meets another value (an infinity, a NaN, one too large or too small) runs on the fp32
+// instruction, with the results that one gives.  What the looking costs: 2 % (120 calls, geometric mean).
+constexpr float kLeastX = 0x1p-64f, kMostX = 0x1p50f;
+constexpr float kLeastS = 0x1p-38f, kMostS = 0x1p43f;
+
+// the smallest and the largest magnitude of what a thread has seen of a step (NaN from a NaN on): half an instruction a value each
+struct Seen {
+  float least, most;
+};
+__device__ __forceinline__ void see(Seen &o, float v)
+{
+  o.least = __builtin_elementwise_minimum(o.least, fabsf(v));
+  o.most = __builtin_elementwise_maximum(o.most, fabsf(v));
+}
+
+// Two values as P pieces each, packed (the first value in the low half)
+template <int P> __device__ __forceinline__ void cut2(float x0, float x1, uint32_t (&p)[P])
 {
   p[0] = pack2<bf16_t>(x0, x1);
-  float r0 = x0 - low_bf16(p[0]), r1 = x1 - high_bf16(p[0]);
-  odd = __builtin_fmaf(r0, 0.0f, __builtin_fmaf(r1, 0.0f, odd));
+  const float r0 = x0 - low_bf16(p[0]), r1 = x1 - high_bf16(p[0]);
   p[1] = pack2<bf16_t>(r0, r1);
   if constexpr (P > 2) p[2] = pack2<bf16_t>(r0 - low_bf16(p[1]), r1 - high_bf16(p[1]));
 }
-// the same for such values.  An infinity or a NaN is its last piece: that one meets no piece but the other operand's first, which
-// has the value's sign and is zero only with it (an infinity times a middle piece would be NaN or of the wrong sign).  Finite
-// values are cut by truncation.
-template <int P> __device__ __forceinline__ void cut2_odd(float x0, float x1, uint32_t (&p)[P])
-{
-  float x[2] = {x0, x1};
-#pragma unroll
-  for (int i = 0; i < P; ++i) p[i] = 0;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const bool finite = fabsf(x[h]) <= 3.4028235e38f;
-    float rest = x[h];
-#pragma unroll
-    for (int i = 0; i < P; ++i) {
-      uint32_t bits = __builtin_bit_cast(uint32_t, rest) >> 16;
-      if (!finite) bits = i < P - 1 ? 0u : (x[h] != x[h] ? 0x7fc0u : bits);
-      else rest -= __builtin_bit_cast(float, bits << 16);
-      p[i] |= bits << (16 * h);
-    }
-  }
-}
 // n values (a multiple of 2) as pieces: out[piece][i] holds values 2 i and 2 i + 1
-template <int P, bool kOdd, int n> __device__ __forceinline__ void cut(const float (&x)[n], uint32_t (&out)[P][n / 2], float &odd)
+template <int P, int n> __device__ __forceinline__ void cut(const float (&x)[n], uint32_t (&out)[P][n / 2])
 {
 #pragma unroll
   for (int i = 0; i < n / 2; ++i) {
     uint32_t p[P];
-    if constexpr (kOdd) cut2_odd<P>(x[2 * i], x[2 * i + 1], p);
-    else cut2<P>(x[2 * i], x[2 * i + 1], p, odd);
+    cut2<P>(x[2 * i], x[2 * i + 1], p);
 #pragma unroll
     for (int k = 0; k < P; ++k) out[k][i] = p[k];
   }
 }
 
 __device__ __forceinline__ int swizzled(int row, int chunk) { return row * 128 + ((chunk ^ ((row ^ (row >> 3)) & 7)) << 4); }
+// the same for rows of 64 fp32 values (a step on the fp32 instruction)
+__device__ __forceinline__ int swizzled32(int row, int chunk) { return row * 256 + ((chunk ^ (row & 15)) << 4); }
 
 // kVec: int8 with a scale vector
 template <typename XT, bool kInt4, bool kVec, bool kBackward, int BM>
@@ -107,6 +102,7 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
   constexpr int TM = BM / 32;              // 16-row blocks of a wave
   __shared__ __attribute__((aligned(16))) unsigned char As[3][BM * 128];
   __shared__ __attribute__((aligned(16))) unsigned char Bs[PW][kPN * 128];
+  __shared__ int fp32_step[2];             // a wave met a value the pieces do not hold, in a step of this parity
 
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -137,16 +133,34 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
     for (int i = 0; i < kALoads; ++i)
       areg[i] = *reinterpret_cast<const u32x4_t *>(a_base + static_cast<int64_t>(s) * (kPK * sizeof(XT)) + a_off[i]);
   };
-  auto store_a = [&](auto odd_path_, float &odd) __attribute__((always_inline)) {
-    constexpr bool kOdd = decltype(odd_path_)::value;
+  // a zero is ordinary, another number below kLeastX is not (fp16 holds none)
+  auto tiny_a = [&]() __attribute__((always_inline)) {
+    bool tiny = false;
+    if constexpr (!std::is_same<XT, f16_t>::value) {
+#pragma unroll
+      for (int i = 0; i < kALoads; ++i) {
+        const XT *h = reinterpret_cast<const XT *>(&areg[i]);
+#pragma unroll
+        for (int e = 0; e < kAV; ++e) {
+          const float x = fabsf(to_f32<XT>(h[e]));
+          tiny = tiny | ((x != 0.0f) & (x < kLeastX));
+        }
+      }
+    }
+    return tiny;
+  };
+  auto store_a = [&](Seen &seen) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kALoads; ++i) {
       const XT *h = reinterpret_cast<const XT *>(&areg[i]);
       float x[kAV];
 #pragma unroll
-      for (int e = 0; e < kAV; ++e) x[e] = to_f32<XT>(h[e]);
+      for (int e = 0; e < kAV; ++e) {
+        x[e] = to_f32<XT>(h[e]);
+        see(seen, x[e]);
+      }
       uint32_t p[3][kAV / 2];
-      cut<3, kOdd>(x, p, odd);
+      cut<3>(x, p);
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         unsigned char *to = As[k] + swizzled(a_row + kARows * i, a_col >> 3) + (a_col & 7) * 2;
@@ -164,7 +178,6 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
       }
     }
   };
-
   // ---- weights: four codes along k of four rows per thread and step.
   // forward: rows n = col0 + t / 16 + 16 r, k = 4 (t % 16) ..; gradient: rows n = 4 (t / 16) + r of the step, columns col0 + 4 (t % 16) ..
   const int b_row = kBackward ? 4 * (t >> 4) : t >> 4, b_col = 4 * (t & 15);
@@ -220,9 +233,7 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
       }
     }
   };
-  auto store_b = [&](auto odd_path_, float &odd) __attribute__((always_inline)) {
-    constexpr bool kOdd = decltype(odd_path_)::value;
-    float w[4][4];          // [row][along k]
+  auto weights = [&](float (&w)[4][4]) __attribute__((always_inline)) {          // [row][along k]
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       if constexpr (kInt4) {
@@ -235,18 +246,65 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
         for (int e = 0; e < 4; ++e) w[r][e] = q[e] * (kVec ? sc[r][kVec ? e : 0] : s_one);
       }
     }
+  };
+  // four weights along the reduction, and the row and the reduction element in LDS where they begin
+  const int b_at = kBackward ? b_row : b_col;
+  auto b_lds_row = [&](int c) __attribute__((always_inline)) { return kBackward ? b_col + c : b_row + 16 * c; };
+  auto store_b = [&](Seen &seen) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (kInt4 || kVec) {
+#pragma unroll
+        for (int e = 0; e < (kVec ? 4 : 1); ++e) see(seen, sc[r][e]);
+      }
+    }
+    float w[4][4];
+    weights(w);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const float x[4] = {kBackward ? w[0][c] : w[c][0], kBackward ? w[1][c] : w[c][1], kBackward ? w[2][c] : w[c][2], kBackward ? w[3][c] : w[c][3]};
       uint32_t p[PW][2];
-      cut<PW, kOdd>(x, p, odd);
-      const int row = kBackward ? b_col + c : b_row + 16 * c, at = kBackward ? b_row : b_col;
+      cut<PW>(x, p);
 #pragma unroll
       for (int k = 0; k < PW; ++k) {
         u32x2_t v;
         v[0] = p[k][0];
         v[1] = p[k][1];
-        *reinterpret_cast<u32x2_t *>(Bs[k] + swizzled(row, at >> 3) + (at & 7) * 2) = v;
+        *reinterpret_cast<u32x2_t *>(Bs[k] + swizzled(b_lds_row(c), b_at >> 3) + (b_at & 7) * 2) = v;
+      }
+    }
+  };
+  // A step's operands as fp32 values in the place of the pieces: read from memory again and in rolled loops, so that this rare
+  // path takes no registers from the other.
+  auto store_fp32 = [&](int s) __attribute__((always_inline)) {
+    const XT *a0 = reinterpret_cast<const XT *>(a_base) + static_cast<int64_t>(s) * kPK + a_col;
+#pragma unroll 1
+    for (int r = a_row; r < BM; r += kARows) {
+      const XT *from = a0 + static_cast<int64_t>(r < rows ? r : rows - 1) * R;
+#pragma unroll
+      for (int c = 0; c < kAV / 4; ++c) {
+        floatx4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = to_f32<XT>(from[4 * c + e]);
+        *reinterpret_cast<floatx4_t *>(As[0] + swizzled32(r, (a_col >> 2) + c)) = v;
+      }
+    }
+#pragma unroll 1
+    for (int r = 0; r < 4; ++r) {
+      int64_t f = flat0 + static_cast<int64_t>(s) * flat_step;
+      if constexpr (kBackward) f += (b_row + r) * g.K + (col0 + b_col + 4 <= g.K ? b_col : g.K - 4 - col0);
+      else f += (col0 + b_row + 16 * r < g.N ? b_row + 16 * r : g.N - 1 - col0) * g.K + b_col;
+      floatx4_t v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (kInt4) v[e] = static_cast<float>(static_cast<int>(static_cast<uint32_t>(g.wq[(f + e) >> 1]) << (28 - 4 * (e & 1))) >> 28) * to_f32(s16[f >> g.group_shift]);
+        else v[e] = static_cast<float>(static_cast<const int8_t *>(static_cast<const void *>(g.wq))[f + e]) * (kVec ? s32[f % g.period + e] : s_one);
+      }
+      if constexpr (kBackward) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) *reinterpret_cast<float *>(Bs[0] + swizzled32(b_col + e, b_row >> 2) + 4 * r) = v[e];
+      } else {
+        *reinterpret_cast<floatx4_t *>(Bs[0] + swizzled32(b_row + 16 * r, b_col >> 2)) = v;
       }
     }
   };
@@ -268,42 +326,72 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
     load_b(at);
     next_scales();
   };
+  // one scale for the weight (or none) is held to its range here
+  const unsigned long long one_scale_odd = !kInt4 && !kVec && s_one != 0.0f && !(fabsf(s_one) >= kLeastS && fabsf(s_one) < kMostS);
   load(0);
+  if (t < 2) fp32_step[t] = 0;
+  meet();
   for (int s = 0; s < steps; ++s) {
-    float odd = 0.0f;
-    store_a(std::false_type{}, odd);
-    store_b(std::false_type{}, odd);
-    if (__ballot(!(odd == 0.0f)) != 0) {          // one branch a step for the whole wave, rarely taken: both operands once more
-      store_a(std::true_type{}, odd);
-      store_b(std::true_type{}, odd);
+    Seen xs{kMostX, 0.0f}, ss{kMostS, kLeastS};
+    store_a(xs);
+    store_b(ss);
+    unsigned long long odd = __ballot(!(xs.most < kMostX)) | one_scale_odd;          // (masks: no lane of the wave leaves the straight line)
+    if constexpr (kInt4) odd |= __ballot(!(ss.most <= 65504.0f));
+    if constexpr (kVec) odd |= __ballot(!(ss.least >= kLeastS)) | __ballot(!(ss.most < kMostS));          // (a scale of zero counts as too small)
+    unsigned long long zero_or_tiny = 0;
+    if constexpr (!std::is_same<XT, f16_t>::value) zero_or_tiny = __ballot(!(xs.least >= kLeastX));
+    if ((odd | zero_or_tiny) != 0) {                    // which of the two is asked only where there is one
+      if ((odd | __ballot(tiny_a())) != 0) fp32_step[s & 1] = 1;
     }
     meet();
+    const int flagged = fp32_step[s & 1];
     load(s + 1);
+    if (t == 0) fp32_step[(s + 1) & 1] = 0;      // read before this step's first barrier, written after its second
+    if (__builtin_amdgcn_readfirstlane(flagged) != 0) {          // the same for the whole workgroup, rare
+      store_fp32(s);
+      meet();
+#pragma unroll 1
+      for (int c = 0; c < 4; ++c) {                              // lane (r16, kq) holds reduction elements 16 c + 4 kq + e in both operands
+        floatx4_t b[2];
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      bf16x8_t b[PW][2];
+        for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const floatx4_t *>(Bs[0] + swizzled32(32 * wn + 16 * j + r16, 4 * c + kq));
 #pragma unroll
-      for (int k = 0; k < PW; ++k)
+        for (int i = 0; i < TM; ++i) {
+          if (i >= mine) break;
+          const floatx4_t a = *reinterpret_cast<const floatx4_t *>(As[0] + swizzled32(16 * (2 * i + wm) + r16, 4 * c + kq));
 #pragma unroll
-        for (int j = 0; j < 2; ++j) b[k][j] = *reinterpret_cast<const bf16x8_t *>(Bs[k] + swizzled(32 * wn + 16 * j + r16, 4 * kk + kq));
+          for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        if (i >= mine) break;                                    // the same for every lane of the wave
-        bf16x8_t a[3];
+            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[j][e], acc[i][j], 0, 0, 0);
+        }
+      }
+    } else {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) a[k] = *reinterpret_cast<const bf16x8_t *>(As[k] + swizzled(16 * (2 * i + wm) + r16, 4 * kk + kq));
+      for (int kk = 0; kk < 2; ++kk) {
+        bf16x8_t b[PW][2];
 #pragma unroll
-        for (int sum = 2; sum >= 0; --sum)
+        for (int k = 0; k < PW; ++k)
 #pragma unroll
-          for (int k = 0; k < PW; ++k) {
-            const int ka = sum - k;
-            if (ka < 0) continue;
+          for (int j = 0; j < 2; ++j) b[k][j] = *reinterpret_cast<const bf16x8_t *>(Bs[k] + swizzled(32 * wn + 16 * j + r16, 4 * kk + kq));
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-              floatx4_t &to = sum == 0 ? acc[i][j] : rest[i][j];
-              to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ka], b[k][j], to, 0, 0, 0);
+        for (int i = 0; i < TM; ++i) {
+          if (i >= mine) break;                                    // the same for every lane of the wave
+          bf16x8_t a[3];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) a[k] = *reinterpret_cast<const bf16x8_t *>(As[k] + swizzled(16 * (2 * i + wm) + r16, 4 * kk + kq));
+#pragma unroll
+          for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+            for (int k = 0; k < PW; ++k) {
+              const int ka = sum - k;
+              if (ka < 0) continue;
+#pragma unroll
+              for (int j = 0; j < 2; ++j) {
+                floatx4_t &to = sum == 0 ? acc[i][j] : rest[i][j];
+                to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ka], b[k][j], to, 0, 0, 0);
+              }
             }
-          }
+        }
       }
     }
     meet();              // the next step overwrites both operands
