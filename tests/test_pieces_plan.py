@@ -36,3 +36,13 @@ def test_every_plan_fits_the_launch_and_the_room(plans):
         assert -(-M // bm) <= 65535, (M, C, R, int4, bm)          # gridDim.y
         assert 1 <= parts <= 65535 and (parts - 1) * per < R // 64 <= parts * per
         assert size == (parts * M * C * 4 if parts > 1 else 0) and size <= min(room, STATIC)
+
+
+# One or two steps in more than one round of the chip, where tiles of 32 rows cut the weight four times as often: int8, us with 32 / 64 /
+# 128 rows 215 / 174 / 165, 118 / 94 / 97, 60 / 53 / 51, 54 / 47 / 46, 133 / 117 / 115 in the order
+# below (int4 161 / 142 / 152 to 44 / 40 / 43; with one step 102 / 97 / 104, left out).
+@pytest.mark.parametrize("int4", [0, 1])
+def test_short_reductions_of_many_rows_take_tall_tiles(plans, int4):
+    calls = [(M, C, R, int4, room) for M, C, R in [(4096, 14336, 128), (4096, 8192, 128), (4096, 4096, 128), (1024, 14336, 128), (4096, 14336, 64)][:4 if int4 else 5]
+             for room in (0, NO_LIMIT)]
+    assert all(bm > 32 for bm, _, _, _ in plans(calls))
