@@ -1,6 +1,6 @@
 // Dequant-GEMM on the fp32 matrix-core instruction: what the products of pieces (caifx_gemm_pieces.hip) do not take, that is
-// float storage, expert segments, reductions that are no multiple of 64, up to 80 rows of a short reduction (640 at most), and
-// scale vectors or groups outside that kernel's forms.  Y[M,N] = X[M,K] * W[N,K]^T and
+// float storage, expert segments, reductions that are no multiple of 64, scale vectors or groups outside that kernel's forms, and up to 128 rows
+// of a short reduction or without room to share a longer one (split_tile_first).  Y[M,N] = X[M,K] * W[N,K]^T and
 // dX[M,K] = dY[M,N] * W[N,K] with W stored int8 or packed int4 and dequantised to fp32 exactly as the
 // reference's dequantise kernels do (fp32 code * scale, no further rounding; ConvertToComputeDtype with
 // ComputeT = float, src/caif_device_frozen_linear.cpp:289-378), activations widened to fp32, fp32
@@ -19,12 +19,12 @@
 #include <type_traits>
 
 #include "caifx_internal.hpp"
+#include "caifx_gemm_pieces_plan.hpp"
 
 namespace caifx {
 namespace {
 
 constexpr int kStep = 32;    // the reduction advances in multiples of this (host-side checks, scale-index steps)
-constexpr int kSplitTileRows = 128;   // up to this many rows the 32 x 32 split tile is used (M = 64: 256 workgroups instead of 64)
 
 struct F32Args {
   int64_t M, N, K;
@@ -410,32 +410,9 @@ int launch_kind(const F32Args &f, int kind, bool int4, bool backward, hipStream_
   return backward ? launch_bm<XT, false, false, true>(f, s) : launch_bm<XT, false, false, false>(f, s);
 }
 
-// Up to 32 rows there are C / 32 split tiles, 128 at C = 4096 (more rows: that many per 32 rows): a chain of R / 128 dependent steps on half of the
-// chip.  With a workspace from the caller up to 4 workgroups share a tile's reduction (at least 8 steps each, about
-// one workgroup per compute unit in total) and a second launch adds their partial tiles in a fixed order.
-struct F32Plan {
-  int parts;
-  int part_steps;
-  size_t bytes;
-};
-F32Plan plan_f32(int64_t M, int64_t C, int64_t R, bool grouped)
+SplitTilePlan plan_f32(int64_t M, int64_t C, int64_t R, bool grouped)
 {
-  F32Plan p{1, 0, 0};
-  if (grouped || M > kSplitTileRows || R % 128 != 0) return p;
-  const int64_t tiles = ((C + 31) / 32) * ((M + 31) / 32);
-  if (tiles > 128) return p;
-  const int64_t steps = R / 128;
-  int64_t k = 256 / tiles;
-  if (k > 4) k = 4;
-  if (k > steps / 8) k = steps / 8;
-  if (k < 2) return p;
-  const int64_t per = (steps + k - 1) / k;
-  k = (steps + per - 1) / per;
-  if (k < 2) return p;
-  p.parts = static_cast<int>(k);
-  p.part_steps = static_cast<int>(per);
-  p.bytes = static_cast<size_t>(k) * static_cast<size_t>(M) * static_cast<size_t>(C) * sizeof(float);
-  return p;
+  return grouped ? SplitTilePlan{1, 0, 0} : plan_split_tile(M, C, R);
 }
 
 int run_f32(const GemmArgs &a, bool backward, hipStream_t s)
@@ -488,7 +465,7 @@ int run_f32(const GemmArgs &a, bool backward, hipStream_t s)
   f.round_dt = float_w ? a.compute_dtype : CAIFX_F32;
   f.parts = 1;
   const int64_t cols = backward ? a.K : a.N;
-  const F32Plan plan = plan_f32(a.M, cols, R, grouped);
+  const SplitTilePlan plan = plan_f32(a.M, cols, R, grouped);
   const bool shared = plan.parts > 1 && a.workspace && a.workspace_bytes >= plan.bytes && aligned_to(a.workspace, 4);
   if (shared) {
     f.parts = plan.parts;

@@ -436,23 +436,30 @@ bool pieces_shape(const GemmArgs &a, bool backward)
   if (a.compute_dtype != CAIFX_F32 || a.offsets || a.addend || a.epilogue) return false;
   if (a.w.kind != CAIFX_W_INT8 && a.w.kind != CAIFX_W_INT4_GROUP) return false;
   const int64_t R = backward ? a.N : a.K, C = backward ? a.K : a.N;
-  // up to five 128-deep steps of the fp32 instruction's kernel, whose waves share them, are done before the pieces pay (M = 65,
-  // R = 512, C = 2176 10.0 us there, 11.6 here; M = 33 and 8 equal; M = 100 12.7 and 12.1; R = 1024 11.6 and 9.4)
-  if (a.M <= 80 && R <= 640 && R % 128 == 0) return false;
   return R >= kPK && R % kPK == 0 && a.K % 16 == 0 && a.M >= 1 && C >= 16 && a.M <= (int64_t{1} << 22) && a.N < (int64_t{1} << 22) && a.K < (int64_t{1} << 22);
+}
+
+// the plan of a call; without tiles where the fp32 instruction's kernel takes it, and sooner
+PiecesPlan plan_of(const GemmArgs &a, bool backward, size_t room)
+{
+  const int64_t C = backward ? a.K : a.N, R = backward ? a.N : a.K;
+  const bool int4 = a.w.kind == CAIFX_W_INT4_GROUP;
+  const PiecesPlan plan = plan_pieces(a.M, C, R, int4, room);
+  return a.K % 32 == 0 && split_tile_first(a.M, C, R, int4, room, plan) ? PiecesPlan{} : plan;
 }
 
 }  // namespace
 
 size_t pieces_workspace_bytes(const GemmArgs &a, bool backward)
 {
-  if (!pieces_shape(a, backward)) return 0;
-  return plan_pieces(a.M, backward ? a.K : a.N, backward ? a.N : a.K, a.w.kind == CAIFX_W_INT4_GROUP, SIZE_MAX).bytes;
+  return pieces_shape(a, backward) ? plan_of(a, backward, SIZE_MAX).bytes : 0;
 }
 
 int pieces_gemm(const GemmArgs &a, bool backward, hipStream_t s)
 {
   if (!pieces_shape(a, backward)) return CAIFX_ERR_UNSUPPORTED;
+  const PiecesPlan plan = plan_of(a, backward, a.workspace && aligned_to(a.workspace, 16) ? a.workspace_bytes : 0);
+  if (plan.bm == 0) return CAIFX_ERR_UNSUPPORTED;
   if (!aligned_to(a.x, 16) || !aligned_to(a.w.q, 16)) return CAIFX_ERR_UNSUPPORTED;
   PiecesArgs g{};
   g.a = a.x;
@@ -475,8 +482,6 @@ int pieces_gemm(const GemmArgs &a, bool backward, hipStream_t s)
       g.step = static_cast<uint32_t>((backward ? static_cast<int64_t>(kPK) * a.K : kPK) % g.period);
     }
   }
-  const int64_t C = backward ? a.K : a.N, R = backward ? a.N : a.K;
-  const PiecesPlan plan = plan_pieces(a.M, C, R, int4, a.workspace && aligned_to(a.workspace, 16) ? a.workspace_bytes : 0);
   const bool shared = plan.parts > 1;
   g.bm = plan.bm;
   g.parts = plan.parts;
@@ -491,7 +496,7 @@ int pieces_gemm(const GemmArgs &a, bool backward, hipStream_t s)
   else if (a.x_dtype == CAIFX_F16) st = launch_kind<f16_t>(g, int4, backward, s);
   else return CAIFX_ERR_UNSUPPORTED;
   if (!shared || st != CAIFX_OK) return st;
-  return splitk_reduce(static_cast<const float *>(a.workspace), plan.parts, a.M * C, a.y, a.y_dtype, nullptr, s);
+  return splitk_reduce(static_cast<const float *>(a.workspace), plan.parts, a.M * (backward ? a.K : a.N), a.y, a.y_dtype, nullptr, s);
 }
 
 }  // namespace caifx

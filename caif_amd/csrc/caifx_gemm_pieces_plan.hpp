@@ -1,5 +1,6 @@
-// How the products of bf16 pieces (caifx_gemm_pieces.hip) are cut into workgroups: host arithmetic alone, so that it can be checked
-// without a GPU.
+// How fp32-compute calls over int8 and int4 codes are cut into workgroups, and which of the two kernels takes them: the products of bf16
+// pieces (caifx_gemm_pieces.hip) or the fp32 instruction's split tile (caifx_gemm_f32.hip).  Host arithmetic alone, so that it can be
+// checked without a GPU.
 #pragma once
 #include "caifx.h"
 
@@ -64,6 +65,57 @@ inline PiecesPlan plan_pieces(int64_t M, int64_t C, int64_t R, bool int4, size_t
     }
   }
   return best;
+}
+
+// The fp32 instruction's tile of 32 x 32 whose waves share 128-deep steps, for up to kSplitTileRows rows and reductions that are a multiple
+// of 128.  There are C / 32 such tiles per 32 rows: a chain of R / 128 dependent steps on half of the chip at 32 rows and C = 4096.
+// With a workspace from the caller up to 4 workgroups share a tile's reduction (at least 8 steps each, about one workgroup per
+// compute unit in total) and a second launch adds their partial tiles in a fixed order.
+constexpr int kSplitTileRows = 128;   // M = 64: 256 workgroups instead of 64
+struct SplitTilePlan {
+  int parts, part_steps;
+  size_t bytes;
+};
+inline SplitTilePlan plan_split_tile(int64_t M, int64_t C, int64_t R)
+{
+  SplitTilePlan p{1, 0, 0};
+  if (M > kSplitTileRows || R % 128 != 0) return p;
+  const int64_t tiles = ((C + 31) / 32) * ((M + 31) / 32);
+  if (tiles > 128) return p;
+  const int64_t steps = R / 128;
+  int64_t k = 256 / tiles;
+  if (k > 4) k = 4;
+  if (k > steps / 8) k = steps / 8;
+  if (k < 2) return p;
+  const int64_t per = (steps + k - 1) / k;
+  k = (steps + per - 1) / per;
+  if (k < 2) return p;
+  p.parts = static_cast<int>(k);
+  p.part_steps = static_cast<int>(per);
+  p.bytes = static_cast<size_t>(k) * static_cast<size_t>(M) * static_cast<size_t>(C) * sizeof(float);
+  return p;
+}
+// us of a call, fitted to 760 of them (4.5 % rms)
+inline double split_tile_us(int64_t M, int64_t C, int64_t R, bool int4, size_t room)
+{
+  const SplitTilePlan p = plan_split_tile(M, C, R);
+  const bool shared = p.parts > 1 && p.bytes <= room;
+  const int64_t parts = shared ? p.parts : 1;
+  const double steps = static_cast<double>(shared ? p.part_steps : R / 128);
+  const double more = static_cast<double>((((C + 31) / 32) * ((M + 31) / 32) * parts + 255) / 256 - 1);
+  const double us = 3.6 + steps * (int4 ? 1.19 + 0.76 * more : 1.28 + 0.81 * more) + 0.4 * more;
+  return shared ? us + 1.6 + 1.6e-6 * static_cast<double>(p.bytes) : us;
+}
+
+// Whether the split tile takes a call that the pieces could take too, by `plan` in that room: where it is estimated to be faster, for short reductions (M = 100, R = 256, int8
+// 6.8 us against 9.1) and, whatever their length, where the room keeps the pieces from sharing a reduction as they would (without a
+// workspace M = 64, C = 1024, R = 4096 44.5 us against 92.5, R = 2048 24.4 against 48.7; M = 33, int4, 43 against 76).  Elsewhere the
+// two are within 20 % of each other, and the pieces have the smaller error.
+inline bool split_tile_first(int64_t M, int64_t C, int64_t R, bool int4, size_t room, const PiecesPlan &plan)
+{
+  if (M > kSplitTileRows || R % 128 != 0) return false;
+  if (R > 640 && plan_pieces(M, C, R, int4, SIZE_MAX).parts == plan.parts) return false;
+  return split_tile_us(M, C, R, int4, room) < plan.us;
 }
 
 }  // namespace caifx
