@@ -681,15 +681,14 @@ int launch_gpw(const MbArgs &m, size_t lds, hipStream_t s)
                   static_cast<unsigned>((m.groups + m.slice_groups - 1) / m.slice_groups));
   const int gpw = (m.slice_groups + kMbWaves - 1) / kMbWaves;
   if (m.M <= 16) {
-    // One row block requested at a time instead of two, by measurement with sixteen waves and one slice (K = 4096,
-    // N = 2048 ... 28672, times in us):
-    // int4 with 4 rows 7.2 -> 6.6, 7.9 -> 7.1, 9.6 -> 9.1, 11.0 -> 10.6, 12.7 -> 12.4, 20.4 -> 19.7; with 16 rows
-    // 9.0 -> 8.4, 9.4 -> 8.9, 11.3 -> 11.2, 12.8 -> 13.1, 14.7 -> 14.9, 23.0 -> 22.4, so two stay only for more than 8
-    // rows with 33..64 weight rows per workgroup; int8 gains up to 32 weight rows per workgroup (10.8 -> 10.6,
-    // 11.5 -> 11.35 at N = 4096) and loses 1.5 us beyond.
+    // One row block requested at a time instead of two, by measurement with the slices that mb_plan chooses (K = 1024 ... 14336, N = 1024 ...
+    // 28672, 3 to 16 rows, 330 calls; time with one over time with two).  One group per wave: 0.97 to 0.99 for 16 weight rows per
+    // workgroup, 0.96 to 1.04 for 32, 1.02 to 1.11 for 56 and more.  Two groups per wave, whose second request is already in flight
+    // beside the first: 0.92 to 0.98, also for int4 with 128 and int8 with 114 rows; 1.00 to 1.02 only for int4 with 33 to 64 weight rows and more
+    // than 8 activation rows.  The chosen one is within 0.3 % of the better in the mean.
     const int64_t rows_class = (m.N + m.V - 1) / m.V;
     const int64_t rows_wg = (rows_class + m.blocks_per_class - 1) / m.blocks_per_class;
-    const bool one_block = kInt4 ? (m.M <= 8 || rows_wg <= 32 || rows_wg > 64) : rows_wg <= 32;
+    const bool one_block = gpw <= 1 ? rows_wg <= 32 : !(kInt4 && m.M > 8 && rows_wg > 32 && rows_wg <= 64);
     if (gpw > 2) return CAIFX_ERR_UNSUPPORTED;
     if (one_block) {
       if (gpw <= 1) hipLaunchKernelGGL((mblock_kernel<CT, XT, kInt4, 1, kF32, 1, 1>), grid, dim3(64 * m.waves), lds, s, m);
