@@ -1,4 +1,5 @@
 import os
+import subprocess
 import sys
 
 import pytest
@@ -18,3 +19,19 @@ def orc():
     from oracle import oracle
     oracle.build()
     return oracle
+
+
+@pytest.fixture(scope="session")
+def pieces_plans(tmp_path_factory):
+    """What the host chooses for fp32-compute calls (M, columns, reduction, int4, room): rows of a tile, workgroups per reduction, their
+    steps, bytes of their sums, and whether the fp32 instruction's split tile takes the call instead."""
+    exe = str(tmp_path_factory.mktemp("plan") / "pieces_plan")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "caif_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "cpp", "pieces_plan.cpp"), "-o", exe], check=True)
+
+    def ask(calls):
+        text = "".join("%d %d %d %d %d\n" % c for c in calls)
+        out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.split("\n")[:-1]
+        assert len(out) == len(calls)
+        return [tuple(int(v) for v in line.split()) for line in out]
+    return ask

@@ -1,6 +1,7 @@
 """fp32 compute over int8 and int4 codes on the 16-bit matrix cores (operands as bf16 pieces), forward and input gradient, against
-the weight (fp32 code * scale) in 64 bits: row counts at the edges of 16-row blocks and of the three tiles, ragged columns, one
-step and many, shared reductions and none, scale vectors that wrap inside a step, extreme values."""
+the weight (fp32 code * scale) in 64 bits: each of the three tiles, with the reduction shared and not, at row counts on the edges of 16-row
+blocks and of tiles, ragged columns, one step and many, scale vectors that wrap inside a step.  The plan that the host makes is asked for
+with each case, so that a case is on the tile that it names.  (Values out of the pieces' range: test_gpu_fp32_pieces_range.py.)"""
 import pytest
 import torch
 
@@ -31,7 +32,43 @@ def _rel(got, want):
     return ((got.double() - want).norm() / want.norm()).item()
 
 
-@pytest.mark.parametrize("kind", ["int4", "channel", "wrap", "one", "none"])
+KINDS = ["int4", "channel", "wrap", "one", "none"]
+NO_LIMIT = 2 ** 63
+# rows of a tile, reduction shared, M, columns, reduction (of the forward: N, K; of the gradient: K, N)
+CASES = [(32, False, 33, 80, 64), (32, False, 65, 2064, 192), (32, True, 33, 80, 320), (32, True, 95, 1104, 704), (32, True, 129, 208, 1088),
+         (64, False, 513, 4112, 64), (64, False, 2095, 1040, 64), (64, True, 33, 4112, 704), (64, True, 600, 1040, 704), (64, True, 2100, 80, 704),
+         (128, False, 513, 6160, 64), (128, False, 1151, 3088, 64), (128, False, 513, 6160, 320), (128, False, 200, 14352, 192)]
+INT8_CASES = [(128, True, 65, 8208, 704), (128, True, 4100, 80, 1088)]
+
+
+def _both_ways(kind, M, C, R):
+    gen = torch.Generator(device="cuda").manual_seed(M + C + R)
+    w, dense = _weight(kind, C, R, gen)
+    x = torch.empty(M, R, device="cuda").normal_(0, 1, generator=gen)
+    assert _rel(T.qlinear_forward(x, w, T.F32), x.double() @ dense.t()) <= _bound(R)
+    w, dense = _weight(kind, R, C, gen)
+    dy = torch.empty(M, R, device="cuda").normal_(0, 1e-3, generator=gen)
+    assert _rel(T.qlinear_backward_input(dy, w, T.F32), dy.double() @ dense) <= _bound(R)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("bm,shared,M,C,R", CASES)
+def test_every_tile(pieces_plans, kind, bm, shared, M, C, R):
+    plan = pieces_plans([(M, C, R, int(kind == "int4"), NO_LIMIT)])[0]
+    assert plan[0] == bm and (plan[1] > 1) == shared and not plan[4], plan
+    _both_ways(kind, M, C, R)
+
+
+@pytest.mark.parametrize("kind", KINDS[1:])
+@pytest.mark.parametrize("bm,shared,M,C,R", INT8_CASES)
+def test_every_tile_int8(pieces_plans, kind, bm, shared, M, C, R):
+    plan = pieces_plans([(M, C, R, 0, NO_LIMIT)])[0]
+    assert plan[0] == bm and (plan[1] > 1) == shared and not plan[4], plan
+    _both_ways(kind, M, C, R)
+
+
+# rows around the tiles' edges, whichever kernel the host chooses, with the workspace and without
+@pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("M", [33, 48, 64, 65, 81, 128, 129, 200])
 @pytest.mark.parametrize("N,K", [(64, 64), (192, 320), (1344, 2048)])
 def test_forward_and_gradient(kind, M, N, K):
@@ -46,7 +83,7 @@ def test_forward_and_gradient(kind, M, N, K):
 
 
 @pytest.mark.parametrize("M", [2, 15, 16, 17, 32])
-@pytest.mark.parametrize("N,K", [(192, 192), (4096, 4096), (80, 128)])
+@pytest.mark.parametrize("N,K", [(192, 192), (4096, 4096), (80, 192)])
 def test_few_rows_int4(M, N, K):
     gen = torch.Generator(device="cuda").manual_seed(M)
     w, dense = _weight("int4", N, K, gen)
@@ -54,20 +91,30 @@ def test_few_rows_int4(M, N, K):
     assert _rel(T.qlinear_forward(x, w, T.F32), x.double() @ dense.t()) <= _bound(K)
 
 
+# 16-bit activations on each tile; results of another type are the fp32 results rounded
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("out", [T.F32, T.BF16, T.F16])
-def test_types(dtype, out):
+@pytest.mark.parametrize("kind,bm,M,C,R", [("channel", 32, 100, 208, 320), ("int4", 32, 100, 208, 320), ("channel", 64, 600, 1040, 704),
+                                           ("int4", 64, 600, 1040, 704), ("channel", 128, 513, 6160, 64), ("int4", 128, 513, 6160, 64)])
+def test_types(pieces_plans, kind, bm, M, C, R, dtype, out):
+    plan = pieces_plans([(M, C, R, int(kind == "int4"), NO_LIMIT)])[0]
+    assert plan[0] == bm and not plan[4]
     gen = torch.Generator(device="cuda").manual_seed(1)
-    w, dense = _weight("channel", 256, 512, gen)
-    x = torch.empty(100, 512, device="cuda").normal_(0, 1, generator=gen).to(dtype)
+    w, dense = _weight(kind, C, R, gen)
+    x = torch.empty(M, R, device="cuda").normal_(0, 1, generator=gen).to(dtype)
     y = T.qlinear_forward(x, w, T.F32, out)
     assert torch.equal(y, T.qlinear_forward(x, w, T.F32, T.F32).to(T.TORCH_DTYPE[out]))
-    assert _rel(T.qlinear_forward(x, w, T.F32), x.double() @ dense.t()) <= _bound(512)
+    assert _rel(T.qlinear_forward(x, w, T.F32), x.double() @ dense.t()) <= _bound(R)
+    w, dense = _weight(kind, R, C, gen)
+    dx = T.qlinear_backward_input(x, w, T.F32, out)
+    assert torch.equal(dx, T.qlinear_backward_input(x, w, T.F32, T.F32).to(T.TORCH_DTYPE[out]))
+    assert _rel(T.qlinear_backward_input(x, w, T.F32), x.double() @ dense) <= _bound(R)
 
 
-def test_extreme_values():
+def test_extreme_values(pieces_plans):
     # codes without zeros, so that an infinity times a weight is one
-    N, K, M = 128, 256, 40
+    N, K, M = 128, 320, 40
+    assert not pieces_plans([(M, N, K, 0, NO_LIMIT)])[0][4]
     codes = torch.randint(1, 128, (N * K,), device="cuda", dtype=torch.int8)
     w = T.FrozenWeight(codes, T.W_INT8, torch.full((1,), 2.0 ** -8, device="cuda"), N, K, 1)
     x = torch.zeros(M, K, device="cuda")

@@ -31,6 +31,10 @@ def _check(got, want):
     assert torch.allclose(got[fin].double(), want[fin].double(), rtol=2.0 ** -22, atol=0)
 
 
+def _on_the_pieces(pieces_plans, *calls):
+    assert not any(split for *_, split in pieces_plans([(*c, 2 ** 63) for c in calls]))
+
+
 def _x(M, R, value, gen):
     # row m holds the value at one place; the other rows are left zero
     x = torch.zeros(M, R, device="cuda")
@@ -42,7 +46,8 @@ def _x(M, R, value, gen):
 @pytest.mark.parametrize("form", ["one", "vector"])
 @pytest.mark.parametrize("value,scale", VALUES)
 @pytest.mark.parametrize("M,N,K", [(40, 192, 320), (100, 320, 192), (200, 1024, 2048)])
-def test_int8(form, value, scale, M, N, K):
+def test_int8(pieces_plans, form, value, scale, M, N, K):
+    _on_the_pieces(pieces_plans, (M, N, K, 0), (M, K, N, 0))
     gen = torch.Generator(device="cuda").manual_seed(M)
     codes = torch.randint(-128, 128, (N, K), device="cuda", generator=gen, dtype=torch.int8)
     codes = torch.where(codes == 0, torch.ones_like(codes), codes)          # (zeros against infinities: test_int4)
@@ -63,7 +68,8 @@ def test_int8(form, value, scale, M, N, K):
 @pytest.mark.parametrize("value,scale", [(1.0, INF), (INF, INF), (-1.5, INF), (1.0, NAN), (INF, 6e-8), (2.99e38, 3000.0), (3.7e-36, 0.0117), (1.0, 6e-8),
                                          (INF, 0.25), (0.0, 0.25)])
 @pytest.mark.parametrize("M,N,K", [(40, 192, 320), (100, 320, 192), (200, 1024, 2048)])
-def test_int4(value, scale, M, N, K):
+def test_int4(pieces_plans, value, scale, M, N, K):
+    _on_the_pieces(pieces_plans, (M, N, K, 1), (M, K, N, 1))
     gen = torch.Generator(device="cuda").manual_seed(M)
     packed = torch.randint(0, 256, (N * K // 2,), device="cuda", generator=gen, dtype=torch.uint8)
     scales = torch.full((N * K // 64,), 0.25, device="cuda", dtype=torch.float16)

@@ -1,6 +1,6 @@
 """GPU parity of the fp32 compute type (ComputeT = float of CAIF_DeviceFrozenLinear, the reference's Accuracy_e
-matmul mode) on the fp32 matrix-core kernel: forward (src/caif_device_frozen_linear.cpp:382-524) and input gradient
-(:528-660) against the oracle, which accumulates in fp64.  Tolerance: 1e-4 of max|ref| (the north star's fp32
+matmul mode), on products of bf16 pieces or the fp32 matrix-core instruction as the dispatcher chooses: forward
+(src/caif_device_frozen_linear.cpp:382-524) and input gradient (:528-660) against the oracle, which accumulates in fp64.  Tolerance: 1e-4 of max|ref| (the north star's fp32
 bar); what is measured is ~1e-6."""
 import numpy as np
 import pytest
@@ -33,6 +33,34 @@ def test_fp32_compute_forward_and_input_gradient(orc, kind, group, M, N, K):
         dx = host(T.qlinear_backward_input(dy, dw, T.F32))
         assert max_rel_err(y, orc.frozen_linear_forward(host(x), ow, orc.F32)) <= TOL, (kind, xdt)
         assert max_rel_err(dx, orc.frozen_linear_backward(host(dy), ow, orc.F32)) <= TOL, (kind, xdt)
+
+
+# what stays on the fp32 instruction: reductions that are a multiple of 32 and not of 64 (tiles of 32 x 128 and of 128 x 128), and up to 128 rows of a
+# short reduction or without room to share a longer one (tiles of 32 x 32)
+@pytest.mark.parametrize("kind,group", [("int8pc", 128), ("int8pt", 128), ("int8raw", 128), ("int4", 32)])
+@pytest.mark.parametrize("M,N,K", [(40, 160, 96), (300, 416, 224), (4100, 1056, 96)])
+def test_fp32_instruction_odd_reductions(orc, kind, group, M, N, K):
+    rng = np.random.default_rng(M + N + K + group)
+    ow, dw = make_weight(orc, rng, N, K, kind, group, std=0.02 if kind != "int8raw" else 1.0)
+    x, dy = dev_as(rng.normal(0, 1, (M, K)), 0), dev_as(rng.normal(0, 1e-3, (M, N)), 0)
+    assert max_rel_err(host(T.qlinear_forward(x, dw, T.F32)), orc.frozen_linear_forward(host(x), ow, orc.F32)) <= TOL
+    assert max_rel_err(host(T.qlinear_backward_input(dy, dw, T.F32)), orc.frozen_linear_backward(host(dy), ow, orc.F32)) <= TOL
+
+
+@pytest.mark.parametrize("kind,group", [("int8pc", 128), ("int8pt", 128), ("int8raw", 128), ("int4", 32)])
+@pytest.mark.parametrize("M,C,R,room", [(33, 208, 128, 2 ** 63), (100, 1040, 256, 2 ** 63), (64, 80, 2048, 0), (128, 208, 1152, 0)])
+def test_fp32_instruction_split_tile(orc, pieces_plans, kind, group, M, C, R, room):
+    import torch
+    assert pieces_plans([(M, C, R, int(kind == "int4"), room)])[0][4]
+    rng = np.random.default_rng(M + C + R + group)
+    ws = torch.empty(0, dtype=torch.uint8, device="cuda") if room == 0 else None
+    ow, dw = make_weight(orc, rng, C, R, kind, group, std=0.02 if kind != "int8raw" else 1.0)
+    x = dev_as(rng.normal(0, 1, (M, R)), 0)
+    assert max_rel_err(host(T.qlinear_forward(x, dw, T.F32, workspace=ws)), orc.frozen_linear_forward(host(x), ow, orc.F32)) <= TOL
+    C -= C % 32                                                  # (the instruction's kernel takes whole 32s along K)
+    ow, dw = make_weight(orc, rng, R, C, kind, group, std=0.02 if kind != "int8raw" else 1.0)
+    dy = dev_as(rng.normal(0, 1e-3, (M, R)), 0)
+    assert max_rel_err(host(T.qlinear_backward_input(dy, dw, T.F32, workspace=ws)), orc.frozen_linear_backward(host(dy), ow, orc.F32)) <= TOL
 
 
 def test_fp32_compute_one_hot_reads_single_weights(orc):

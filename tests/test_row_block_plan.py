@@ -46,6 +46,7 @@ def _tiled(M, N, K, compute, kind):
 
 
 def test_degenerate_sizes():
+    # refused calls (no rows, no reduction) ask for nothing, a reduction that is no multiple of 64 fits no kernel that shares it
     query = capi.lib().caifx_qlinear_workspace_bytes
     for M, N, K in [(0, 64, 128), (4, 64, 0), (4, 64, 100)]:
-        query(M, N, K, BF16, BF16, INT8, 0)
+        assert query(M, N, K, BF16, BF16, INT8, 0) == 0
