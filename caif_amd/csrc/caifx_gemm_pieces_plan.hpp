@@ -24,17 +24,16 @@ struct PiecesTile {
 constexpr PiecesTile kTiles4[3] = {{32, 4, 1.035, 0.32, 2.07}, {64, 3, 1.63, 0.32, 2.60}, {128, 2, 2.78, 0.29, 2.97}};
 constexpr PiecesTile kTiles8[3] = {{32, 4, 1.33, 0.42, 2.68}, {64, 3, 1.82, 0.46, 3.09}, {128, 2, 2.90, 0.46, 3.34}};
 
-inline double pieces_us(const PiecesTile &tile, int64_t groups, int64_t per, int64_t parts, size_t sum_bytes)
+inline double pieces_us(const PiecesTile &tile, int64_t groups, int per)
 {
-  const int64_t residents = (groups + 255) / 256, last = residents % tile.slots;
+  const int64_t residents = (groups + 255) >> 8;
   const double steps = static_cast<double>(per), full = steps * tile.full + 0.042 * tile.bm;
   const auto some = [&](int64_t n) { return steps * (tile.alone + tile.more * static_cast<double>(n - 1)); };
-  double us = 4.9;
-  if (residents <= tile.slots) us += some(residents);
-  else if (tile.slots == 2) us += full * static_cast<double>(residents / tile.slots) + (last > 0 ? 0.85 * some(last) : 0.0);
-  else us += full * static_cast<double>(residents) / tile.slots;
-  return parts > 1 ? us + 1.0 + 0.086 * static_cast<double>(parts) + 0.59e-6 * static_cast<double>(sum_bytes) : us;
+  if (residents <= tile.slots) return 4.9 + some(residents);
+  if (tile.slots == 2) return 4.9 + full * static_cast<double>(residents >> 1) + ((residents & 1) != 0 ? 0.85 * some(1) : 0.0);
+  return 4.9 + full * static_cast<double>(residents) * (tile.slots == 3 ? 1.0 / 3.0 : 0.25);
 }
+inline double pieces_sums_us(int parts, size_t bytes) { return parts > 1 ? 1.0 + 0.086 * parts + 0.59e-6 * static_cast<double>(bytes) : 0.0; }
 
 // Rows of a tile and workgroups that share its reduction: the plan of the least cost.  It is within 0.6 % of the fastest in the mean, 19 %
 // at the worst (fixed: 32 rows up to M = 32, 64 up to 64, 128 beyond, as many parts as fill the chip: M = 200, N = 3456, K = 3712 70 us
@@ -43,27 +42,35 @@ struct PiecesPlan {
   int bm, parts, part_steps;
   size_t bytes;
   double us;
+  bool limited;          // with more room another plan would be faster
 };
+// (made for every call, and for every question how much workspace one takes: no division but those of the steps)
 inline PiecesPlan plan_pieces(int64_t M, int64_t C, int64_t R, bool int4, size_t room)
 {
   constexpr int kMostParts = 12;
   constexpr int64_t kMostRowTiles = 65535;        // gridDim.y
-  const int64_t steps = R / kPK;
+  const int steps = static_cast<int>(R / kPK);
+  const size_t part_bytes = static_cast<size_t>(M) * static_cast<size_t>(C) * sizeof(float);
   PiecesPlan best{};
-  for (int t = 0; t < 3; ++t) {
-    const PiecesTile &tile = (int4 ? kTiles4 : kTiles8)[t];
-    if (t > 0 && M <= tile.bm / 2) break;
-    const int64_t row_tiles = (M + tile.bm - 1) / tile.bm;
-    if (row_tiles > kMostRowTiles) continue;
-    for (int k = 1; k <= kMostParts; ++k) {
-      const int64_t per = (steps + k - 1) / k, parts = (steps + per - 1) / per;
-      if (k > 1 && (per < 2 || parts < k)) continue;
-      const size_t bytes = parts > 1 ? static_cast<size_t>(parts) * static_cast<size_t>(M) * static_cast<size_t>(C) * sizeof(float) : 0;
-      if (bytes > CAIFX_STATIC_SCRATCH_BYTES || bytes > room) continue;
-      const double us = pieces_us(tile, row_tiles * ((C + kPN - 1) / kPN) * parts, per, parts, bytes);
-      if (best.bm == 0 || us < best.us) best = PiecesPlan{tile.bm, static_cast<int>(parts), static_cast<int>(per), bytes, us};
+  double least = 0.0;
+  for (int k = 1; k <= kMostParts; ++k) {
+    const int per = (steps + k - 1) / k, parts = (steps + per - 1) / per;
+    if (k > 1 && per < 2) break;
+    if (parts < k) continue;
+    const size_t bytes = parts > 1 ? static_cast<size_t>(parts) * part_bytes : 0;
+    if (bytes > CAIFX_STATIC_SCRATCH_BYTES) break;
+    const double sums = pieces_sums_us(parts, bytes);
+    for (int t = 0; t < 3; ++t) {
+      const PiecesTile &tile = (int4 ? kTiles4 : kTiles8)[t];
+      if (t > 0 && M <= tile.bm / 2) break;
+      const int64_t row_tiles = (M + tile.bm - 1) >> (5 + t);
+      if (row_tiles > kMostRowTiles) continue;
+      const double us = sums + pieces_us(tile, row_tiles * ((C + kPN - 1) / kPN) * parts, per);
+      if (least == 0.0 || us < least) least = us;
+      if (bytes <= room && (best.bm == 0 || us < best.us)) best = PiecesPlan{tile.bm, parts, per, bytes, us, false};
     }
   }
+  best.limited = least < best.us;
   return best;
 }
 
@@ -114,7 +121,7 @@ inline double split_tile_us(int64_t M, int64_t C, int64_t R, bool int4, size_t r
 inline bool split_tile_first(int64_t M, int64_t C, int64_t R, bool int4, size_t room, const PiecesPlan &plan)
 {
   if (M > kSplitTileRows || R % 128 != 0) return false;
-  if (R > 640 && plan_pieces(M, C, R, int4, SIZE_MAX).parts == plan.parts) return false;
+  if (R > 640 && !plan.limited) return false;
   return split_tile_us(M, C, R, int4, room) < plan.us;
 }
 
