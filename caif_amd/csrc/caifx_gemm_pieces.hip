@@ -53,9 +53,9 @@ __device__ __forceinline__ float high_bf16(uint32_t p) { return __builtin_bit_ca
 // would be a subnormal number (2^-64 * 2^-38 = 2^-102, its last bits 2^-125); above, sums of fewer than 2^22 products could pass the
 // largest number in acc and its negative in rest.  Weights are held to theirs by their scales (int8 codes: 2^-38 to 2^43; every finite
 // fp16 scale does).  A step of a tile that meets another value (an infinity, a NaN, one too large or too small) runs on the fp32
-// instruction, with the results that one gives.  What the looking costs: 1 % with int4 and 2 with int8 (628 calls, geometric means), 4 to 11 %
-// where zeros make every step ask for the second look (half of the activations zero, M = 200 and 2048).  M = 200, N = 3456, K = 3712
-// takes 62 (int4) and 67 us (int8) with ordinary values, the same with one tiny value in a million, and 136 and 139 where all are tiny.
+// instruction, with the results that one gives.  What the looking costs: 1 % with int4 and 2 with int8 (628 calls, geometric means),
+// up to 3 more where zeros make every step look twice (half of the activations zero).  M = 200, N = 3456, K = 3712 takes 62 (int4) and
+// 67 us (int8) with ordinary values, the same with one tiny value in a million, and 157 and 163 where all are tiny.
 constexpr float kLeastX = 0x1p-64f, kMostX = 0x1p50f;
 constexpr float kLeastS = 0x1p-38f, kMostS = 0x1p43f;
 
@@ -135,21 +135,22 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
     for (int i = 0; i < kALoads; ++i)
       areg[i] = *reinterpret_cast<const u32x4_t *>(a_base + static_cast<int64_t>(s) * (kPK * sizeof(XT)) + a_off[i]);
   };
-  // a zero is ordinary, another number below kLeastX is not (fp16 holds none)
+  // A zero is ordinary, another number below kLeastX is not (fp16 holds none).  The bits without the sign, less one: a zero becomes the
+  // largest, and a minimum of three is one instruction (two comparisons a value and their masks cost 10 % of a call with zeros).
   auto tiny_a = [&]() __attribute__((always_inline)) {
-    bool tiny = false;
+    uint32_t least = 0xffffffffu;
     if constexpr (!std::is_same<XT, f16_t>::value) {
 #pragma unroll
       for (int i = 0; i < kALoads; ++i) {
         const XT *h = reinterpret_cast<const XT *>(&areg[i]);
 #pragma unroll
         for (int e = 0; e < kAV; ++e) {
-          const float x = fabsf(to_f32<XT>(h[e]));
-          tiny = tiny | ((x != 0.0f) & (x < kLeastX));
+          const uint32_t b = (__builtin_bit_cast(uint32_t, to_f32<XT>(h[e])) << 1) - 1u;
+          least = b < least ? b : least;
         }
       }
     }
-    return tiny;
+    return least < (__builtin_bit_cast(uint32_t, kLeastX) << 1) - 1u;
   };
   auto store_a = [&](Seen &seen) __attribute__((always_inline)) {
 #pragma unroll
