@@ -5,12 +5,14 @@
 // an 11-bit scale has 15 bits).  The products of pieces are exact in the matrix core and are summed in fp32; left out are those
 // below 2^-25 of the largest (middle x last and last x last): six products for int8, five for int4, at 16 times the rate of
 // the fp32 instruction.  Error against 64 bits (2-norm, relative; N(0,1) x N(0,0.02)), fp32 instruction -> here: M = 185, N = 3456,
-// K = 3712 int4 1.0e-6 -> 1.6e-7, int8 1.1e-6 -> 2.1e-7; M = 256, 8192 x 4096 1.1e-6 -> 3.3e-7 and 3.9e-7; M = 40, 1024 x 512 1.9e-7 ->
-// 7.4e-8 and 2.1e-7 -> 9.2e-8.  us, forward / gradient: M = 200, N = 3456, K = 3712, int4 120 / 123 -> 60 / 62; M = 66, 6720 x 3584
-// 85 / 235 -> 43 / 42; M = 2048, 4096 x 4096 549 / 570 -> 420 / 403 (int8 590 / 594 -> 496 / 456).
+// K = 3712 int4 1.0e-6 -> 1.6e-7, int8 1.1e-6 -> 2.1e-7; M = 256, 8192 x 4096 1.1e-6 -> 3.3e-7 and 4.0e-7; M = 40, N = 1024, K = 512, gradient
+// 2.7e-7 -> 7.6e-8 and 2.9e-7 -> 8.9e-8.  us, forward / gradient (int8 in brackets): M = 200, N = 3456, K = 3712 118 / 121 -> 55 / 60
+// (124 / 129 -> 65 / 67); M = 66, 6720 x 3584 81 / 231 -> 52 / 51 (88 / 244 -> 54 / 58); M = 256, 8192 x 4096 189 / 277 -> 130 / 132 (199 / 296 ->
+// 152 / 146); M = 2048, 4096 x 4096 540 / 563 -> 402 / 404 (561 / 579 -> 440 / 438).
 //
-// What bounds it with up to a few hundred rows is not the products but cutting the operands (6 to 8 VALU instructions a value,
-// a tile of 64 x 64 x 64 as long as its 48 products per wave) and the latency of a step, so two to four workgroups share a
+// What bounds it with up to a few hundred rows is not the products but cutting the operands (6 to 8 VALU instructions a value, a
+// tile of 64 x 64 x 64 as long as its 48 products per wave) and the latency of a step: at M = 200 the VALU is busy 0.40 to 0.44 of the time,
+// the matrix pipes 0.17 to 0.19, waves wait 0.3 of theirs (M = 2048: 0.50, 0.33 to 0.37, 0.23 to 0.31).  So two to four workgroups share a
 // compute unit and take turns, and the reduction is shared out until they do: `parts` workgroups write fp32 sums to the
 // caller's workspace, a second launch adds them in order.
 //
@@ -51,10 +53,11 @@ __device__ __forceinline__ float high_bf16(uint32_t p) { return __builtin_bit_ca
 
 // Pieces are the value where it is zero or its magnitude lies in these ranges.  Below, a piece or a product of first and last pieces
 // would be a subnormal number (2^-64 * 2^-38 = 2^-102, its last bits 2^-125); above, sums of fewer than 2^22 products could pass the
-// largest number in acc and its negative in rest.  Weights are held to theirs by their scales (int8 codes: 2^-38 to 2^43; every finite
-// fp16 scale does).  A step of a tile that meets another value (an infinity, a NaN, one too large or too small) runs on the fp32
-// instruction, with the results that one gives.  What the looking costs: 1 % with int4 and 2 with int8 (628 calls, geometric means),
-// up to 3 more where zeros make every step look twice (half of the activations zero).  M = 200, N = 3456, K = 3712 takes 62 (int4) and
+// largest number in acc and its negative in rest.  Weights are held to theirs by their scales (int8 codes: zero, or 2^-38 to 2^43; every
+// finite fp16 scale does).  A step of a tile that meets another value (an infinity, a NaN, one too large or too small) runs on the fp32
+// instruction, with the results that one gives.  What the looking costs: 1 % (int4 628 calls, geometric mean; int8 M = 200 to 2048),
+// up to 3 more where zero activations make every step look twice (half of them zero) and 6 where zero scales do (M = 2048, 4096 x 4096,
+// gradient 462 us with a zero scale, 438 without; held to be too small they took 1147).  M = 200, N = 3456, K = 3712 takes 62 (int4) and
 // 67 us (int8) with ordinary values, the same with one tiny value in a million, and 157 and 163 where all are tiny.
 constexpr float kLeastX = 0x1p-64f, kMostX = 0x1p50f;
 constexpr float kLeastS = 0x1p-38f, kMostS = 0x1p43f;
@@ -250,6 +253,20 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
       }
     }
   };
+  // the same question of the scales (those of a channel of zeros may be zero)
+  auto tiny_s = [&]() __attribute__((always_inline)) {
+    uint32_t least = 0xffffffffu;
+    if constexpr (kVec) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t b = (__builtin_bit_cast(uint32_t, sc[r][kVec ? e : 0]) << 1) - 1u;
+          least = b < least ? b : least;
+        }
+    }
+    return least < (__builtin_bit_cast(uint32_t, kLeastS) << 1) - 1u;
+  };
   // four weights along the reduction, and the row and the reduction element in LDS where they begin
   const int b_at = kBackward ? b_row : b_col;
   auto b_lds_row = [&](int c) __attribute__((always_inline)) { return kBackward ? b_col + c : b_row + 16 * c; };
@@ -340,11 +357,12 @@ __global__ __launch_bounds__(256, BM == 128 ? 2 : 3) void pieces_gemm_kernel(Pie
     store_b(ss);
     unsigned long long odd = __ballot(!(xs.most < kMostX)) | one_scale_odd;          // (masks: no lane of the wave leaves the straight line)
     if constexpr (kInt4) odd |= __ballot(!(ss.most <= 65504.0f));
-    if constexpr (kVec) odd |= __ballot(!(ss.least >= kLeastS)) | __ballot(!(ss.most < kMostS));          // (a scale of zero counts as too small)
+    if constexpr (kVec) odd |= __ballot(!(ss.most < kMostS));
     unsigned long long zero_or_tiny = 0;
     if constexpr (!std::is_same<XT, f16_t>::value) zero_or_tiny = __ballot(!(xs.least >= kLeastX));
+    if constexpr (kVec) zero_or_tiny |= __ballot(!(ss.least >= kLeastS));
     if ((odd | zero_or_tiny) != 0) {                    // which of the two is asked only where there is one
-      if ((odd | __ballot(tiny_a())) != 0) fp32_step = s + 1;
+      if ((odd | __ballot(tiny_a() | tiny_s())) != 0) fp32_step = s + 1;
     }
     meet();
     const int flagged = fp32_step;          // (written again after this step's last barrier)

@@ -14,7 +14,7 @@ INF, NAN = float("inf"), float("nan")
 # zero, numbers whose last piece bf16 would cut off (3.7e-36), a NaN that truncation would make an infinity
 VALUES = [(2.99e38, 30.0), (-2.99e38, 30.0), (1.003e30, 1e10), (3.4028234e38, 2.0 ** -8), (-3.4028234e38, 2.0 ** -8), (INF, INF), (-INF, INF),
           (1.0, INF), (0.0, INF), (INF, 2.0 ** -145), (INF, 2.0 ** -8), (-INF, 2.0 ** -8), (NAN, 1.0), (1.0, NAN), (3.7e-36, 0.0117), (1.7e-36, 0.5), (2.0 ** -100, 2.0 ** -8),
-          (1.1e-33, 1.3e-5), (1.2345678, 1.2345678e-13), (1.2345678e-19, 1.2345678e-11), (1.2345678e15, 1.2345678e15), (0.0, 0.0), (5.0, 0.0)]
+          (1.1e-33, 1.3e-5), (1.2345678, 1.2345678e-13), (1.2345678e-19, 1.2345678e-11), (1.2345678e15, 1.2345678e15), (0.0, 0.0), (5.0, 0.0), (INF, 0.0), (NAN, 0.0), (2.0 ** -100, 0.0)]
 
 
 def _expected(x, dense):
