@@ -85,12 +85,13 @@ void mfma_grouped_tile_stamps(void *buf, int64_t tiles);
 int mfma_regw_forward(const GemmArgs &a, hipStream_t s);
 
 // fp32 compute type over quantised storage on the 16-bit matrix cores, operands cut into bf16 pieces that add up to them; plain form,
-// reductions that are a multiple of 64.  CAIFX_ERR_UNSUPPORTED for everything else.
+// reductions that are a multiple of 64.  CAIFX_ERR_UNSUPPORTED for everything else, and where the kernel on the fp32 instruction is
+// estimated to be faster in the workspace at hand.
 int pieces_gemm(const GemmArgs &a, bool backward, hipStream_t s);
 size_t pieces_workspace_bytes(const GemmArgs &a, bool backward);
 
-// fp32 compute type on the matrix cores (v_mfma_f32_32x32x2_f32), forward and input gradient, any M, plain
-// and grouped.  CAIFX_ERR_UNSUPPORTED for an addend, reductions that are not a multiple of 32,
+// fp32 compute type on the matrix cores, forward and input gradient, any M, plain and grouped: pieces_gemm, and
+// v_mfma_f32_32x32x2_f32 for what that leaves.  CAIFX_ERR_UNSUPPORTED for an addend, reductions that are not a multiple of 32,
 // int4 groups below 16 or not a power of two, int8 scale vectors shorter than 32 or not a multiple of 4 long.
 int mfma_f32_forward(const GemmArgs &a, hipStream_t s);
 int mfma_f32_backward(const GemmArgs &a, hipStream_t s);
