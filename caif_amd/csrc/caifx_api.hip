@@ -380,15 +380,11 @@ static int grouped(bool backward, int num_experts, const int32_t *offsets, int64
   a.num_experts = num_experts;
   if (addend && (addend == y || !aligned_to(addend, dtype_size(y_dtype)))) return CAIFX_ERR_INVALID_ARGUMENT;
   hipStream_t s = as_stream(stream);
+  a.zero_rest = zero_rest;      // the 16-bit kernels clear the rows outside the segments themselves, in front of the others a launch does
   if (!backward && !addend && !float_kind(w_kind) && compute_dtype != CAIFX_F32) {
-    // few rows per expert (MoE decode): memory bound on the touched experts' weights; it clears the other rows itself
-    a.zero_rest = zero_rest;
+    // few rows per expert (MoE decode): memory bound on the touched experts' weights
     st = mblock_grouped_forward(a, s);
     if (st != CAIFX_ERR_UNSUPPORTED) return st;
-  }
-  if (zero_rest) {
-    st = caifx_qlinear_grouped_zero_rest(num_experts, offsets, total_rows, row_bytes, y, stream);
-    if (st != CAIFX_OK) return st;
   }
   if (same_16bit(w_kind, compute_dtype)) {
     a.addend = addend;
@@ -396,20 +392,23 @@ static int grouped(bool backward, int num_experts, const int32_t *offsets, int64
     if (st != CAIFX_ERR_UNSUPPORTED) return st;
     a.addend = nullptr;
   }
-  if ((compute_dtype == CAIFX_F32 || float_kind(w_kind)) && !addend) {
-    st = backward ? mfma_f32_backward(a, s) : mfma_f32_forward(a, s);
+  const bool f32_path = compute_dtype == CAIFX_F32 || float_kind(w_kind);
+  if (!f32_path) {
+    a.addend = addend;
+    st = backward ? mfma_backward(a, s) : mfma_forward(a, s);
     if (st != CAIFX_ERR_UNSUPPORTED) return st;
   }
-  if (float_kind(w_kind)) {
-    if (addend) return CAIFX_ERR_UNSUPPORTED;
-    return backward ? generic_backward(a, s) : generic_forward(a, s);
-  }
-  a.addend = addend;
-  st = backward ? mfma_backward(a, s) : mfma_forward(a, s);
-  if (st != CAIFX_ERR_UNSUPPORTED) return st;
   // the shape-agnostic kernels have no fused add, and rows past offsets[E] must stay untouched, which a
   // plain element-wise pass over the buffer would not respect
   if (addend) return CAIFX_ERR_UNSUPPORTED;
+  if (zero_rest) {
+    st = caifx_qlinear_grouped_zero_rest(num_experts, offsets, total_rows, row_bytes, y, stream);
+    if (st != CAIFX_OK) return st;
+  }
+  if (f32_path) {
+    st = backward ? mfma_f32_backward(a, s) : mfma_f32_forward(a, s);
+    if (st != CAIFX_ERR_UNSUPPORTED) return st;
+  }
   return backward ? generic_backward(a, s) : generic_forward(a, s);
 }
 

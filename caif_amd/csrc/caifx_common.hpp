@@ -114,13 +114,16 @@ __device__ __forceinline__ void int8x4_to_f32(uint32_t p, float (&e)[4])
 
 // Rows [lo, hi) of expert e, forced into 0 <= lo <= hi <= M: offsets that are not non-decreasing or that
 // run past the buffer (a caller's mistake) then lose rows instead of sending loads and stores out of bounds.
-__device__ __forceinline__ void segment_rows(const int32_t *offsets, int e, int64_t M, int &lo, int &hi)
+// Returns whether the entries step down there.
+__device__ __forceinline__ bool segment_rows(const int32_t *offsets, int e, int64_t M, int &lo, int &hi)
 {
   const int m = static_cast<int>(M);          // M <= 2^30 is checked on the host
   lo = offsets[e];
   hi = offsets[e + 1];
+  const bool down = hi < lo;
   lo = lo < 0 ? 0 : (lo > m ? m : lo);
   hi = hi < lo ? lo : (hi > m ? m : hi);
+  return down;
 }
 
 // Zeroes bytes [a, b) of y by `threads` threads of which this is the t-th: whole aligned 16-byte pieces, single bytes at the ends.
@@ -159,21 +162,37 @@ struct GroupedTile {
   int64_t pos;
   const void *wq;
   const void *scales;      // null when scales_ptrs is
+  // what the segments cover, also where the workgroup has no tile: rows [first, end) if the offsets never step down
+  int first, end;
+  bool ordered;
 };
-template <int BM>
+template <int BM, bool kEven> __device__ __forceinline__ void grouped_rows(int lo, int hi, int tiles, int t, GroupedTile &out)
+{
+  const int height = kEven ? ((hi - lo + tiles - 1) / tiles + 31) & ~31 : BM;
+  out.row0 = lo + static_cast<int64_t>(t) * height;
+  out.row_end = kEven && hi - out.row0 > height ? out.row0 + height : hi;
+}
+// kEven: an expert's rows are cut into tiles of equal height (a multiple of 32 of at most `height`, the last one what is left), and
+// row_end is the end of the tile's rows.
+template <int BM, bool kEven = false>
 __device__ __forceinline__ bool grouped_tile(const int32_t *offsets, int num_experts, int64_t M, int64_t col_tiles,
                                              const void *const *wq_ptrs, const void *const *scales_ptrs, int lane,
-                                             GroupedTile &out)
+                                             GroupedTile &out, int height = BM)
 {
+  if (!kEven) height = BM;
   if (num_experts <= 64) {
     int my_lo = 0, my_hi = 0;
+    bool down = false;
     uint64_t my_w = 0, my_s = 0;
     if (lane < num_experts) {
-      segment_rows(offsets, lane, M, my_lo, my_hi);
+      down = segment_rows(offsets, lane, M, my_lo, my_hi);
       my_w = reinterpret_cast<uint64_t>(wq_ptrs[lane]);
       if (scales_ptrs) my_s = reinterpret_cast<uint64_t>(scales_ptrs[lane]);
     }
-    const int tiles = (my_hi - my_lo + BM - 1) / BM;
+    out.first = __shfl(my_lo, 0, 64);
+    out.end = __shfl(my_hi, num_experts - 1, 64);
+    out.ordered = __ballot(down) == 0;
+    const int tiles = (my_hi - my_lo + height - 1) / height;
     int incl = tiles;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -192,8 +211,7 @@ __device__ __forceinline__ bool grouped_tile(const int32_t *offsets, int num_exp
     out.e = src;
     out.pos = pos;
     out.col_tile = pos - static_cast<int64_t>(t) * col_tiles;
-    out.row0 = __shfl(my_lo, src, 64) + static_cast<int64_t>(t - __shfl(incl - tiles, src, 64)) * BM;
-    out.row_end = __shfl(my_hi, src, 64);
+    grouped_rows<BM, kEven>(__shfl(my_lo, src, 64), __shfl(my_hi, src, 64), __shfl(tiles, src, 64), t - __shfl(incl - tiles, src, 64), out);
     const uint32_t wl = __shfl(static_cast<uint32_t>(my_w), src, 64), wh = __shfl(static_cast<uint32_t>(my_w >> 32), src, 64);
     const uint32_t sl = __shfl(static_cast<uint32_t>(my_s), src, 64), sh = __shfl(static_cast<uint32_t>(my_s >> 32), src, 64);
     out.wq = reinterpret_cast<const void *>((static_cast<uint64_t>(wh) << 32) | wl);
@@ -201,14 +219,18 @@ __device__ __forceinline__ bool grouped_tile(const int32_t *offsets, int num_exp
     return true;
   }
   int total_rt = 0;
+  out.ordered = true;
   for (int base = 0; base < num_experts; base += 64) {
     const int my = base + lane;
-    int tiles = 0;
+    int tiles = 0, slo = 0, shi = 0;
+    bool down = false;
     if (my < num_experts) {
-      int slo, shi;
-      segment_rows(offsets, my, M, slo, shi);
-      tiles = (shi - slo + BM - 1) / BM;
+      down = segment_rows(offsets, my, M, slo, shi);
+      tiles = (shi - slo + height - 1) / height;
     }
+    if (base == 0) out.first = __shfl(slo, 0, 64);
+    out.end = __shfl(shi, num_experts - 1 - base < 63 ? num_experts - 1 - base : 63, 64);
+    out.ordered = out.ordered && __ballot(down) == 0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) tiles += __shfl_xor(tiles, o, 64);
     total_rt += tiles;
@@ -225,7 +247,7 @@ __device__ __forceinline__ bool grouped_tile(const int32_t *offsets, int num_exp
     const int my = base + lane;
     int my_lo = 0, my_hi = 0;
     if (my < num_experts) segment_rows(offsets, my, M, my_lo, my_hi);
-    const int tiles = (my_hi - my_lo + BM - 1) / BM;
+    const int tiles = (my_hi - my_lo + height - 1) / height;
     int incl = tiles;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -236,8 +258,7 @@ __device__ __forceinline__ bool grouped_tile(const int32_t *offsets, int num_exp
     if (owners != 0) {
       const int src = __builtin_ctzll(owners);
       out.e = base + src;
-      out.row0 = __shfl(my_lo, src, 64) + static_cast<int64_t>(t - __shfl(incl - tiles, src, 64)) * BM;
-      out.row_end = __shfl(my_hi, src, 64);
+      grouped_rows<BM, kEven>(__shfl(my_lo, src, 64), __shfl(my_hi, src, 64), __shfl(tiles, src, 64), t - __shfl(incl - tiles, src, 64), out);
       out.wq = wq_ptrs[out.e];
       out.scales = scales_ptrs ? scales_ptrs[out.e] : nullptr;
       return true;
@@ -245,6 +266,34 @@ __device__ __forceinline__ bool grouped_tile(const int32_t *offsets, int num_exp
     t -= __shfl(incl, 63, 64);
   }
   return false;
+}
+
+// Zeroes the rows of a grouped result that no segment covers, the launch's workgroups sharing them: [0, first) and [end, rows),
+// none of which a tile writes.  Offsets that step down somewhere (a caller's mistake) may also leave rows in between, or cover
+// some of those: then each row is looked up.  (As a launch of its own in front of each product it took 4.7 us, any does: 28
+// of the 1250 us that 4096 tokens through 64 experts take forward and backward, 28 of 150 at 650 tokens and 8 experts.)
+__device__ __forceinline__ void zero_uncovered(const int32_t *offsets, int num_experts, int64_t total_rows, int first, int end, bool ordered, void *result,
+                                               int64_t row_bytes)
+{
+  const int rows = static_cast<int>(total_rows);
+  if (ordered && first == 0 && end == rows) return;
+  unsigned char *y = static_cast<unsigned char *>(result);
+  if (ordered) {
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x, threads = static_cast<int64_t>(gridDim.x) * blockDim.x;
+    zero_bytes(y, 0, first * row_bytes, t, threads);
+    zero_bytes(y, end * row_bytes, rows * row_bytes, t, threads);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  for (int r = static_cast<int>(blockIdx.x); r < rows; r += static_cast<int>(gridDim.x)) {
+    bool covered = false;
+    for (int e = lane; e < num_experts; e += 64) {
+      int lo, hi;
+      segment_rows(offsets, e, total_rows, lo, hi);
+      covered = covered || (lo <= r && r < hi);
+    }
+    if (__ballot(covered) == 0) zero_bytes(y, r * row_bytes, (r + 1) * row_bytes, threadIdx.x, blockDim.x);
+  }
 }
 
 // v_mfma_f32_32x32x16 in the 16-bit compute type CT: A is 32 rows x 16 (lane l supplies row l % 32, reduction
@@ -265,6 +314,17 @@ template <> struct Mfma32<f16_t> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }
 };
+
+// acc += a b, 16 x 16 x 32: lane l supplies row (column) l % 16, reduction elements 8 (l / 16) .. + 7; the result's
+// register r holds row 4 (l / 16) + r, column l % 16.  Written as asm so that the accumulators stay in accumulation
+// registers: with the builtin the compiler moves a part of 256 of them between the two files in every step.
+template <typename CT> __device__ __forceinline__ void mfma16(floatx4_t &acc, const typename Mfma32<CT>::vec_t &a, const typename Mfma32<CT>::vec_t &b)
+{
+  if constexpr (sizeof(CT) == 2 && dtype_code<CT>::value == CAIFX_BF16)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
 
 // two fp32 values rounded to CT (nearest even), the first in the low half
 template <typename CT> __device__ __forceinline__ uint32_t pack2(float lo, float hi)

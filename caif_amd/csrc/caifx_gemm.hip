@@ -142,6 +142,7 @@ int run(const GemmArgs &a, bool backward, hipStream_t s)
   t.wq_ptrs = a.wq_ptrs;
   t.scales_ptrs = a.scales_ptrs;
   t.num_experts = a.num_experts;
+  t.zero_rest = a.zero_rest;
   if (dense) {
     if (!grouped && !aligned_to(a.w.q, 16)) return CAIFX_ERR_UNSUPPORTED;
     t.scales = nullptr;
@@ -228,7 +229,8 @@ int splitk_reduce(const float *partial, int parts, int64_t n, void *y, int y_dty
 int mfma_tiled(const GemmArgs &a, bool backward, hipStream_t s) { return run(a, backward, s); }
 int mfma_backward(const GemmArgs &a, hipStream_t s)
 {
-  const int st = mfma_wide(a, true, s);
+  int st = mfma_wide(a, true, s);
+  if (st == CAIFX_ERR_UNSUPPORTED) st = mfma_tall(a, true, s);
   return st == CAIFX_ERR_UNSUPPORTED ? mfma_tiled(a, true, s) : st;
 }
 void mfma_grouped_stamp_target(unsigned long long **buf, long long *capacity)

@@ -62,6 +62,7 @@ struct Regw8Args {
   const void *const *wq_ptrs;
   const void *const *scales_ptrs;
   int num_experts;
+  bool zero_rest;
   unsigned long long *stamps;       // grouped form, measurement only
   long long stamps_capacity;
 };
@@ -84,7 +85,9 @@ __global__ __launch_bounds__(512, 2) void qgemm_regw8_kernel(Regw8Args g)
   const int64_t col_tiles = (g.N + kBN - 1) / kBN;
   if constexpr (kGrouped) {
     GroupedTile gt;
-    if (!grouped_tile<BM>(g.offsets, g.num_experts, g.M, col_tiles, g.wq_ptrs, g.scales_ptrs, lane, gt)) return;
+    const bool has_tile = grouped_tile<BM>(g.offsets, g.num_experts, g.M, col_tiles, g.wq_ptrs, g.scales_ptrs, lane, gt);
+    if (g.zero_rest) zero_uncovered(g.offsets, g.num_experts, g.M, gt.first, gt.end, gt.ordered, g.d, g.N * (g.d_dtype == CAIFX_F32 ? 4 : 2));
+    if (!has_tile) return;
     const int e = gt.e;
     const int64_t pos = gt.pos;
     col0 = gt.col_tile * kBN;
@@ -459,6 +462,7 @@ static int prepare(const GemmArgs &a, Regw8Args &t)
   t.wq_ptrs = a.wq_ptrs;
   t.scales_ptrs = a.scales_ptrs;
   t.num_experts = a.num_experts;
+  t.zero_rest = a.zero_rest;
   const bool has_scales = grouped ? a.scales_ptrs != nullptr : a.w.scales != nullptr;
   const int64_t P = a.w.scale_period;
   if (!has_scales || P <= 1) {

@@ -69,6 +69,7 @@ struct TileArgs {
   const void *const *wq_ptrs;
   const void *const *scales_ptrs;
   int num_experts;
+  bool zero_rest;             // rows that no segment covers are to be zero
   // plain form with few tiles: ksplit workgroups share a tile, each takes split_steps 64-deep steps of the
   // reduction and writes its fp32 partial tile to d + split * M * C (d is then the caller's workspace)
   int ksplit;
@@ -133,7 +134,9 @@ __global__ __launch_bounds__(2 * kCW * 64, (kCW == 8 || (BM == 128 && (kW == W_C
     // list per XCD (grouped_tile); the grid is an upper bound padded to a multiple of 8
     const int64_t col_tiles = (C + BC - 1) / BC;
     GroupedTile gt;
-    if (!grouped_tile<BM>(g.offsets, g.num_experts, g.M, col_tiles, g.wq_ptrs, g.scales_ptrs, lane, gt)) return;
+    const bool has_tile = grouped_tile<BM>(g.offsets, g.num_experts, g.M, col_tiles, g.wq_ptrs, g.scales_ptrs, lane, gt);
+    if (g.zero_rest) zero_uncovered(g.offsets, g.num_experts, g.M, gt.first, gt.end, gt.ordered, g.d, (kBackward ? g.K : g.N) * (g.d_dtype == CAIFX_F32 ? 4 : 2));
+    if (!has_tile) return;
     const int e = gt.e;
     const int64_t pos = gt.pos;
     col_tile = gt.col_tile;

@@ -37,20 +37,10 @@ struct WideArgs {
   const int32_t *offsets;
   const void *const *wq_ptrs;
   int num_experts;
+  bool zero_rest;
   unsigned long long *stamps;      // measurement only, see mfma_grouped_tile_stamps
   long long stamps_capacity;
 };
-
-// acc += a b, 16 x 16 x 32: lane l supplies row (column) l % 16, reduction elements 8 (l / 16) .. + 7; the result's
-// register r holds row 4 (l / 16) + r, column l % 16.  Written as asm so that the accumulators stay in accumulation
-// registers: with the builtin the compiler moves a part of the 256 between the two files in every step.
-template <typename CT> __device__ __forceinline__ void mfma16(floatx4_t &acc, const typename Mfma32<CT>::vec_t &a, const typename Mfma32<CT>::vec_t &b)
-{
-  if constexpr (std::is_same<CT, bf16_t>::value)
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-  else
-    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-}
 
 // A result tile has 64 WI rows and 64 WJ columns.  Wave (wm, wn) owns rows h 32 WI + wm 16 WI + [0, 16 WI) and columns
 // g 32 WJ + wn 16 WJ + [0, 16 WJ) of it for h, g in {0, 1}: four quadrants of WI x WJ products.  LDS holds four half
@@ -85,7 +75,9 @@ __global__ __launch_bounds__(256, WI + WJ <= 4 ? 2 : 1) void wide_gemm_kernel(Wi
   int64_t stamp_pos = -1;
   if constexpr (kGrouped) {
     GroupedTile gt;
-    if (!grouped_tile<BM>(g.offsets, g.num_experts, g.M, col_tiles, g.wq_ptrs, nullptr, lane, gt)) return;
+    const bool has_tile = grouped_tile<BM>(g.offsets, g.num_experts, g.M, col_tiles, g.wq_ptrs, nullptr, lane, gt);
+    if (g.zero_rest) zero_uncovered(g.offsets, g.num_experts, g.M, gt.first, gt.end, gt.ordered, g.d, g.C * (g.d_dtype == CAIFX_F32 ? 4 : 2));
+    if (!has_tile) return;
     // the search's results are the same in every lane: into scalar registers with them
     row0 = uniform64(static_cast<uint64_t>(gt.row0));
     row_end = uniform64(static_cast<uint64_t>(gt.row_end));
@@ -685,6 +677,7 @@ int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s)
     g.offsets = a.offsets;
     g.wq_ptrs = a.wq_ptrs;
     g.num_experts = a.num_experts;
+    g.zero_rest = a.zero_rest;
     mfma_grouped_stamp_target(&g.stamps, &g.stamps_capacity);
   }
   const auto product = [&]() { return a.compute_dtype == CAIFX_BF16 ? pick_form<bf16_t>(g, s) : pick_form<f16_t>(g, s); };

@@ -568,35 +568,6 @@ struct MbGroup {
   bool zero_rest;                         // zero the result's rows that no segment covers
 };
 
-// Zeroes the rows of a grouped result that no segment covers, the launch's workgroups sharing them: [0, offsets[0]) and
-// [offsets[E], rows), none of which a unit writes.  Offsets that step down somewhere (a caller's mistake) may also leave rows in
-// between, or cover some of those: then each row is looked up.  As a launch of its own in front of each
-// of the three products it was a quarter of the smallest MoE decode passes (ten of them, geometric mean: 1.25x without).
-__device__ __forceinline__ void zero_uncovered(const MbGroup &g, unsigned char *y, int64_t row_bytes)
-{
-  const int lane = threadIdx.x & 63;
-  const int rows = static_cast<int>(g.total_rows);
-  const int first = g.offsets[0], end = g.offsets[g.num_experts];
-  bool down = false;
-  for (int e = lane; e < g.num_experts; e += 64) down = down || g.offsets[e + 1] < g.offsets[e];
-  if (__ballot(down) == 0) {
-    const int lo = first < 0 ? 0 : first > rows ? rows : first, hi = end < 0 ? 0 : end > rows ? rows : end;
-    if (lo == 0 && hi == rows) return;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x, threads = static_cast<int64_t>(gridDim.x) * blockDim.x;
-    zero_bytes(y, 0, lo * row_bytes, t, threads);
-    zero_bytes(y, hi * row_bytes, rows * row_bytes, t, threads);
-    return;
-  }
-  for (int r = static_cast<int>(blockIdx.x); r < rows; r += static_cast<int>(gridDim.x)) {
-    bool covered = false;
-    for (int e = lane; e < g.num_experts; e += 64) {
-      int lo, hi;
-      segment_rows(g.offsets, e, g.total_rows, lo, hi);
-      covered = covered || (lo <= r && r < hi);
-    }
-    if (__ballot(covered) == 0) zero_bytes(y, r * row_bytes, (r + 1) * row_bytes, threadIdx.x, blockDim.x);
-  }
-}
 template <typename CT, typename XT, bool kInt4, int GPW>
 __global__ __launch_bounds__(kMbThreads) void mblock_grouped_kernel(MbArgs a, MbGroup g)
 {
@@ -624,7 +595,14 @@ __global__ __launch_bounds__(kMbThreads) void mblock_grouped_kernel(MbArgs a, Mb
   int u = static_cast<int>(start / g.unit_blocks);                               // unit, and the run's first block in it
   int first = static_cast<int>(start - u * g.unit_blocks);
   const size_t ybytes = a.y_dtype == CAIFX_F32 ? 4 : 2;
-  if (g.zero_rest) zero_uncovered(g, static_cast<unsigned char *>(a.y), a.N * static_cast<int64_t>(ybytes));
+  if (g.zero_rest) {
+    bool down = false;
+    for (int e = lane; e < g.num_experts; e += 64) down = down || g.offsets[e + 1] < g.offsets[e];
+    int first, end, x;
+    segment_rows(g.offsets, 0, g.total_rows, first, x);
+    segment_rows(g.offsets, g.num_experts - 1, g.total_rows, x, end);
+    zero_uncovered(g.offsets, g.num_experts, g.total_rows, first, end, __ballot(down) == 0, a.y, a.N * static_cast<int64_t>(ybytes));
+  }
   int base = g.num_experts <= 64 ? 0 : -1;          // which 64 experts the lanes hold
   int before = 0;                                   // units of the experts in front of them
   while (todo > 0) {

@@ -27,7 +27,7 @@ struct GemmArgs {
   const void *const *wq_ptrs;
   const void *const *scales_ptrs;
   int num_experts;
-  bool zero_rest;         // grouped: y holds nothing yet, rows that no segment covers are to be zero (mblock_grouped_forward alone looks)
+  bool zero_rest;         // grouped: y holds nothing yet, rows that no segment covers are to be zero (the 16-bit matrix-core kernels see to it)
   void *workspace;
   size_t workspace_bytes;
   // optional: y = T(float(T(acc)) + float(addend)), addend [M, columns of y] of y_dtype (may alias y)
@@ -74,6 +74,9 @@ size_t mfma_workspace_bytes(const GemmArgs &a, bool backward);
 // not take, CAIFX_ERR_UNSUPPORTED.
 int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s);
 size_t mfma_wide_workspace_bytes(const GemmArgs &a, bool backward);
+// Expert segments, int8 codes with a scale vector of at most 32 classes of weight rows, forward (K a multiple of 128) and input
+// gradient: tiles of up to 256 rows whose waves dequantise their own columns.  CAIFX_ERR_UNSUPPORTED for everything else.
+int mfma_tall(const GemmArgs &a, bool backward, hipStream_t s);
 // Measurement only: grouped launches of the matrix-core GEMM issued after this call record, per tile of their own
 // numbering (expert by expert, row tile by row tile, column tile last), four 64-bit words {expert, rows in the
 // tile, start, end} with the times in ticks of the 100 MHz wall clock, into buf (device memory for `tiles` tiles);
