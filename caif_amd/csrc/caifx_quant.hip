@@ -276,6 +276,111 @@ __global__ __launch_bounds__(256) void quantize_int8_columns_x4_kernel(const flo
   }
 }
 
+// Per-column int8 in one launch that reads the tensor once: a workgroup takes a strip of 4 kLanes columns (8 lanes: one 128-byte
+// line of every row) of up to kThreads / kLanes x (kRegs + kLds) rows and keeps it, kRegs 16-byte pieces per thread in registers and
+// kLds in LDS, while its maxima are found.  4096 rows of 32 columns are 512 KB, a compute unit's registers and LDS
+// together; with 24 + 8 pieces instead of 32 in registers two workgroups of 512 threads fit one (2048 x 14336: 46 us without, 41 with).
+// Bound by HBM where there are enough strips (4096 x 14336: 3.6 TB/s of input, whose lines of 128 bytes lie 57 KB apart), by
+// the launch and one round trip for small tensors.  Neighbouring strips run on one XCD at a time (workgroup id mod 8), so that
+// their pieces of a row's codes, and of an input line where a strip is narrower than that, meet in one L2.
+template <int kThreads, int kRegs, int kLds, int kLanes>
+__global__ __launch_bounds__(kThreads) void quantize_int8_strip_kernel(const float *__restrict__ in, int8_t *__restrict__ out,
+                                                                       float *__restrict__ scales, int rows, int cols)
+{
+  constexpr int kPass = kThreads / kLanes, kWaves = kThreads / 64, kStripCols = 4 * kLanes;
+  __shared__ __attribute__((aligned(16))) floatx4_t part[kWaves][kLanes];
+  __shared__ __attribute__((aligned(16))) floatx4_t held[kLds > 0 ? kLds : 1][kLds > 0 ? kThreads : 1];
+  const int strips = (cols + kStripCols - 1) / kStripCols, per_xcd = (strips + 7) / 8;
+  const int strip = static_cast<int>(blockIdx.x & 7) * per_xcd + static_cast<int>(blockIdx.x >> 3);
+  if (static_cast<int>(blockIdx.x >> 3) >= per_xcd || strip >= strips) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = strip * kStripCols + 4 * (threadIdx.x & (kLanes - 1));
+  const bool mine = c < cols;                            // cols is a multiple of 4
+  const int r0 = threadIdx.x / kLanes;
+  const float *p = in + (mine ? c : 0);
+  const int64_t pitch = cols;
+  // rows past the end repeat the last one: no influence on a maximum
+  const auto piece = [&](int i) __attribute__((always_inline)) {
+    return __builtin_nontemporal_load(reinterpret_cast<const floatx4_t *>(p + min(r0 + i * kPass, rows - 1) * pitch));
+  };
+  floatx4_t m = {0.0f, 0.0f, 0.0f, 0.0f};
+  const auto take = [&](const floatx4_t &v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = fabsf(v[j]);
+      if (a > m[j]) m[j] = a;
+    }
+  };
+  // passes in groups of four; a group without rows is left out
+  floatx4_t v[kRegs];
+  if constexpr (kLds > 0) {
+    if (kRegs * kPass < rows) {
+      floatx4_t w[kLds];
+#pragma unroll
+      for (int i = 0; i < kLds; ++i) w[i] = piece(kRegs + i);
+#pragma unroll
+      for (int i = 0; i < kRegs - kLds; ++i) v[i] = piece(i);
+#pragma unroll
+      for (int i = 0; i < kLds; ++i) {
+        take(w[i]);
+        held[i][threadIdx.x] = w[i];                     // read back by the thread that wrote it
+      }
+#pragma unroll
+      for (int i = kRegs - kLds; i < kRegs; ++i) v[i] = piece(i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kRegs; ++i) v[i] = piece(i);
+    }
+  } else {
+#pragma unroll
+    for (int g = 0; g < kRegs; g += 4)
+      if (g * kPass < rows) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[g + i] = piece(g + i);
+      }
+  }
+#pragma unroll
+  for (int g = 0; g < kRegs; g += 4)
+    if (g * kPass < rows) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) take(v[g + i]);
+    }
+#pragma unroll
+  for (int o = kLanes; o < 64; o <<= 1)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) m[j] = fmaxf(m[j], __shfl_xor(m[j], o, 64));
+  if (lane < kLanes) part[wave][lane] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) take(part[w][lane & (kLanes - 1)]);
+  float inv[4];
+  floatx4_t s;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    s[j] = (m[j] > 0.0f) ? m[j] / kInt8Max : 1.0f;
+    inv[j] = (s[j] > 0.0f) ? 1.0f / s[j] : 0.0f;
+  }
+  if (!mine) return;
+  if (threadIdx.x < kLanes) *reinterpret_cast<floatx4_any_t *>(scales + c) = s;
+  int8_t *q = out + c;
+  const auto put = [&](int i, const floatx4_t &x) __attribute__((always_inline)) {
+    const int r = r0 + i * kPass;
+    if (r < rows) *reinterpret_cast<uint32_t *>(q + r * pitch) = quantize_int8_x4(x, inv);
+  };
+#pragma unroll
+  for (int g = 0; g < kRegs; g += 4)
+    if (g * kPass < rows) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) put(g + i, v[g + i]);
+    }
+  if constexpr (kLds > 0) {
+    if (kRegs * kPass < rows) {
+#pragma unroll
+      for (int i = 0; i < kLds; ++i) put(kRegs + i, held[i][threadIdx.x]);
+    }
+  }
+}
+
 __global__ void dequantize_int8_kernel(const int8_t *__restrict__ in, float *__restrict__ out,
                                        const float *__restrict__ scales, int64_t n, int period)
 {
@@ -521,6 +626,22 @@ int caifx_quantize_int8_per_channel(const float *input, void *output, void *scal
   // four columns per thread when every row starts 16-byte aligned (and the codes of a row 4-byte aligned)
   if (cols % 4 == 0 && rows >= 8 && aligned_to(input, 16) && aligned_to(output, 4) && aligned_to(scales, 16) &&
       (rows + 31) / 32 <= 65535) {
+    // One launch over strips of columns where they fill the chip: us, three launches / this with strips of 32, 16 and 8 columns.
+    // 8 columns up to 2048: 2048 x 2048 14.4 / 18.7, 19.0, 13.8; 1536 x 640 13.2 / -, -, 10.5; 512 x 512 10.7 / -, -, 5.2.  16 up to 5000:
+    // 1024 x 4096 13.1 / 14.5, 11.4, 12.1; 640 x 3264 13.3 / 10.1, 7.6, 7.9.  32 beyond: 2048 x 14336 43.2 / 41.2, 46.4, 67.6; 1536 x 8192
+    // 25.0 / 19.6, 23.2, 30.5; 512 x 14336 15.0 / 13.2, 13.6, 17.7; 4096 x 14336 84.3 / 81.0, 100, 153.  Not here: 2048 x 4096 17.9 /
+    // 19.8, 20.0, 22.2; 1024 x 6144 14.8 / 15.7, 15.9, 16.8; 4096 x 9000 62.1 / 65.7, 76.4, 90.3; 2560 x 1024 15.0 / -, -, 15.4.
+    const auto strips_of = [&](auto kern, int threads, int lanes) {
+      const int strips = (cols / 4 + lanes - 1) / lanes;
+      hipLaunchKernelGGL(kern, dim3((strips + 7) / 8 * 8), dim3(threads), 0, s, input, static_cast<int8_t *>(output), static_cast<float *>(scales), rows,
+                         cols);
+      return launch_status();
+    };
+    if (cols >= 7000 && rows <= 1024) return strips_of(quantize_int8_strip_kernel<256, 24, 8, 8>, 256, 8);
+    if (cols >= 7000 && rows <= 2048) return strips_of(quantize_int8_strip_kernel<512, 24, 8, 8>, 512, 8);
+    if (cols >= 12288 && rows <= 4096) return strips_of(quantize_int8_strip_kernel<1024, 24, 8, 8>, 1024, 8);
+    if (cols <= 2048 && rows <= 2048) return strips_of(quantize_int8_strip_kernel<256, 32, 0, 2>, 256, 2);
+    if (cols > 2048 && cols <= 5000 && rows <= 1024) return strips_of(quantize_int8_strip_kernel<256, 32, 0, 4>, 256, 4);
     const int colblocks = grid_for(cols / 4, 64);
     // rows per chunk: 256, fewer where that gives less than four workgroups per compute unit
     int chunk = 256;

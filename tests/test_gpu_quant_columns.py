@@ -29,8 +29,22 @@ def test_bit_exact(orc, rows, cols):
     assert torch.equal(q2, q) and torch.equal(s2, s)
 
 
+# strips of 32, 16 and 8 columns held by one workgroup: with and without the pieces in LDS, the most rows of each form and one
+# more, a last strip that is not full
+@pytest.mark.parametrize("rows,cols", [(8, 7000), (768, 7004), (769, 7168), (1024, 7000), (1025, 7004), (1537, 7000), (2048, 7000), (2049, 12288),
+                                       (3073, 12292), (4096, 12288), (4097, 12288), (1024, 5000), (1025, 2052), (65, 2052), (2048, 2048), (2049, 36)])
+def test_strips(orc, rows, cols):
+    rng = np.random.default_rng(rows + cols)
+    w = rng.standard_normal((rows, cols), dtype=np.float32)
+    w[:, 1] = 0.0
+    w[rows - 1, cols - 1], w[0, cols - 2], w[rows // 2, 5] = -9.0, 8.0, 7.0
+    q, s = T.quantize_int8(dev(w), True)
+    qo, so = orc.quantize_int8_per_channel(w)
+    assert np.array_equal(s.cpu().numpy(), so) and np.array_equal(q.cpu().numpy(), qo)
+
+
 @pytest.mark.parametrize("offset", [4, 8, 12, 1])
-@pytest.mark.parametrize("rows,cols", [(8, 4), (65, 260), (1031, 1028)])
+@pytest.mark.parametrize("rows,cols", [(8, 4), (65, 260), (1031, 1028), (2100, 260)])
 def test_codes_at_any_address(orc, rows, cols, offset):
     # a slice of a packed checkpoint: the partial maxima wait in the codes' memory whatever its alignment
     w = np.random.default_rng(rows + cols).normal(0, 0.02, (rows, cols)).astype(np.float32)
