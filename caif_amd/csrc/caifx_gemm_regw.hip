@@ -377,6 +377,7 @@ int mfma_regw_forward(const GemmArgs &a, hipStream_t s)
 int mfma_forward(const GemmArgs &a, hipStream_t s)
 {
   int st = mfma_wide(a, false, s);
+  if (st == CAIFX_ERR_UNSUPPORTED) st = mfma_few_forward(a, s);
   if (st == CAIFX_ERR_UNSUPPORTED) st = mfma_tall(a, false, s);
   if (st == CAIFX_ERR_UNSUPPORTED) st = mfma_regw_forward(a, s);
   if (st == CAIFX_ERR_UNSUPPORTED) st = mfma_regw8_forward(a, s);

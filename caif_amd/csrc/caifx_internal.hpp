@@ -77,6 +77,9 @@ size_t mfma_wide_workspace_bytes(const GemmArgs &a, bool backward);
 // Expert segments, int8 codes with a scale vector of at most 32 classes of weight rows, forward (K a multiple of 128) and input
 // gradient: tiles of up to 256 rows whose waves dequantise their own columns.  CAIFX_ERR_UNSUPPORTED for everything else.
 int mfma_tall(const GemmArgs &a, bool backward, hipStream_t s);
+// Forward for a few dozen to a few hundred rows of int8 or int4 codes, the reduction split among a workgroup's waves.  Needs the
+// workspace mfma_workspace_bytes reports where it shares the reduction among workgroups too.  CAIFX_ERR_UNSUPPORTED for everything else.
+int mfma_few_forward(const GemmArgs &a, hipStream_t s);
 // Measurement only: grouped launches of the matrix-core GEMM issued after this call record, per tile of their own
 // numbering (expert by expert, row tile by row tile, column tile last), four 64-bit words {expert, rows in the
 // tile, start, end} with the times in ticks of the 100 MHz wall clock, into buf (device memory for `tiles` tiles);
