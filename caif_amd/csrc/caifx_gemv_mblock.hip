@@ -596,11 +596,12 @@ __global__ __launch_bounds__(kMbThreads) void mblock_grouped_kernel(MbArgs a, Mb
   int first = static_cast<int>(start - u * g.unit_blocks);
   const size_t ybytes = a.y_dtype == CAIFX_F32 ? 4 : 2;
   if (g.zero_rest) {
+    const int rows = static_cast<int>(g.total_rows);
+    int first = g.offsets[0], end = g.offsets[g.num_experts];
     bool down = false;
     for (int e = lane; e < g.num_experts; e += 64) down = down || g.offsets[e + 1] < g.offsets[e];
-    int first, end, x;
-    segment_rows(g.offsets, 0, g.total_rows, first, x);
-    segment_rows(g.offsets, g.num_experts - 1, g.total_rows, x, end);
+    first = first < 0 ? 0 : first > rows ? rows : first;
+    end = end < 0 ? 0 : end > rows ? rows : end;
     zero_uncovered(g.offsets, g.num_experts, g.total_rows, first, end, __ballot(down) == 0, a.y, a.N * static_cast<int64_t>(ybytes));
   }
   int base = g.num_experts <= 64 ? 0 : -1;          // which 64 experts the lanes hold
