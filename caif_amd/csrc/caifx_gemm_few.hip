@@ -396,10 +396,11 @@ template <typename CT> int pick_kind(const FewArgs &g, int kind, hipStream_t s)
 // 29.8 and 31.2) and up to 64 rows, which leave half of a 128-row tile idle (N = 14336, K = 4096: M = 64 29.5 and 27.9, M = 33
 // 29.0 and 21.1).  int8 with a scale vector and more than 256 rows: up to twice that share (N = K = 2048, M = 512 23.1 and 18.3; above it
 // N = 2048, K = 4096, M = 320 21.8 and 23.8).  With one scale the tiled kernel takes twice as long.
+// Reductions below 512 leave waves without a unit, and stay with the kernel that adds up in the order of the grouped ones.
 bool plan_few(const GemmArgs &a, int kind, FewArgs &g)
 {
   const int unit = kind == FK_INT4 ? 128 : 64;
-  if (a.M < 17 || a.K % unit != 0 || a.N % 8 != 0 || a.N * a.K >= (int64_t{1} << 32) || a.M * a.K >= (int64_t{1} << 31)) return false;
+  if (a.M < 17 || a.K < 512 || a.K % unit != 0 || a.N % 8 != 0 || a.N * a.K >= (int64_t{1} << 32) || a.M * a.K >= (int64_t{1} << 31)) return false;
   const int64_t col_tiles = (a.N + kCols - 1) / kCols, units = a.K / unit;
   int64_t best = 0;
   for (int blocks = 2; blocks <= 7; ++blocks) {

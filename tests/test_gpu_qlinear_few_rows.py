@@ -16,8 +16,8 @@ from gpu_helpers import dev_as, host, make_weight, max_rel_err        # noqa: E4
 # tiles of two to seven 16-row blocks, and the last of several that begins before its own rows; columns that end inside a 64-column
 # tile; reductions of fewer units than waves, of an odd number per wave, shared among workgroups or not
 @pytest.mark.parametrize("kind,group", [("int4", 128), ("int4", 32), ("int8pc", 128), ("int8pt", 128), ("int8", 128)])
-@pytest.mark.parametrize("M,N,K,dt", [(33, 512, 512, 2), (48, 64, 128, 1), (65, 200, 1152, 2), (96, 512, 4096, 2), (40, 8448, 640, 2), (60, 8448, 384, 1),
-                                      (75, 8456, 640, 2), (90, 8448, 128, 2), (100, 8448, 640, 2), (150, 8192, 640, 1), (220, 8192, 256, 2),
+@pytest.mark.parametrize("M,N,K,dt", [(33, 512, 512, 2), (48, 64, 512, 1), (65, 200, 1152, 2), (96, 512, 4096, 2), (40, 8448, 640, 2), (60, 8448, 640, 1),
+                                      (75, 8456, 640, 2), (90, 8448, 512, 2), (100, 8448, 640, 2), (150, 8192, 640, 1), (220, 8192, 512, 2),
                                       (130, 1024, 1024, 2), (200, 448, 3200, 2), (700, 320, 2176, 2)])
 def test_against_the_oracle(orc, kind, group, M, N, K, dt):
     rng = np.random.default_rng(M + N + K)
