@@ -34,7 +34,7 @@ EXPORTS = [
     "caifx_swiglu_backward",
     "caifx_moe_dispatch_map_workspace_bytes", "caifx_moe_build_dispatch_map", "caifx_moe_dispatch",
     "caifx_moe_combine", "caifx_moe_combine_backward_grad_expert", "caifx_moe_combine_backward_grad_weights",
-    "caifx_moe_dispatch_backward",
+    "caifx_moe_dispatch_backward", "caifx_moe_dispatch_fresh", "caifx_moe_combine_backward_grad_expert_fresh",
 ]
 
 
@@ -110,6 +110,8 @@ def lib():
         L.caifx_moe_dispatch_map_workspace_bytes.argtypes = [_i64, _int, _int]
         L.caifx_moe_build_dispatch_map.argtypes = [_p, _i64, _int, _int, _int, _p, _p, _p, _sz, _p]
         L.caifx_moe_dispatch.argtypes = [_p, _p, _p, _p, _p, _i64, _i64, _int, _int, _int, _p]
+        L.caifx_moe_dispatch_fresh.argtypes = [_p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _int, _int, _p]
+        L.caifx_moe_combine_backward_grad_expert_fresh.argtypes = [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _int, _int, _int, _p]
         L.caifx_moe_combine.argtypes = [_p, _p, _p, _p, _p, _p, _i64, _i64, _int, _int, _int, _p]
         L.caifx_moe_combine_backward_grad_expert.argtypes = [_p, _p, _p, _p, _p, _p, _i64, _i64, _int, _int, _int, _p]
         L.caifx_moe_combine_backward_grad_weights.argtypes = [_p, _p, _p, _p, _p, _p, _i64, _i64, _int, _int, _int, _p]

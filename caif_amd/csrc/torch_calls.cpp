@@ -28,7 +28,8 @@ namespace {
   X(caifx_qlinear_grouped_workspace_bytes) X(caifx_qlinear_grouped_fresh) X(caifx_silu) X(caifx_silu_backward) X(caifx_multiply) X(caifx_add)           \
   X(caifx_silu_multiply) X(caifx_swiglu_backward) X(caifx_moe_dispatch_map_workspace_bytes)                              \
   X(caifx_moe_build_dispatch_map) X(caifx_moe_dispatch) X(caifx_moe_combine) X(caifx_moe_combine_backward_grad_expert)   \
-  X(caifx_moe_combine_backward_grad_weights) X(caifx_moe_dispatch_backward) X(caifx_quantize_int8_per_channel)           \
+  X(caifx_moe_combine_backward_grad_weights) X(caifx_moe_dispatch_backward) X(caifx_moe_dispatch_fresh)                  \
+  X(caifx_moe_combine_backward_grad_expert_fresh) X(caifx_quantize_int8_per_channel)           \
   X(caifx_quantize_int8_per_tensor) X(caifx_quantize_to_int4)
 
 struct Api {
@@ -441,8 +442,12 @@ PyObject *moe_dispatch(PyObject *, PyObject *const *a, Py_ssize_t n)
   return guarded(n, 6, [&]() -> PyObject * {
     const at::Tensor &x = device_tensor(a[0]), &ids = device_tensor(a[1]), &offsets = device_tensor(a[3]);
     const int64_t tokens = matrix(x).size(0), dim = x.size(1), top_k = columns(ids);
-    const at::Tensor buf = a[5] != Py_None ? tensor(a[5]) : at::zeros({integer(a[4]), dim}, x.options());
+    const bool fresh = a[5] == Py_None;
+    const at::Tensor buf = fresh ? at::empty({integer(a[4]), dim}, x.options()) : tensor(a[5]);
     const int32_t *i1 = ints(a[1]); const int32_t *i2 = ints(a[2]); const int32_t *i3 = ints(a[3]); const int dt = code_of(x.scalar_type());
+    if (fresh)
+      return result(launch(api.caifx_moe_dispatch_fresh, x.data_ptr(), i1, i2, i3, buf.data_ptr(), buf.size(0), tokens, dim,
+                                               static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1), dt, stream()), buf);
     return result(launch(api.caifx_moe_dispatch, x.data_ptr(), i1, i2, i3, buf.data_ptr(), tokens, dim,
                                          static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1), dt, stream()), buf);
   });
@@ -467,8 +472,12 @@ PyObject *moe_combine_backward_grad_expert(PyObject *, PyObject *const *a, Py_ss
   return guarded(n, 7, [&]() -> PyObject * {
     const at::Tensor &g = device_tensor(a[0]), &ids = device_tensor(a[1]), &w = device_tensor(a[2]), &offsets = device_tensor(a[4]);
     const int64_t tokens = matrix(g).size(0), dim = g.size(1), top_k = columns(ids);
-    const at::Tensor buf = a[6] != Py_None ? tensor(a[6]) : at::zeros({integer(a[5]), dim}, g.options());
+    const bool fresh = a[6] == Py_None;
+    const at::Tensor buf = fresh ? at::empty({integer(a[5]), dim}, g.options()) : tensor(a[6]);
     const int32_t *i1 = ints(a[1]); const int32_t *i3 = ints(a[3]); const int32_t *i4 = ints(a[4]); const int dt = code_of(g.scalar_type());
+    if (fresh)
+      return result(launch(api.caifx_moe_combine_backward_grad_expert_fresh, g.data_ptr(), i1, w.data_ptr(), i3, i4, buf.data_ptr(), buf.size(0), tokens,
+                                                                   dim, static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1), dt, stream()), buf);
     return result(launch(api.caifx_moe_combine_backward_grad_expert, g.data_ptr(), i1, w.data_ptr(), i3, i4, buf.data_ptr(), tokens, dim,
                                                              static_cast<int>(top_k), static_cast<int>(offsets.numel() - 1),
                                                              dt, stream()), buf);

@@ -402,6 +402,11 @@ CAIFX_API int caifx_moe_dispatch(const void *input, const int32_t *expert_indice
                        const int32_t *expert_offsets, void *expert_buffer, int64_t num_tokens, int64_t dim,
                        int top_k, int num_experts, int dtype, caifx_stream_t stream);
 
+/* The same into a buffer of total_rows that holds nothing yet: rows no assignment maps to are zeroed. */
+CAIFX_API int caifx_moe_dispatch_fresh(const void *input, const int32_t *expert_indices, const int32_t *dispatch_map,
+                             const int32_t *expert_offsets, void *expert_buffer, int64_t total_rows, int64_t num_tokens,
+                             int64_t dim, int top_k, int num_experts, int dtype, caifx_stream_t stream);
+
 /* Zeroes the rows of a grouped result that no segment covers, [0, offsets[0]) and [offsets[num_experts], total_rows), each
  * row_bytes long: what a result tensor that was not cleared as a whole needs in front of the launch that fills it. */
 CAIFX_API int caifx_qlinear_grouped_zero_rest(int num_experts, const int32_t *offsets, int64_t total_rows, int64_t row_bytes,
@@ -432,6 +437,13 @@ CAIFX_API int caifx_moe_combine_backward_grad_expert(const void *grad_output, co
                                            const int32_t *expert_offsets, void *grad_expert_buffer,
                                            int64_t num_tokens, int64_t dim, int top_k, int num_experts, int dtype,
                                            caifx_stream_t stream);
+
+/* The same into a buffer of total_rows that holds nothing yet: rows no assignment maps to are zeroed. */
+CAIFX_API int caifx_moe_combine_backward_grad_expert_fresh(const void *grad_output, const int32_t *expert_indices,
+                                                 const void *expert_weights, const int32_t *dispatch_map,
+                                                 const int32_t *expert_offsets, void *grad_expert_buffer, int64_t total_rows,
+                                                 int64_t num_tokens, int64_t dim, int top_k, int num_experts, int dtype,
+                                                 caifx_stream_t stream);
 
 /* launch_moe_combine_backward_grad_weights (caif_cuda_kernels_moe.cuh:349-358, caif_cuda_kernels_moe.cu:915-990):
  * grad_weights[t,k] = T( sum over d of float(grad_output[t,d]) * float(buffer[row(t,k), d]) ), fp32
