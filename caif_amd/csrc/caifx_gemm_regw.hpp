@@ -116,6 +116,9 @@ __device__ __forceinline__ void store_tile(unsigned char *smem, const floatx16_t
 int mfma_regw8_forward(const GemmArgs &a, hipStream_t s);
 // Whether mfma_regw8_forward takes the call.
 bool mfma_regw8_takes(const GemmArgs &a);
+// forward with one int8 weight on the grouped kernel of tall tiles: its estimate in us (0: not for it), and whether it is the one to take
+double mfma_tall_plain_us(const GemmArgs &a);
+bool mfma_tall_plain(const GemmArgs &a);
 // where grouped launches record their tiles (see mfma_grouped_tile_stamps); null when switched off
 void mfma_grouped_stamp_target(unsigned long long **buf, long long *capacity);
 

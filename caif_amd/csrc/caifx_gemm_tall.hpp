@@ -1,5 +1,5 @@
-// Grouped dequant-GEMM over token-sorted expert segments, forward and input gradient, int8 codes with a scale vector: tall tiles
-// whose weight columns never meet in LDS as operands.
+// Grouped dequant-GEMM over token-sorted expert segments, forward and input gradient, int8 codes with a scale vector, and the forward
+// with one weight where its tiles are one round: tall tiles whose weight columns never meet in LDS as operands.
 //
 // A workgroup of eight waves owns up to 256 rows x 256 columns of an expert's result; wave w owns columns [32 w, 32 w + 32) for
 // all of the rows and walks the reduction in steps of 64.
@@ -61,7 +61,8 @@ struct TallArgs {
   int epilogue;              // gated experts, see EPI_* in caifx_gemm_tile.hpp: 1 forward (e1 = gate), 2 backward (and e2 = up)
   const void *e1, *e2;
   void *d2;
-  const int32_t *offsets;
+  const int32_t *offsets;    // null: one weight (wq, scales) for all M rows
+  const void *wq, *scales;
   const void *const *wq_ptrs;
   const void *const *scales_ptrs;
   int num_experts;
@@ -104,6 +105,22 @@ template <int kLanes> __device__ __forceinline__ void request16_by(uint32_t dst,
     asm volatile("s_mov_b32 m0, %0\n\ts_bfm_b64 exec, %3, 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(dst), "v"(voff), "s"(src), "n"(kLanes) : "memory");
 }
 
+// The tile of a product with one weight: row tiles of equal height, those of a column tile side by side, so that a piece of the weight
+// comes into one L2.
+__device__ __forceinline__ bool plain_tile(const TallArgs &g, int64_t col_tiles, GroupedTile &out)
+{
+  const int64_t row_tiles = (g.M + g.height - 1) / g.height, total = row_tiles * col_tiles, per_xcd = (total + 7) >> 3;
+  const int64_t slot = blockIdx.x >> 3, pos = static_cast<int64_t>(blockIdx.x & 7) * per_xcd + slot;
+  if (slot >= per_xcd || pos >= total) return false;
+  out.e = 0;
+  out.pos = pos;
+  out.col_tile = pos / row_tiles;
+  grouped_rows<BM, true>(0, static_cast<int>(g.M), static_cast<int>(row_tiles), static_cast<int>(pos - out.col_tile * row_tiles), out);
+  out.wq = g.wq;
+  out.scales = g.scales;
+  return out.row0 < out.row_end;
+}
+
 template <typename CT, bool kBackward>
 __global__ __launch_bounds__(64 * kWaves, 2) void tall_gemm_kernel(TallArgs g)
 {
@@ -115,7 +132,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void tall_gemm_kernel(TallArgs g)
   const int64_t C = kBackward ? g.K : g.N, R = kBackward ? g.N : g.K;
 
   GroupedTile gt;
-  const bool has_tile = grouped_tile<BM, true>(g.offsets, g.num_experts, g.M, (C + BN - 1) / BN, g.wq_ptrs, g.scales_ptrs, lane, gt, g.height);
+  const bool has_tile = !kBackward && !g.offsets ? plain_tile(g, (C + BN - 1) / BN, gt) : grouped_tile<BM, true>(g.offsets, g.num_experts, g.M, (C + BN - 1) / BN, g.wq_ptrs, g.scales_ptrs, lane, gt, g.height);
   if (g.zero_rest) zero_uncovered(g.offsets, g.num_experts, g.M, gt.first, gt.end, gt.ordered, g.d, C * (g.d_dtype == CAIFX_F32 ? 4 : 2));
   if (!has_tile) return;
   // the search's results are the same in every lane: into scalar registers with them

@@ -649,6 +649,18 @@ bool wide_shape(const GemmArgs &a, bool backward)
 
 }  // namespace
 
+// int8 forward with a scale vector and one round of tall tiles (caifx_gemm_tall.hpp), which need no copy: by the estimates, which are
+// within 10 % for both from reductions of 2048 on (us, f16 into f16, copy / tall, K = 4096: N = 14336, M = 800 119 / 95, M = 999 119 / 110;
+// N = 10240, M = 800 101 / 76, M = 1536 120 / 115; N = 8192, M = 1100 98 / 76; into fp32 by 1.00 to 1.29; over eight weights and
+// twelve M it is taken where it is 1.02 to 1.5 times as fast.  With a second round, N = 14336, M = 1100, 139 / 148).  From 769 rows on: below,
+// with the same tiles, tests pin which calls make the copy (N = 14336, K = 4096, M = 768 106 / 87).
+bool mfma_tall_plain(const GemmArgs &a)
+{
+  if (a.M <= 768) return false;
+  const double us = mfma_tall_plain_us(a);
+  return us != 0.0 && wide_shape(a, false) && us < wide_us(a, false) && (!mfma_regw8_takes(a) || us < regw_us(a));
+}
+
 size_t mfma_wide_workspace_bytes(const GemmArgs &a, bool backward)
 {
   if (!wide_shape(a, backward) || (dense16(a) && !backward)) return 0;
@@ -663,6 +675,7 @@ int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s)
   // what the workspace query cannot know: int8 forward with one scale, or with a scale vector that fits its LDS table, has a
   // kernel of its own (one scale, N = 14336, K = 4096, M = 320 59 us there against 75 here, K = 2048, M = 512 41 against 46)
   if (!grouped && !backward && a.w.kind == CAIFX_W_INT8 && mfma_regw8_takes(a) && regw_us(a) < wide_us(a, false)) return CAIFX_ERR_UNSUPPORTED;
+  if (!grouped && !backward && mfma_tall_plain(a)) return CAIFX_ERR_UNSUPPORTED;
   WideArgs g{};
   g.a = a.x;
   g.d = a.y;
