@@ -413,8 +413,8 @@ CAIFX_API int caifx_qlinear_grouped_zero_rest(int num_experts, const int32_t *of
                                     void *y, caifx_stream_t stream);
 
 /* caifx_qlinear_grouped_forward (backward = 0), caifx_qlinear_grouped_backward_input or, with an addend, _backward_input_add (backward
- * != 0) into a result that holds nothing yet: rows that no segment covers are zeroed too (caifx_qlinear_grouped_zero_rest), by the
- * decode kernel in its own launch and in front of it otherwise. */
+ * != 0) into a result that holds nothing yet: rows that no segment covers are zeroed too, by the 16-bit kernels in their own launch, with
+ * fp32 compute by caifx_qlinear_grouped_zero_rest in front of it. */
 CAIFX_API int caifx_qlinear_grouped_fresh(int backward, int num_experts, const int32_t *offsets, int64_t total_rows, int64_t N,
                                 int64_t K, const void *x, int x_dtype, int compute_dtype, const void *const *wq_ptrs,
                                 int w_kind, const void *const *scales_ptrs, int64_t scale_period, int group_size,
