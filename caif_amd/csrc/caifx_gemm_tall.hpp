@@ -33,6 +33,7 @@
 #pragma once
 
 #include "caifx_gemm_regw.hpp"
+#include "caifx_gemm_tall_plan.hpp"
 
 #include <atomic>
 #include <type_traits>
@@ -43,7 +44,7 @@ namespace tall {
 
 typedef __attribute__((__vector_size__(2 * sizeof(float)))) float floatx2_t;
 
-constexpr int BM = 256, BN = 256;
+constexpr int BM = kTallRows, BN = kTallCols;
 constexpr int kWaves = 8, kCols = 32;         // columns of a wave: two column tiles of 16
 constexpr int kHalf = 16 * 1024;             // LDS of half an activation tile: 128 rows of 128 bytes
 constexpr int kCodes = 4 * kHalf;            // codes: forward 8 waves x 8 KiB, gradient 3 steps x 16 KiB
