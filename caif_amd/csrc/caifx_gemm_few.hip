@@ -19,6 +19,7 @@
 //   * Operands of X are loaded a step ahead, each into registers whose operand has just been used; the weight operands of one half
 //     step are formed while the other's products run.
 //   * The operand is the reference's: code * scale in fp32, rounded once to the compute type.
+#include "caifx_gemm_few_plan.hpp"
 #include "caifx_internal.hpp"
 
 #include <atomic>
@@ -27,7 +28,7 @@
 namespace caifx {
 namespace {
 
-constexpr int kCols = 64, kWaves = 8;
+constexpr int kCols = kFewCols, kWaves = kFewWaves;
 constexpr int kScaleBytes = 64 * 1024;      // of a scale vector in LDS
 
 struct FewArgs {
@@ -42,8 +43,7 @@ struct FewArgs {
   void *d;                  // Y, or the partial tiles [parts][M][N] in fp32
   int d_dtype;
   const void *addend;       // optional [M, N] of d_dtype: d = T(float(T(acc)) + float(addend))
-  int row_tiles, col_tiles, tile_rows;
-  int parts, part_units;
+  FewPlan plan;
 };
 
 // Eight int4 codes (element j in nibble j) times one scale, rounded to CT: fma(code + 8, s, -8 s) rounds the exact product once.  The
@@ -60,8 +60,6 @@ template <typename CT> __device__ __forceinline__ u32x4_t int4_operand(uint32_t 
   v[3] = pack2<CT>(__builtin_fmaf(ubyte3_f32(lo), s, m8), __builtin_fmaf(ubyte3_f32(hi), s16, m8));
   return v;
 }
-
-enum { FK_INT4 = 0, FK_INT8 = 1, FK_INT8_ONE = 2 };      // int8 with a scale vector; with one scale or none
 
 // A lane loads 16 neighbouring bytes of its weight row: the four lanes of a row (q) cover 64 of them, a unit of two steps of int4 or
 // one of int8.  What it multiplies are the codes of reduction elements 32 h + 8 q .. + 7 for every half step h: of int4, dword q
@@ -108,20 +106,20 @@ __global__ __launch_bounds__(64 * kWaves, 2) void few_rows_gemm_kernel(FewArgs g
   // XCD x (workgroup id mod 8) takes the x-th contiguous eighth of the tiles, the row tiles of one piece of the weight side by side
   const int per_xcd = static_cast<int>(gridDim.x >> 3);
   const int pos = static_cast<int>(blockIdx.x & 7) * per_xcd + static_cast<int>(blockIdx.x >> 3);
-  if (pos >= g.row_tiles * g.col_tiles * g.parts) return;
-  const int row_tile = pos % g.row_tiles, part = pos / g.row_tiles % g.parts, col_tile = pos / g.row_tiles / g.parts;
+  if (pos >= g.plan.row_tiles * g.plan.col_tiles * g.plan.parts) return;
+  const int row_tile = pos % g.plan.row_tiles, part = pos / g.plan.row_tiles % g.plan.parts, col_tile = pos / g.plan.row_tiles / g.plan.parts;
   // the last row tile begins early enough to be a whole one; rows in front of `skip` are its predecessor's and not stored
-  int64_t row0 = static_cast<int64_t>(row_tile) * g.tile_rows;
+  int64_t row0 = static_cast<int64_t>(row_tile) * g.plan.tile_rows;
   int skip = 0;
-  if (row0 + g.tile_rows > g.M && row_tile > 0) {
-    skip = static_cast<int>(row0 + g.tile_rows - g.M);
+  if (row0 + g.plan.tile_rows > g.M && row_tile > 0) {
+    skip = static_cast<int>(row0 + g.plan.tile_rows - g.M);
     row0 -= skip;
   }
-  const int rows = static_cast<int>(g.M - row0 < g.tile_rows ? g.M - row0 : g.tile_rows);      // more than 16 (NB - 1)
+  const int rows = static_cast<int>(g.M - row0 < g.plan.tile_rows ? g.M - row0 : g.plan.tile_rows);      // more than 16 (NB - 1)
   const int64_t col0 = static_cast<int64_t>(col_tile) * kCols;
   constexpr int kHalves = kKind == FK_INT4 ? 4 : 2, kUnit = 32 * kHalves;      // reduction elements of a unit
   const int units = static_cast<int>(g.K / kUnit);
-  const int first = part * g.part_units, end = first + g.part_units < units ? first + g.part_units : units;
+  const int first = part * g.plan.part_units, end = first + g.plan.part_units < units ? first + g.plan.part_units : units;
   const int mine = first + wave < end ? (end - first - wave + kWaves - 1) / kWaves : 0;      // units first + wave + 8 t
 
   // rows and columns past the end are loaded from the last one and never stored
@@ -363,13 +361,13 @@ template <typename CT, int kKind, int NB> int launch(const FewArgs &g, hipStream
       return CAIFX_ERR_LAUNCH_FAILED;
     raised.store(true, std::memory_order_relaxed);
   }
-  const unsigned tiles = static_cast<unsigned>(g.row_tiles * g.col_tiles * g.parts);
+  const unsigned tiles = static_cast<unsigned>(g.plan.row_tiles * g.plan.col_tiles * g.plan.parts);
   hipLaunchKernelGGL(kern, dim3((tiles + 7) / 8 * 8), dim3(64 * kWaves), kLds, s, g);
   return launch_status();
 }
 template <typename CT, int kKind> int pick_rows(const FewArgs &g, hipStream_t s)
 {
-  switch ((g.tile_rows + 15) / 16) {
+  switch ((g.plan.tile_rows + 15) / 16) {
     case 2: return launch<CT, kKind, 2>(g, s);
     case 3: return launch<CT, kKind, 3>(g, s);
     case 4: return launch<CT, kKind, 4>(g, s);
@@ -382,50 +380,6 @@ template <typename CT> int pick_kind(const FewArgs &g, int kind, hipStream_t s)
 {
   if (kind == FK_INT4) return pick_rows<CT, FK_INT4>(g, s);
   return kind == FK_INT8 ? pick_rows<CT, FK_INT8>(g, s) : pick_rows<CT, FK_INT8_ONE>(g, s);
-}
-
-// Tiles and parts; false where the kernel does not take the sizes, or is not the faster one.
-//
-// Whole rounds: with more tiles than compute units a second round costs as much as the first (int8 per channel, N = 11008, K = 4096:
-// M = 100, 172 tiles, 39.4 us here and 45.3 tiled; M = 128, 344 of 64 rows, 56.0 and 46.0).  Among the row tiles that fit, the height
-// whose estimate is the least: low ones repeat the dequantisation, which beats few parts of a long reduction (M = 256, N = K = 2048,
-// int8: 32 rows 13.3 us, 64 16.2, 112 18.3) but not many parts (M = 33, N = 5952, K = 3072, int4: 48 rows 12.6 us, 32 14.2).
-//
-// int4 runs the tiled kernel faster, four steps of codes to a line: here where a workgroup's share is short (units x 16-row blocks up
-// to 64; N = K = 2048, M = 256 16.6 tiled, 12.4 here; above it N = K = 4096, M = 200 25.4 and 27.7, N = 14336, K = 4096, M = 80
-// 29.8 and 31.2) and up to 64 rows, which leave half of a 128-row tile idle (N = 14336, K = 4096: M = 64 29.5 and 27.9, M = 33
-// 29.0 and 21.1).  int8 with a scale vector and more than 256 rows: up to twice that share (N = K = 2048, M = 512 23.1 and 18.3; above it
-// N = 2048, K = 4096, M = 320 21.8 and 23.8).  With one scale the tiled kernel takes twice as long.
-// Reductions below 512 leave waves without a unit, and stay with the kernel that adds up in the order of the grouped ones.
-bool plan_few(const GemmArgs &a, int kind, FewArgs &g)
-{
-  const int unit = kind == FK_INT4 ? 128 : 64;
-  if (a.M < 17 || a.K < 512 || a.K % unit != 0 || a.N % 8 != 0 || a.N * a.K >= (int64_t{1} << 32) || a.M * a.K >= (int64_t{1} << 31)) return false;
-  const int64_t col_tiles = (a.N + kCols - 1) / kCols, units = a.K / unit;
-  int64_t best = 0;
-  for (int blocks = 2; blocks <= 7; ++blocks) {
-    const int64_t row_tiles = (a.M + 16 * blocks - 1) / (16 * blocks), tiles = row_tiles * col_tiles;
-    if (tiles > 256) continue;
-    const int64_t tile_rows = ((a.M + row_tiles - 1) / row_tiles + 15) / 16 * 16, nb = tile_rows / 16;
-    int64_t parts = 256 / tiles;
-    if (parts > units / kWaves) parts = units / kWaves;
-    if (parts > 8) parts = 8;
-    if (parts < 1) parts = 1;
-    const int64_t per = (units + parts - 1) / parts;
-    // beginning and end of a workgroup, and its share of the reduction, in units of about 0.15 us
-    const int64_t cost = 8 * (4 + 2 * nb) + per * (1 + nb);
-    if (best != 0 && cost >= best) continue;
-    best = cost;
-    g.row_tiles = static_cast<int>(row_tiles);
-    g.col_tiles = static_cast<int>(col_tiles);
-    g.tile_rows = static_cast<int>(tile_rows);
-    g.parts = static_cast<int>((units + per - 1) / per);
-    g.part_units = static_cast<int>(per);
-  }
-  if (best == 0) return false;
-  const int64_t share = static_cast<int64_t>(g.part_units) * (g.tile_rows / 16);
-  if (kind == FK_INT4) return a.M <= 64 || share <= 64;
-  return kind == FK_INT8_ONE || a.M <= 256 || share <= 128;
 }
 
 }  // namespace
@@ -460,7 +414,8 @@ int mfma_few_forward(const GemmArgs &a, hipStream_t s)
   } else {
     return CAIFX_ERR_UNSUPPORTED;
   }
-  if (!plan_few(a, kind, g)) return CAIFX_ERR_UNSUPPORTED;
+  g.plan = plan_few(a.M, a.N, a.K, kind);
+  if (g.plan.parts == 0) return CAIFX_ERR_UNSUPPORTED;
   g.M = a.M;
   g.N = a.N;
   g.K = a.K;
@@ -470,10 +425,10 @@ int mfma_few_forward(const GemmArgs &a, hipStream_t s)
   g.d = a.y;
   g.d_dtype = a.y_dtype;
   g.addend = a.addend;
-  const bool split = g.parts > 1;
+  const bool split = g.plan.parts > 1;
   if (split) {
     // no more than the tiled kernel's parts ask for: its tiles are as high or higher and twice as wide
-    if (!a.workspace || a.workspace_bytes < static_cast<size_t>(g.parts) * static_cast<size_t>(a.M) * static_cast<size_t>(a.N) * 4 || !aligned_to(a.workspace, 16))
+    if (!a.workspace || a.workspace_bytes < static_cast<size_t>(g.plan.parts) * static_cast<size_t>(a.M) * static_cast<size_t>(a.N) * 4 || !aligned_to(a.workspace, 16))
       return CAIFX_ERR_UNSUPPORTED;
     g.d = a.workspace;
     g.d_dtype = CAIFX_F32;
@@ -481,7 +436,7 @@ int mfma_few_forward(const GemmArgs &a, hipStream_t s)
   }
   const int st = a.compute_dtype == CAIFX_BF16 ? pick_kind<bf16_t>(g, kind, s) : pick_kind<f16_t>(g, kind, s);
   if (!split || st != CAIFX_OK) return st;
-  return splitk_reduce(static_cast<const float *>(a.workspace), g.parts, a.M * a.N, a.y, a.y_dtype, a.addend, s);
+  return splitk_reduce(static_cast<const float *>(a.workspace), g.plan.parts, a.M * a.N, a.y, a.y_dtype, a.addend, s);
 }
 
 }  // namespace caifx

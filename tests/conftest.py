@@ -46,3 +46,10 @@ def pieces_plans(tmp_path_factory):
 def tall_plans(tmp_path_factory):
     """Height of the tall kernel's row tiles for grouped int8 calls (rows, experts, columns, reduction), and the estimate in us."""
     return _plans(tmp_path_factory, "tall_plan", float)
+
+
+@pytest.fixture(scope="session")
+def few_plans(tmp_path_factory):
+    """How the few-row forward kernel cuts calls (rows, columns, reduction, kind): row tiles, their 16-row blocks, workgroups per reduction
+    and the units of each; zeros where another kernel takes the call."""
+    return _plans(tmp_path_factory, "few_plan")
