@@ -96,7 +96,8 @@ def test_rows_outside_the_segments(kind, shift, offsets, rows):
     assert not want[~covered].any() and want[covered].any(dim=1).all()
 
 
-# the paths that clear in a launch of their own: the gradient with an addend and without, and a forward of more rows than the decode kernel takes
+# the tiled kernel: the gradient with an addend and without, and a forward of more rows than the decode kernel takes (the other grouped
+# kernels, and offsets out of order, in test_gpu_grouped_clearing.py)
 @pytest.mark.parametrize("kind", ["int8", "int4"])
 @pytest.mark.parametrize("form", ["gradient", "addend", "forward"])
 @pytest.mark.parametrize("offsets,rows", [([2, 30, 41], 50), ([0, 33, 40], 40), ([5, 5, 5], 40)])
