@@ -456,9 +456,15 @@ int check_route(const void *a, const void *b, const int32_t *idx, const int32_t 
 unsigned wave_blocks(int64_t waves) { return static_cast<unsigned>((waves * 64 + kRouteThreads - 1) / kRouteThreads); }
 
 constexpr int64_t kClearAssignments = 1024, kClearRows = 1024;
+// A 16-byte piece a thread and no loop, as fast as the framework's fill (with zero_bytes' loop, four pieces a thread, up to 0.2 us slower: 1716
+// rows of 1288 columns and the launch behind it 5.6 us, 5.4 here); single bytes at the ends by the first workgroup.
 __global__ __launch_bounds__(256) void zero_all_kernel(unsigned char *y, int64_t bytes)
 {
-  zero_bytes(y, 0, bytes, static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, static_cast<int64_t>(gridDim.x) * 256);
+  const int64_t before = (16 - (reinterpret_cast<uintptr_t>(y) & 15)) & 15, head = before < bytes ? before : bytes;
+  const int64_t pieces = (bytes - head) / 16, i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, tail = head + 16 * pieces;
+  if (i < pieces) reinterpret_cast<u32x4_t *>(y + head)[i] = u32x4_t{0, 0, 0, 0};
+  if (i < head) y[i] = 0;
+  if (i < 16 && tail + i < bytes) y[tail + i] = 0;
 }
 
 // How a buffer of total_rows that holds nothing yet gets its unmapped rows zeroed.  Few rows and assignments: by the launch that fills
@@ -476,11 +482,13 @@ int plan_clear(void *buf, int64_t total_rows, int64_t dim, int64_t assignments, 
     c.blocks = static_cast<int>(wave_blocks(total_rows));
     return CAIFX_OK;
   }
-  const int64_t bytes = total_rows * row_bytes, grid = bytes / (256 * 16 * 4) + 1;
-  hipLaunchKernelGGL(zero_all_kernel, dim3(static_cast<unsigned>(grid < (1 << 20) ? grid : 1 << 20)), dim3(256), 0, s, static_cast<unsigned char *>(buf), bytes);
+  const int64_t bytes = total_rows * row_bytes, most = int64_t{1} << 34;      // of a launch: 2^22 workgroups
+  for (int64_t at = 0; at < bytes; at += most) {
+    const int64_t part = bytes - at < most ? bytes - at : most;
+    hipLaunchKernelGGL(zero_all_kernel, dim3(static_cast<unsigned>(part / (256 * 16) + 1)), dim3(256), 0, s, static_cast<unsigned char *>(buf) + at, part);
+  }
   return launch_status();
 }
-
 
 }  // namespace
 }  // namespace caifx
