@@ -645,14 +645,14 @@ def moe_rows(torch, T, dev, gen):
     ms_f, ms_b = timed(fwd), timed(bwd)
     ms_f_fused, ms_b_fused = timed(fwd_gating_in_store), timed(bwd_gating_in_store)
 
-    # Per-expert-segment GEMM efficiency (outside the timed runs): the grouped kernel stamps every 128 x 128 tile
+    # Per-expert-segment GEMM efficiency (outside the timed runs): the grouped kernel stamps every tile
     # with its expert, row count, start and end (100 MHz wall clock).  An expert's efficiency is the flops of its
     # segment over what the matrix pipes offer during its tiles' lifetimes, 2 cnt K N / (sum of tile durations x
     # peak / (256 compute units x the workgroups that share one)); partial last tiles and everything a tile waits
     # for count against it.
     def segment_efficiency(launch, n_cols, k_red):
         from caif_amd import capi
-        tiles = ((rows + 127) // 128 + E) * ((n_cols + 127) // 128)
+        tiles = ((rows + 63) // 64 + E) * ((n_cols + 127) // 128)
         stamps = torch.zeros(tiles * 4, dtype=torch.int64, device=dev)
         capi.call("caifx_qlinear_grouped_tile_stamps", stamps.data_ptr(), tiles)
         try:

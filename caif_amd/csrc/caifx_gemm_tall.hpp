@@ -11,7 +11,7 @@
 // 0.3 more, operand reads 0.1, dequantisation 0.2 to 0.35: 1.2 in all, issue of the two waves of a SIMD being what most of it
 // has in common (a wave alone issues a VALU instruction every eight clocks: four waves of 64 columns are no faster).
 // 64 experts, 24576 rows, 1408 x 2048 and 2048 x 1408, bf16, us, before (those two kernels) / now: forward 263 / 189 and 226 / 169,
-// gradient 290 / 166 and 242 / 155, 0.84 to 0.92 PFLOP/s.
+// gradient 290 / 166 and 242 / 155, 0.75 to 0.91 PFLOP/s.
 //   * Row tiles: a segment is cut into tiles of equal height (a multiple of 32), so 384 rows make two of 192 and not one of
 //     256 and one of 128 that costs as much dequantisation.  The reduction loop is instantiated for 64, 96, .. 256 rows.
 //   * The weight: every wave dequantises the 64 x 32 piece of its own columns for the next step in registers, float(code) *

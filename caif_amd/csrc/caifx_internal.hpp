@@ -74,8 +74,9 @@ size_t mfma_workspace_bytes(const GemmArgs &a, bool backward);
 // not take, CAIFX_ERR_UNSUPPORTED.
 int mfma_wide(const GemmArgs &a, bool backward, hipStream_t s);
 size_t mfma_wide_workspace_bytes(const GemmArgs &a, bool backward);
-// Expert segments, int8 codes with a scale vector of at most 32 classes of weight rows, forward (K a multiple of 128) and input
-// gradient: tiles of up to 256 rows whose waves dequantise their own columns.  CAIFX_ERR_UNSUPPORTED for everything else.
+// int8 codes with a scale vector of at most 32 classes of weight rows, 16-bit compute: tiles of up to 256 rows whose waves dequantise their
+// own columns.  Expert segments, forward (K a multiple of 128, N of 64) and input gradient (N of 128 too); one weight, forward, where
+// mfma_tall_plain says so.  CAIFX_ERR_UNSUPPORTED for everything else.
 int mfma_tall(const GemmArgs &a, bool backward, hipStream_t s);
 // Forward for a few dozen to a few hundred rows of int8 or int4 codes, the reduction split among a workgroup's waves.  Needs the
 // workspace mfma_workspace_bytes reports where it shares the reduction among workgroups too.  CAIFX_ERR_UNSUPPORTED for everything else.

@@ -366,9 +366,12 @@ __global__ __launch_bounds__(kThreads) void quantize_int8_strip_kernel(const flo
   const auto put = [&](int i, const floatx4_t &x) __attribute__((always_inline)) {
     const int r = r0 + i * kPass;
     if (r >= rows) return;
-    // Small tensors are often experts' weights, quantised one after the other and read by the next pass: with streaming stores that pass is
-    // faster (64 experts of 1408 x 2048, 16 tokens, first pass 180 us without, 150 to 155 with, the old launches 155 to 163), this launch
-    // up to 1.3 us slower (2048 x 512 10.5 / 11.8).  Whole-line strips of large tensors lose more (4096 x 14336, both forms 128 / 164).
+    // Strips narrower than a line: streaming stores, so that what a strip writes of a line is not left in its XCD's L2 for the next kernel to wait
+    // for.  The launch alone, replayed, us, plain / streaming / three launches: 1024 x 512 6.3 / 7.5 / 11.5, 2048 x 512 8.8 / 9.8 / 12.3, 1408 x 2048
+    // 9.2 / 11.5 / 12.9, 2048 x 1024 10.4 / 13.2 / 13.0 (2048 rows are the most, there alone are the three as fast).  Launch and
+    // a product that reads the codes: 2048 x 512, one row 27.7 / 22.2 / 26.5, 2048 x 2048, 16 rows 28.1 / 25.8 / 28.5, 1024 x 4096, 200 rows 34.8 /
+    // 30.4 / 57.  64 experts of 1408 x 2048, 16 tokens, first pass behind the three banks 180 / 150 to 155 / 155 to 163; one bank alone 896 / 952 / 1018
+    // to quantise and read.  Whole-line strips of large tensors stay with plain stores (4096 x 14336 and the int4 form 128 / 164).
     if constexpr (kLanes < 8) __builtin_nontemporal_store(quantize_int8_x4(x, inv), reinterpret_cast<uint32_t *>(q + r * pitch));
     else *reinterpret_cast<uint32_t *>(q + r * pitch) = quantize_int8_x4(x, inv);
   };

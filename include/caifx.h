@@ -241,12 +241,14 @@ CAIFX_API int caifx_qlinear_forward_static(int64_t M, int64_t N, int64_t K,
 
 /* Measurement only, no counterpart in the reference (whose per-expert loop, src/caif_device_moe_layer.cpp:534-557,
  * can simply be timed expert by expert on the host): grouped launches of the matrix-core GEMM issued after this
- * call record four 64-bit words per tile (128 rows x 128 columns, x 256 for the int8 forward kernel that keeps
- * the weight out of LDS, and 128 x 128, 128 x 256 or 256 x 256 where the experts' weights are copied first) - {expert, rows of the segment inside the tile (low 32 bits; from bit 32 up, when not 0,
- * how many workgroups share a compute unit instead of two), start, end}, times in ticks of the
- * GPU's 100 MHz wall clock - into `stamps` (device memory for `tiles` tiles, 32 bytes each; sizing for 128 x 128
- * tiles covers all of them; tiles are numbered expert by expert, row tile by row tile, column tile last; clear it before
- * a launch, words of tiles that do not exist stay as they are).  stamps = NULL switches the recording off.
+ * call record four 64-bit words per tile (128 rows x 128 columns, x 256 for the int8 forward that keeps the weight out of LDS; int8 with
+ * a scale vector of few classes of weight rows, both directions, 64, 96 .. or 256 x 256, a segment's tiles being of equal height;
+ * 128 x 128, 128 x 256 or 256 x 256 where the experts' weights are copied first) - {expert, rows of the segment inside the tile
+ * (low 32 bits; from bit 32 up, when not 0, how many workgroups share a compute unit instead of two), start, end}, times in ticks of
+ * the GPU's 100 MHz wall clock - into `stamps` (device memory for `tiles` tiles, 32 bytes each; (total_rows / 64 + experts) x
+ * ceil(columns / 128) covers all of them, tiles beyond what there is room for are not recorded; tiles are numbered expert by
+ * expert, row tile by row tile, column tile last; clear it before a launch, words of tiles that do not exist stay as they
+ * are).  stamps = NULL switches the recording off.
  * Process-wide state; not meant for timed runs (one more store per workgroup). */
 CAIFX_API int caifx_qlinear_grouped_tile_stamps(void *stamps, int64_t tiles);
 
