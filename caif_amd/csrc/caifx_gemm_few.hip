@@ -7,9 +7,9 @@
 // the tiles do not fill the chip the reduction is shared among workgroups too, as in the tiled kernel (fp32 partial tiles in the
 // workspace, a second launch adds them).
 //
-// Bound by the way of its loads: a wave's operands of X are asked for one to two half steps ahead, its codes a unit, and 45 to 60 % of the waves'
-// time is waiting (counters: matrix cores 13 to 17 % busy, VALU 15 to 22 % of a wave's time, two waves a SIMD; a compute unit takes
-// in 9 to 14 bytes a clock, its share of the codes and all rows of X along its share of the reduction).  The tiled kernel before it (128 x 128 tiles, 64-deep steps that eight waves pass through together) took 1.1 us a step
+// Bound by the way of its loads: a wave's operands of X are asked for one to two half steps ahead, its codes a unit, and 48 to 60 % of the waves'
+// time is waiting (counters: matrix cores 7 to 16 % busy, VALU 15 to 23 % of a wave's time, two waves a SIMD; a compute unit takes
+// in 8 to 13 bytes a clock, its share of the codes and all rows of X along its share of the reduction).  The tiled kernel before it (128 x 128 tiles, 64-deep steps that eight waves pass through together) took 1.1 us a step
 // however few of its rows were there.  Graph replay, before / now in us, bf16, int4 | int8 per channel | int8 with one scale:
 //     N = K = 4096,          M = 33    15.7 / 15.1 | 19.4 / 13.3 | 29.1 / 12.1        M = 64   17.8 / 15.3 | 22.5 / 16.1 | 32.2 / 14.6
 //     N = 11008, K = 4096,   M = 33    27.7 / 20.5 | 42.9 / 23.4 | 86.8 / 20.6        M = 100  (tiled)     | 45.3 / 39.4 | 98.3 / 37.3
